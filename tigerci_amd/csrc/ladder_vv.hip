@@ -22,15 +22,12 @@
 // outside a walk's domain are zero once per plan and never written again, so a
 // sigma writes only the sum_P d_P (d_P + 1) / 2 entries its walks own.
 //
-// Layouts (row-major): V+ [n_p][n_p], V- [n_m][n_m] (FP64, plan lifetime);
-// X+ [P][n_p], X- [P'][n_m]; S+, S- the same shapes, one copy per K-split.
-// Split precisions keep V+- and X+- as split rows (hi/lo 16-bit parts,
-// common.hpp) and compute S = X V^T on the split GEMM; FP64 uses the dense
-// FP64 GEMM with V as the K x N operand.  The split product can also run as
-// S^T = V X^T: with a few hundred walks, the walks then lie along the tiles'
-// N side, where 192-wide tiles cover 518 walks in three tiles (V read three
-// times) against five 128-row tiles the other way round; S^T is transposed
-// back before the gather.
+// Layouts (row-major): V+ [n_p][n_p], V- [n_m][n_m] (FP64, plan lifetime),
+// X+ [P][n_p], X- [P'][n_m], both with rows padded to an even count (16-byte
+// rows); S+, S- [P][n_p], [P'][n_m], one copy per K-split.  V+- are symmetric,
+// so S = X V^T with both operands k-contiguous: every precision runs on the NT
+// GEMM with direct-load stages (ngemm.hpp); the split precisions keep V+- and
+// X+- as split rows (hi/lo 16-bit parts, common.hpp).
 #include <algorithm>
 #include <cmath>
 
@@ -75,7 +72,8 @@ __global__ void vv_assemble_kernel(const double* __restrict__ W, int n_v, int a0
   const int al = (int)blockIdx.y / n_v, b = (int)blockIdx.y % n_v;
   const int a = a0 + al;
   if (b > a) return;
-  const int64_t nv2 = (int64_t)n_v * n_v, np = tri(n_v), nm = tri(n_v - 1);
+  const int64_t nv2 = (int64_t)n_v * n_v, np = tri(n_v);
+  const int64_t ldp = (np + 1) & ~(int64_t)1, ldm = (tri(n_v - 1) + 1) & ~(int64_t)1;  // even rows
   const double* Wa = W + (int64_t)al * n_v * nv2 + (int64_t)b * n_v;
   const int64_t rp = tri(a) + b, rm = a > b ? tri(a - 1) + b : -1;
   for (int64_t col = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; col < np; col += (int64_t)gridDim.x * blockDim.x) {
@@ -83,8 +81,8 @@ __global__ void vv_assemble_kernel(const double* __restrict__ W, int n_v, int a0
     untri(col, c, d);
     const double x = Wa[(int64_t)c * nv2 + d];  // (ac|bd)
     const double y = Wa[(int64_t)d * nv2 + c];  // (ad|bc)
-    Vp[rp * np + col] = x + y;
-    if (rm >= 0 && c > d) Vm[rm * nm + tri(c - 1) + d] = x - y;
+    Vp[rp * ldp + col] = x + y;
+    if (rm >= 0 && c > d) Vm[rm * ldm + tri(c - 1) + d] = x - y;
   }
 }
 
@@ -103,8 +101,8 @@ __device__ __forceinline__ void put_split1(uint16_t* p, double v, float s, int f
   }
 }
 
-// split rows of a row-major FP64 n x n matrix: out[r ldo + xidx(k)] (k padded to 8)
-__global__ void split_square_kernel(const double* __restrict__ src, int64_t n, uint16_t* __restrict__ out,
+// split rows of a row-major FP64 n x n matrix of row stride ld: out[r ldo + xidx(k)] (k padded to 8)
+__global__ void split_square_kernel(const double* __restrict__ src, int64_t n, int64_t ld, uint16_t* __restrict__ out,
                                     int64_t ldo, const float* scl, int f16) {
   const float s = scale_at(scl);
   const int64_t nch = ((n + 7) & ~(int64_t)7) >> 3;
@@ -112,7 +110,7 @@ __global__ void split_square_kernel(const double* __restrict__ src, int64_t n, u
     const int64_t r = e / nch, c = 8 * (e - r * nch);
     float v[8];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) v[t] = c + t < n ? (float)src[r * n + c + t] : 0.f;
+    for (int t = 0; t < 8; ++t) v[t] = c + t < n ? (float)src[r * ld + c + t] : 0.f;
     put_split8(out + r * ldo + xidx(c), v, s, f16 != 0);
   }
 }
@@ -211,27 +209,6 @@ __global__ void vv_gather_kernel(PairTab T, const double* __restrict__ Sp, int64
   }
 }
 
-// S[r][c] = sum over the nparts K-split partials of ST[c][r] (ST: [cols][rows]
-// per partial, S: [rows][cols]); 32 x 32 tiles through LDS, 256 threads
-__global__ void vv_untranspose_kernel(const double* __restrict__ ST, int64_t part, int64_t rows, int64_t cols,
-                                      int nparts, double* __restrict__ S) {
-  __shared__ double t[32][33];
-  const int64_t c0 = (int64_t)blockIdx.x * 32, r0 = (int64_t)blockIdx.y * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  for (int i = ty; i < 32; i += 8) {
-    const int64_t c = c0 + i, r = r0 + tx;
-    double v = 0.0;
-    if (c < cols && r < rows)
-      for (int k = 0; k < nparts; ++k) v += ST[k * part + c * rows + r];
-    t[i][tx] = v;
-  }
-  __syncthreads();
-  for (int i = ty; i < 32; i += 8) {
-    const int64_t r = r0 + i, c = c0 + tx;
-    if (r < rows && c < cols) S[r * cols + c] = t[tx][i];
-  }
-}
-
 inline unsigned blocks(int64_t work, unsigned cap) {
   return (unsigned)std::min<int64_t>(std::max<int64_t>(cdiv(work, 256), 1), cap);
 }
@@ -261,90 +238,52 @@ Seg vseg(const Op& A, const Op& B, int K) {
 // (slot 1 holds the scale of C, set per sigma by the split ladder's helper).
 constexpr int kScV = 9, kScOut = 10, kScC = 1;
 
-// S = X V (FP64: V as K x N; split: X V^T over split rows) for both parts as
-// one program: tasks ordered by column block of V, then K-split, then row
-// block of X, so the row tiles that read one V panel are neighbours.
-void build_products(tci_plan& P, GemmProgram& g, bool split, int tile, int tile_n, int dma, int ks, bool trans,
-                    hipStream_t st) {
+inline int64_t even(int64_t n) { return (n + 1) & ~(int64_t)1; }
+
+// S = X V^T for both parts as one program: tasks ordered by column block of V,
+// then K-split, then row block of X, so the row tiles that read one V panel
+// are neighbours.
+void build_products(tci_plan& P, NProgram& g, bool split, int shape, int ks, hipStream_t st) {
   tci_plan::VVLadder& V = P.vv;
   g.clear();
-  g.dense = !split;
   g.split = split;
-  g.tile = tile;
-  g.tile_n = split ? tile_n : 0;
-  // 256 x 256 split tiles take `dma` as their wave count (4, 8 or 16); others as direct-load stages
-  g.dma = split && tile == 256 ? 0 : dma;
-  g.waves = split && tile == 256 && (dma == 8 || dma == 16) ? dma : 4;
-  const int tn = split ? tile_n : tile;
+  g.shape = shape;
+  const int tn = g.tn(), esz = split ? 4 : 8;
   struct Part {
     const void* X;
     const void* Vm;
     double* S;
-    int64_t n, rows, ldx;
+    int64_t n, rows, ld;
   };
-  const int64_t lx_p = split ? 2 * xpad(V.np) : V.np, lx_m = split ? 2 * xpad(V.nm) : V.nm;
-  std::vector<Part> parts = {{split ? V.Xpx.p : V.Xp.p, split ? V.Vpx.p : V.Vp.p,
-                              (trans ? V.STp : V.Sp).as<double>(), V.np, (int64_t)P.n_pairs, lx_p}};
+  auto ld = [&](int64_t n) { return split ? xpad(n) : even(n); };
+  std::vector<Part> parts = {{split ? V.Xpx.p : V.Xp.p, split ? V.Vpx.p : V.Vp.p, V.Sp.as<double>(), V.np,
+                              (int64_t)P.n_pairs, ld(V.np)}};
   if (V.ncm > 0)
-    parts.push_back({split ? V.Xmx.p : V.Xm.p, split ? V.Vmx.p : V.Vm.p, (trans ? V.STm : V.Sm).as<double>(), V.nm,
-                     (int64_t)V.ncm, lx_m});
-  if (trans) {
-    TCI_REQUIRE(split, "the transposed product is a split-precision schedule");
-    // S^T = V X^T: tasks by row block of V (tile rows of pairs), then K-split;
-    // the program tiles the walks along N
-    for (const Part& pt : parts) {
-      const int64_t K = xpad(pt.n);
-      const int64_t spart = pt.rows * pt.n;
-      for (int64_t m0 = 0; m0 < pt.n; m0 += tile) {
-        const int mm = (int)std::min<int64_t>(tile, pt.n - m0);
-        for (int k = 0; k < ks; ++k) {
-          const int64_t k0 = (K * k / ks) & ~(int64_t)15, k1 = k + 1 == ks ? K : (K * (k + 1) / ks) & ~(int64_t)15;
-          TCI_REQUIRE(k1 > k0, "empty K-split range");
-          const uint16_t* Vb = static_cast<const uint16_t*>(pt.Vm) + m0 * pt.ldx + 2 * k0;
-          const uint16_t* Xb = static_cast<const uint16_t*>(pt.X) + 2 * k0;
-          g.add(pt.S + k * spart + m0 * pt.rows, pt.rows, mm, (int)pt.rows,
-                {vseg(vop(Vb, pt.ldx), vop(Xb, pt.ldx), (int)(k1 - k0))}, false, false, 0, Blocking(), kScOut);
-        }
-      }
-    }
-    g.upload_tables(st);
-    return;
-  }
+    parts.push_back({split ? V.Xmx.p : V.Xm.p, split ? V.Vmx.p : V.Vm.p, V.Sm.as<double>(), V.nm, (int64_t)V.ncm,
+                     ld(V.nm)});
   for (const Part& pt : parts) {
-    const int64_t K = split ? xpad(pt.n) : pt.n;
+    const int64_t K = pt.ld;               // padding columns of X and V are zero
     const int64_t spart = pt.rows * pt.n;  // elements of one partial S
     for (int64_t n0 = 0; n0 < pt.n; n0 += tn) {
       const int nn = (int)std::min<int64_t>(tn, pt.n - n0);
       for (int k = 0; k < ks; ++k) {
-        // K ranges on multiples of 16 (8 for split rows suffices; 16 keeps both aligned)
-        const int64_t k0 = (K * k / ks) & ~(int64_t)15, k1 = k + 1 == ks ? K : (K * (k + 1) / ks) & ~(int64_t)15;
+        const int64_t k0 = (K * k / ks) & ~(int64_t)31, k1 = k + 1 == ks ? K : (K * (k + 1) / ks) & ~(int64_t)31;
         TCI_REQUIRE(k1 > k0, "empty K-split range");
-        Seg s;
-        if (split) {
-          const uint16_t* Xb = static_cast<const uint16_t*>(pt.X) + 2 * k0;
-          const uint16_t* Vb = static_cast<const uint16_t*>(pt.Vm) + n0 * pt.ldx + 2 * k0;
-          s = vseg(vop(Xb, pt.ldx), vop(Vb, pt.ldx), (int)(k1 - k0));
-        } else {
-          const double* Xb = static_cast<const double*>(pt.X) + k0;
-          const double* Vb = static_cast<const double*>(pt.Vm) + k0 * pt.n + n0;
-          s = vseg(vop(Xb, pt.ldx), vop(Vb, pt.n), (int)(k1 - k0));
-        }
-        g.add(pt.S + k * spart + n0, pt.n, (int)pt.rows, nn, {s}, false, false, 0, Blocking(), split ? kScOut : -1);
+        const char* Xb = static_cast<const char*>(pt.X) + k0 * esz;
+        const char* Vb = static_cast<const char*>(pt.Vm) + (n0 * pt.ld + k0) * esz;
+        g.add(pt.S + k * spart + n0, pt.n, (int)pt.rows, nn, {nseg(Xb, pt.ld, Vb, pt.ld, k1 - k0, esz)}, false,
+              Blocking(), split ? kScOut : -1);
       }
     }
   }
   g.upload_tables(st);
 }
 
-void alloc_partials(tci_plan& P, int ks, bool trans) {
+void alloc_partials(tci_plan& P, int ks) {
   tci_plan::VVLadder& V = P.vv;
   const size_t need_p = (size_t)ks * P.n_pairs * V.np * 8, need_m = (size_t)ks * std::max(V.ncm, 1) * V.nm * 8;
   if (V.Sp.bytes < need_p) V.Sp.alloc(need_p);
   if (V.Sm.bytes < need_m) V.Sm.alloc(need_m);
-  if (trans) {
-    if (V.STp.bytes < need_p) V.STp.alloc(need_p);
-    if (V.STm.bytes < need_m) V.STm.alloc(need_m);
-  }
 }
 
 }  // namespace
@@ -382,8 +321,11 @@ void vv_build(tci_plan& P, hipStream_t st) {
   for (int Q = 0; Q < P.n_pairs; ++Q)
     if (P.h_pairs[2 * Q] != P.h_pairs[2 * Q + 1]) colm[Q] = V.ncm++;
   upload(V.colm, colm, st);
-  V.Vp.alloc((size_t)V.np * V.np * 8);
-  V.Vm.alloc((size_t)std::max<int64_t>(V.nm, 1) * std::max<int64_t>(V.nm, 1) * 8);
+  V.Vp.alloc((size_t)V.np * even(V.np) * 8);
+  V.Vm.alloc((size_t)std::max<int64_t>(V.nm, 1) * even(std::max<int64_t>(V.nm, 1)) * 8);
+  // the padding column of odd sizes must read as zero
+  if (V.np != even(V.np)) launch_fill(V.Vp.as<double>(), (int64_t)(V.Vp.bytes / 8), 0.0, st);
+  if (V.nm != even(V.nm)) launch_fill(V.Vm.as<double>(), (int64_t)(V.Vm.bytes / 8), 0.0, st);
   {
     DevBuf LT;
     LT.alloc((size_t)nv2 * P.n_chol * 8);
@@ -416,29 +358,27 @@ void vv_build(tci_plan& P, hipStream_t st) {
       TCI_HIP(hipStreamSynchronize(st));  // the tables and W are reused by the next slab
     }
   }
-  V.Xp.alloc((size_t)P.n_pairs * V.np * 8);
-  V.Xm.alloc((size_t)std::max(V.ncm, 1) * V.nm * 8);
+  V.Xp.alloc((size_t)P.n_pairs * even(V.np) * 8);
+  V.Xm.alloc((size_t)std::max(V.ncm, 1) * even(V.nm) * 8);
   launch_fill(V.Xp.as<double>(), (int64_t)(V.Xp.bytes / 8), 0.0, st);
   launch_fill(V.Xm.as<double>(), (int64_t)(V.Xm.bytes / 8), 0.0, st);
   V.built = true;
-  vv_set_schedule(P, TCI_SIGMA_FP64, 128, 0, 0, 1, st);
+  vv_set_schedule(P, TCI_SIGMA_FP64, N128, 1, st);
   TCI_HIP(hipStreamSynchronize(st));
 }
 
-void vv_set_schedule(tci_plan& P, int precision, int tile, int tile_n, int dma, int ks, hipStream_t st, bool trans) {
+void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t st) {
   tci_plan::VVLadder& V = P.vv;
   // every K-split range non-empty (at least 64 long), so every partial of S is written
   const int64_t kmin = V.ncm > 0 ? std::min(V.np, V.nm) : V.np;
   ks = (int)std::max<int64_t>(1, std::min<int64_t>(ks, kmin / 64));
+  alloc_partials(P, ks);
   if (precision == TCI_SIGMA_FP64) {
-    alloc_partials(P, ks, false);
     V.ks = ks;
-    build_products(P, V.g64, false, tile, 0, 0, ks, false, st);
+    build_products(P, V.g64, false, shape, ks, st);
   } else {
-    alloc_partials(P, ks, trans);
     V.ksx = ks;
-    V.xtrans = trans;
-    build_products(P, V.gx, true, tile, tile_n, dma, ks, trans, st);
+    build_products(P, V.gx, true, shape, ks, st);
   }
 }
 
@@ -452,11 +392,11 @@ void vv_prepare_split(tci_plan& P, int precision, hipStream_t st) {
   if (f16) {
     unsigned* mx = P.mx.maxbits.as<unsigned>() + 3;
     hipLaunchKernelGGL(vv_zero_kernel, dim3(1), dim3(64), 0, st, mx);
-    hipLaunchKernelGGL(vv_absmax_kernel, dim3(blocks(V.np * V.np, 8192)), dim3(256), 0, st, V.Vp.as<double>(),
-                       V.np * V.np, mx);
+    hipLaunchKernelGGL(vv_absmax_kernel, dim3(blocks(V.np * even(V.np), 1024)), dim3(256), 0, st, V.Vp.as<double>(),
+                       V.np * even(V.np), mx);
     if (V.nm > 0)
-      hipLaunchKernelGGL(vv_absmax_kernel, dim3(blocks(V.nm * V.nm, 8192)), dim3(256), 0, st, V.Vm.as<double>(),
-                         V.nm * V.nm, mx);
+      hipLaunchKernelGGL(vv_absmax_kernel, dim3(blocks(V.nm * even(V.nm), 1024)), dim3(256), 0, st, V.Vm.as<double>(),
+                         V.nm * even(V.nm), mx);
     hipLaunchKernelGGL(vv_set_vscale_kernel, dim3(1), dim3(64), 0, st, mx, sc, kScV);
     TCI_HIP(hipGetLastError());
   }
@@ -464,31 +404,21 @@ void vv_prepare_split(tci_plan& P, int precision, hipStream_t st) {
   V.Vpx.alloc((size_t)V.np * lp * 2);
   V.Vmx.alloc((size_t)std::max<int64_t>(V.nm, 1) * lm * 2);
   hipLaunchKernelGGL(split_square_kernel, dim3(blocks(V.np * (lp / 16), 16384)), dim3(256), 0, st, V.Vp.as<double>(),
-                     V.np, V.Vpx.as<uint16_t>(), lp, sc + kScV, f16);
+                     V.np, even(V.np), V.Vpx.as<uint16_t>(), lp, sc + kScV, f16);
   if (V.nm > 0)
     hipLaunchKernelGGL(split_square_kernel, dim3(blocks(V.nm * (lm / 16), 16384)), dim3(256), 0, st,
-                       V.Vm.as<double>(), V.nm, V.Vmx.as<uint16_t>(), lm, sc + kScV, f16);
+                       V.Vm.as<double>(), V.nm, even(V.nm), V.Vmx.as<uint16_t>(), lm, sc + kScV, f16);
   TCI_HIP(hipGetLastError());
   V.Xpx.alloc((size_t)P.n_pairs * lp * 2);
   V.Xmx.alloc((size_t)std::max(V.ncm, 1) * lm * 2);
   launch_fill(static_cast<double*>(V.Xpx.p), (int64_t)(V.Xpx.bytes / 8), 0.0, st);
   launch_fill(static_cast<double*>(V.Xmx.p), (int64_t)(V.Xmx.bytes / 8), 0.0, st);
   V.prec = precision;
-  // untuned schedule: 128 x 192 tiles, TCI_VV_TILE=256 (256w8, 256w16) for the
-  // 32 x 32-MFMA kernel, TCI_VV_TILE=128x192T (128x192T<k>: k K-splits) for
-  // the transposed product, TCI_VV_TILE=128x192d2 or 128x192d3 for two or
-  // three direct-load stages
+  // untuned schedule: 128 x 192 tiles; TCI_VV_TILE=256.. or 128x128.. for the others
   const char* te = std::getenv("TCI_VV_TILE");
   const std::string ts = te ? te : "";
-  if (te && std::atoi(te) == 256)
-    vv_set_schedule(P, precision, 256, 256, ts == "256w8" ? 8 : (ts == "256w16" ? 16 : 0), 2, st);
-  else if (ts.rfind("128x192T", 0) == 0)
-    vv_set_schedule(P, precision, 128, 192, 0, ts.size() > 8 ? std::max(1, std::atoi(te + 8)) : 1, st, true);
-  else if (ts == "128x192d2" || ts == "128x192d3")
-    vv_set_schedule(P, precision, 128, 192, ts == "128x192d2" ? 2 : 3, 1, st);
-  else if (ts == "128x128d2")
-    vv_set_schedule(P, precision, 128, 128, 2, 1, st);
-  else vv_set_schedule(P, precision, 128, 192, 0, 1, st);
+  const int shape = ts.rfind("256", 0) == 0 ? N256 : ts.rfind("128x128", 0) == 0 || ts.rfind("128d", 0) == 0 ? N128 : N128x192;
+  vv_set_schedule(P, precision, shape, 1, st);
   TCI_HIP(hipStreamSynchronize(st));
 }
 
@@ -511,29 +441,14 @@ void vv_ladder(tci_plan& P, int precision, hipStream_t st) {
                        V.Xpx.p, 2 * xpad(V.np), V.Xmx.p, 2 * xpad(V.nm), f16 ? sc + kScC : nullptr, f16);
   } else {
     hipLaunchKernelGGL(vv_scatter_kernel<false>, gs, dim3(256), 0, st, P.tab, P.C.as<double>(), V.colm.as<int32_t>(),
-                       V.Xp.p, V.np, V.Xm.p, V.nm, nullptr, 0);
+                       V.Xp.p, even(V.np), V.Xm.p, even(V.nm), nullptr, 0);
   }
   TCI_HIP(hipGetLastError());
   P.kt_end(e0, pn + " ladder vv_scatter_kernel", 0.0, precision, st);
-  const GemmProgram& g = split ? V.gx : V.g64;
-  int ks = split ? V.ksx : V.ks;  // K-splits change the launch (and its traffic), so they name it
+  const NProgram& g = split ? V.gx : V.g64;
+  const int ks = split ? V.ksx : V.ks;  // K-splits change the launch (and its traffic), so they name it
   P.kt_run(pn + " ladder (ab|cd) product" + (ks > 1 ? " K-split " + std::to_string(ks) : std::string()), g,
-           precision, st, [&] {
-    if (split) g.launch_split(precision, st, 0, sc);
-    else g.launch(st);
-  });
-  if (split && V.xtrans) {  // S^T partials -> S (summed)
-    e0 = P.kt_begin(st);
-    const int64_t rp = P.n_pairs, rm = std::max(V.ncm, 1);
-    hipLaunchKernelGGL(vv_untranspose_kernel, dim3((unsigned)cdiv(V.np, 32), (unsigned)cdiv(rp, 32)), dim3(256), 0,
-                       st, V.STp.as<double>(), rp * V.np, rp, V.np, ks, V.Sp.as<double>());
-    if (V.ncm > 0)
-      hipLaunchKernelGGL(vv_untranspose_kernel, dim3((unsigned)cdiv(V.nm, 32), (unsigned)cdiv(rm, 32)), dim3(256), 0,
-                         st, V.STm.as<double>(), rm * V.nm, rm, V.nm, ks, V.Sm.as<double>());
-    TCI_HIP(hipGetLastError());
-    P.kt_end(e0, pn + " ladder vv_untranspose_kernel", 0.0, precision, st);
-    ks = 1;
-  }
+           precision, st, [&] { g.launch(precision, st, 0, sc); });
   e0 = P.kt_begin(st);
   hipLaunchKernelGGL(vv_gather_kernel, dim3(blocks((int64_t)P.dmax * P.dmax, 64), (unsigned)P.n_pairs), dim3(256), 0,
                      st, P.tab, V.Sp.as<double>(), (int64_t)P.n_pairs * V.np, V.np, V.Sm.as<double>(),
@@ -546,65 +461,48 @@ void vv_ladder(tci_plan& P, int precision, hipStream_t st) {
 // Returns the time of the whole resident ladder with the chosen schedule.
 double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
   tci_plan::VVLadder& V = P.vv;
-  struct Cand {
-    int tile, tile_n, dma, ks;
-    bool trans = false;
-  };
-  std::vector<Cand> cands;
-  if (precision == TCI_SIGMA_FP64) {
-    for (int t : {128, 192})
-      for (int ks : {1, 2, 4}) cands.push_back({t, 0, 0, ks});
-  } else {
-    for (int ks : {1, 2, 4}) {
-      cands.push_back({128, 128, 0, ks});
-      cands.push_back({128, 192, 0, ks});
-      cands.push_back({192, 192, 0, ks});
-      cands.push_back({192, 192, 3, ks});
-      cands.push_back({256, 256, 0, ks});
-      cands.push_back({256, 256, 8, ks});  // dma field: eight waves
-      cands.push_back({256, 256, 16, ks});  // sixteen waves
-      cands.push_back({128, 192, 2, ks});  // 128 x 192 with two or three direct-load stages
-      cands.push_back({128, 192, 3, ks});
-      cands.push_back({128, 128, 2, ks});
-      cands.push_back({128, 192, 0, ks, true});  // S^T = V X^T
-      cands.push_back({128, 128, 0, ks, true});
-      cands.push_back({192, 192, 3, ks, true});
-      cands.push_back({128, 192, 3, ks, true});
-    }
+  const bool split = precision != TCI_SIGMA_FP64;
+  std::vector<int> shapes = {N128, N192};
+  if (split) shapes = {N128, N128x192, N192, N256};
+  // tiles that leave the chip idle at 128 x 128 also try the small ones
+  if (cdiv(V.np, 128) * cdiv(P.n_pairs, 128) < 512) {
+    shapes.push_back(N64);
+    shapes.push_back(N32K4);
   }
-  auto label = [](const Cand& c) {
-    return std::to_string(c.tile) + (c.tile_n ? "x" + std::to_string(c.tile_n) : "") +
-           (c.dma ? (c.tile == 256 ? "w" + std::to_string(c.dma) : "d" + (c.tile == 192 ? "" : std::to_string(c.dma)))
-                  : "") +
-           (c.trans ? "T" : "") + "/" + std::to_string(c.ks);
-  };
+  // FP32 sums of scaled fp16x3 products lose about as much to the length of
+  // the chain as the operands do to their split: four K-splits at least
+  const int kmin = precision == TCI_SIGMA_FP16X3 ? 4 : 1;
   double best = 1e300;
-  Cand bc = cands[0];
-  for (const Cand& c : cands) {
-    vv_set_schedule(P, precision, c.tile, c.tile_n, c.dma, c.ks, st, c.trans);
-    const double ms = time_ms(st, 2, [&] { vv_ladder(P, precision, st); });
-    log += " " + label(c) + ":" + fmt_ms(ms);
-    if (ms < best * 0.98) {
-      best = ms;
-      bc = c;
+  int bs = N128, bk = kmin, bo = 0;
+  NProgram& g = split ? V.gx : V.g64;
+  const int orders = xcd_remap_forced() ? 1 : 2;
+  for (int ks : {1, 2, 4}) {
+    if (ks < kmin) continue;
+    for (int sh : shapes) {
+      vv_set_schedule(P, precision, sh, ks, st);
+      for (int o = 0; o < orders; ++o) {
+        g.remap = o;
+        const double ms = time_ms(st, 2, [&] { vv_ladder(P, precision, st); });
+        log += " " + std::to_string(g.tm()) + "x" + std::to_string(g.tn()) + "/" + std::to_string(ks) + (o ? "x:" : ":") +
+               fmt_ms(ms);
+        if (ms < best * 0.98) {
+          best = ms;
+          bs = sh;
+          bk = ks;
+          bo = o;
+        }
+      }
     }
   }
-  vv_set_schedule(P, precision, bc.tile, bc.tile_n, bc.dma, bc.ks, st, bc.trans);
-  GemmProgram& g = precision == TCI_SIGMA_FP64 ? V.g64 : V.gx;
-  const float* sc = P.mx.scales.as<float>();
-  const int o = tune_order(g, st, [&] {
-    if (precision == TCI_SIGMA_FP64) g.launch(st);
-    else g.launch_split(precision, st, 0, sc);
-  });
-  if (precision != TCI_SIGMA_FP64) {
-    V.split_tile = bc.tile;
-    V.split_tile_n = bc.tile_n;
-    V.split_dma = bc.dma;
-    V.split_ks = bc.ks;
-    V.split_order = o;
-    V.split_trans = bc.trans;
+  vv_set_schedule(P, precision, bs, bk, st);
+  g.remap = bo;
+  if (split) {
+    V.split_shape = bs;
+    V.split_ks = bk;
+    V.split_order = bo;
   }
-  log += " -> " + label(bc) + " order " + std::to_string(o);
+  log += " -> " + std::to_string(g.tm()) + "x" + std::to_string(g.tn()) + "/" + std::to_string(bk) + " order " +
+         std::to_string(bo);
   TCI_HIP(hipStreamSynchronize(st));
   return time_ms(st, 2, [&] { vv_ladder(P, precision, st); });
 }
@@ -612,7 +510,7 @@ double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
 int64_t vv_device_bytes(const tci_plan& P) {
   const tci_plan::VVLadder& V = P.vv;
   int64_t b = 0;
-  for (const DevBuf* x : {&V.Vp, &V.Vm, &V.Vpx, &V.Vmx, &V.Xp, &V.Xm, &V.Xpx, &V.Xmx, &V.Sp, &V.Sm, &V.STp, &V.STm,
+  for (const DevBuf* x : {&V.Vp, &V.Vm, &V.Vpx, &V.Vmx, &V.Xp, &V.Xm, &V.Xpx, &V.Xmx, &V.Sp, &V.Sm,
                           &V.colm})
     b += (int64_t)x->bytes;
   return b;

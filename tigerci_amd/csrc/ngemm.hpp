@@ -1,0 +1,98 @@
+// Grouped GEMM over k-contiguous operands with direct global-to-LDS stages:
+//   C[tile] (+)= s sum_seg A_seg B_seg^T,   A_seg: M x K,  B_seg: N x K,
+// both operands as rows of bytes: FP64 (16 values of k per 128 bytes) or split
+// rows (common.hpp: 32 values of k, hi and lo parts, per 128 bytes).  The two
+// types share the staging: a k-step is 128 bytes of every row, copied by
+// global_load_lds_dwordx4 into LDS rows of 128 bytes whose 16-byte chunks are
+// XOR-swizzled on the source side.  Rows may be gathered through a row map, so
+// one launch covers pair blocks over local domains without packed copies of
+// operands that already have their k contiguous.
+//
+// What the loop avoids, against a staging that reads its segment descriptor
+// and forms 64-bit row addresses for every load: each lane keeps one 32-bit
+// offset per load for a whole segment, the segment's base is scalar and moves
+// by 128 bytes a step, and nothing between two barriers waits on scalar
+// memory, so the loads of the next stage cost a few issue slots and the MFMAs
+// follow at once.
+//
+// Rows beyond M or N load a valid row again (their products are not stored);
+// k beyond the segment loads zeros.
+//
+// Waves: NWM x NWN over the tile, blocks of 16 rows (columns) dealt
+// round-robin, so that a ragged tile (a domain below the tile's size) loads
+// every wave about equally; NWK groups of waves take alternate 128-byte
+// k-chunks of one deeper stage and meet in LDS at the end (small outputs,
+// whose few tiles would otherwise run a long chain of dependent k-steps on a
+// mostly idle chip).
+#pragma once
+
+#include "common.hpp"
+
+namespace tci {
+
+// One contraction range of a task.  kbytes: valid bytes of k per row, a
+// multiple of 16; lda / ldb row strides in bytes (multiples of 16); am / bm
+// row maps or null; ja / jb bytes per unit of the launch argument J0.
+struct NSeg {
+  const void* A;
+  const void* B;
+  const int32_t* am;
+  const int32_t* bm;
+  int64_t lda, ldb, ja, jb;
+  int64_t kbytes;
+  int64_t pad_;
+};
+
+// Tile shapes (rows x columns; K-groups).
+enum NShape {
+  N128 = 0,    // 128 x 128, 4 waves, two workgroups per CU
+  N192 = 1,    // 192 x 192, 8 waves, one workgroup per CU
+  N64 = 2,     // 64 x 64, 4 waves
+  N32K4 = 3,   // 32 x 32, 4 waves each on a quarter of k
+  N256 = 4,    // split only: 256 x 256 on 32 x 32 MFMAs, 8 waves
+  N128x192 = 5 // split only: 128 x 192, 4 waves
+};
+
+struct NProgram {
+  int shape = N128;
+  bool split = false;
+  int remap = 0;
+  double alg_flops = 0.0;
+  std::vector<Task> tasks;
+  std::vector<NSeg> segs;
+  DevBuf d_tasks, d_segs;
+  void clear() {
+    tasks.clear();
+    segs.clear();
+  }
+  int tm() const { return shape == N192 ? 192 : shape == N64 ? 64 : shape == N32K4 ? 32 : shape == N256 ? 256 : 128; }
+  int tn() const { return shape == N128x192 ? 192 : tm(); }
+  // adds the tiles of one M x N output; rows / cols of the stored element are
+  // offset by the blocking as in GemmProgram
+  void add(double* C, int64_t ldc, int M, int N, const std::vector<NSeg>& s, bool accumulate, Blocking blk = Blocking(),
+           int oscale = -1, bool out_split = false);
+  void upload_tables(hipStream_t st);
+  void launch(int precision, hipStream_t st, int64_t J0 = 0, const float* scales = nullptr) const;
+  std::string kernel_name() const;
+};
+
+// segment over rows of elements of `esz` bytes per value of k (8: FP64, 4: split rows)
+inline NSeg nseg(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t K, int esz,
+                 const int32_t* am = nullptr, const int32_t* bm = nullptr) {
+  NSeg s{};
+  s.A = A;
+  s.B = B;
+  s.am = am;
+  s.bm = bm;
+  s.lda = lda * esz;
+  s.ldb = ldb * esz;
+  s.kbytes = K * esz;
+  return s;
+}
+
+void launch_ngemm64(int shape, const Task* tasks, const NSeg* segs, int64_t ntasks, int64_t J0, hipStream_t st,
+                    int remap);
+void launch_ngemm16(int precision, int shape, const Task* tasks, const NSeg* segs, int64_t ntasks, int64_t J0,
+                    const float* scales, hipStream_t st, int remap);
+
+}  // namespace tci

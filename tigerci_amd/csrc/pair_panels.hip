@@ -1,0 +1,894 @@
+// Pair-pair terms as per-walk products over packed panels.
+//
+// For an internal orbital i let K_i be the list of all (k, c) with the walk
+// {i, k} strong and c in its domain D_ik: blocks by k, each padded to a
+// multiple of 8.  C^{pq} is the walk's dense block (p >= q) or its transpose.
+// Panels over K_i, rows a over all virtuals (zero outside the domains):
+//   CR_i[a][(k,c)] = C^{ik}[a][c],  CC_i[a][(k,c)] = C^{ki}[a][c],  CT_i = 2 CR_i - CC_i
+// (written from C in every sigma) and, once per plan, for every strong ordered
+// pair (i, j) over the rows x of D_ij, and for every i over the Cholesky vectors,
+//   JP_ij[x][(k,c)] = -(kj|c D_ij[x]),   LP_i[J][(k,c)] = L^J_kc.
+// With U[(i,a)][J] = Y[i][J][a] + W[i][J][a],
+//   Y[i][J][a] = sum_c L^J_ac s_i^c,  W_i = LP_i CT_i^T  ([i][J][a]),
+// the ring and 3-external terms of the walk P = (i, j), rows and columns over
+// D_P, are one contraction (Kov = Lov^T Lov puts C~ K into U Lov):
+//   R_P += CR_i JP_ij^T + JP_ij CC_i^T + JP_ji CR_j^T + CC_j JP_ji^T
+//        + U_i Lov_j + (U_j Lov_i)^T
+// and the 3-internal singles terms are two more ranges of it (FP64):
+//        + s_i O_ij^T + O_ji s^T,   O_ij[b][k] = -(ki|bj).
+// All operands have their k contiguous and rows gathered through D_P, so they
+// run on the NT GEMM (ngemm.hpp): flops 2 d_P^2 (2 |K_i| + 2 |K_j| + 2 n_chol)
+// per walk, the count of the gathered per-walk products, at the rate of the
+// dense ones.  Embedding every block in the full virtual space instead
+// (4 N^3 + 6 N^2 n_chol, N = n_int n_v) costs 4.4 times the flops at 34
+// internal, 192 virtual orbitals with domains of 60 to 192.  W serves U and
+// the singles (g += W L): it is computed once.
+//
+// The 4-internal term sum_Q [(ki|lj) C_Q + (li|kj) C_Q^T] acts on the symmetric
+// and antisymmetric parts of C_Q separately, over packed virtual pairs:
+//   H+[P][p] = sum_Q h+_PQ X+_Q[p],  H-[P'][q] = sum_Q h-_PQ X-_Q[q],
+//   h+- = (ki|lj) +- (li|kj),
+// products over k = walk with X+- transposed to [pair][walk].  The final kernel
+// (pack_panels_kernel) adds everything of one CSF: K-split partials, S+- of
+// the resident ladder, H+-, c0 (ia|jb) and the CSF factors.
+#include "plan.hpp"
+
+#include <algorithm>
+#include <cstdlib>
+#include <string>
+
+namespace tci {
+
+namespace {
+
+constexpr double SQRT2 = 1.41421356237309504880;
+constexpr double INV_SQRT2 = 0.70710678118654752440;
+constexpr double SQRT3 = 1.73205080756887729353;
+
+__host__ __device__ __forceinline__ int64_t tri(int64_t a) { return a * (a + 1) / 2; }
+__device__ __forceinline__ void untri32(int t, int& x, int& y) {  // t = x(x+1)/2 + y, y <= x
+  int r = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
+  while ((r + 1) * (r + 2) / 2 <= t) ++r;
+  while (r * (r + 1) / 2 > t) --r;
+  x = r;
+  y = t - r * (r + 1) / 2;
+}
+inline int64_t up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
+
+// Offsets are in values; a value is 8 bytes (FP64) or 4 (split rows).
+struct PanelTab {
+  const int32_t* koff;   // [i n_int + k] -> column of block k in panel i, or -1
+  const int64_t* ld;     // [i] row stride of panel i
+  const int64_t* poff;   // [i] start of panel i (n_v rows)
+  const int64_t* jpoff;  // [i n_int + j] start of JP_ij
+  const int64_t* lpoff;  // [i] start of LP_i (n_chol rows)
+  const int32_t* pairid;
+};
+
+__device__ __forceinline__ uint16_t* srow(void* base, int64_t row_start, int64_t col) {
+  return static_cast<uint16_t*>(base) + 2 * row_start + xidx(col);
+}
+
+// CR, CC and CT of both panels of walk Q from its C block: 32 x 32 tiles, the
+// tile and its transpose read once.  Rows outside the domain and padding
+// columns are zero from set-up and never written.
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void panels_kernel(PairTab T, PanelTab K, const double* __restrict__ C, void* CR,
+                                                     void* CC, void* CT, const float* scl, const float* sclt, int f16,
+                                                     int what) {
+  __shared__ double ta[32][33], tb[32][33];
+  const int Q = blockIdx.y;
+  const int64_t o = T.dom_off[Q];
+  const int d = (int)(T.dom_off[Q + 1] - o), nt = (d + 31) >> 5;
+  if ((int)blockIdx.x >= nt * nt) return;
+  const int x0 = ((int)blockIdx.x / nt) * 32, y0 = ((int)blockIdx.x % nt) * 32;
+  const int i = T.pairs[2 * Q], j = T.pairs[2 * Q + 1];
+  const double* Cq = C + T.cd_off[Q];
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  for (int r = ty; r < 32; r += 8) {
+    const int x = x0 + r, y = y0 + tx;
+    ta[r][tx] = x < d && y < d ? Cq[(int64_t)x * d + y] : 0.0;     // C^{ij}[x][y]
+    const int yr = y0 + r, xc = x0 + tx;
+    tb[tx][r] = yr < d && xc < d ? Cq[(int64_t)yr * d + xc] : 0.0;  // C^{ji}[x][y] = C_Q[y][x]
+  }
+  __syncthreads();
+  const int two = i != j ? 2 : 1;
+  if (!SPLIT) {
+    for (int p = 0; p < two; ++p) {
+      const int u = p ? j : i, v = p ? i : j;
+      const int64_t base = K.poff[u] + K.koff[u * T.n_int + v], ld = K.ld[u];
+      for (int r = ty; r < 32; r += 8) {
+        const int x = x0 + r, y = y0 + tx;
+        if (x >= d || y >= d) continue;
+        const double a = p ? tb[r][tx] : ta[r][tx], b = p ? ta[r][tx] : tb[r][tx];
+        const int64_t e = base + (int64_t)T.dom_idx[o + x] * ld + y;
+        static_cast<double*>(CR)[e] = a;
+        static_cast<double*>(CC)[e] = b;
+        static_cast<double*>(CT)[e] = 2.0 * a - b;
+      }
+    }
+  } else {
+    const float s = scale_at(scl), st = scale_at(sclt);
+    // 128 chunks of 8 per array (row r, chunk ch); arrays CR, CC (what & 1), CT (what & 2), per panel
+    for (int t = threadIdx.x; t < 128 * 3 * two; t += 256) {
+      const int arr = (t >> 7) % 3, p = (t >> 7) / 3;
+      if (!(what & (arr == 2 ? 2 : 1))) continue;
+      const int r = (t & 127) >> 2, c = 8 * (t & 3);
+      const int x = x0 + r, y = y0 + c;
+      if (x >= d || y >= d) continue;
+      const int u = p ? j : i, v = p ? i : j;
+      float w[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const double a = p ? tb[r][c + q] : ta[r][c + q], b = p ? ta[r][c + q] : tb[r][c + q];
+        w[q] = (float)(arr == 0 ? a : arr == 1 ? b : 2.0 * a - b);
+      }
+      void* dst = arr == 0 ? CR : arr == 1 ? CC : CT;
+      put_split8(srow(dst, K.poff[u] + (int64_t)T.dom_idx[o + x] * K.ld[u], K.koff[u * T.n_int + v] + y), w,
+                 arr == 2 ? st : s, f16 != 0);
+    }
+  }
+}
+
+// JP_ij block k: rows x of D_ij, columns c of D_ik.  Grid (k, (i,j)).
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void jp_kernel(PairTab T, PanelTab K, const double* __restrict__ Jvv, void* JP,
+                                                 const float* scl, int f16) {
+  const int n = T.n_int, k = blockIdx.x, i = blockIdx.y / n, j = blockIdx.y % n;
+  const int P = K.pairid[i * n + j], Q = K.pairid[i * n + k];
+  if (P < 0 || Q < 0) return;
+  const int64_t oP = T.dom_off[P], oQ = T.dom_off[Q];
+  const int dP = (int)(T.dom_off[P + 1] - oP), dQ = (int)(T.dom_off[Q + 1] - oQ);
+  const int hi = max(k, j), lo = min(k, j);
+  const int64_t nv = T.n_v;
+  const double* J = Jvv + ((int64_t)hi * (hi + 1) / 2 + lo) * nv * nv;
+  const int64_t ld = K.ld[i], base = K.jpoff[i * n + j];
+  const int64_t col = K.koff[i * n + k];
+  const float s = SPLIT ? scale_at(scl) : 1.f;
+  const int nch = (dQ + 7) >> 3;
+  if (SPLIT) {
+    for (int t = threadIdx.x; t < dP * nch; t += 256) {
+      const int x = t / nch, c = 8 * (t - x * nch);
+      const double* row = J + (int64_t)T.dom_idx[oP + x] * nv;
+      float w[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w[q] = c + q < dQ ? (float)-row[T.dom_idx[oQ + c + q]] : 0.f;
+      put_split8(srow(JP, base + x * ld, col + c), w, s, f16 != 0);
+    }
+  } else {
+    for (int t = threadIdx.x; t < dP * dQ; t += 256) {
+      const int x = t / dQ, c = t - x * dQ;
+      static_cast<double*>(JP)[base + x * ld + col + c] = -J[(int64_t)T.dom_idx[oP + x] * nv + T.dom_idx[oQ + c]];
+    }
+  }
+}
+
+// LP_i[J][(k,c)] = L^J_kc.  Grid (J, i).
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void lp_kernel(PairTab T, PanelTab K, const double* __restrict__ Lov, void* LP,
+                                                 const float* scl, int f16) {
+  const int n = T.n_int, i = blockIdx.y;
+  const int64_t J = blockIdx.x, nv = T.n_v;
+  const int64_t row = K.lpoff[i] + J * K.ld[i];
+  const float s = SPLIT ? scale_at(scl) : 1.f;
+  for (int k = 0; k < n; ++k) {
+    const int Q = K.pairid[i * n + k];
+    if (Q < 0) continue;
+    const int64_t o = T.dom_off[Q];
+    const int d = (int)(T.dom_off[Q + 1] - o);
+    const double* L = Lov + (J * n + k) * nv;
+    const int64_t col = K.koff[i * n + k];
+    if (SPLIT) {
+      for (int c = 8 * (int)threadIdx.x; c < d; c += 8 * 256) {
+        float w[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) w[q] = c + q < d ? (float)L[T.dom_idx[o + c + q]] : 0.f;
+        put_split8(srow(LP, row, col + c), w, s, f16 != 0);
+      }
+    } else {
+      for (int c = threadIdx.x; c < d; c += 256) static_cast<double*>(LP)[row + col + c] = L[T.dom_idx[o + c]];
+    }
+  }
+}
+
+// U[(i,a)][J] = Y[i][J][a] + W[i][J][a] (Y null: W alone, for the transposed
+// Lov), 32 x 32 tiles through LDS; row stride ldu values.  Grid (J tiles, a
+// tiles, i).
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void u_kernel(const double* __restrict__ Y, const double* __restrict__ W, int n_v,
+                                                int64_t n_chol, int64_t wstride_i, int64_t wstride_J, void* U,
+                                                int64_t ldu, const float* scl, int f16) {
+  __shared__ double tile[32][33];
+  const int i = blockIdx.z;
+  const int64_t J0 = (int64_t)blockIdx.x * 32;
+  const int a0 = blockIdx.y * 32;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  for (int r = ty; r < 32; r += 8) {
+    const int64_t J = J0 + r;
+    const int a = a0 + tx;
+    double v = 0.0;
+    if (J < n_chol && a < n_v) {
+      const int64_t e = i * wstride_i + J * wstride_J + a;
+      v = W[e];
+      if (Y) v += Y[e];
+    }
+    tile[r][tx] = v;
+  }
+  __syncthreads();
+  if (!SPLIT) {
+    for (int r = ty; r < 32; r += 8) {
+      const int a = a0 + r;
+      const int64_t J = J0 + tx;
+      if (J < n_chol && a < n_v) static_cast<double*>(U)[((int64_t)i * n_v + a) * ldu + J] = tile[tx][r];
+    }
+  } else if (threadIdx.x < 128) {
+    const int r = threadIdx.x >> 2, c = 8 * (threadIdx.x & 3);
+    const int a = a0 + r;
+    if (a < n_v && J0 + c < n_chol) {
+      float w[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w[q] = (float)tile[c + q][r];  // zero beyond n_chol
+      put_split8(srow(U, ((int64_t)i * n_v + a) * ldu, J0 + c), w, scale_at(scl), f16 != 0);
+    }
+  }
+}
+
+// max |Y + W| into *out (float bits)
+__global__ __launch_bounds__(256) void u_absmax_kernel(const double* __restrict__ Y, const double* __restrict__ W,
+                                                       int64_t n, unsigned* __restrict__ out) {
+  __shared__ float part[4];
+  float m = 0.f;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
+    m = fmaxf(m, fabsf((float)(Y[e] + W[e])));
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_down(m, off, 64));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicMax(out, __float_as_uint(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]))));
+}
+
+// XT+[p(a,b)][Q] = C+_ab, XT-[q(a,b)][Q] = C-_ab of walk Q (0 outside its
+// domain), rows of ldw values.  Block: one a, 32 b and 32 walks; the walks'
+// elements are read along b and leave through LDS along Q.
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void xt_kernel(PairTab T, const int32_t* __restrict__ pos, const double* __restrict__ C,
+                                                 void* XTp, void* XTm, int64_t ldw, const float* scl, int f16) {
+  __shared__ double tp[32][33], tm[32][33];
+  const int nv = T.n_v, a = blockIdx.x, b0 = blockIdx.y * 32, Q0 = blockIdx.z * 32;
+  if (b0 > a) return;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int b = b0 + tx;
+  for (int r = ty; r < 32; r += 8) {
+    const int Q = Q0 + r;
+    double vp = 0.0, vm = 0.0;
+    if (Q < T.n_pairs && b <= a) {
+      const int32_t* ps = pos + (int64_t)Q * nv;
+      const int pa = ps[a], pb = ps[b];
+      if (pa >= 0 && pb >= 0) {
+        const int d = (int)(T.dom_off[Q + 1] - T.dom_off[Q]);
+        const double* Cq = C + T.cd_off[Q];
+        const double x = Cq[(int64_t)pa * d + pb], y = Cq[(int64_t)pb * d + pa];
+        vp = 0.5 * (x + y);
+        vm = 0.5 * (x - y);
+      }
+    }
+    tp[r][tx] = vp;
+    tm[r][tx] = vm;
+  }
+  __syncthreads();
+  if (!SPLIT) {
+    for (int r = ty; r < 32; r += 8) {
+      const int bb = b0 + r, Q = Q0 + tx;
+      if (bb > a || Q >= T.n_pairs) continue;
+      static_cast<double*>(XTp)[(tri(a) + bb) * ldw + Q] = tp[tx][r];
+      if (bb < a) static_cast<double*>(XTm)[(tri(a - 1) + bb) * ldw + Q] = tm[tx][r];
+    }
+  } else {
+    const int t = threadIdx.x & 127, r = t >> 2, c = 8 * (t & 3);
+    const bool minus = threadIdx.x >= 128;
+    const int bb = b0 + r;
+    if (bb <= a && Q0 + c < T.n_pairs && !(minus && bb == a)) {
+      float w[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w[q] = (float)(minus ? tm[c + q][r] : tp[c + q][r]);
+      put_split8(srow(minus ? XTm : XTp, (minus ? tri(a - 1) + bb : tri(a) + bb) * ldw, Q0 + c), w, scale_at(scl),
+                 f16 != 0);
+    }
+  }
+}
+
+// split rows of an FP64 matrix (rows x K values, stride ld) into stride ldo values
+__global__ void split_matrix_kernel(const double* __restrict__ src, int64_t rows, int64_t K, int64_t ld, void* out,
+                                    int64_t ldo, const float* scl, int f16) {
+  const float s = scale_at(scl);
+  const int64_t nch = (K + 7) >> 3;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < rows * nch; e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r = e / nch, c = 8 * (e - r * nch);
+    float w[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) w[q] = c + q < K ? (float)src[r * ld + c + q] : 0.f;
+    put_split8(srow(out, r * ldo, c), w, s, f16 != 0);
+  }
+}
+
+// O_ij[b][k] = -(ki|bj) = -O3[k][i][j][b], rows of nk values; grid (i n_int + j)
+__global__ __launch_bounds__(256) void o3t_kernel(const double* __restrict__ O3, int n, int nv, int nk,
+                                                  double* __restrict__ O) {
+  const int i = blockIdx.x / n, j = blockIdx.x % n;
+  for (int t = threadIdx.x; t < nv * nk; t += 256) {
+    const int k = t / nv, b = t - k * nv;
+    O[((int64_t)blockIdx.x * nv + b) * nk + k] = k < n ? -O3[(((int64_t)k * n + i) * n + j) * nv + b] : 0.0;
+  }
+}
+
+// sT[a][k] = s[k][a], rows of nk values, zero padded
+__global__ void st_kernel(const double* __restrict__ s, int n, int nv, int nk, double* __restrict__ sT) {
+  const int64_t tot = (int64_t)nv * nk;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot; e += (int64_t)gridDim.x * blockDim.x) {
+    const int a = (int)(e / nk), k = (int)(e - (int64_t)a * nk);
+    sT[e] = k < n ? s[(int64_t)k * nv + a] : 0.0;
+  }
+}
+
+// Everything of one CSF of the pair walks: R_P[x][y] and R_P[y][x] from the
+// K-split partials (d x d each), the packed S+- and H+-, c0 (ia|jb), and R
+// itself when another term went there; then the CSF factors of pack_kernel.
+// Block: one walk, one pair of 32 x 32 tiles (X >= Y); the transposed elements
+// come through LDS.  blockIdx.y == n_pairs: valence and singles.
+struct PackSrc {
+  const double* Rp;     // [nrp][sum_d2]
+  int64_t rstride;
+  int nrp;
+  const double* R;      // null: no further terms
+  const double* Sp;     // [nsp][n_pairs][np], null: no resident ladder
+  const double* Sm;     // [nsp][ncm][nm]
+  int64_t sp_part, sm_part;
+  int nsp;
+  const double* Hp;     // [n_pairs][np]
+  const double* Hm;     // [ncm][nm]
+  int64_t np, nm;
+  const int32_t* colm;
+  const double* Kov;
+};
+
+__global__ __launch_bounds__(256) void pack_panels_kernel(PairTab T, PackSrc S, const double* __restrict__ x,
+                                                          const double* __restrict__ g,
+                                                          const double* __restrict__ sig0, double e_ref, int flags,
+                                                          double* __restrict__ sigma, const IoSlot* __restrict__ io) {
+  if (io) {
+    x = io->x;
+    sigma = io->y;
+  }
+  const bool accum = (flags & TCI_ACCUMULATE) != 0;
+  const double eadd = (flags & TCI_ADD_EREF) ? e_ref : 0.0;
+  const int P = blockIdx.y, no = T.n_int, nv = T.n_v;
+  if (P == T.n_pairs) {
+    const int64_t n = 1 + (int64_t)no * nv;
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
+      double v;
+      if (k == 0) {
+        v = *sig0 + eadd * x[0];
+      } else {
+        const int64_t w = (k - 1) / nv;  // N-1 walk rank: hole no - 1 - w
+        const int i = no - 1 - (int)w, a = (int)(k - 1 - w * nv);
+        v = SQRT2 * g[(int64_t)i * nv + a] + (T.eps[no + a] - T.eps[i] + eadd) * x[k];
+      }
+      sigma[k] = accum ? sigma[k] + v : v;
+    }
+    return;
+  }
+  const int64_t off = T.dom_off[P];
+  const int d = (int)(T.dom_off[P + 1] - off), nt = (d + 31) >> 5;
+  if ((int)blockIdx.x >= nt * (nt + 1) / 2) return;
+  int X, Yt;
+  untri32((int)blockIdx.x, X, Yt);
+  const int x0 = X * 32, y0 = Yt * 32;
+  const int i = T.pairs[2 * P], j = T.pairs[2 * P + 1];
+  const int64_t niv = (int64_t)no * nv, m2 = (int64_t)d * (d - 1) / 2;
+  const double* Rp = S.Rp + T.cd_off[P];
+  const double* R = S.R ? S.R + T.cd_off[P] : nullptr;
+  const int32_t* D = T.dom_idx + off;
+  const int cm = S.colm[P];
+  const double c0 = x[0], ei = T.eps[i], ej = T.eps[j];
+  __shared__ double tile[32][33];
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  auto elem = [&](int r, int c) {  // [r][c] without the packed parts
+    const int64_t e = (int64_t)r * d + c;
+    double v = c0 * S.Kov[((int64_t)i * nv + D[r]) * niv + (int64_t)j * nv + D[c]];
+    for (int q = 0; q < S.nrp; ++q) v += Rp[q * S.rstride + e];
+    if (R) v += R[e];
+    return v;
+  };
+  for (int r = ty; r < 32; r += 8) {
+    const int yr = y0 + r, xc = x0 + tx;
+    tile[r][tx] = yr < d && xc < d ? elem(yr, xc) : 0.0;
+  }
+  __syncthreads();
+  for (int r = ty; r < 32; r += 8) {
+    const int xr = x0 + r, yc = y0 + tx;
+    if (xr >= d || yc > xr) continue;
+    double A = elem(xr, yc), B = tile[tx][r];
+    const int gx = D[xr], gy = D[yc];  // domains are sorted: gx >= gy
+    const int64_t p = P * S.np + tri(gx) + gy;
+    double sp = S.Hp[p];
+    for (int q = 0; q < S.nsp; ++q) sp += S.Sp[q * S.sp_part + p];
+    A += sp;
+    B += sp;
+    if (cm >= 0 && gx != gy) {
+      const int64_t m = cm * S.nm + tri(gx - 1) + gy;
+      double sm = S.Hm[m];
+      for (int q = 0; q < S.nsp; ++q) sm += S.Sm[q * S.sm_part + m];
+      A += sm;
+      B -= sm;
+    }
+    const double fock = T.eps[no + gx] + T.eps[no + gy] - ei - ej + eadd;
+    auto put = [&](int64_t k, double v) {
+      v += fock * x[k];
+      sigma[k] = accum ? sigma[k] + v : v;
+    };
+    if (xr == yc) {
+      put(T.aa_off[P] + xr, i == j ? A : -SQRT2 * A);
+    } else {
+      const int64_t k = T.ab_off[P] + (int64_t)xr * (xr - 1) / 2 + yc;
+      if (i == j) {
+        put(k, (A + B) * INV_SQRT2);
+      } else {  // aa and singlet CSFs with a minus sign (see pack_kernel)
+        put(k, -(A + B));
+        put(k + m2, SQRT3 * (B - A));
+      }
+    }
+  }
+}
+
+// fp16x3 scales of the panel products: mode 0 (slots 11, 12) for W from
+// max|C|; mode 1 (slots 6, 5) for the pair products and the 4-internal product
+// from max|C| and max|U|
+__global__ void panel_scales_kernel(int mode, const unsigned* __restrict__ mx, float* __restrict__ sc) {
+  if (threadIdx.x != 0) return;
+  const float mc = __uint_as_float(mx[0]);
+  const float m = mode == 0 ? 3.f * mc : fmaxf(3.f * mc, __uint_as_float(mx[1]));
+  const float s = m > 0.f ? ldexpf(1.f, 13 - ilogbf(m)) : 1.f;
+  if (mode == 0) {
+    sc[11] = s;
+    sc[12] = 1.f / (sc[0] * s);
+  } else {
+    sc[6] = s;
+    sc[5] = 1.f / (sc[0] * s);
+  }
+}
+__global__ void zero_word_kernel(unsigned* p) {
+  if (threadIdx.x == 0) *p = 0u;
+}
+
+inline unsigned gsz(int64_t work, unsigned cap = 16384) {
+  return (unsigned)std::min<int64_t>(std::max<int64_t>(cdiv(work, 256), 1), cap);
+}
+
+PanelTab ptab(const tci_plan& P) {
+  const auto& Z = P.pp;
+  return PanelTab{Z.koff.as<int32_t>(), Z.ld.as<int64_t>(), Z.poff.as<int64_t>(), Z.jpoff.as<int64_t>(),
+                  Z.lpoff.as<int64_t>(), Z.pairid.as<int32_t>()};
+}
+
+void zero(DevBuf& b, size_t bytes, hipStream_t st) {
+  b.alloc((size_t)up((int64_t)std::max<size_t>(bytes, 16), 16));
+  launch_fill(b.as<double>(), (int64_t)(b.bytes / 8), 0.0, st);
+}
+
+// tile shape of a d x d pair block under a tiling mode: 0 by size (64, 128,
+// 192; 128-wide tiles above), 1 all 128, 2 all 64, 3 all 32 x 32 in four K-groups
+int shape_of(int mode, int d) {
+  if (mode == 3) return N32K4;
+  if (mode == 2 || d <= 64) return N64;
+  if (mode == 1 || d <= 128) return N128;
+  return d <= 192 ? N192 : N128;
+}
+
+}  // namespace
+
+// Panels hold |K_i| columns for n_v rows three times, for every ordered strong
+// pair's domain once (JP) and for n_chol rows once (LP).
+bool panels_choose(const tci_plan& P) {
+  if (P.n_pairs == 0) return false;
+  const char* env = std::getenv("TCI_DENSE_PAIRS");
+  if (env && env[0] == '0') return false;
+  const int n = P.n_int;
+  double vals = 0.0;
+  for (int i = 0; i < n; ++i) {
+    double kp = 0.0, rows = 3.0 * P.n_v + (double)P.n_chol;
+    for (int k = 0; k < n; ++k) {
+      const int Q = P.pairid[(size_t)i * n + k];
+      if (Q < 0) continue;
+      const double d = (double)(P.h_dom_off[Q + 1] - P.h_dom_off[Q]);
+      kp += (double)up((int64_t)d, 8);
+      rows += d;
+    }
+    vals += (kp + 16.0) * rows;
+  }
+  const double np = (double)tri(P.n_v);
+  vals += 2.0 * np * (double)up(P.n_pairs, 16) + 2.0 * np * P.n_pairs;  // XT+-, H+-
+  vals += (double)n * n * P.n_v * (n + 1);
+  size_t freeb = 0, totalb = 0;
+  if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) return false;
+  // FP64 and one split copy, the K-split partials, and room for the rest of
+  // the plan (the ladder's buffers above all)
+  const double need = 12.0 * vals + 8.0 * 8.0 * (double)P.sum_d2;
+  return need <= 72.0e9 && need + 160.0e9 <= (double)freeb + 0.0 && (double)P.n_chol * P.n_v < 2.0e9;
+}
+
+void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st) {
+  auto& Z = P.pp;
+  const int n = P.n_int, nv = P.n_v, np_w = P.n_pairs;
+  Z.h_koff.assign((size_t)n * n, -1);
+  Z.h_ld.assign(n, 0);
+  Z.h_poff.assign(n, 0);
+  Z.h_lpoff.assign(n, 0);
+  Z.h_jpoff.assign((size_t)n * n, 0);
+  Z.n_panel = Z.n_jp = Z.n_lp = 0;
+  for (int i = 0; i < n; ++i) {
+    int64_t w = 0;
+    for (int k = 0; k < n; ++k) {
+      const int Q = P.pairid[(size_t)i * n + k];
+      if (Q < 0) continue;
+      Z.h_koff[(size_t)i * n + k] = (int32_t)w;
+      w += up(P.h_dom_off[Q + 1] - P.h_dom_off[Q], 8);
+    }
+    Z.h_ld[i] = std::max<int64_t>(up(w, 16), 16);
+    Z.h_poff[i] = Z.n_panel;
+    Z.n_panel += nv * Z.h_ld[i];
+    Z.h_lpoff[i] = Z.n_lp;
+    Z.n_lp += P.n_chol * Z.h_ld[i];
+    for (int j = 0; j < n; ++j) {
+      const int Q = P.pairid[(size_t)i * n + j];
+      if (Q < 0) continue;
+      Z.h_jpoff[(size_t)i * n + j] = Z.n_jp;
+      Z.n_jp += (P.h_dom_off[Q + 1] - P.h_dom_off[Q]) * Z.h_ld[i];
+    }
+  }
+  upload(Z.koff, Z.h_koff, st);
+  upload(Z.ld, Z.h_ld, st);
+  upload(Z.poff, Z.h_poff, st);
+  upload(Z.lpoff, Z.h_lpoff, st);
+  upload(Z.jpoff, Z.h_jpoff, st);
+  upload(Z.pairid, P.pairid, st);
+  Z.np = tri(nv);
+  Z.nm = tri(nv - 1);
+  Z.ldw = up(np_w, 16);
+  Z.ldu = up(P.n_chol, 16);
+  std::vector<int32_t> colm(np_w, -1);
+  Z.ncm = 0;
+  for (int Q = 0; Q < np_w; ++Q)
+    if (P.h_pairs[2 * Q] != P.h_pairs[2 * Q + 1]) colm[Q] = Z.ncm++;
+  upload(Z.colm, colm, st);
+  // 4-internal coefficients (o4[((k n + i) n + l) n + j] = (ki|lj))
+  std::vector<double> hp((size_t)np_w * Z.ldw, 0.0), hm((size_t)std::max(Z.ncm, 1) * Z.ldw, 0.0);
+  for (int X = 0; X < np_w; ++X) {
+    const size_t i = P.h_pairs[2 * X], j = P.h_pairs[2 * X + 1];
+    for (int Q = 0; Q < np_w; ++Q) {
+      const size_t k = P.h_pairs[2 * Q], l = P.h_pairs[2 * Q + 1];
+      const double a = o4[((k * n + i) * n + l) * n + j], b = k != l ? o4[((l * n + i) * n + k) * n + j] : 0.0;
+      hp[(size_t)X * Z.ldw + Q] = a + b;
+      if (colm[X] >= 0 && k != l) hm[(size_t)colm[X] * Z.ldw + Q] = a - b;
+    }
+  }
+  upload(Z.holeP, hp, st);
+  upload(Z.holeM, hm, st);
+  Z.Hp.alloc((size_t)np_w * Z.np * 8);
+  Z.Hm.alloc((size_t)std::max(Z.ncm, 1) * std::max<int64_t>(Z.nm, 1) * 8);
+  // 3-internal singles factors
+  Z.nk = (int)up(n, 2);
+  Z.O3T.alloc((size_t)n * n * nv * Z.nk * 8);
+  hipLaunchKernelGGL(o3t_kernel, dim3((unsigned)(n * n)), dim3(256), 0, st, P.O3.as<double>(), n, nv, Z.nk,
+                     Z.O3T.as<double>());
+  Z.sTp.alloc((size_t)nv * Z.nk * 8);
+  // FP64 operands
+  auto& F = Z.f64;
+  for (DevBuf* b : {&F.CR, &F.CC, &F.CT}) zero(*b, (size_t)Z.n_panel * 8, st);
+  zero(F.JP, (size_t)Z.n_jp * 8, st);
+  zero(F.LP, (size_t)Z.n_lp * 8, st);
+  zero(F.U, (size_t)n * nv * Z.ldu * 8, st);
+  zero(F.LovT, (size_t)n * nv * Z.ldu * 8, st);
+  zero(F.XTp, (size_t)Z.np * Z.ldw * 8, st);
+  zero(F.XTm, (size_t)std::max<int64_t>(Z.nm, 1) * Z.ldw * 8, st);
+  const PanelTab K = ptab(P);
+  hipLaunchKernelGGL(jp_kernel<false>, dim3(n, n * n), dim3(256), 0, st, P.tab, K, P.Jvv.as<double>(), F.JP.p, nullptr, 0);
+  hipLaunchKernelGGL(lp_kernel<false>, dim3((unsigned)P.n_chol, n), dim3(256), 0, st, P.tab, K, P.Lov.as<double>(),
+                     F.LP.p, nullptr, 0);
+  // LovT[(i,a)][J] = Lov[J][(i,a)]
+  hipLaunchKernelGGL(u_kernel<false>, dim3((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n), dim3(256), 0, st,
+                     nullptr, P.Lov.as<double>(), nv, P.n_chol, (int64_t)nv, (int64_t)n * nv, F.LovT.p, Z.ldu, nullptr, 0);
+  TCI_HIP(hipGetLastError());
+  panels_programs(P, false, 0, 1, st);
+}
+
+// Split copies of the constant operands (scale slot 0) and zeroed panels.
+void panels_build_split(tci_plan& P, hipStream_t st) {
+  auto& Z = P.pp;
+  auto& F = Z.s16;
+  const int n = P.n_int, nv = P.n_v;
+  const int f16 = P.mx.prec == TCI_SIGMA_FP16X3 ? 1 : 0;
+  const float* s0 = P.mx.scales.as<float>();
+  for (DevBuf* b : {&F.CR, &F.CC, &F.CT}) zero(*b, (size_t)Z.n_panel * 4, st);
+  zero(F.JP, (size_t)Z.n_jp * 4, st);
+  zero(F.LP, (size_t)Z.n_lp * 4, st);
+  zero(F.U, (size_t)n * nv * Z.ldu * 4, st);
+  zero(F.LovT, (size_t)n * nv * Z.ldu * 4, st);
+  zero(F.XTp, (size_t)Z.np * Z.ldw * 4, st);
+  zero(F.XTm, (size_t)std::max<int64_t>(Z.nm, 1) * Z.ldw * 4, st);
+  zero(F.hP, (size_t)P.n_pairs * Z.ldw * 4, st);
+  zero(F.hM, (size_t)std::max(Z.ncm, 1) * Z.ldw * 4, st);
+  const PanelTab K = ptab(P);
+  hipLaunchKernelGGL(jp_kernel<true>, dim3(n, n * n), dim3(256), 0, st, P.tab, K, P.Jvv.as<double>(), F.JP.p, s0, f16);
+  hipLaunchKernelGGL(lp_kernel<true>, dim3((unsigned)P.n_chol, n), dim3(256), 0, st, P.tab, K, P.Lov.as<double>(),
+                     F.LP.p, s0, f16);
+  hipLaunchKernelGGL(u_kernel<true>, dim3((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n), dim3(256), 0, st,
+                     nullptr, P.Lov.as<double>(), nv, P.n_chol, (int64_t)nv, (int64_t)n * nv, F.LovT.p, Z.ldu, s0, f16);
+  hipLaunchKernelGGL(split_matrix_kernel, dim3(gsz(P.n_pairs * Z.ldw / 8)), dim3(256), 0, st, Z.holeP.as<double>(),
+                     (int64_t)P.n_pairs, Z.ldw, Z.ldw, F.hP.p, Z.ldw, s0, f16);
+  hipLaunchKernelGGL(split_matrix_kernel, dim3(gsz(std::max(Z.ncm, 1) * Z.ldw / 8)), dim3(256), 0, st,
+                     Z.holeM.as<double>(), (int64_t)std::max(Z.ncm, 1), Z.ldw, Z.ldw, F.hM.p, Z.ldw, s0, f16);
+  TCI_HIP(hipGetLastError());
+  P.mx.bytes += 0;
+  for (DevBuf* b : {&F.CR, &F.CC, &F.CT, &F.JP, &F.LP, &F.U, &F.LovT, &F.XTp, &F.XTm, &F.hP, &F.hM})
+    P.mx.bytes += (int64_t)b->bytes;
+}
+
+// Programs of one element type: W per internal orbital, the 4-internal product
+// over packed pairs, and the pair products with `mode` (shape_of) and `ks`
+// K-splits; for a split type also the FP64 3-internal products.
+void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st) {
+  auto& Z = P.pp;
+  auto& F = split ? Z.s16 : Z.f64;
+  const int n = P.n_int, nv = P.n_v, es = split ? 4 : 8;
+  auto at = [&](const DevBuf& b, int64_t values) { return static_cast<const char*>(b.p) + values * es; };
+  F.W.clear();
+  F.W.split = split;
+  F.hole.clear();
+  F.hole.split = split;
+  // shapes of the side products: large tiles when they fill the chip
+  auto fill = [](int64_t m, int64_t nn, int64_t cnt, int t) { return cdiv(m, t) * cdiv(nn, t) * cnt; };
+  F.W.shape = fill(P.n_chol, nv, n, 128) >= 512 ? N128 : fill(P.n_chol, nv, n, 64) >= 256 ? N64 : N32K4;
+  F.hole.shape = fill(P.n_pairs, Z.np, 2, 128) >= 512 ? N128 : fill(P.n_pairs, Z.np, 2, 64) >= 256 ? N64 : N32K4;
+  for (int i = 0; i < n; ++i) {
+    F.W.add(P.W.as<double>() + (int64_t)i * P.n_chol * nv, nv, (int)P.n_chol, nv,
+            {nseg(at(F.LP, Z.h_lpoff[i]), Z.h_ld[i], at(F.CT, Z.h_poff[i]), Z.h_ld[i], Z.h_ld[i], es)}, false,
+            Blocking(), split ? 12 : -1);
+  }
+  F.W.upload_tables(st);
+  const void* hP = split ? F.hP.p : Z.holeP.p;
+  const void* hM = split ? F.hM.p : Z.holeM.p;
+  F.hole.add(Z.Hp.as<double>(), Z.np, P.n_pairs, (int)Z.np, {nseg(hP, Z.ldw, F.XTp.p, Z.ldw, Z.ldw, es)}, false,
+             Blocking(), split ? 5 : -1);
+  if (Z.ncm > 0 && Z.nm > 0)
+    F.hole.add(Z.Hm.as<double>(), Z.nm, Z.ncm, (int)Z.nm, {nseg(hM, Z.ldw, F.XTm.p, Z.ldw, Z.ldw, es)}, false,
+               Blocking(), split ? 5 : -1);
+  F.hole.upload_tables(st);
+  // pair products
+  F.ks = ks;
+  F.pair.clear();
+  F.pair.resize(4);
+  for (int s = 0; s < 4; ++s) {
+    F.pair[s].split = split;
+    F.pair[s].shape = s;
+  }
+  const int slots = ks + (split ? 1 : 0);
+  if (Z.Rp.bytes < (size_t)slots * P.sum_d2 * 8) Z.Rp.alloc((size_t)slots * P.sum_d2 * 8);
+  Z.rank.clear();
+  Z.rank.shape = P.dmax <= 64 ? N64 : N128;
+  std::vector<int> order(P.n_pairs);
+  for (int Q = 0; Q < P.n_pairs; ++Q) order[Q] = Q;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return P.h_dom_off[a + 1] - P.h_dom_off[a] > P.h_dom_off[b + 1] - P.h_dom_off[b];
+  });
+  for (int Q : order) {
+    const int i = P.h_pairs[2 * Q], j = P.h_pairs[2 * Q + 1];
+    const int d = (int)(P.h_dom_off[Q + 1] - P.h_dom_off[Q]);
+    const int32_t* D = P.dom_idx.as<int32_t>() + P.h_dom_off[Q];
+    const int64_t li = Z.h_ld[i], lj = Z.h_ld[j];
+    const char *CRi = at(F.CR, Z.h_poff[i]), *CRj = at(F.CR, Z.h_poff[j]), *CCi = at(F.CC, Z.h_poff[i]),
+               *CCj = at(F.CC, Z.h_poff[j]);
+    const char *Jij = at(F.JP, Z.h_jpoff[(size_t)i * n + j]), *Jji = at(F.JP, Z.h_jpoff[(size_t)j * n + i]);
+    const char *Ui = at(F.U, (int64_t)i * nv * Z.ldu), *Uj = at(F.U, (int64_t)j * nv * Z.ldu);
+    const char *Li = at(F.LovT, (int64_t)i * nv * Z.ldu), *Lj = at(F.LovT, (int64_t)j * nv * Z.ldu);
+    std::vector<NSeg> sg = {nseg(CRi, li, Jij, li, li, es, D, nullptr), nseg(Jij, li, CCi, li, li, es, nullptr, D),
+                            nseg(Jji, lj, CRj, lj, lj, es, nullptr, D), nseg(CCj, lj, Jji, lj, lj, es, D, nullptr),
+                            nseg(Ui, Z.ldu, Lj, Z.ldu, Z.ldu, es, D, D), nseg(Li, Z.ldu, Uj, Z.ldu, Z.ldu, es, D, D)};
+    const double* Oij = Z.O3T.as<double>() + ((int64_t)i * n + j) * nv * Z.nk;
+    const double* Oji = Z.O3T.as<double>() + ((int64_t)j * n + i) * nv * Z.nk;
+    const NSeg r1 = nseg(Z.sTp.p, Z.nk, Oij, Z.nk, Z.nk, 8, D, D), r2 = nseg(Oji, Z.nk, Z.sTp.p, Z.nk, Z.nk, 8, D, D);
+    if (split) {
+      Z.rank.add(Z.Rp.as<double>() + (int64_t)ks * P.sum_d2 + P.h_cd_off[Q], d, d, d, {r1, r2}, false);
+    } else {
+      sg.push_back(r1);
+      sg.push_back(r2);
+    }
+    int64_t tot = 0;
+    for (const NSeg& s : sg) tot += s.kbytes;
+    NProgram& g = F.pair[shape_of(mode, d)];
+    for (int s = 0; s < ks; ++s) {
+      const int64_t b0 = (tot * s / ks) & ~(int64_t)127, b1 = s + 1 == ks ? tot : (tot * (s + 1) / ks) & ~(int64_t)127;
+      std::vector<NSeg> part;
+      int64_t pos = 0;
+      for (const NSeg& q : sg) {
+        const int64_t u = std::max(b0, pos), v = std::min(b1, pos + q.kbytes);
+        if (u < v) {
+          NSeg c = q;
+          c.A = static_cast<const char*>(q.A) + (u - pos);
+          c.B = static_cast<const char*>(q.B) + (v > u ? u - pos : 0);
+          c.kbytes = v - u;
+          part.push_back(c);
+        }
+        pos += q.kbytes;
+      }
+      g.add(Z.Rp.as<double>() + (int64_t)s * P.sum_d2 + P.h_cd_off[Q], d, d, d, part, false, Blocking(),
+            split ? 5 : -1);
+    }
+  }
+  for (auto& g : F.pair) g.upload_tables(st);
+  if (split) Z.rank.upload_tables(st);
+}
+
+// Times tilings and K-splits of the pair products and keeps the fastest.
+void panels_tune(tci_plan& P, int precision, hipStream_t st) {
+  const bool split = precision != TCI_SIGMA_FP64;
+  auto& Z = P.pp;
+  auto& F = split ? Z.s16 : Z.f64;
+  const float* sc = P.mx.scales.as<float>();
+  // split types keep an FP32 chain no longer than about a quarter of the
+  // contraction (the partial sums meet in FP64)
+  const int kmin = split ? 4 : 1;
+  if (!autotune_enabled()) {
+    panels_programs(P, split, 0, kmin, st);
+    return;
+  }
+  if (split && Z.tuned_mode >= 0) {  // tuned for the other split precision: same tiles, same sums
+    panels_programs(P, split, Z.tuned_mode, Z.tuned_ks, st);
+    for (auto& g : F.pair) g.remap = Z.tuned_order;
+    return;
+  }
+  static const char* mname[4] = {"by size", "128", "64", "32k4"};
+  double tiles128 = 0.0;
+  for (int Q = 0; Q < P.n_pairs; ++Q) {
+    const int64_t c = cdiv(P.h_dom_off[Q + 1] - P.h_dom_off[Q], 128);
+    tiles128 += (double)(c * c);
+  }
+  std::string log = std::string(split ? "split" : "fp64") + " pair panels:";
+  double best = 1e300;
+  int bm = 0, bk = kmin, bo = 0;
+  for (int mode = 0; mode < 4; ++mode) {
+    if (mode == 3 && tiles128 > 256) continue;  // enough tiles without K-groups
+    if (mode == 2 && tiles128 > 4096) continue;
+    for (int ks : {1, 2, 4, 8}) {
+      if (ks < kmin || (ks > kmin && tiles128 * ks > 8192)) continue;
+      panels_programs(P, split, mode, ks, st);
+      for (int o = 0; o < (xcd_remap_forced() ? 1 : 2); ++o) {
+        for (auto& g : F.pair) g.remap = o;
+        const double ms = time_ms(st, 2, [&] {
+          for (const auto& g : F.pair) g.launch(precision, st, 0, sc);
+        });
+        log += std::string(" ") + mname[mode] + "/" + std::to_string(ks) + (o ? "x:" : ":") + fmt_ms(ms);
+        if (ms < best * 0.98) {
+          best = ms;
+          bm = mode;
+          bk = ks;
+          bo = o;
+        }
+      }
+    }
+  }
+  panels_programs(P, split, bm, bk, st);
+  for (auto& g : F.pair) g.remap = bo;
+  if (split) {
+    Z.tuned_mode = bm;
+    Z.tuned_ks = bk;
+    Z.tuned_order = bo;
+  }
+  P.tuning += log + " -> " + mname[bm] + "/" + std::to_string(bk) + (bo ? "x" : "") + "\n";
+  TCI_HIP(hipStreamSynchronize(st));
+}
+
+// Pair terms of one sigma into the K-split partials and H+-; needs C, s and Y.
+void panels_terms(tci_plan& P, int precision, hipStream_t st) {
+  auto& Z = P.pp;
+  const bool split = precision != TCI_SIGMA_FP64;
+  auto& F = split ? Z.s16 : Z.f64;
+  const int n = P.n_int, nv = P.n_v;
+  const int f16 = precision == TCI_SIGMA_FP16X3 ? 1 : 0;
+  const std::string pn = precision == TCI_SIGMA_FP64 ? "fp64" : (f16 ? "fp16x3" : "bf16x3");
+  float* sc = split ? P.mx.scales.as<float>() : nullptr;
+  unsigned* mx = f16 ? P.mx.maxbits.as<unsigned>() : nullptr;
+  const PanelTab K = ptab(P);
+  const int nt = (P.dmax + 31) / 32;
+  auto run = [&](const std::string& role, const NProgram& g, int prec) {
+    if (!g.tasks.empty()) P.kt_run(pn + " " + role, g, precision, st, [&] { g.launch(prec, st, 0, sc); });
+  };
+  auto panels = [&](int what) {
+    const dim3 g(nt * nt, P.n_pairs);
+    if (split)
+      hipLaunchKernelGGL(panels_kernel<true>, g, dim3(256), 0, st, P.tab, K, P.C.as<double>(), F.CR.p, F.CC.p, F.CT.p,
+                         sc + 6, sc + (f16 ? 11 : 6), f16, what);
+    else
+      hipLaunchKernelGGL(panels_kernel<false>, g, dim3(256), 0, st, P.tab, K, P.C.as<double>(), F.CR.p, F.CC.p, F.CT.p,
+                         nullptr, nullptr, 0, 3);
+  };
+  int e0 = P.kt_begin(st);
+  if (f16) hipLaunchKernelGGL(panel_scales_kernel, dim3(1), dim3(64), 0, st, 0, mx, sc);
+  panels(f16 ? 2 : 3);  // fp16x3: the scale of CR and CC waits for max|U|
+  hipLaunchKernelGGL(st_kernel, dim3(gsz((int64_t)nv * Z.nk)), dim3(256), 0, st, P.s.as<double>(), n, nv, Z.nk,
+                     Z.sTp.as<double>());
+  TCI_HIP(hipGetLastError());
+  P.kt_end(e0, pn + " pair panels", 0.0, precision, st);
+  run("pair product W", F.W, precision);
+  e0 = P.kt_begin(st);
+  if (f16) {
+    hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(64), 0, st, mx + 1);
+    hipLaunchKernelGGL(u_absmax_kernel, dim3(gsz((int64_t)n * nv * P.n_chol, 1024)), dim3(256), 0, st,
+                       P.Y.as<double>(), P.W.as<double>(), (int64_t)n * nv * P.n_chol, mx + 1);
+    hipLaunchKernelGGL(panel_scales_kernel, dim3(1), dim3(64), 0, st, 1, mx, sc);
+    panels(1);
+  }
+  const dim3 gu((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n);
+  const dim3 gx((unsigned)nv, (unsigned)cdiv(nv, 32), (unsigned)cdiv(P.n_pairs, 32));
+  const int64_t wi = P.n_chol * nv;
+  if (split) {
+    hipLaunchKernelGGL(u_kernel<true>, gu, dim3(256), 0, st, P.Y.as<double>(), P.W.as<double>(), nv, P.n_chol, wi,
+                       (int64_t)nv, F.U.p, Z.ldu, sc + 6, f16);
+    hipLaunchKernelGGL(xt_kernel<true>, gx, dim3(256), 0, st, P.tab, P.pos.as<int32_t>(), P.C.as<double>(), F.XTp.p,
+                       F.XTm.p, Z.ldw, sc + 6, f16);
+  } else {
+    hipLaunchKernelGGL(u_kernel<false>, gu, dim3(256), 0, st, P.Y.as<double>(), P.W.as<double>(), nv, P.n_chol, wi,
+                       (int64_t)nv, F.U.p, Z.ldu, nullptr, 0);
+    hipLaunchKernelGGL(xt_kernel<false>, gx, dim3(256), 0, st, P.tab, P.pos.as<int32_t>(), P.C.as<double>(), F.XTp.p,
+                       F.XTm.p, Z.ldw, nullptr, 0);
+  }
+  TCI_HIP(hipGetLastError());
+  P.kt_end(e0, pn + " pair panels", 0.0, precision, st);
+  for (const auto& g : F.pair) run("pair products", g, precision);
+  if (split && !Z.rank.tasks.empty())
+    P.kt_run(pn + " 3-internal products", Z.rank, precision, st, [&] { Z.rank.launch(TCI_SIGMA_FP64, st); });
+  run("4-internal product", F.hole, precision);
+}
+
+// sigma from the pair terms' partials, the ladder (packed S+- when `packed`,
+// otherwise R) and the singles
+void panels_pack(tci_plan& P, int precision, bool packed, bool use_r, const double* x, const IoSlot* io, int flags,
+                 double* y, hipStream_t st) {
+  auto& Z = P.pp;
+  const bool split = precision != TCI_SIGMA_FP64;
+  PackSrc S{};
+  S.Rp = Z.Rp.as<double>();
+  S.rstride = P.sum_d2;
+  S.nrp = (split ? Z.s16.ks : Z.f64.ks) + (split ? 1 : 0);
+  S.R = use_r ? P.R.as<double>() : nullptr;
+  S.np = Z.np;
+  S.nm = Z.nm;
+  if (packed) {
+    S.nsp = split ? P.vv.ksx : P.vv.ks;
+    S.Sp = P.vv.Sp.as<double>();
+    S.Sm = P.vv.Sm.as<double>();
+    S.sp_part = (int64_t)P.n_pairs * Z.np;
+    S.sm_part = (int64_t)std::max(Z.ncm, 1) * Z.nm;
+  }
+  S.Hp = Z.Hp.as<double>();
+  S.Hm = Z.Hm.as<double>();
+  S.colm = Z.colm.as<int32_t>();
+  S.Kov = P.Kov.as<double>();
+  const int nt = (P.dmax + 31) / 32;
+  hipLaunchKernelGGL(pack_panels_kernel, dim3((unsigned)std::max<int64_t>(nt * (nt + 1) / 2, 4), P.n_pairs + 1),
+                     dim3(256), 0, st, P.tab, S, x, P.g.as<double>(), P.sig0.as<double>(), P.e_ref, flags, y, io);
+  TCI_HIP(hipGetLastError());
+}
+
+int64_t panels_device_bytes(const tci_plan& P) {
+  const auto& Z = P.pp;
+  int64_t b = 0;
+  for (const auto* F : {&Z.f64, &Z.s16})
+    for (const DevBuf* x : {&F->CR, &F->CC, &F->CT, &F->JP, &F->LP, &F->U, &F->LovT, &F->XTp, &F->XTm, &F->hP, &F->hM})
+      b += (int64_t)x->bytes;
+  for (const DevBuf* x : {&Z.koff, &Z.ld, &Z.poff, &Z.jpoff, &Z.lpoff, &Z.pairid, &Z.colm, &Z.holeP, &Z.holeM, &Z.Hp,
+                          &Z.Hm, &Z.O3T, &Z.sTp, &Z.Rp})
+    b += (int64_t)x->bytes;
+  return b;
+}
+
+}  // namespace tci

@@ -6,6 +6,7 @@
 #include "common.hpp"
 #include "ladder.hpp"
 #include "ladder_fused.hpp"
+#include "ngemm.hpp"
 #include "terms.hpp"
 
 struct tci_plan {
@@ -167,19 +168,13 @@ struct tci_plan {
     tci::DevBuf Vpx, Vmx;           // split rows of V+-
     tci::DevBuf Xp, Xm, Xpx, Xmx;   // X+- (FP64 rows, split rows)
     tci::DevBuf Sp, Sm;             // S+- partials of the K-splits
-    // split product run transposed, S^T = V X^T (pairs x walks, the walks as
-    // the tiles' N side), then transposed back into Sp / Sm
-    bool xtrans = false;
-    tci::DevBuf STp, STm;
     tci::DevBuf colm;               // [n_pairs] row of the walk in X- or -1
     int ks = 1, ksx = 1;            // K-splits of the FP64 / split products
-    tci::GemmProgram g64, gx;       // the products (both parts in one launch)
+    tci::NProgram g64, gx;          // the products (both parts in one launch)
     // split schedule chosen on the first split preparation (kept for both
-    // split precisions, so a plan's split sigma does not change): tile,
-    // tile_n, dma (wave count for 256 tiles), K-split, order; use: -1 not yet
-    // decided, 0 Cholesky-direct, 1 resident
-    int split_tile = 0, split_tile_n = 0, split_dma = 0, split_ks = 1, split_order = 0, split_use = -1;
-    bool split_trans = false;
+    // split precisions, so a plan's split sigma does not change): tile shape,
+    // K-split, order; use: -1 not yet decided, 0 Cholesky-direct, 1 resident
+    int split_shape = -1, split_ks = 1, split_order = 0, split_use = -1;
   } vv;
   tci::PairTab tab{};
   // accounting
@@ -228,8 +223,8 @@ struct tci_plan {
   void kt_end(int e0, const std::string& name, double flops, int prec, hipStream_t st);
   void kt_collect();
   // time one program launch under its role name and the program's algorithmic flops
-  template <class F>
-  void kt_run(const std::string& role, const tci::GemmProgram& g, int prec, hipStream_t st, F&& launch) {
+  template <class G, class F>
+  void kt_run(const std::string& role, const G& g, int prec, hipStream_t st, F&& launch) {
     const int e0 = kt_begin(st);
     launch();
     if (e0 >= 0) kt_end(e0, role + " " + g.kernel_name(), g.alg_flops, prec, st);
@@ -276,8 +271,8 @@ void launch_split_scales(int mode, const double* x, int64_t n, unsigned* mx, int
 bool vv_fits(const tci_plan& P, double* bytes_out);
 double vv_flops(const tci_plan& P);
 void vv_build(tci_plan& P, hipStream_t st);
-void vv_set_schedule(tci_plan& P, int precision, int tile, int tile_n, int dma, int ks, hipStream_t st,
-                     bool trans = false);
+// shape: an NShape of ngemm.hpp
+void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t st);
 void vv_prepare_split(tci_plan& P, int precision, hipStream_t st);
 void vv_ladder(tci_plan& P, int precision, hipStream_t st);
 double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log);
