@@ -167,7 +167,6 @@ __device__ __forceinline__ float p2scale(float m) { return m > 0.f ? ldexpf(1.f,
 
 // Scales of the scaled-FP16 split (indices documented at MixedLadder::scales).
 //   mode 0: constants from mx[2]     mode 1: ladder from mx[0] = max|C|
-//   mode 2: pair products from mx[0], mx[1] = max|Yt|
 __global__ void set_scales_kernel(int mode, const unsigned* __restrict__ mx, float* __restrict__ sc, float dmax) {
   if (threadIdx.x != 0) return;
   if (mode == 0) {
@@ -180,10 +179,6 @@ __global__ void set_scales_kernel(int mode, const unsigned* __restrict__ mx, flo
     sc[2] = p2scale(dmax * sc[8] * mc);  // |T| <= d max|L| max|C|
     sc[3] = sc[2] / (sc[0] * sc[1]);
     sc[4] = 1.f / (sc[2] * sc[0]);
-  } else {
-    const float mv = fmaxf(3.f * __uint_as_float(mx[0]), __uint_as_float(mx[1]));  // |Ct| <= 3 max|C|
-    sc[6] = p2scale(mv);
-    sc[5] = 1.f / (sc[0] * sc[6]);
   }
 }
 
@@ -217,7 +212,7 @@ Seg xseg(const Op& A, const Op& B, int K) {
 void launch_split_scales(int mode, const double* x, int64_t n, unsigned* mx, int slot, float* sc, float dmax,
                          hipStream_t st) {
   hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, st, mx + slot, 1);
-  if (n > 0) hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(n, 8192)), dim3(256), 0, st, x, n, mx + slot);
+  if (n > 0) hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(n, 1024)), dim3(256), 0, st, x, n, mx + slot);
   hipLaunchKernelGGL(set_scales_kernel, dim3(1), dim3(64), 0, st, mode, mx, sc, dmax);
   TCI_HIP(hipGetLastError());
 }
@@ -281,23 +276,20 @@ void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
   if (f16) {
     unsigned* mx = M.maxbits.as<unsigned>();
     const int64_t nvv = P.n_chol * (int64_t)P.n_v * P.n_v, nov = P.n_chol * (int64_t)P.n_int * P.n_v;
-    const int64_t niv = (int64_t)P.n_int * P.n_v;
     if (P.lvv_f32)
-      hipLaunchKernelGGL(absmax_kernel<float>, dim3(blocks_for(nvv, 8192)), dim3(256), 0, st, P.Lvv.as<float>(), nvv,
+      hipLaunchKernelGGL(absmax_kernel<float>, dim3(blocks_for(nvv, 1024)), dim3(256), 0, st, P.Lvv.as<float>(), nvv,
                          mx + 2);
     else
-      hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(nvv, 8192)), dim3(256), 0, st, P.Lvv.as<double>(), nvv,
+      hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(nvv, 1024)), dim3(256), 0, st, P.Lvv.as<double>(), nvv,
                          mx + 2);
-    if (P.dense_pairs) {
-      hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(niv * niv, 8192)), dim3(256), 0, st,
-                         P.Kov.as<double>(), niv * niv, mx + 2);
-      hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(niv * niv, 8192)), dim3(256), 0, st,
-                         P.Jbig.as<double>(), niv * niv, mx + 2);
-      hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(nov, 8192)), dim3(256), 0, st, P.Lov.as<double>(),
-                         nov, mx + 2);
-      const int64_t nh = 2 * (int64_t)P.n_pairs * P.n_pairs;  // 4-internal coefficients
-      hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(nh, 8192)), dim3(256), 0, st, P.holeA.as<double>(),
-                         nh, mx + 2);
+    if (P.pp.on) {
+      auto amax = [&](const DevBuf& x, int64_t n) {
+        hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(n, 1024)), dim3(256), 0, st, x.as<double>(), n, mx + 2);
+      };
+      amax(P.Jvv, (int64_t)(P.Jvv.bytes / 8));
+      amax(P.Lov, nov);
+      amax(P.pp.holeP, (int64_t)(P.pp.holeP.bytes / 8));  // 4-internal coefficients
+      amax(P.pp.holeM, (int64_t)(P.pp.holeM.bytes / 8));
     }
     hipLaunchKernelGGL(set_scales_kernel, dim3(1), dim3(64), 0, st, 0, mx, sc, (float)P.dmax);
     TCI_HIP(hipGetLastError());
@@ -870,70 +862,9 @@ void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
     M.tuned_fused_target = bft;
     P.tuning += log + "\n";
   }
-  if (P.dense_pairs) {
-    const float* scl = M.scales.as<float>();
-    auto pair_programs = [&] {
-      std::vector<GemmProgram*> gs;
-      if (M.pairs_merged) gs = {&M.pairsUWx, &M.pairsx};
-      else gs = {&M.progUx, &M.ringZx, &M.ringZ3x, &M.progWx, &M.holeGx};
-      return gs;
-    };
-    auto run_pairs = [&] {
-      for (GemmProgram* g : pair_programs())
-        if (!g->tasks.empty()) g->launch_split(precision, st, 0, scl);
-    };
-    const char* te = std::getenv("TCI_PAIRS_TILE");
-    if (autotune_enabled() && !te) {
-      // tiles of the split pair products (128 x 128, or 256 x 256 on 32 x 32
-      // MFMAs with 4, 8 or 16 waves): Z, Z3 and the 4-internal product first,
-      // then U and W; then their tile order
-      std::string log = (precision == TCI_SIGMA_FP16X3 ? "fp16x3" : "bf16x3") + std::string(" pair products: tile");
-      static const char* cname[6] = {"128", "256w4", "256w8", "256w16", "128x192d2", "128d2"};
-      const int64_t bytes0 = M.bytes;  // each build counts its split copies again
-      auto trial = [&](int cz, int cu) {
-        M.bytes = bytes0;
-        dense_pairs_build_split(P, st, cz, cu);
-        return time_ms(st, 2, run_pairs);
-      };
-      double best = 1e300;
-      int bz = 0, bu = 0;
-      if (M.tuned_pairs_z >= 0) {  // tuned for the other split precision: same tiles, same sums
-        bz = M.tuned_pairs_z;
-        bu = M.tuned_pairs_uw;
-        log += " kept";
-        trial(bz, bu);
-      } else {
-        for (int cz = 0; cz < 6; ++cz) {
-          const double ms = trial(cz, 0);
-          log += std::string(" z") + cname[cz] + ":" + fmt_ms(ms);
-          if (ms < best * 0.98) {
-            best = ms;
-            bz = cz;
-          }
-        }
-        if (M.z_lowrank) {  // U and W go out as a launch of their own
-          for (int cu : {2, 4, 5}) {
-            const double ms = trial(bz, cu);
-            log += std::string(" uw") + cname[cu] + ":" + fmt_ms(ms);
-            if (ms < best * 0.98) {
-              best = ms;
-              bu = cu;
-            }
-          }
-        } else {
-          bu = bz;
-        }
-        if (!(M.z_lowrank && bu == 5)) trial(bz, bu);  // unless the last trial built the chosen tiles
-        M.tuned_pairs_z = bz;
-        M.tuned_pairs_uw = bu;
-      }
-      log += std::string(" -> z") + cname[bz] + " uw" + cname[bu] + "; order";
-      for (GemmProgram* g : pair_programs())
-        if (!g->tasks.empty()) log += " " + tune_block_order(*g, st, [&] { g->launch_split(precision, st, 0, scl); });
-      P.tuning += log + "\n";
-    } else {
-      dense_pairs_build_split(P, st);
-    }
+  if (P.pp.on) {
+    panels_build_split(P, st);
+    panels_tune(P, precision, st);
   }
   // ladder from the resident (ab|cd) block when the plan holds it: timed
   // against the split Cholesky-direct ladder above (kept when faster) unless
@@ -986,7 +917,7 @@ void mixed_ladder_run(tci_plan& P, int precision, hipStream_t st) {
   if (f16) {  // scale of C and of the intermediate from max|C|
     unsigned* mx = M.maxbits.as<unsigned>();
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, st, mx, 2);
-    hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(P.sum_d2, 8192)), dim3(256), 0, st, P.C.as<double>(),
+    hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(P.sum_d2, 1024)), dim3(256), 0, st, P.C.as<double>(),
                        P.sum_d2, mx);
     hipLaunchKernelGGL(set_scales_kernel, dim3(1), dim3(64), 0, st, 1, mx, sc, (float)P.dmax);
     TCI_HIP(hipGetLastError());
@@ -1037,7 +968,7 @@ void mixed_ladder_run(tci_plan& P, int precision, hipStream_t st) {
 void mixed_ladder(tci_plan& P, int precision, hipStream_t st) {
   mixed_prepare(P, precision, st);
   if (P.vv.split) {
-    vv_ladder(P, precision, st);
+    vv_ladder(P, precision, st, !P.pp.on);
     if (P.timing()) TCI_HIP(hipEventRecord(P.ev[3], st));
     return;
   }
@@ -1189,7 +1120,7 @@ void mixed_batch_prepare(tci_plan& P, int precision, int nvec, hipStream_t st) {
 void mixed_batch_absmax(tci_plan& P, bool first, hipStream_t st) {
   unsigned* mx = P.mx.maxbits.as<unsigned>();
   if (first) hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, st, mx, 2);
-  hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(P.sum_d2, 8192)), dim3(256), 0, st, P.C.as<double>(),
+  hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(P.sum_d2, 1024)), dim3(256), 0, st, P.C.as<double>(),
                      P.sum_d2, mx);
   TCI_HIP(hipGetLastError());
 }

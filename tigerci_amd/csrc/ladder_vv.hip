@@ -279,20 +279,15 @@ void build_products(tci_plan& P, NProgram& g, bool split, int shape, int ks, hip
   g.upload_tables(st);
 }
 
-void alloc_partials(tci_plan& P, int ks) {
-  tci_plan::VVLadder& V = P.vv;
-  const size_t need_p = (size_t)ks * P.n_pairs * V.np * 8, need_m = (size_t)ks * std::max(V.ncm, 1) * V.nm * 8;
-  if (V.Sp.bytes < need_p) V.Sp.alloc(need_p);
-  if (V.Sm.bytes < need_m) V.Sm.alloc(need_m);
-}
+constexpr int kMaxSplits = 4;  // K-splits of the products
 
 }  // namespace
 
 bool vv_fits(const tci_plan& P, double* bytes_out) {
   const int64_t n_v = P.n_v, np = tri(n_v), nm = tri(n_v - 1);
   const double v64 = 8.0 * ((double)np * np + (double)nm * nm);
-  // resident V (FP64 and one split copy), X and two K-split partials of S
-  const double need = 1.5 * v64 + 8.0 * 3.0 * (double)P.n_pairs * (np + nm);
+  // resident V (FP64 and one split copy), X and four K-split partials of S
+  const double need = 1.5 * v64 + 8.0 * 5.0 * (double)P.n_pairs * (np + nm);
   if (bytes_out) *bytes_out = need;
   size_t freeb = 0, totalb = 0;
   if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) return false;
@@ -362,6 +357,9 @@ void vv_build(tci_plan& P, hipStream_t st) {
   V.Xm.alloc((size_t)std::max(V.ncm, 1) * even(V.nm) * 8);
   launch_fill(V.Xp.as<double>(), (int64_t)(V.Xp.bytes / 8), 0.0, st);
   launch_fill(V.Xm.as<double>(), (int64_t)(V.Xm.bytes / 8), 0.0, st);
+  // partials for every schedule of both precisions: the programs keep their address
+  V.Sp.alloc((size_t)kMaxSplits * P.n_pairs * V.np * 8);
+  V.Sm.alloc((size_t)kMaxSplits * std::max(V.ncm, 1) * V.nm * 8);
   V.built = true;
   vv_set_schedule(P, TCI_SIGMA_FP64, N128, 1, st);
   TCI_HIP(hipStreamSynchronize(st));
@@ -371,8 +369,7 @@ void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t 
   tci_plan::VVLadder& V = P.vv;
   // every K-split range non-empty (at least 64 long), so every partial of S is written
   const int64_t kmin = V.ncm > 0 ? std::min(V.np, V.nm) : V.np;
-  ks = (int)std::max<int64_t>(1, std::min<int64_t>(ks, kmin / 64));
-  alloc_partials(P, ks);
+  ks = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(ks, kMaxSplits), kmin / 64));
   if (precision == TCI_SIGMA_FP64) {
     V.ks = ks;
     build_products(P, V.g64, false, shape, ks, st);
@@ -422,8 +419,9 @@ void vv_prepare_split(tci_plan& P, int precision, hipStream_t st) {
   TCI_HIP(hipStreamSynchronize(st));
 }
 
-// R = ladder of the unpacked C (overwrites R), FP64 or the prepared split precision.
-void vv_ladder(tci_plan& P, int precision, hipStream_t st) {
+// R = ladder of the unpacked C (overwrites R), FP64 or the prepared split
+// precision; without `gather` the result stays packed in S+-.
+void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool gather) {
   tci_plan::VVLadder& V = P.vv;
   const bool split = precision != TCI_SIGMA_FP64;
   TCI_REQUIRE(V.built && (!split || V.prec == precision), "resident (ab|cd) block not prepared for this precision");
@@ -449,6 +447,7 @@ void vv_ladder(tci_plan& P, int precision, hipStream_t st) {
   const int ks = split ? V.ksx : V.ks;  // K-splits change the launch (and its traffic), so they name it
   P.kt_run(pn + " ladder (ab|cd) product" + (ks > 1 ? " K-split " + std::to_string(ks) : std::string()), g,
            precision, st, [&] { g.launch(precision, st, 0, sc); });
+  if (!gather) return;
   e0 = P.kt_begin(st);
   hipLaunchKernelGGL(vv_gather_kernel, dim3(blocks((int64_t)P.dmax * P.dmax, 64), (unsigned)P.n_pairs), dim3(256), 0,
                      st, P.tab, V.Sp.as<double>(), (int64_t)P.n_pairs * V.np, V.np, V.Sm.as<double>(),
@@ -482,7 +481,7 @@ double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
       vv_set_schedule(P, precision, sh, ks, st);
       for (int o = 0; o < orders; ++o) {
         g.remap = o;
-        const double ms = time_ms(st, 2, [&] { vv_ladder(P, precision, st); });
+        const double ms = time_ms(st, 2, [&] { vv_ladder(P, precision, st, !P.pp.on); });
         log += " " + std::to_string(g.tm()) + "x" + std::to_string(g.tn()) + "/" + std::to_string(ks) + (o ? "x:" : ":") +
                fmt_ms(ms);
         if (ms < best * 0.98) {
@@ -504,7 +503,7 @@ double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
   log += " -> " + std::to_string(g.tm()) + "x" + std::to_string(g.tn()) + "/" + std::to_string(bk) + " order " +
          std::to_string(bo);
   TCI_HIP(hipStreamSynchronize(st));
-  return time_ms(st, 2, [&] { vv_ladder(P, precision, st); });
+  return time_ms(st, 2, [&] { vv_ladder(P, precision, st, !P.pp.on); });
 }
 
 int64_t vv_device_bytes(const tci_plan& P) {

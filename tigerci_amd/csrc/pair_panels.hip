@@ -55,6 +55,8 @@ __device__ __forceinline__ void untri32(int t, int& x, int& y) {  // t = x(x+1)/
 }
 inline int64_t up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 
+constexpr int kMaxKs = 8;  // K-splits of the pair products
+
 // Offsets are in values; a value is 8 bytes (FP64) or 4 (split rows).
 struct PanelTab {
   const int32_t* koff;   // [i n_int + k] -> column of block k in panel i, or -1
@@ -493,7 +495,7 @@ bool panels_choose(const tci_plan& P) {
   const char* env = std::getenv("TCI_DENSE_PAIRS");
   if (env && env[0] == '0') return false;
   const int n = P.n_int;
-  double vals = 0.0;
+  double vals = 0.0, kmax = 0.0;
   for (int i = 0; i < n; ++i) {
     double kp = 0.0, rows = 3.0 * P.n_v + (double)P.n_chol;
     for (int k = 0; k < n; ++k) {
@@ -504,16 +506,18 @@ bool panels_choose(const tci_plan& P) {
       rows += d;
     }
     vals += (kp + 16.0) * rows;
+    kmax = std::max(kmax, kp + 16.0);
   }
   const double np = (double)tri(P.n_v);
   vals += 2.0 * np * (double)up(P.n_pairs, 16) + 2.0 * np * P.n_pairs;  // XT+-, H+-
   vals += (double)n * n * P.n_v * (n + 1);
   size_t freeb = 0, totalb = 0;
   if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) return false;
-  // FP64 and one split copy, the K-split partials, and room for the rest of
-  // the plan (the ladder's buffers above all)
-  const double need = 12.0 * vals + 8.0 * 8.0 * (double)P.sum_d2;
-  return need <= 72.0e9 && need + 160.0e9 <= (double)freeb + 0.0 && (double)P.n_chol * P.n_v < 2.0e9;
+  // FP64 and one split copy and the K-split partials, with room left for the
+  // ladder; gathered rows are addressed by 32-bit byte offsets from a panel
+  const double need = 12.0 * vals + 8.0 * 9.0 * (double)P.sum_d2;
+  return need <= 72.0e9 && need + 64.0e9 <= (double)freeb && 8.0 * kmax * P.n_v < 4.0e9 &&
+         8.0 * ((double)P.n_chol + 16.0) * P.n_v < 4.0e9;
 }
 
 void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st) {
@@ -581,6 +585,9 @@ void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st) {
   hipLaunchKernelGGL(o3t_kernel, dim3((unsigned)(n * n)), dim3(256), 0, st, P.O3.as<double>(), n, nv, Z.nk,
                      Z.O3T.as<double>());
   Z.sTp.alloc((size_t)nv * Z.nk * 8);
+  // one buffer for every schedule of both element types: the programs keep its
+  // address (kMaxKs partials and the 3-internal products of a split sigma)
+  Z.Rp.alloc((size_t)(kMaxKs + 1) * P.sum_d2 * 8);
   // FP64 operands
   auto& F = Z.f64;
   for (DevBuf* b : {&F.CR, &F.CC, &F.CT}) zero(*b, (size_t)Z.n_panel * 8, st);
@@ -628,7 +635,6 @@ void panels_build_split(tci_plan& P, hipStream_t st) {
   hipLaunchKernelGGL(split_matrix_kernel, dim3(gsz(std::max(Z.ncm, 1) * Z.ldw / 8)), dim3(256), 0, st,
                      Z.holeM.as<double>(), (int64_t)std::max(Z.ncm, 1), Z.ldw, Z.ldw, F.hM.p, Z.ldw, s0, f16);
   TCI_HIP(hipGetLastError());
-  P.mx.bytes += 0;
   for (DevBuf* b : {&F.CR, &F.CC, &F.CT, &F.JP, &F.LP, &F.U, &F.LovT, &F.XTp, &F.XTm, &F.hP, &F.hM})
     P.mx.bytes += (int64_t)b->bytes;
 }
@@ -671,8 +677,7 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st) 
     F.pair[s].split = split;
     F.pair[s].shape = s;
   }
-  const int slots = ks + (split ? 1 : 0);
-  if (Z.Rp.bytes < (size_t)slots * P.sum_d2 * 8) Z.Rp.alloc((size_t)slots * P.sum_d2 * 8);
+  TCI_REQUIRE(ks >= 1 && ks <= kMaxKs, "K-splits of the pair products out of range");
   Z.rank.clear();
   Z.rank.shape = P.dmax <= 64 ? N64 : N128;
   std::vector<int> order(P.n_pairs);
@@ -714,7 +719,7 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st) 
         if (u < v) {
           NSeg c = q;
           c.A = static_cast<const char*>(q.A) + (u - pos);
-          c.B = static_cast<const char*>(q.B) + (v > u ? u - pos : 0);
+          c.B = static_cast<const char*>(q.B) + (u - pos);
           c.kbytes = v - u;
           part.push_back(c);
         }

@@ -416,21 +416,7 @@ void tci_plan::build(const tci_problem& p) {
     const double* b = X + h_cd_off[Q];
     return transposed ? op(b, 1, d, rm, cm) : op(b, d, 1, rm, cm);
   };
-  {
-    // flops of the per-walk gathered ring and 3-external products
-    double fg = 0.0;
-    for (int P = 0; P < n_pairs; ++P) {
-      const double d = dsz(P);
-      const int i = h_pairs[2 * P], j = h_pairs[2 * P + 1];
-      for (int k = 0; k < n_int; ++k) {
-        const int Q1 = pairid[(size_t)i * n_int + k], Q2 = pairid[(size_t)j * n_int + k];
-        if (Q1 >= 0) fg += 3.0 * 2.0 * d * d * dsz(Q1);
-        if (Q2 >= 0) fg += 3.0 * 2.0 * d * d * dsz(Q2);
-      }
-      fg += 2.0 * 2.0 * d * d * (double)n_chol + 2.0 * d * n_v * (double)n_chol;
-    }
-    dense_pairs = dense_pairs_choose(*this, fg);
-  }
+  pp.on = panels_choose(*this);
   ring.clear();
   ring.tile = 128;
   for (int P = 0; P < n_pairs; ++P) {
@@ -438,7 +424,7 @@ void tci_plan::build(const tci_problem& p) {
     const int d = dsz(P);
     const int32_t* DP = DL(P);
     std::vector<Seg> sg;
-    for (int k = 0; k < n_int && !dense_pairs; ++k) {
+    for (int k = 0; k < n_int && !pp.on; ++k) {
       const int Q1 = pairid[(size_t)i * n_int + k];
       if (Q1 >= 0) {  // Z^{ij}: Ct^{ik} K^{kj} - C^{ik} J^{kj} - J^{kj} C^{ik}
         const int dq = dsz(Q1);
@@ -459,12 +445,12 @@ void tci_plan::build(const tci_problem& p) {
         sg.push_back(seg(blk(Cp, Q2, tr, m, nullptr), Jop(k, i, DL(Q2), DP), dq, -1.0));
       }
     }
-    if (dense_pairs) continue;
-    // 3-external singles: X^{ij}_ab + X^{ji}_ba, X^{ij}_ab = sum_J Y[J][a][i] L^J_{jb}
+    if (pp.on) continue;
+    // 3-external singles: X^{ij}_ab + X^{ji}_ba, X^{ij}_ab = sum_J Y[i][J][a] L^J_{jb}
     const double* Yp = Y.as<double>();
     const double* Lo = Lov.as<double>();
-    sg.push_back(seg(op(Yp + i, n_int, niv, DP, nullptr), op(Lo + (int64_t)j * n_v, niv, 1, nullptr, DP), (int)n_chol, 1.0));
-    sg.push_back(seg(op(Lo + (int64_t)i * n_v, 1, niv, DP, nullptr), op(Yp + j, niv, n_int, nullptr, DP), (int)n_chol, 1.0));
+    sg.push_back(seg(op(Yp + (int64_t)i * n_chol * n_v, 1, n_v, DP, nullptr), op(Lo + (int64_t)j * n_v, niv, 1, nullptr, DP), (int)n_chol, 1.0));
+    sg.push_back(seg(op(Lo + (int64_t)i * n_v, 1, niv, DP, nullptr), op(Yp + (int64_t)j * n_chol * n_v, n_v, 1, nullptr, DP), (int)n_chol, 1.0));
     ring.add(R.as<double>() + h_cd_off[P], d, d, d, sg, true);
   }
   ring.upload_tables(st);
@@ -484,19 +470,32 @@ void tci_plan::build(const tci_problem& p) {
     }
     fockvv.upload_tables(st);
   }
-  if (dense_pairs) dense_pairs_build(*this, o4, st);
-  // Y[(J,a)][i] = sum_c L^J_ac s_i^c
-  // (a dense product: L^J rows are contiguous, and s is transposed into sT per sigma)
+  if (pp.on) panels_build(*this, o4, st);
+  // Y[i][J][a] = sum_c L^J_ac s_i^c: s rows against the rows (J, a) of L^J on
+  // the NT GEMM where those rows are 16-byte aligned FP64; otherwise L^J sT on
+  // the dense kernel, its columns i stored n_chol n_v apart
+  const bool nt_ok = !lvv_f32 && n_v % 2 == 0;
   progY.clear();
-  progY.dense = true;
-  progY.tile = 64;
-  progY.add(Y.as<double>(), n_int, (int)(n_chol * n_v), n_int,
-            {seg(op(Lvv.p, n_v, 1, nullptr, nullptr, lvv_f32), op(sT.as<double>(), n_int, 1), n_v, 1.0)}, false);
-  progY.upload_tables(st);
+  nprogY.clear();
+  if (nt_ok) {
+    nprogY.shape = N64;
+    nprogY.add(Y.as<double>(), n_chol * n_v, n_int, (int)(n_chol * n_v), {nseg(s.p, n_v, Lvv.p, n_v, n_v, 8)}, false);
+    nprogY.upload_tables(st);
+  } else {
+    Blocking by;
+    by.cdiv = 1;
+    by.cstride = n_chol * n_v;
+    progY.dense = true;
+    progY.tile = 64;
+    progY.add(Y.as<double>(), 1, (int)(n_chol * n_v), n_int,
+              {seg(op(Lvv.p, n_v, 1, nullptr, nullptr, lvv_f32), op(sT.as<double>(), n_int, 1), n_v, 1.0)}, false,
+              false, 0, by);
+    progY.upload_tables(st);
+  }
   // W[i][J][b] = sum_j sum_c Ct^{ij}[pos(b)][c] L^J_{j D[c]}
   progW.clear();
   progW.tile = 128;
-  for (int i = 0; i < n_int && !dense_pairs; ++i) {
+  for (int i = 0; i < n_int && !pp.on; ++i) {
     std::vector<Seg> sg;
     for (int j = 0; j < n_int; ++j) {
       const int Q = pairid[(size_t)i * n_int + j];
@@ -512,19 +511,30 @@ void tci_plan::build(const tci_problem& p) {
     progW.add(W.as<double>() + (int64_t)i * n_chol * n_v, n_v, (int)n_chol, n_v, sg, false);
   }
   progW.upload_tables(st);
-  // gW[s][i][a] = sum_{J in split s} sum_b W[i][J][b] L^J_ba (a dense product)
+  // gW[s][i][a] = sum_{J in split s} sum_b W[i][J][b] L^J_ab
   progGW.clear();
+  nprogGW.clear();
   progGW.dense = true;
   progGW.tile = 64;
+  nprogGW.shape = N64;
   for (int sp = 0; sp < n_split; ++sp) {
     const int64_t J0 = n_chol * sp / n_split, J1 = n_chol * (sp + 1) / n_split;
+    double* out = gW.as<double>() + (int64_t)sp * niv;
+    if (nt_ok) {
+      std::vector<NSeg> sg;
+      for (int64_t J = J0; J < J1; ++J)
+        sg.push_back(nseg(W.as<double>() + J * n_v, n_chol * n_v, Lvv.as<double>() + J * n_v * n_v, n_v, n_v, 8));
+      nprogGW.add(out, n_v, n_int, n_v, sg, false);
+      continue;
+    }
     const void* Lb = lvv_f32 ? (const void*)(Lvv.as<float>() + J0 * n_v * n_v) : (const void*)(Lvv.as<double>() + J0 * n_v * n_v);
-    progGW.add(gW.as<double>() + (int64_t)sp * niv, n_v, n_int, n_v,
+    progGW.add(out, n_v, n_int, n_v,
                {seg(op(W.as<double>() + J0 * n_v, n_chol * n_v, 1), op(Lb, n_v, 1, nullptr, nullptr, lvv_f32),
                     (int)((J1 - J0) * n_v), 1.0)},
                false);
   }
   progGW.upload_tables(st);
+  nprogGW.upload_tables(st);
   // gss = (2K - J) s runs as a GEMV (launch_gemv) inside every sigma
 
   // ---- ladder work items -------------------------------------------------------
@@ -602,14 +612,7 @@ void tci_plan::build(const tci_problem& p) {
     }
   }
 
-  // order of the dense pair products' tiles (plain, or XCD-contiguous in
-  // blocks of tiles that share operand panels in one XCD's L2)
-  if (dense_pairs && autotune_enabled()) {
-    std::string log = "fp64 pair products: order";
-    for (GemmProgram* g : {&ringZ, &ringZ3, &progU, &progWd, &holeG})
-      if (!g->tasks.empty()) log += " " + tune_block_order(*g, st, [&] { g->launch(st); });
-    tuning += log + "\n";
-  }
+  if (pp.on) panels_tune(*this, TCI_SIGMA_FP64, st);
 
   // ---- accounting ---------------------------------------------------------------
   flops_ladder = 0.0;
@@ -627,21 +630,19 @@ void tci_plan::build(const tci_problem& p) {
     f_ring += 2.0 * 2.0 * d * d * (double)n_chol;
   }
   bytes_ladder = bytes;
-  if (dense_pairs) {  // executed products: Z (two or three terms), U, Z3, W, the 4-internal GEMM
-    const double N = (double)niv, d2 = (double)n_v * n_v;
-    f_ring = (z_lowrank ? 4.0 * N * N * N + 6.0 * N * N * (double)n_chol : 6.0 * N * N * N + 4.0 * N * N * (double)n_chol) +
-             2.0 * n_pairs * 2.0 * n_pairs * d2;
+  if (pp.on) {  // executed products: the pair products, W, the 4-internal product
+    f_ring = pp.f64.W.alg_flops + pp.f64.hole.alg_flops;
+    for (const auto& gq : pp.f64.pair) f_ring += gq.alg_flops;
   }
   flops_sigma = flops_ladder + f_ring + 2.0 * (double)n_chol * n_v * niv * 3.0 + 2.0 * (double)niv * niv;
   TCI_HIP(hipDeviceSynchronize());
   device_bytes = 0;
   for (DevBuf* b : {&pairs, &dom_off, &dom_idx, &cd_off, &aa_off, &ab_off, &eps, &pos, &xmap, &isect_off, &isect,
                     &inv_off, &inv_q, &inv_pos, &gpart_off, &Lvv, &Lov, &Kov, &Jvv, &Mss, &O4, &O3, &vvd, &vvx,
-                    &diag, &C, &Ct, &R, &s, &sT, &g, &gss, &gW, &Y, &W, &gpart, &part, &sig0, &lad_part, &Jbig, &CRb,
-                    &CtRb, &CCb, &Zb, &Z3b, &Cemb, &CTemb, &Remb, &Yt, &holeA, &LovT, &Tbuf, &Rpart, &Lp, &Cw, &lp_off_all, &Fm,
+                    &diag, &C, &Ct, &R, &s, &sT, &g, &gss, &gW, &Y, &W, &gpart, &part, &sig0, &lad_part, &Tbuf, &Rpart, &Lp, &Cw, &lp_off_all, &Fm,
                     &Fvvp, &Fov})
     device_bytes += (int64_t)b->bytes;
-  device_bytes += vv_device_bytes(*this);
+  device_bytes += vv_device_bytes(*this) + panels_device_bytes(*this);
 }
 
 void tci_plan::drop_graphs() {
@@ -1029,7 +1030,7 @@ void tci_plan::unpack_and_ladder(const double* x, const IoSlot* io, int precisio
     return;
   }
   if (vv.fp64) {
-    vv_ladder(*this, TCI_SIGMA_FP64, st);
+    vv_ladder(*this, TCI_SIGMA_FP64, st, !pp.on);
     if (timing()) TCI_HIP(hipEventRecord(ev[3], st));
     return;
   }
@@ -1063,14 +1064,23 @@ void tci_plan::sigma_body(const double* x, double* y, const IoSlot* io, int flag
 // ladder's R
 void tci_plan::sigma_rest(const double* x, double* y, const IoSlot* io, int flags, hipStream_t st) {
   const int precision = flags & 0xff;
-  int e0 = kt_begin(st);
-  launch_rterms(tab, dmax, x, s.as<double>(), Kov.as<double>(), O3.as<double>(), R.as<double>(), st, io);
-  kt_end(e0, "rterms_kernel", 0.0, precision, st);
-  launch_transpose_small(s.as<double>(), n_int, n_v, sT.as<double>(), st);
-  kt_run("singles Y", progY, precision, st, [&] { progY.launch(st); });
-  if (dense_pairs) {
-    dense_pairs_terms(*this, precision, st);
+  int e0;
+  if (!nprogY.tasks.empty()) {
+    kt_run("singles Y", nprogY, precision, st, [&] { nprogY.launch(TCI_SIGMA_FP64, st); });
   } else {
+    launch_transpose_small(s.as<double>(), n_int, n_v, sT.as<double>(), st);
+    kt_run("singles Y", progY, precision, st, [&] { progY.launch(st); });
+  }
+  // with the panels the ladder's packed S+- and the pair terms meet in the
+  // final kernel; R then holds a Cholesky-direct ladder and the virtual Fock
+  // products only
+  const bool packed = pp.on && (precision == TCI_SIGMA_FP64 ? vv.fp64 : vv.split);
+  if (pp.on) {
+    panels_terms(*this, precision, st);
+  } else {
+    e0 = kt_begin(st);
+    launch_rterms(tab, dmax, x, s.as<double>(), Kov.as<double>(), O3.as<double>(), R.as<double>(), st, io);
+    kt_end(e0, "rterms_kernel", 0.0, precision, st);
     HoleTab H{isect_off.as<int64_t>(), isect.as<int32_t>()};
     e0 = kt_begin(st);
     launch_hole(tab, H, dmax, C.as<double>(), O4.as<double>(), R.as<double>(), st);
@@ -1079,16 +1089,19 @@ void tci_plan::sigma_rest(const double* x, double* y, const IoSlot* io, int flag
     kt_run("singles W", progW, precision, st, [&] { progW.launch(st); });
   }
   launch_gemv(Mss.as<double>(), (int64_t)n_int * n_v, s.as<double>(), gss.as<double>(), st);
-  progGW.launch(st);
+  if (!nprogGW.tasks.empty()) nprogGW.launch(TCI_SIGMA_FP64, st);
+  else progGW.launch(st);
   launch_s3int_singles(tab, dmax, gpart_off.as<int64_t>(), Ct.as<double>(), O3.as<double>(), gpart.as<double>(), st);
   InvTab I{inv_off.as<int64_t>(), inv_q.as<int32_t>(), inv_pos.as<int32_t>()};
   launch_singles_reduce(tab, I, gpart_off.as<int64_t>(), gpart.as<double>(), gss.as<double>(), gW.as<double>(), n_split,
                         g.as<double>(), st);
   launch_ref_dot(tab, Kov.as<double>(), Ct.as<double>(), part.as<double>(), sig0.as<double>(), st);
+  if (has_fvv && packed) launch_fill(R.as<double>(), sum_d2, 0.0, st);
   if (has_fvv) kt_run("virtual Fock", fockvv, precision, st, [&] { fockvv.launch(st); });
   if (has_fov) launch_fov_terms(x, s.as<double>(), Fov.as<double>(), (int64_t)n_int * n_v, g.as<double>(),
                                 sig0.as<double>(), st, io);
-  launch_pack(tab, dmax, x, R.as<double>(), g.as<double>(), sig0.as<double>(), e_ref, flags, y, st, io);
+  if (pp.on) panels_pack(*this, precision, packed, !packed || has_fvv, x, io, flags, y, st);
+  else launch_pack(tab, dmax, x, R.as<double>(), g.as<double>(), sig0.as<double>(), e_ref, flags, y, st, io);
 }
 
 // The whole build as one graph launch: the first call with a flag set captures

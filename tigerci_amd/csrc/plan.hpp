@@ -40,13 +40,27 @@ struct tci_plan {
   int lad_chunks = 1;
   // programs
   tci::GemmProgram ring, progY, progW, progGW;
-  // pair terms as dense products over embedded pair blocks (pairs_full.hip)
-  bool dense_pairs = false;
-  tci::DevBuf pairid_d, Jbig, CRb, CtRb, CCb, Zb, Z3b, Cemb, CTemb, Remb, Yt, holeA, LovT;
-  tci::GemmProgram ringZ, ringZ3, holeG, progWd, progU;
-  // Kov = Lov^T Lov: the C~R Kov part of Z runs as U = Yt + C~R Lov^T, then
-  // U Lov (2 N^2 n_chol flops in place of 2 N^3); TCI_Z_LOWRANK=0 keeps C~R Kov
-  bool z_lowrank = false;
+  tci::NProgram nprogY, nprogGW;   // the same on the NT GEMM (even n_v, FP64 L^J)
+  // pair terms as per-walk products over packed panels (pair_panels.hip)
+  struct PairPanels {
+    bool on = false;
+    std::vector<int32_t> h_koff;
+    std::vector<int64_t> h_ld, h_poff, h_jpoff, h_lpoff;
+    tci::DevBuf koff, ld, poff, jpoff, lpoff, pairid, colm;
+    int64_t n_panel = 0, n_jp = 0, n_lp = 0;  // values of one panel set, of JP, of LP
+    int64_t np = 0, nm = 0, ldw = 0, ldu = 0; // packed pair counts; row strides over walks and over Cholesky vectors
+    int ncm = 0, nk = 0;                      // walks with i != j; n_int rounded up to even
+    tci::DevBuf holeP, holeM, Hp, Hm;         // 4-internal coefficients and results
+    tci::DevBuf O3T, sTp, Rp;                 // 3-internal factors, s transposed, K-split partials of R
+    struct Set {                              // operands of one element type
+      tci::DevBuf CR, CC, CT, JP, LP, U, LovT, XTp, XTm, hP, hM;
+      tci::NProgram W, hole;
+      std::vector<tci::NProgram> pair;        // one per tile shape
+      int ks = 1;
+    } f64, s16;
+    tci::NProgram rank;                       // FP64 3-internal products of a split sigma
+    int tuned_mode = -1, tuned_ks = 1, tuned_order = 0;  // split schedule, kept for both split precisions
+  } pp;
   tci::LadderLaunch ladder;        // fused single-kernel ladder (TCI_LADDER=fused)
   bool ladder_fused = false;
   // two-phase ladder: per J-chunk of length Lc, T_P = L[D,D] C_P then R_P += sum T L
@@ -85,9 +99,10 @@ struct tci_plan {
     // scales (fp16x3; all 1 for bf16x3): [0] constants (L, Kov, Jbig, Lov,
     // the 4-internal coefficients),
     // [1] C of the ladder, [2] ladder intermediate, [3] phase-1 output,
-    // [4] phase-2 output, [5] pair-product output, [6] C and Yt of the pair
-    // products, [8] max of the constants; maxbits: [0] max|C|, [1] max|Yt|,
-    // [2] max over the constants (float bits)
+    // [4] phase-2 output, [5] pair-product output, [6] C and U of the pair
+    // products, [8] max of the constants, [9] and [10] V and the output of the
+    // resident ladder, [11] CT and [12] the output of W; maxbits: [0] max|C|,
+    // [1] max|U|, [2] max over the constants, [3] max|V| (float bits)
     tci::DevBuf scales, maxbits;
     tci::DevBuf lp_off_all;         // offsets of the local pairs in a prepacked Lpx
     tci::DevBuf Cx, cx_off;         // split rows of the C_P blocks (of C_P^T when merged)
@@ -96,22 +111,6 @@ struct tci_plan {
     tci::DevBuf Tx;                 // T' of one chunk
     tci::DevBuf Rpart;              // partial R buffers of phase 2 K-splits
     int rpart_n = 1;
-    // dense pair terms in split precision (full domains)
-    tci::DevBuf Kx, Jx, CRx, CtRx, CCx, Lovx, LovTx, Ytx;
-    tci::GemmProgram ringZx, ringZ3x, progWx;
-    // bf16x3 with the low-rank Z: U (into Yt) and W as one launch before Z
-    bool z_lowrank = false;
-    tci::GemmProgram progUx, pairsUWx;
-    // 4-internal product in split precision: the coefficient matrix and the
-    // embedded [C; C^T] blocks as split rows over k = walk
-    tci::DevBuf holeAx, embTx;
-    tci::GemmProgram holeGx;
-    // Z, Z3, W and the 4-internal product as one task list (128 x 128 tiles)
-    tci::GemmProgram pairsx;
-    bool pairs_merged = false;
-    // tile configurations of the split pair products, tuned on the first split
-    // preparation and kept for both split precisions (-1: not yet tuned)
-    int tuned_pairs_z = -1, tuned_pairs_uw = -1;
     std::vector<LadderPhase> phase;
     std::vector<std::pair<int64_t, int>> chunks;
     int64_t bytes = 0;
@@ -274,14 +273,18 @@ void vv_build(tci_plan& P, hipStream_t st);
 // shape: an NShape of ngemm.hpp
 void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t st);
 void vv_prepare_split(tci_plan& P, int precision, hipStream_t st);
-void vv_ladder(tci_plan& P, int precision, hipStream_t st);
+// gather: unpack S+- into R (otherwise the caller reads the packed S+-)
+void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool gather);
 double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log);
 int64_t vv_device_bytes(const tci_plan& P);
-// dense pair terms (pairs_full.hip)
-bool dense_pairs_choose(const tci_plan& P, double f_gather);
-void dense_pairs_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st);
-// cfg_z (Z, Z3, 4-internal) and cfg_uw (U, W): 0 = 128 x 128 tiles, 1 / 2 =
-// 256 x 256 with 4 / 8 waves, -1 = the TCI_PAIRS_TILE choice
-void dense_pairs_build_split(tci_plan& P, hipStream_t st, int cfg_z = -1, int cfg_uw = -1);
-void dense_pairs_terms(tci_plan& P, int precision, hipStream_t st);
+// pair terms over packed panels (pair_panels.hip)
+bool panels_choose(const tci_plan& P);
+void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st);
+void panels_build_split(tci_plan& P, hipStream_t st);
+void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st);
+void panels_tune(tci_plan& P, int precision, hipStream_t st);
+void panels_terms(tci_plan& P, int precision, hipStream_t st);
+void panels_pack(tci_plan& P, int precision, bool packed, bool use_r, const double* x, const tci::IoSlot* io,
+                 int flags, double* y, hipStream_t st);
+int64_t panels_device_bytes(const tci_plan& P);
 }  // namespace tci
