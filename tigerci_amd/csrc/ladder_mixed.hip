@@ -282,7 +282,7 @@ void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
     else
       hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(nvv, 1024)), dim3(256), 0, st, P.Lvv.as<double>(), nvv,
                          mx + 2);
-    if (P.pp.on) {
+    if (P.pp.on && P.pp.split) {
       auto amax = [&](const DevBuf& x, int64_t n) {
         hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(n, 1024)), dim3(256), 0, st, x.as<double>(), n, mx + 2);
       };
@@ -862,7 +862,7 @@ void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
     M.tuned_fused_target = bft;
     P.tuning += log + "\n";
   }
-  if (P.pp.on) {
+  if (P.pp.on && P.pp.split) {
     panels_build_split(P, st);
     panels_tune(P, precision, st);
   }
@@ -965,10 +965,11 @@ void mixed_ladder_run(tci_plan& P, int precision, hipStream_t st) {
   if (M.rpart_n > 1) ladder_reduce(M.Rpart.as<double>(), P.sum_d2, M.rpart_n, P.R.as<double>(), P.sum_d2, st);
 }
 
-void mixed_ladder(tci_plan& P, int precision, hipStream_t st) {
+void mixed_ladder(tci_plan& P, int precision, bool expanded, const double* x, const IoSlot* io, hipStream_t st) {
   mixed_prepare(P, precision, st);
   if (P.vv.split) {
-    vv_ladder(P, precision, st, !P.pp.on);
+    if (panels_hole_in_ladder(P, precision)) panels_xt(P, precision, x, io, st);
+    vv_ladder(P, precision, st, !expanded, !P.pp.on);
     if (P.timing()) TCI_HIP(hipEventRecord(P.ev[3], st));
     return;
   }

@@ -15,7 +15,8 @@
 // (a > b, n_m of them):
 //   V+[p(a,b)][p(c,d)] = (ac|bd) + (ad|bc)      X+[P][p(c,d)] = C+_cd (c > d), C_cc / 2
 //   V-[q(a,b)][q(c,d)] = (ac|bd) - (ad|bc)      X-[P][q(c,d)] = C-_cd
-//   S+ = X+ V+,  S- = X- V-   (V+- symmetric)
+//   S+ = X+ V+,  S- = X- V-   (V+- symmetric; with the pair panels S+- also
+//   hold the 4-internal term, one more K-range over the walks)
 //   R_P[a][b] = S+[p(a,b)] + S-[q(a,b)],  R_P[b][a] = S+[p(a,b)] - S-[q(a,b)]  (a > b),
 //   R_P[a][a] = S+[p(a,a)].
 // Walks with i == j have symmetric C_P and take no row of X-.  Entries of X
@@ -240,27 +241,30 @@ constexpr int kScV = 9, kScOut = 10, kScC = 1;
 
 inline int64_t even(int64_t n) { return (n + 1) & ~(int64_t)1; }
 
-// S = X V^T for both parts as one program: tasks ordered by column block of V,
-// then K-split, then row block of X, so the row tiles that read one V panel
-// are neighbours.
-void build_products(tci_plan& P, NProgram& g, bool split, int shape, int ks, hipStream_t st) {
+}  // namespace
+
+// S = X V^T for both parts: tasks ordered by column block of V, then K-split,
+// then row block of X, so the row tiles that read one V panel are neighbours.
+void vv_add_products(tci_plan& P, NProgram& g, bool split, int ks) {
   tci_plan::VVLadder& V = P.vv;
-  g.clear();
-  g.split = split;
-  g.shape = shape;
   const int tn = g.tn(), esz = split ? 4 : 8;
   struct Part {
     const void* X;
     const void* Vm;
     double* S;
     int64_t n, rows, ld;
+    const void *hc, *hx;  // 4-internal coefficients and X^T, both over k = walk
   };
   auto ld = [&](int64_t n) { return split ? xpad(n) : even(n); };
+  // with the pair panels the 4-internal product over the walks is one more
+  // K-range of the last split, except in fp16x3, whose scales differ
+  const bool hole = P.pp.on && (!split || (P.pp.split && P.mx.prec != TCI_SIGMA_FP16X3));
+  const auto& H = split ? P.pp.s16 : P.pp.f64;
   std::vector<Part> parts = {{split ? V.Xpx.p : V.Xp.p, split ? V.Vpx.p : V.Vp.p, V.Sp.as<double>(), V.np,
-                              (int64_t)P.n_pairs, ld(V.np)}};
+                              (int64_t)P.n_pairs, ld(V.np), split ? H.hP.p : P.pp.holeP.p, H.XTp.p}};
   if (V.ncm > 0)
     parts.push_back({split ? V.Xmx.p : V.Xm.p, split ? V.Vmx.p : V.Vm.p, V.Sm.as<double>(), V.nm, (int64_t)V.ncm,
-                     ld(V.nm)});
+                     ld(V.nm), split ? H.hM.p : P.pp.holeM.p, H.XTm.p});
   for (const Part& pt : parts) {
     const int64_t K = pt.ld;               // padding columns of X and V are zero
     const int64_t spart = pt.rows * pt.n;  // elements of one partial S
@@ -271,11 +275,24 @@ void build_products(tci_plan& P, NProgram& g, bool split, int shape, int ks, hip
         TCI_REQUIRE(k1 > k0, "empty K-split range");
         const char* Xb = static_cast<const char*>(pt.X) + k0 * esz;
         const char* Vb = static_cast<const char*>(pt.Vm) + (n0 * pt.ld + k0) * esz;
-        g.add(pt.S + k * spart + n0, pt.n, (int)pt.rows, nn, {nseg(Xb, pt.ld, Vb, pt.ld, k1 - k0, esz)}, false,
-              Blocking(), split ? kScOut : -1);
+        std::vector<NSeg> sg = {nseg(Xb, pt.ld, Vb, pt.ld, k1 - k0, esz)};
+        if (hole && k + 1 == ks) {
+          const int64_t ldw = P.pp.ldw;
+          sg.push_back(nseg(pt.hc, ldw, static_cast<const char*>(pt.hx) + n0 * ldw * esz, ldw, ldw, esz));
+        }
+        g.add(pt.S + k * spart + n0, pt.n, (int)pt.rows, nn, sg, false, Blocking(), split ? kScOut : -1);
       }
     }
   }
+}
+
+namespace {
+
+void build_products(tci_plan& P, NProgram& g, bool split, int shape, int ks, hipStream_t st) {
+  g.clear();
+  g.split = split;
+  g.shape = shape;
+  vv_add_products(P, g, split, ks);
   g.upload_tables(st);
 }
 
@@ -420,8 +437,9 @@ void vv_prepare_split(tci_plan& P, int precision, hipStream_t st) {
 }
 
 // R = ladder of the unpacked C (overwrites R), FP64 or the prepared split
-// precision; without `gather` the result stays packed in S+-.
-void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool gather) {
+// precision; without `scatter` X+- hold the vector already, without `gather` the
+// result stays packed in S+-.
+void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool scatter, bool gather) {
   tci_plan::VVLadder& V = P.vv;
   const bool split = precision != TCI_SIGMA_FP64;
   TCI_REQUIRE(V.built && (!split || V.prec == precision), "resident (ab|cd) block not prepared for this precision");
@@ -429,20 +447,20 @@ void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool gather) {
   const int f16 = precision == TCI_SIGMA_FP16X3 ? 1 : 0;
   float* sc = P.mx.scales.as<float>();
   const dim3 gs(blocks((int64_t)P.dmax * (P.dmax + 1) / 2, 64), (unsigned)P.n_pairs);
-  int e0 = P.kt_begin(st);
-  if (split) {
+  int e0 = scatter ? P.kt_begin(st) : -1;
+  if (scatter && split) {
     if (f16) {  // scale of C from max|C|, then the output scale 1 / (s_V s_C)
       launch_split_scales(1, P.C.as<double>(), P.sum_d2, P.mx.maxbits.as<unsigned>(), 0, sc, (float)P.dmax, st);
       hipLaunchKernelGGL(vv_set_oscale_kernel, dim3(1), dim3(64), 0, st, sc, kScV, kScC, kScOut);
     }
     hipLaunchKernelGGL(vv_scatter_kernel<true>, gs, dim3(256), 0, st, P.tab, P.C.as<double>(), V.colm.as<int32_t>(),
                        V.Xpx.p, 2 * xpad(V.np), V.Xmx.p, 2 * xpad(V.nm), f16 ? sc + kScC : nullptr, f16);
-  } else {
+  } else if (scatter) {
     hipLaunchKernelGGL(vv_scatter_kernel<false>, gs, dim3(256), 0, st, P.tab, P.C.as<double>(), V.colm.as<int32_t>(),
                        V.Xp.p, even(V.np), V.Xm.p, even(V.nm), nullptr, 0);
   }
   TCI_HIP(hipGetLastError());
-  P.kt_end(e0, pn + " ladder vv_scatter_kernel", 0.0, precision, st);
+  if (scatter) P.kt_end(e0, pn + " ladder vv_scatter_kernel", 0.0, precision, st);
   const NProgram& g = split ? V.gx : V.g64;
   const int ks = split ? V.ksx : V.ks;  // K-splits change the launch (and its traffic), so they name it
   P.kt_run(pn + " ladder (ab|cd) product" + (ks > 1 ? " K-split " + std::to_string(ks) : std::string()), g,
@@ -481,7 +499,7 @@ double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
       vv_set_schedule(P, precision, sh, ks, st);
       for (int o = 0; o < orders; ++o) {
         g.remap = o;
-        const double ms = time_ms(st, 2, [&] { vv_ladder(P, precision, st, !P.pp.on); });
+        const double ms = time_ms(st, 2, [&] { vv_ladder(P, precision, st, true, !P.pp.on); });
         log += " " + std::to_string(g.tm()) + "x" + std::to_string(g.tn()) + "/" + std::to_string(ks) + (o ? "x:" : ":") +
                fmt_ms(ms);
         if (ms < best * 0.98) {
@@ -503,7 +521,7 @@ double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
   log += " -> " + std::to_string(g.tm()) + "x" + std::to_string(g.tn()) + "/" + std::to_string(bk) + " order " +
          std::to_string(bo);
   TCI_HIP(hipStreamSynchronize(st));
-  return time_ms(st, 2, [&] { vv_ladder(P, precision, st, !P.pp.on); });
+  return time_ms(st, 2, [&] { vv_ladder(P, precision, st, true, !P.pp.on); });
 }
 
 int64_t vv_device_bytes(const tci_plan& P) {

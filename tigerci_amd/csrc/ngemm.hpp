@@ -32,7 +32,9 @@ namespace tci {
 
 // One contraction range of a task.  kbytes: valid bytes of k per row, a
 // multiple of 16; lda / ldb row strides in bytes (multiples of 16); am / bm
-// row maps or null; ja / jb bytes per unit of the launch argument J0.
+// row maps or null; ja / jb bytes per unit of the launch argument J0.  The range
+// is taken `reps` times (at least once), A and B moving by sa and sb bytes from
+// one to the next (the Cholesky vectors of one walk): the row offsets stay.
 struct NSeg {
   const void* A;
   const void* B;
@@ -40,6 +42,7 @@ struct NSeg {
   const int32_t* bm;
   int64_t lda, ldb, ja, jb;
   int64_t kbytes;
+  int64_t reps, sa, sb;
   int64_t pad_;
 };
 
@@ -68,7 +71,8 @@ struct NProgram {
   int tm() const { return shape == N192 ? 192 : shape == N64 ? 64 : shape == N32K4 ? 32 : shape == N256 ? 256 : 128; }
   int tn() const { return shape == N128x192 ? 192 : tm(); }
   // adds the tiles of one M x N output; rows / cols of the stored element are
-  // offset by the blocking as in GemmProgram
+  // offset by the blocking as in GemmProgram.  out_split: C is a split-row
+  // matrix (the operand of a following split product), ldc in 16-bit elements
   void add(double* C, int64_t ldc, int M, int N, const std::vector<NSeg>& s, bool accumulate, Blocking blk = Blocking(),
            int oscale = -1, bool out_split = false);
   void upload_tables(hipStream_t st);
@@ -87,6 +91,7 @@ inline NSeg nseg(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t
   s.lda = lda * esz;
   s.ldb = ldb * esz;
   s.kbytes = K * esz;
+  s.reps = 1;
   return s;
 }
 

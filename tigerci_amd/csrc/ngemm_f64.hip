@@ -34,10 +34,13 @@ void NProgram::add(double* C, int64_t ldc, int M, int N, const std::vector<NSeg>
                    int oscale, bool out_split) {
   if (M <= 0 || N <= 0) return;
   TCI_REQUIRE(oscale < 0 || split, "output scales belong to split programs");
-  TCI_REQUIRE(!out_split, "NT programs write FP64 output");
+  TCI_REQUIRE(!out_split || (split && !accumulate && blk.rdiv == 0 && blk.cdiv == 0 && ldc % 16 == 0 &&
+                             (reinterpret_cast<uintptr_t>(C) & 31) == 0),
+              "split-row output needs a split program, no accumulation or blocking, and 32-byte rows");
   for (const NSeg& x : s)
     TCI_REQUIRE(x.A && x.B && x.kbytes % 16 == 0 && x.lda % 16 == 0 && x.ldb % 16 == 0 && x.ja % 16 == 0 &&
-                    x.jb % 16 == 0 && (reinterpret_cast<uintptr_t>(x.A) & 15) == 0 &&
+                    x.jb % 16 == 0 && x.kbytes < ((int64_t)1 << 30) && x.reps >= 1 && x.reps < ((int64_t)1 << 30) && x.sa % 16 == 0 && x.sb % 16 == 0 &&
+                    (reinterpret_cast<uintptr_t>(x.A) & 15) == 0 &&
                     (reinterpret_cast<uintptr_t>(x.B) & 15) == 0,
                 "NT GEMM operands need 16-byte aligned rows and ranges");
   // plain rows: a lane's offset spans one tile (gathered rows: the caller keeps
@@ -60,6 +63,7 @@ void NProgram::add(double* C, int64_t ldc, int M, int N, const std::vector<NSeg>
       t.seg0 = seg0;
       t.seg1 = seg1;
       t.accumulate = accumulate ? 1 : 0;
+      t.out_split = out_split ? 1 : 0;
       t.rdiv = blk.rdiv;
       t.cdiv = blk.cdiv;
       t.rstride = blk.rstride;
@@ -74,7 +78,7 @@ void NProgram::upload_tables(hipStream_t st) {
   const double esz = split ? 4.0 : 8.0;
   for (const Task& t : tasks) {
     const double mv = std::min(tm(), t.M - t.m0), nv = std::min(tn(), t.N - t.n0);
-    for (int q = t.seg0; q < t.seg1; ++q) alg_flops += 2.0 * mv * nv * (double)segs[q].kbytes / esz;
+    for (int q = t.seg0; q < t.seg1; ++q) alg_flops += 2.0 * mv * nv * (double)segs[q].kbytes / esz * (double)segs[q].reps;
   }
   upload(d_tasks, tasks, st);
   upload(d_segs, segs, st);

@@ -34,9 +34,13 @@ struct F64T {
 };
 
 template <int PREC>
+struct NV;
+
+template <int PREC>
 struct S16T {
   static constexpr int BS = 16;
   typedef f4 Acc;
+  typedef typename NV<PREC>::T T16;
   static __device__ __forceinline__ int sw(int r) { return ((r >> 1) & 1) | (((r >> 2) & 1) << 2); }
   static __device__ __forceinline__ Acc zero() { return f4{0.f, 0.f, 0.f, 0.f}; }
 };
@@ -45,6 +49,7 @@ template <int PREC>
 struct S32T {
   static constexpr int BS = 32;
   typedef f16v Acc;
+  typedef typename NV<PREC>::T T16;
   static __device__ __forceinline__ int sw(int r) { return ((r >> 1) & 3) | (((r >> 4) & 1) << 2); }
   static __device__ __forceinline__ Acc zero() {
     f16v z;
@@ -54,8 +59,6 @@ struct S32T {
   }
 };
 
-template <int PREC>
-struct NV;
 template <>
 struct NV<TCI_SIGMA_BF16X3> {
   typedef __bf16 T;
@@ -74,7 +77,10 @@ struct NV<TCI_SIGMA_FP16X3> {
 // ---- staging ------------------------------------------------------------------
 // NI loads of one wave for one operand of R rows and NWK k-chunks: load q
 // covers 8 rows (lane / 8) of k-chunk sub(q).
-template <class TT, int R, int NWK, int NW>
+// Groups of 8 rows wholly outside the output are not loaded when SKIP is set
+// (their LDS rows then hold anything, which only reaches products that are not
+// stored); three-stage kernels count their loads in flight and load them all.
+template <class TT, int R, int NWK, int NW, bool SKIP>
 struct NStage {
   static constexpr int NI = NWK * R / (8 * NW);
   static_assert(NI * 8 * NW == NWK * R, "loads divide evenly over the waves");
@@ -103,12 +109,13 @@ struct NStage {
     }
   }
   // rem: bytes of k left in the segment from this step on
-  __device__ __forceinline__ void issue(int w, int lane, const char* base, int64_t rem, char* lds, int rowbase,
-                                        int stride) const {
+  __device__ __forceinline__ void issue(int w, int lane, const char* base, int rem, char* lds, int rowbase,
+                                        int stride, int valid) const {
     const bool whole = rem >= NWK * 128;
 #pragma unroll
     for (int q = 0; q < NI; ++q) {
       const int ins = w * NI + q, sub = ins / (R / 8), r8 = ins % (R / 8);
+      if (SKIP && r8 * 8 >= valid) continue;
       char* dst = lds + sub * stride + (rowbase + r8 * 8) * 128;
       if (whole) {
         __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(base + off[q]),
@@ -246,7 +253,7 @@ __device__ __forceinline__ void nput(const Task& t, int64_t o, double v) {
   *p = t.accumulate ? *p + v : v;
 }
 
-template <int NWM, int NWN, int BM, int BN>
+template <class TT, int NWM, int NWN, int BM, int BN>
 __device__ __forceinline__ void nstore(const Task& t, const float*, const d4 (&acc)[BM][BN], int wr, int wc, int lane) {
   const int li = lane & 15, lg = lane >> 4;
   int64_t co[BN];
@@ -265,9 +272,28 @@ __device__ __forceinline__ void nstore(const Task& t, const float*, const d4 (&a
     }
 }
 
-// four consecutive columns col .. col+3 of one row
+// four consecutive columns col .. col+3 of one row; split-row output writes
+// their hi and lo parts as 8-byte groups (columns beyond N up to the padding
+// to a multiple of 8 receive zeros: the caller's B rows are clamped, so they
+// are masked here)
+template <class T16>
 __device__ __forceinline__ void nput4(const Task& t, int row, int col, const float* v) {
   const int64_t ro = nrow_off(t, row);
+  if (t.out_split) {
+    typedef T16 b4 __attribute__((ext_vector_type(4)));
+    b4 h, l;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float x = col + r < t.N ? v[r] : 0.f;
+      h[r] = (T16)x;
+      l[r] = (T16)(x - (float)h[r]);
+    }
+    __attribute__((address_space(1))) b4* p =
+        (__attribute__((address_space(1))) b4*)(reinterpret_cast<uint16_t*>(t.C) + ro + xidx(col));
+    p[0] = h;
+    p[2] = l;
+    return;
+  }
   const int cc = t.cdiv ? col % t.cdiv : col;
   if (t.cdiv ? ((cc & 3) == 0 && cc + 3 < t.cdiv && col + 3 < t.N) : col + 3 < t.N) {
     typedef double d4u __attribute__((ext_vector_type(4), aligned(8)));  // ldc is arbitrary
@@ -282,7 +308,7 @@ __device__ __forceinline__ void nput4(const Task& t, int row, int col, const flo
   }
 }
 
-template <int NWM, int NWN, int BM, int BN>
+template <class TT, int NWM, int NWN, int BM, int BN>
 __device__ __forceinline__ void nstore(const Task& t, const float* scales, const f4 (&acc)[BM][BN], int wr, int wc,
                                        int lane) {
   const int li = lane & 15, lg = lane >> 4;
@@ -296,12 +322,12 @@ __device__ __forceinline__ void nstore(const Task& t, const float* scales, const
       const int col = t.n0 + 16 * (wc + NWN * j) + 4 * lg;
       const f4 v = acc[i][j] * osc;
       const float x[4] = {v[0], v[1], v[2], v[3]};
-      if (col < t.N) nput4(t, row, col, x);
+      if (col < t.N) nput4<typename TT::T16>(t, row, col, x);
     }
   }
 }
 
-template <int NWM, int NWN, int BM, int BN>
+template <class TT, int NWM, int NWN, int BM, int BN>
 __device__ __forceinline__ void nstore(const Task& t, const float* scales, const f16v (&acc)[BM][BN], int wr, int wc,
                                        int lane) {
   const int lr = lane & 31, hs = lane >> 5;
@@ -317,23 +343,31 @@ __device__ __forceinline__ void nstore(const Task& t, const float* scales, const
         const int col = t.n0 + 32 * (wc + NWN * j) + 8 * g + 4 * hs;
         const float x[4] = {acc[i][j][4 * g] * osc, acc[i][j][4 * g + 1] * osc, acc[i][j][4 * g + 2] * osc,
                             acc[i][j][4 * g + 3] * osc};
-        if (col < t.N) nput4(t, row, col, x);
+        if (col < t.N) nput4<typename TT::T16>(t, row, col, x);
       }
   }
 }
 
 // ---- kernel ---------------------------------------------------------------------
+// Column of wave wq.  With 2 x 4 waves, w and w + 4 share a SIMD: the second
+// row of waves is rotated by two columns, so that in a ragged tile (say 10
+// column blocks: 3, 3, 2, 2) every SIMD gets one long and one short wave.
+template <int NWM, int NWN>
+__device__ __forceinline__ int nwave_col(int wq) {
+  return NWM == 2 && NWN == 4 ? (wq + 2 * (wq >> 2)) & 3 : wq % NWN;
+}
+
 template <class TT, int NWM, int NWN, int NWK, int BM, int BN, int NST, bool FULL>
 __device__ __forceinline__ void nbody(const Task& t, const NSeg* __restrict__ segs, int64_t J0,
                                       const float* __restrict__ scales, char* sm, int w, int lane, int nbm, int nbn) {
   constexpr int NW = NWM * NWN * NWK;
   constexpr int TM = TT::BS * NWM * BM, TN = TT::BS * NWN * BN;
   constexpr int SUB = (TM + TN) * 128, STG = NWK * SUB;
-  typedef NStage<TT, TM, NWK, NW> SA;
-  typedef NStage<TT, TN, NWK, NW> SB;
+  typedef NStage<TT, TM, NWK, NW, NST == 2 && !FULL> SA;
+  typedef NStage<TT, TN, NWK, NW, NST == 2 && !FULL> SB;
   constexpr int PER = SA::NI + SB::NI;
   static_assert(NST == 2 || (NST == 3 && PER <= 15), "two stages, or three within the vmcnt field");
-  const int kg = w / (NWM * NWN), wq = w % (NWM * NWN), wr = wq / NWN, wc = wq % NWN;
+  const int kg = w / (NWM * NWN), wq = w % (NWM * NWN), wr = wq / NWN, wc = nwave_col<NWM, NWN>(wq);
   typename TT::Acc acc[BM][BN];
 #pragma unroll
   for (int i = 0; i < BM; ++i)
@@ -343,17 +377,18 @@ __device__ __forceinline__ void nbody(const Task& t, const NSeg* __restrict__ se
   SB lb;
   int seg = t.seg0;
   const char *pa = nullptr, *pb = nullptr;
-  int64_t rem = 0;
+  int rem = 0, reps = 0;  // bytes left of this pass over the range, passes left
   // first segment with work from `seg` on: sets the load state, false at the end
   auto open = [&]() -> bool {
     while (seg < t.seg1) {
       const NSeg& S = segs[seg];
-      rem = S.kbytes;
+      rem = (int)S.kbytes;
       if (rem > 0) {
         pa = static_cast<const char*>(S.A) + J0 * S.ja + (S.am ? 0 : (int64_t)t.m0 * S.lda);
         pb = static_cast<const char*>(S.B) + J0 * S.jb + (S.bm ? 0 : (int64_t)t.n0 * S.ldb);
         la.set(w, lane, S.am, S.lda, t.m0, t.M);
         lb.set(w, lane, S.bm, S.ldb, t.n0, t.N);
+        reps = (int)S.reps - 1;
         return true;
       }
       seg = __builtin_amdgcn_readfirstlane(seg + 1);
@@ -361,14 +396,23 @@ __device__ __forceinline__ void nbody(const Task& t, const NSeg* __restrict__ se
     return false;
   };
   auto issue = [&](char* buf) {
-    la.issue(w, lane, pa, rem, buf, 0, SUB);
-    lb.issue(w, lane, pb, rem, buf, TM, SUB);
+    la.issue(w, lane, pa, rem, buf, 0, SUB, t.M - t.m0);
+    lb.issue(w, lane, pb, rem, buf, TM, SUB, t.N - t.n0);
     pa += NWK * 128;
     pb += NWK * 128;
     rem -= NWK * 128;
   };
   auto step = [&]() -> bool {  // is there a further stage to load?
     if (rem > 0) return true;
+    if (reps > 0) {  // the same rows again, sa and sb bytes further
+      const NSeg& S = segs[seg];
+      const int kb = (int)S.kbytes, used = kb - rem;  // rem <= 0: what the last step ran over
+      --reps;
+      pa += S.sa - used;
+      pb += S.sb - used;
+      rem = kb;
+      return true;
+    }
     seg = __builtin_amdgcn_readfirstlane(seg + 1);
     return open();
   };
@@ -420,7 +464,7 @@ __device__ __forceinline__ void nbody(const Task& t, const NSeg* __restrict__ se
 #pragma unroll
         for (int j = 0; j < BN; ++j) acc[i][j] += red[(((g * NWM * NWN + wq) * BM + i) * BN + j) * 64 + lane];
   }
-  nstore<NWM, NWN, BM, BN>(t, scales, acc, wr, wc, lane);
+  nstore<TT, NWM, NWN, BM, BN>(t, scales, acc, wr, wc, lane);
 }
 
 // FULL bodies have no block predicates; a wave takes the predicated body when
@@ -434,7 +478,7 @@ __global__ __launch_bounds__(64 * NWM * NWN * NWK, OCC) void ngemm_kernel(const 
   const Task t = tasks[remap ? xcd_task(blockIdx.x, gridDim.x) : blockIdx.x];
   __shared__ __attribute__((aligned(16))) char sm[NST * NWK * (TM + TN) * 128];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wq = w % (NWM * NWN), wr = wq / NWN, wc = wq % NWN;
+  const int wq = w % (NWM * NWN), wr = wq / NWN, wc = nwave_col<NWM, NWN>(wq);
   const int nbm = __builtin_amdgcn_readfirstlane(max(0, min(BM, (t.M - t.m0 - BS * wr + BS * NWM - 1) / (BS * NWM))));
   const int nbn = __builtin_amdgcn_readfirstlane(max(0, min(BN, (t.N - t.n0 - BS * wc + BS * NWN - 1) / (BS * NWN))));
   if (nbm == BM && nbn == BN)

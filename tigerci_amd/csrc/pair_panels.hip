@@ -132,6 +132,163 @@ __global__ __launch_bounds__(256) void panels_kernel(PairTab T, PanelTab K, cons
   }
 }
 
+// Everything a sigma derives from the CI vector alone, in one pass over it:
+// the panels, Ct (and C where a term reads it), the rows X+- of the resident
+// ladder, s and its transpose.  Block: one walk, one pair of 32 x 32 tiles
+// (X >= Y) of the packed triangle; each vector element is read once and both
+// orientations leave along rows.  FP64 and bf16x3 (the scales of fp16x3 need
+// max|C| first: unpack_kernel, vv_scatter_kernel and panels_kernel there).
+// Bound by its writes: 116 us (bf16x3) and 157 us (FP64) at 34/192/1200, against
+// 98 + 50 + 100 us for unpack, scatter and panels one after the other.
+struct ExpandOut {
+  double *C, *Ct, *s, *sT;  // C null: not needed
+  int nk;
+  void *CR, *CC, *CT;
+  void *Xp, *Xm;            // null: no resident ladder
+  int64_t ldp, ldm;         // values
+  const int32_t* colm;
+};
+
+__device__ __forceinline__ void put_bf(uint16_t* p, double v) {
+  const float x = (float)v;
+  const __bf16 h = (__bf16)x;
+  const __bf16 l = (__bf16)(x - (float)h);
+  p[0] = __builtin_bit_cast(uint16_t, h);
+  p[8] = __builtin_bit_cast(uint16_t, l);
+}
+
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void expand_kernel(PairTab T, PanelTab K, const double* __restrict__ x,
+                                                     const IoSlot* __restrict__ io, ExpandOut O) {
+  if (io) x = io->x;
+  const int Q = blockIdx.y, n = T.n_int, nv = T.n_v;
+  if (Q == T.n_pairs) {  // singles (walks by descending hole)
+    const int64_t tot = (int64_t)nv * O.nk;
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot; e += (int64_t)gridDim.x * blockDim.x) {
+      const int k = (int)(e / nv), a = (int)(e - (int64_t)k * nv);
+      const double v = k < n ? x[1 + (int64_t)(n - 1 - k) * nv + a] * INV_SQRT2 : 0.0;
+      if (k < n) O.s[e] = v;
+      O.sT[(int64_t)a * O.nk + k] = v;
+    }
+    return;
+  }
+  __shared__ double ta[32][33], tb[32][33];  // C[x][y] and C[y][x], x in tile X, y in tile Y
+  const int64_t o = T.dom_off[Q];
+  const int d = (int)(T.dom_off[Q + 1] - o), nt = (d + 31) >> 5;
+  if ((int)blockIdx.x >= nt * (nt + 1) / 2) return;
+  int X, Y;
+  untri32((int)blockIdx.x, X, Y);
+  const int x0 = X * 32, y0 = Y * 32;
+  const int i = T.pairs[2 * Q], j = T.pairs[2 * Q + 1];
+  const int64_t m2 = (int64_t)d * (d - 1) / 2;
+  const double *xa = x + T.aa_off[Q], *xb = x + T.ab_off[Q];
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  constexpr double INV_2SQRT3 = 0.28867513459481288225;
+  const int cm = O.colm[Q];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int r = ty + 8 * u, xr = x0 + r, yc = y0 + tx;
+    double A = 0.0, B = 0.0;
+    if (xr < d && yc <= xr) {
+      if (xr == yc) {
+        A = B = i == j ? xa[xr] : -xa[xr] * INV_SQRT2;
+      } else {
+        const int64_t idx = (int64_t)xr * (xr - 1) / 2 + yc;
+        if (i == j) {
+          A = B = xb[idx] * INV_SQRT2;
+        } else {
+          const double vs = -0.5 * xb[idx], q = xb[m2 + idx] * INV_2SQRT3;
+          A = vs - q;
+          B = vs + q;
+        }
+      }
+      if (O.Xp) {
+        const int gx = T.dom_idx[o + xr], gy = T.dom_idx[o + yc];
+        const double vp = xr == yc ? 0.5 * A : 0.5 * (A + B);
+        const int64_t kp = tri(gx) + gy;
+        if (SPLIT) put_bf(static_cast<uint16_t*>(O.Xp) + 2 * Q * O.ldp + xidx(kp), vp);
+        else static_cast<double*>(O.Xp)[Q * O.ldp + kp] = vp;
+        if (cm >= 0 && xr != yc) {
+          const int64_t km = tri(gx - 1) + gy;
+          const double vm = 0.5 * (A - B);
+          if (SPLIT) put_bf(static_cast<uint16_t*>(O.Xm) + 2 * cm * O.ldm + xidx(km), vm);
+          else static_cast<double*>(O.Xm)[cm * O.ldm + km] = vm;
+        }
+      }
+    }
+    ta[r][tx] = A;
+    tb[r][tx] = B;
+  }
+  __syncthreads();
+  if (X == Y) {  // fill the upper half of the diagonal tile
+    double up[4], lo[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = ty + 8 * u;
+      up[u] = tx > r ? tb[tx][r] : ta[r][tx];
+      lo[u] = tx > r ? ta[tx][r] : tb[r][tx];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      ta[ty + 8 * u][tx] = up[u];
+      tb[ty + 8 * u][tx] = lo[u];
+    }
+    __syncthreads();
+  }
+  // orientation 0: rows in X, columns in Y, C[row][col] = ta; 1: rows in Y,
+  // columns in X, C[row][col] = tb^T (the diagonal tile is whole after 0)
+  const int no = X == Y ? 1 : 2;
+  for (int w = 0; w < no; ++w) {
+    const int r0 = w ? y0 : x0, c0 = w ? x0 : y0;
+    double* Cq = O.C ? O.C + T.cd_off[Q] : nullptr;
+    double* Ctq = O.Ct + T.cd_off[Q];
+    const int two = i != j ? 2 : 1;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = ty + 8 * u, row = r0 + r, col = c0 + tx;
+      if (row >= d || col >= d) continue;
+      const double a = w ? tb[tx][r] : ta[r][tx], b = w ? ta[tx][r] : tb[r][tx];  // C[row][col], C[col][row]
+      const int64_t e = (int64_t)row * d + col;
+      if (Cq) Cq[e] = a;
+      Ctq[e] = 2.0 * a - b;
+      if (!SPLIT) {
+        const int64_t g = T.dom_idx[o + row];
+        for (int p = 0; p < two; ++p) {
+          const int iu = p ? j : i, iv = p ? i : j;
+          const int64_t q = K.poff[iu] + K.koff[iu * n + iv] + g * K.ld[iu] + col;
+          const double aa = p ? b : a, bb = p ? a : b;
+          static_cast<double*>(O.CR)[q] = aa;
+          static_cast<double*>(O.CC)[q] = bb;
+          static_cast<double*>(O.CT)[q] = 2.0 * aa - bb;
+        }
+      }
+    }
+    if (SPLIT) {
+      for (int t = threadIdx.x; t < 128 * 3 * two; t += 256) {
+        const int arr = (t >> 7) % 3, p = (t >> 7) / 3;
+        const int r = (t & 127) >> 2, c = 8 * (t & 3);
+        const int row = r0 + r, col = c0 + c;
+        if (row >= d || col >= d) continue;
+        const int iu = p ? j : i, iv = p ? i : j;
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          double a = w ? tb[c + q][r] : ta[r][c + q], b = w ? ta[c + q][r] : tb[r][c + q];
+          if (p) {
+            const double h = a;
+            a = b;
+            b = h;
+          }
+          v[q] = col + q < d ? (float)(arr == 0 ? a : arr == 1 ? b : 2.0 * a - b) : 0.f;
+        }
+        void* dst = arr == 0 ? O.CR : arr == 1 ? O.CC : O.CT;
+        put_split8(srow(dst, K.poff[iu] + (int64_t)T.dom_idx[o + row] * K.ld[iu], K.koff[iu * n + iv] + col), v);
+      }
+    }
+  }
+}
+
 // JP_ij block k: rows x of D_ij, columns c of D_ik.  Grid (k, (i,j)).
 template <bool SPLIT>
 __global__ __launch_bounds__(256) void jp_kernel(PairTab T, PanelTab K, const double* __restrict__ Jvv, void* JP,
@@ -250,11 +407,14 @@ __global__ __launch_bounds__(256) void u_absmax_kernel(const double* __restrict_
 }
 
 // XT+[p(a,b)][Q] = C+_ab, XT-[q(a,b)][Q] = C-_ab of walk Q (0 outside its
-// domain), rows of ldw values.  Block: one a, 32 b and 32 walks; the walks'
-// elements are read along b and leave through LDS along Q.
+// domain), rows of ldw values, from the CI vector (the symmetric part of C_Q
+// is its singlet-coupled block, the antisymmetric part its triplet-coupled
+// one).  Block: one a, 32 b and 32 walks; the walks' elements are read along b
+// and leave through LDS along Q.
 template <bool SPLIT>
-__global__ __launch_bounds__(256) void xt_kernel(PairTab T, const int32_t* __restrict__ pos, const double* __restrict__ C,
-                                                 void* XTp, void* XTm, int64_t ldw, const float* scl, int f16) {
+__global__ __launch_bounds__(256) void xt_kernel(PairTab T, const int32_t* __restrict__ pos, const double* __restrict__ x,
+                                                 const IoSlot* __restrict__ io, void* XTp, void* XTm, int64_t ldw, const float* scl, int f16) {
+  if (io) x = io->x;
   __shared__ double tp[32][33], tm[32][33];
   const int nv = T.n_v, a = blockIdx.x, b0 = blockIdx.y * 32, Q0 = blockIdx.z * 32;
   if (b0 > a) return;
@@ -268,10 +428,14 @@ __global__ __launch_bounds__(256) void xt_kernel(PairTab T, const int32_t* __res
       const int pa = ps[a], pb = ps[b];
       if (pa >= 0 && pb >= 0) {
         const int d = (int)(T.dom_off[Q + 1] - T.dom_off[Q]);
-        const double* Cq = C + T.cd_off[Q];
-        const double x = Cq[(int64_t)pa * d + pb], y = Cq[(int64_t)pb * d + pa];
-        vp = 0.5 * (x + y);
-        vm = 0.5 * (x - y);
+        const bool same = T.pairs[2 * Q] == T.pairs[2 * Q + 1];
+        if (pa == pb) {
+          vp = same ? x[T.aa_off[Q] + pa] : -x[T.aa_off[Q] + pa] * INV_SQRT2;
+        } else {  // domains are sorted: pa > pb
+          const int64_t idx = T.ab_off[Q] + (int64_t)pa * (pa - 1) / 2 + pb;
+          vp = same ? x[idx] * INV_SQRT2 : -0.5 * x[idx];
+          if (!same) vm = -x[idx + (int64_t)d * (d - 1) / 2] * 0.28867513459481288225;  // 1 / (2 sqrt3)
+        }
       }
     }
     tp[r][tx] = vp;
@@ -346,7 +510,7 @@ struct PackSrc {
   const double* Sm;     // [nsp][ncm][nm]
   int64_t sp_part, sm_part;
   int nsp;
-  const double* Hp;     // [n_pairs][np]
+  const double* Hp;     // [n_pairs][np], null: part of S+-
   const double* Hm;     // [ncm][nm]
   int64_t np, nm;
   const int32_t* colm;
@@ -394,39 +558,67 @@ __global__ __launch_bounds__(256) void pack_panels_kernel(PairTab T, PackSrc S, 
   const double c0 = x[0], ei = T.eps[i], ej = T.eps[j];
   __shared__ double tile[32][33];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  auto elem = [&](int r, int c) {  // [r][c] without the packed parts
-    const int64_t e = (int64_t)r * d + c;
-    double v = c0 * S.Kov[((int64_t)i * nv + D[r]) * niv + (int64_t)j * nv + D[c]];
-    for (int q = 0; q < S.nrp; ++q) v += Rp[q * S.rstride + e];
-    if (R) v += R[e];
-    return v;
-  };
-  for (int r = ty; r < 32; r += 8) {
-    const int yr = y0 + r, xc = x0 + tx;
-    tile[r][tx] = yr < d && xc < d ? elem(yr, xc) : 0.0;
-  }
-  __syncthreads();
-  for (int r = ty; r < 32; r += 8) {
-    const int xr = x0 + r, yc = y0 + tx;
-    if (xr >= d || yc > xr) continue;
-    double A = elem(xr, yc), B = tile[tx][r];
-    const int gx = D[xr], gy = D[yc];  // domains are sorted: gx >= gy
-    const int64_t p = P * S.np + tri(gx) + gy;
-    double sp = S.Hp[p];
-    for (int q = 0; q < S.nsp; ++q) sp += S.Sp[q * S.sp_part + p];
-    A += sp;
-    B += sp;
-    if (cm >= 0 && gx != gy) {
-      const int64_t m = cm * S.nm + tri(gx - 1) + gy;
-      double sm = S.Hm[m];
-      for (int q = 0; q < S.nsp; ++q) sm += S.Sm[q * S.sm_part + m];
-      A += sm;
-      B -= sm;
+  // elements [r + 8 u][c] (u < 4) without the packed parts, four rows' loads
+  // in flight together
+  auto elems = [&](int r, int rmax, int c, bool cok, double (&v)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = 0.0;
+    if (!cok) return;
+    int64_t e[4];
+    const int64_t kc = (int64_t)j * nv + D[c];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int rr = min(r + 8 * u, rmax);
+      e[u] = (int64_t)rr * d + c;
+      v[u] = c0 * S.Kov[((int64_t)i * nv + D[rr]) * niv + kc];
     }
-    const double fock = T.eps[no + gx] + T.eps[no + gy] - ei - ej + eadd;
-    auto put = [&](int64_t k, double v) {
-      v += fock * x[k];
-      sigma[k] = accum ? sigma[k] + v : v;
+#pragma unroll 2
+    for (int q = 0; q < S.nrp; ++q)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] += Rp[q * S.rstride + e[u]];
+    if (R)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] += R[e[u]];
+  };
+  double v[4];
+  elems(y0 + ty, d - 1, x0 + tx, x0 + tx < d, v);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) tile[ty + 8 * u][tx] = v[u];
+  __syncthreads();
+  const int yc = y0 + tx;
+  if (yc >= d) return;
+  elems(x0 + ty, d - 1, yc, true, v);
+  const int gy = D[yc];
+  double sp[4], sm[4];
+  int gx[4];
+  int64_t p[4], m[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    // clamped where the element lies outside (above the diagonal, beyond d):
+    // the loads stay in bounds and nothing is stored
+    const int xr = max(min(x0 + ty + 8 * u, d - 1), yc);
+    gx[u] = D[xr];  // domains are sorted: gx >= gy
+    p[u] = P * S.np + tri(gx[u]) + gy;
+    m[u] = cm >= 0 && gx[u] != gy ? cm * S.nm + tri(gx[u] - 1) + gy : -1;
+    sp[u] = S.Hp ? S.Hp[p[u]] : 0.0;
+    sm[u] = S.Hm && m[u] >= 0 ? S.Hm[m[u]] : 0.0;
+  }
+#pragma unroll 2
+  for (int q = 0; q < S.nsp; ++q)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      sp[u] += S.Sp[q * S.sp_part + p[u]];
+      if (m[u] >= 0) sm[u] += S.Sm[q * S.sm_part + m[u]];
+    }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int xr = x0 + ty + 8 * u;
+    if (xr >= d || yc > xr) continue;
+    const double A = v[u] + sp[u] + sm[u], B = tile[tx][ty + 8 * u] + sp[u] - sm[u];
+    const double fock = T.eps[no + gx[u]] + T.eps[no + gy] - ei - ej + eadd;
+    auto put = [&](int64_t k, double w) {
+      w += fock * x[k];
+      sigma[k] = accum ? sigma[k] + w : w;
     };
     if (xr == yc) {
       put(T.aa_off[P] + xr, i == j ? A : -SQRT2 * A);
@@ -520,8 +712,33 @@ bool panels_choose(const tci_plan& P) {
          8.0 * ((double)P.n_chol + 16.0) * P.n_v < 4.0e9;
 }
 
+// Do the pair terms of a split build run in split precision?  Where the
+// embedded products (6 N^3 + 4 N^2 n_chol, N = n_int n_v) cost at most eight
+// times the per-walk ones, i.e. the domains fill a good part of the virtual
+// space.  Elsewhere (small domains in a wide space) the pair terms are a few
+// percent of the ladder's work: they stay FP64, and the split error is the
+// ladder's alone.
+bool panels_split_rule(const tci_plan& P) {
+  const double N = (double)P.n_int * P.n_v;
+  if (8.0 * (6.0 * N * N + 3.0 * P.n_pairs * (double)P.n_v * P.n_v) > 48.0e9 || N >= 46340.0) return false;
+  const char* env = std::getenv("TCI_DENSE_PAIRS");
+  if (env && env[0] == '1') return true;
+  double f = 0.0;
+  for (int Q = 0; Q < P.n_pairs; ++Q) {
+    const double d = (double)(P.h_dom_off[Q + 1] - P.h_dom_off[Q]);
+    for (int e = 0; e < 2; ++e)
+      for (int k = 0; k < P.n_int; ++k) {
+        const int R = P.pairid[(size_t)P.h_pairs[2 * Q + e] * P.n_int + k];
+        if (R >= 0) f += 6.0 * d * d * (double)(P.h_dom_off[R + 1] - P.h_dom_off[R]);
+      }
+    f += 4.0 * d * d * (double)P.n_chol + 2.0 * d * P.n_v * (double)P.n_chol;
+  }
+  return 6.0 * N * N * N + 4.0 * N * N * (double)P.n_chol <= 8.0 * f;
+}
+
 void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st) {
   auto& Z = P.pp;
+  Z.split = panels_split_rule(P);
   const int n = P.n_int, nv = P.n_v, np_w = P.n_pairs;
   Z.h_koff.assign((size_t)n * n, -1);
   Z.h_ld.assign(n, 0);
@@ -605,7 +822,6 @@ void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st) {
   hipLaunchKernelGGL(u_kernel<false>, dim3((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n), dim3(256), 0, st,
                      nullptr, P.Lov.as<double>(), nv, P.n_chol, (int64_t)nv, (int64_t)n * nv, F.LovT.p, Z.ldu, nullptr, 0);
   TCI_HIP(hipGetLastError());
-  panels_programs(P, false, 0, 1, st);
 }
 
 // Split copies of the constant operands (scale slot 0) and zeroed panels.
@@ -639,28 +855,45 @@ void panels_build_split(tci_plan& P, hipStream_t st) {
     P.mx.bytes += (int64_t)b->bytes;
 }
 
-// Programs of one element type: W per internal orbital, the 4-internal product
-// over packed pairs, and the pair products with `mode` (shape_of) and `ks`
-// K-splits; for a split type also the FP64 3-internal products.
-void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st) {
+// W of every internal orbital.
+void add_w(tci_plan& P, NProgram& g, bool split) {
   auto& Z = P.pp;
   auto& F = split ? Z.s16 : Z.f64;
   const int n = P.n_int, nv = P.n_v, es = split ? 4 : 8;
   auto at = [&](const DevBuf& b, int64_t values) { return static_cast<const char*>(b.p) + values * es; };
-  F.W.clear();
-  F.W.split = split;
-  F.hole.clear();
-  F.hole.split = split;
-  // shapes of the side products: large tiles when they fill the chip
-  auto fill = [](int64_t m, int64_t nn, int64_t cnt, int t) { return cdiv(m, t) * cdiv(nn, t) * cnt; };
-  F.W.shape = fill(P.n_chol, nv, n, 128) >= 512 ? N128 : fill(P.n_chol, nv, n, 64) >= 256 ? N64 : N32K4;
-  F.hole.shape = fill(P.n_pairs, Z.np, 2, 128) >= 512 ? N128 : fill(P.n_pairs, Z.np, 2, 64) >= 256 ? N64 : N32K4;
-  for (int i = 0; i < n; ++i) {
-    F.W.add(P.W.as<double>() + (int64_t)i * P.n_chol * nv, nv, (int)P.n_chol, nv,
+  for (int i = 0; i < n; ++i)
+    g.add(P.W.as<double>() + (int64_t)i * P.n_chol * nv, nv, (int)P.n_chol, nv,
             {nseg(at(F.LP, Z.h_lpoff[i]), Z.h_ld[i], at(F.CT, Z.h_poff[i]), Z.h_ld[i], Z.h_ld[i], es)}, false,
             Blocking(), split ? 12 : -1);
-  }
-  F.W.upload_tables(st);
+}
+
+void panels_w_program(tci_plan& P, bool split, int shape, hipStream_t st) {
+  NProgram& g = (split ? P.pp.s16 : P.pp.f64).W;
+  g.clear();
+  g.split = split;
+  g.shape = shape;
+  add_w(P, g, split);
+  g.upload_tables(st);
+}
+
+// Programs of one element type: the 4-internal product over packed pairs, and
+// the pair products with `mode` (shape_of), `ks` K-splits and `order` (0:
+// walks by descending domain, so that the smallest tasks fill the tail of the
+// launch; 1: walks in plan order, dealt XCD-contiguously, so that the walks of
+// one i share its panels in an L2); for a split type also the FP64 3-internal
+// products.
+// With `into` the pair products' tasks go there instead (its shape is set).
+void panels_programs(tci_plan& P, bool split, int mode, int ks, int order, hipStream_t st, NProgram* into = nullptr) {
+  auto& Z = P.pp;
+  auto& F = split ? Z.s16 : Z.f64;
+  const int n = P.n_int, nv = P.n_v, es = split ? 4 : 8;
+  auto at = [&](const DevBuf& b, int64_t values) { return static_cast<const char*>(b.p) + values * es; };
+  if (!into) {
+  F.hole.clear();
+  F.hole.split = split;
+  // large tiles when they fill the chip
+  auto fill = [](int64_t m, int64_t nn, int64_t cnt, int t) { return cdiv(m, t) * cdiv(nn, t) * cnt; };
+  F.hole.shape = fill(P.n_pairs, Z.np, 2, 128) >= 512 ? N128 : fill(P.n_pairs, Z.np, 2, 64) >= 256 ? N64 : N32K4;
   const void* hP = split ? F.hP.p : Z.holeP.p;
   const void* hM = split ? F.hM.p : Z.holeM.p;
   F.hole.add(Z.Hp.as<double>(), Z.np, P.n_pairs, (int)Z.np, {nseg(hP, Z.ldw, F.XTp.p, Z.ldw, Z.ldw, es)}, false,
@@ -669,23 +902,28 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st) 
     F.hole.add(Z.Hm.as<double>(), Z.nm, Z.ncm, (int)Z.nm, {nseg(hM, Z.ldw, F.XTm.p, Z.ldw, Z.ldw, es)}, false,
                Blocking(), split ? 5 : -1);
   F.hole.upload_tables(st);
+  }
   // pair products
   F.ks = ks;
-  F.pair.clear();
-  F.pair.resize(4);
-  for (int s = 0; s < 4; ++s) {
+  if (!into) {
+    F.pair.clear();
+    F.pair.resize(4);
+  }
+  for (int s = 0; s < (into ? 0 : 4); ++s) {
     F.pair[s].split = split;
     F.pair[s].shape = s;
+    F.pair[s].remap = order;
   }
   TCI_REQUIRE(ks >= 1 && ks <= kMaxKs, "K-splits of the pair products out of range");
-  Z.rank.clear();
+  if (split) Z.rank.clear();
   Z.rank.shape = P.dmax <= 64 ? N64 : N128;
-  std::vector<int> order(P.n_pairs);
-  for (int Q = 0; Q < P.n_pairs; ++Q) order[Q] = Q;
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-    return P.h_dom_off[a + 1] - P.h_dom_off[a] > P.h_dom_off[b + 1] - P.h_dom_off[b];
-  });
-  for (int Q : order) {
+  std::vector<int> walks(P.n_pairs);
+  for (int Q = 0; Q < P.n_pairs; ++Q) walks[Q] = Q;
+  if (order == 0)
+    std::stable_sort(walks.begin(), walks.end(), [&](int a, int b) {
+      return P.h_dom_off[a + 1] - P.h_dom_off[a] > P.h_dom_off[b + 1] - P.h_dom_off[b];
+    });
+  for (int Q : walks) {
     const int i = P.h_pairs[2 * Q], j = P.h_pairs[2 * Q + 1];
     const int d = (int)(P.h_dom_off[Q + 1] - P.h_dom_off[Q]);
     const int32_t* D = P.dom_idx.as<int32_t>() + P.h_dom_off[Q];
@@ -695,9 +933,24 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st) 
     const char *Jij = at(F.JP, Z.h_jpoff[(size_t)i * n + j]), *Jji = at(F.JP, Z.h_jpoff[(size_t)j * n + i]);
     const char *Ui = at(F.U, (int64_t)i * nv * Z.ldu), *Uj = at(F.U, (int64_t)j * nv * Z.ldu);
     const char *Li = at(F.LovT, (int64_t)i * nv * Z.ldu), *Lj = at(F.LovT, (int64_t)j * nv * Z.ldu);
-    std::vector<NSeg> sg = {nseg(CRi, li, Jij, li, li, es, D, nullptr), nseg(Jij, li, CCi, li, li, es, nullptr, D),
-                            nseg(Jji, lj, CRj, lj, lj, es, nullptr, D), nseg(CCj, lj, Jji, lj, lj, es, D, nullptr),
-                            nseg(Ui, Z.ldu, Lj, Z.ldu, Z.ldu, es, D, D), nseg(Li, Z.ldu, Uj, Z.ldu, Z.ldu, es, D, D)};
+    // the two ranges that read one JP run interleaved in chunks of k, so that
+    // its second read finds it in cache
+    std::vector<NSeg> sg;
+    auto two = [&](const NSeg& u, const NSeg& v) {
+      constexpr int64_t chunk = 4096;  // bytes of k: 512 FP64 values, 1024 split ones
+      for (int64_t k = 0; k < u.kbytes; k += chunk)
+        for (const NSeg* q : {&u, &v}) {
+          NSeg c = *q;
+          c.A = static_cast<const char*>(q->A) + k;
+          c.B = static_cast<const char*>(q->B) + k;
+          c.kbytes = std::min(chunk, q->kbytes - k);
+          sg.push_back(c);
+        }
+    };
+    two(nseg(CRi, li, Jij, li, li, es, D, nullptr), nseg(Jij, li, CCi, li, li, es, nullptr, D));
+    two(nseg(Jji, lj, CRj, lj, lj, es, nullptr, D), nseg(CCj, lj, Jji, lj, lj, es, D, nullptr));
+    sg.push_back(nseg(Ui, Z.ldu, Lj, Z.ldu, Z.ldu, es, D, D));
+    sg.push_back(nseg(Li, Z.ldu, Uj, Z.ldu, Z.ldu, es, D, D));
     const double* Oij = Z.O3T.as<double>() + ((int64_t)i * n + j) * nv * Z.nk;
     const double* Oji = Z.O3T.as<double>() + ((int64_t)j * n + i) * nv * Z.nk;
     const NSeg r1 = nseg(Z.sTp.p, Z.nk, Oij, Z.nk, Z.nk, 8, D, D), r2 = nseg(Oji, Z.nk, Z.sTp.p, Z.nk, Z.nk, 8, D, D);
@@ -709,7 +962,7 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st) 
     }
     int64_t tot = 0;
     for (const NSeg& s : sg) tot += s.kbytes;
-    NProgram& g = F.pair[shape_of(mode, d)];
+    NProgram& g = into ? *into : F.pair[shape_of(mode, d)];
     for (int s = 0; s < ks; ++s) {
       const int64_t b0 = (tot * s / ks) & ~(int64_t)127, b1 = s + 1 == ks ? tot : (tot * (s + 1) / ks) & ~(int64_t)127;
       std::vector<NSeg> part;
@@ -729,6 +982,7 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st) 
             split ? 5 : -1);
     }
   }
+  if (into) return;
   for (auto& g : F.pair) g.upload_tables(st);
   if (split) Z.rank.upload_tables(st);
 }
@@ -742,32 +996,63 @@ void panels_tune(tci_plan& P, int precision, hipStream_t st) {
   // split types keep an FP32 chain no longer than about a quarter of the
   // contraction (the partial sums meet in FP64)
   const int kmin = split ? 4 : 1;
+  auto wrule = [&] {
+    auto fill = [&](int t) { return cdiv(P.n_chol, t) * cdiv(P.n_v, t) * P.n_int; };
+    return fill(128) >= 512 ? N128 : fill(64) >= 256 ? N64 : N32K4;
+  };
   if (!autotune_enabled()) {
-    panels_programs(P, split, 0, kmin, st);
+    panels_w_program(P, split, wrule(), st);
+    panels_programs(P, split, 0, kmin, 0, st);
     return;
   }
   if (split && Z.tuned_mode >= 0) {  // tuned for the other split precision: same tiles, same sums
-    panels_programs(P, split, Z.tuned_mode, Z.tuned_ks, st);
-    for (auto& g : F.pair) g.remap = Z.tuned_order;
+    panels_w_program(P, split, Z.tuned_w, st);
+    panels_programs(P, split, Z.tuned_mode, Z.tuned_ks, Z.tuned_order, st);
     return;
   }
+  // operands of a random vector (scales of fp16x3 included) before the timing
+  panels_w_program(P, split, wrule(), st);
+  panels_programs(P, split, 0, kmin, 0, st);
+  DevBuf xr;
+  P.tune_vector(xr, st);
+  if (precision == TCI_SIGMA_FP16X3)
+    launch_split_scales(1, P.C.as<double>(), P.sum_d2, P.mx.maxbits.as<unsigned>(), 0, P.mx.scales.as<float>(),
+                        (float)P.dmax, st);
+  P.run_Y(precision, st);
+  panels_terms(P, precision, false, xr.as<double>(), nullptr, st);
+  TCI_HIP(hipStreamSynchronize(st));
   static const char* mname[4] = {"by size", "128", "64", "32k4"};
   double tiles128 = 0.0;
   for (int Q = 0; Q < P.n_pairs; ++Q) {
     const int64_t c = cdiv(P.h_dom_off[Q + 1] - P.h_dom_off[Q], 128);
     tiles128 += (double)(c * c);
   }
-  std::string log = std::string(split ? "split" : "fp64") + " pair panels:";
+  std::string log = std::string(split ? "split" : "fp64") + " pair panels: W";
   double best = 1e300;
+  int bw = N128;
+  std::vector<int> wshapes = {N128, N192, N64};
+  if (split) wshapes.push_back(N128x192);
+  if (wrule() == N32K4) wshapes.push_back(N32K4);
+  for (int sh : wshapes) {
+    panels_w_program(P, split, sh, st);
+    const double ms = time_ms(st, 2, [&] { F.W.launch(precision, st, 0, sc); });
+    log += " " + std::to_string(F.W.tm()) + "x" + std::to_string(F.W.tn()) + ":" + fmt_ms(ms);
+    if (ms < best * 0.98) {
+      best = ms;
+      bw = sh;
+    }
+  }
+  panels_w_program(P, split, bw, st);
+  log += "; products";
+  best = 1e300;
   int bm = 0, bk = kmin, bo = 0;
   for (int mode = 0; mode < 4; ++mode) {
     if (mode == 3 && tiles128 > 256) continue;  // enough tiles without K-groups
     if (mode == 2 && tiles128 > 4096) continue;
     for (int ks : {1, 2, 4, 8}) {
       if (ks < kmin || (ks > kmin && tiles128 * ks > 8192)) continue;
-      panels_programs(P, split, mode, ks, st);
       for (int o = 0; o < (xcd_remap_forced() ? 1 : 2); ++o) {
-        for (auto& g : F.pair) g.remap = o;
+        panels_programs(P, split, mode, ks, o, st);
         const double ms = time_ms(st, 2, [&] {
           for (const auto& g : F.pair) g.launch(precision, st, 0, sc);
         });
@@ -781,20 +1066,178 @@ void panels_tune(tci_plan& P, int precision, hipStream_t st) {
       }
     }
   }
-  panels_programs(P, split, bm, bk, st);
-  for (auto& g : F.pair) g.remap = bo;
+  panels_programs(P, split, bm, bk, bo, st);
   if (split) {
     Z.tuned_mode = bm;
     Z.tuned_ks = bk;
     Z.tuned_order = bo;
+    Z.tuned_w = bw;
   }
-  P.tuning += log + " -> " + mname[bm] + "/" + std::to_string(bk) + (bo ? "x" : "") + "\n";
+  P.tuning += log + " -> W " + std::to_string(F.W.tm()) + "x" + std::to_string(F.W.tn()) + ", " + mname[bm] + "/" +
+              std::to_string(bk) + (bo ? "x" : "") + "\n";
   TCI_HIP(hipStreamSynchronize(st));
 }
 
-// Pair terms of one sigma into the K-split partials and H+-; needs C, s and Y.
-void panels_terms(tci_plan& P, int precision, hipStream_t st) {
+// Small FP64 builds: S+-, W and Y do not depend on each other and none fills
+// the chip, so they go out as one launch on small tiles; likewise the pair
+// products and gW.  Kept where the one launch beats the separate ones: at
+// 5/30/175 the first group takes 12 us instead of 35, the second 12 instead of 25.
+void panels_merge(tci_plan& P, hipStream_t st) {
   auto& Z = P.pp;
+  auto& F = Z.f64;
+  Z.m1on = Z.m2on = false;
+  double fl = F.W.alg_flops;
+  for (const auto& g : F.pair) fl += g.alg_flops;
+  if (!autotune_enabled() || !P.vv.fp64 || fl + P.vv.g64.alg_flops > 4.0e10) return;
+  const bool sing = P.singles_nt();
+  Z.m1_singles = Z.m2_singles = sing;
+  std::string log = "fp64 merged launches:";
+  const int kp0 = F.ks;
+  // S, W, Y
+  double t0 = time_ms(st, 3, [&] {
+    P.vv.g64.launch(TCI_SIGMA_FP64, st);
+    F.W.launch(TCI_SIGMA_FP64, st);
+    if (sing) P.nprogY.launch(TCI_SIGMA_FP64, st);
+  });
+  log += " S, W, Y separate:" + fmt_ms(t0);
+  double best = t0 * 0.98;
+  int bs = -1, bk = 1;
+  auto build1 = [&](int sh, int ks) {
+    Z.m1.clear();
+    Z.m1.shape = sh;
+    vv_add_products(P, Z.m1, false, ks);
+    add_w(P, Z.m1, false);
+    if (sing) P.add_singles_Y(Z.m1);
+    Z.m1.upload_tables(st);
+  };
+  const int64_t kmin = P.vv.ncm > 0 ? std::min(P.vv.np, P.vv.nm) : P.vv.np;
+  for (int sh : {(int)N64, (int)N32K4})
+    for (int ks : {1, 2, 4}) {
+      if (ks > 1 && ks > kmin / 64) continue;
+      build1(sh, ks);
+      const double ms = time_ms(st, 3, [&] { Z.m1.launch(TCI_SIGMA_FP64, st); });
+      log += std::string(sh == N64 ? " 64/" : " 32k4/") + std::to_string(ks) + ":" + fmt_ms(ms);
+      if (ms < best) {
+        best = ms;
+        bs = sh;
+        bk = ks;
+      }
+    }
+  if (bs >= 0) {
+    build1(bs, bk);
+    Z.m1on = true;
+    Z.m1_ks = bk;
+  } else {
+    Z.m1.clear();
+  }
+  // pair products, gW
+  t0 = time_ms(st, 3, [&] {
+    for (const auto& g : F.pair) g.launch(TCI_SIGMA_FP64, st);
+    if (sing) P.nprogGW.launch(TCI_SIGMA_FP64, st);
+  });
+  log += "; pairs, gW separate:" + fmt_ms(t0);
+  best = t0 * 0.98;
+  bs = -1;
+  auto build2 = [&](int sh, int ks) {
+    Z.m2.clear();
+    Z.m2.shape = sh;
+    panels_programs(P, false, 0, ks, 0, st, &Z.m2);
+    if (sing) P.add_singles_GW(Z.m2);
+    Z.m2.upload_tables(st);
+  };
+  for (int sh : {(int)N64, (int)N32K4})
+    for (int ks : {1, 2, 4, 8}) {
+      build2(sh, ks);
+      const double ms = time_ms(st, 3, [&] { Z.m2.launch(TCI_SIGMA_FP64, st); });
+      log += std::string(sh == N64 ? " 64/" : " 32k4/") + std::to_string(ks) + ":" + fmt_ms(ms);
+      if (ms < best) {
+        best = ms;
+        bs = sh;
+        bk = ks;
+      }
+    }
+  if (bs >= 0) {
+    build2(bs, bk);
+    Z.m2on = true;
+    Z.m2_ks = bk;
+  } else {
+    Z.m2.clear();
+  }
+  F.ks = kp0;  // of the separate programs, which split builds may run
+  P.tuning += log + " -> " + (Z.m1on ? "merged " : "separate ") + (Z.m2on ? "merged" : "separate") + "\n";
+  TCI_HIP(hipStreamSynchronize(st));
+}
+
+// arithmetic of the pair terms in a build of this precision
+int panels_precision(const tci_plan& P, int precision) {
+  return precision != TCI_SIGMA_FP64 && P.pp.split ? precision : (int)TCI_SIGMA_FP64;
+}
+
+// Is the 4-internal product a K-range of the resident ladder's product?  Then
+// its operand XT+- is written before the ladder and no H+- exists.  Not where
+// the two differ in arithmetic or (fp16x3) in their scales.
+bool panels_hole_in_ladder(const tci_plan& P, int precision) {
+  return P.pp.on && panels_precision(P, precision) == precision &&
+         (precision == TCI_SIGMA_FP64 ? P.vv.fp64 : precision == TCI_SIGMA_BF16X3 && P.vv.split);
+}
+
+// One pass over the CI vector for everything the build reads of it (FP64 and
+// bf16x3); false where the separate kernels are needed.
+bool panels_expand(tci_plan& P, int precision, const double* x, const IoSlot* io, hipStream_t st) {
+  if (!P.pp.on) return false;
+  auto& Z = P.pp;
+  const bool vv = precision != TCI_SIGMA_FP64 ? P.vv.split : P.vv.fp64;
+  const int pp = panels_precision(P, precision);
+  if (pp == TCI_SIGMA_FP16X3 || (vv && pp != precision)) return false;
+  const bool split = pp != TCI_SIGMA_FP64;
+  auto& F = split ? Z.s16 : Z.f64;
+  ExpandOut O{};
+  // C itself is read by the Cholesky-direct ladders and the virtual Fock products
+  O.C = !vv || P.has_fvv ? P.C.as<double>() : nullptr;
+  O.Ct = P.Ct.as<double>();
+  O.s = P.s.as<double>();
+  O.sT = Z.sTp.as<double>();
+  O.nk = Z.nk;
+  O.CR = F.CR.p;
+  O.CC = F.CC.p;
+  O.CT = F.CT.p;
+  if (vv) {
+    O.Xp = split ? P.vv.Xpx.p : P.vv.Xp.p;
+    O.Xm = split ? P.vv.Xmx.p : P.vv.Xm.p;
+    O.ldp = split ? xpad(Z.np) : up(Z.np, 2);
+    O.ldm = split ? xpad(Z.nm) : up(Z.nm, 2);
+  }
+  O.colm = Z.colm.as<int32_t>();
+  const int nt = (P.dmax + 31) / 32;
+  const dim3 g((unsigned)std::max(nt * (nt + 1) / 2, 4), P.n_pairs + 1);
+  const PanelTab K = ptab(P);
+  if (split) hipLaunchKernelGGL(expand_kernel<true>, g, dim3(256), 0, st, P.tab, K, x, io, O);
+  else hipLaunchKernelGGL(expand_kernel<false>, g, dim3(256), 0, st, P.tab, K, x, io, O);
+  TCI_HIP(hipGetLastError());
+  return true;
+}
+
+// XT+- from the CI vector (needs no scale but that of fp16x3's pair products)
+void panels_xt(tci_plan& P, int precision, const double* x, const IoSlot* io, hipStream_t st) {
+  auto& Z = P.pp;
+  precision = panels_precision(P, precision);
+  const bool split = precision != TCI_SIGMA_FP64;
+  const int f16 = precision == TCI_SIGMA_FP16X3 ? 1 : 0;
+  const dim3 g((unsigned)P.n_v, (unsigned)cdiv(P.n_v, 32), (unsigned)cdiv(P.n_pairs, 32));
+  if (split)
+    hipLaunchKernelGGL(xt_kernel<true>, g, dim3(256), 0, st, P.tab, P.pos.as<int32_t>(), x, io, Z.s16.XTp.p, Z.s16.XTm.p,
+                       Z.ldw, P.mx.scales.as<float>() + 6, f16);
+  else
+    hipLaunchKernelGGL(xt_kernel<false>, g, dim3(256), 0, st, P.tab, P.pos.as<int32_t>(), x, io,
+                       Z.f64.XTp.p, Z.f64.XTm.p, Z.ldw, nullptr, 0);
+  TCI_HIP(hipGetLastError());
+}
+
+// Pair terms of one sigma into the K-split partials and H+-; needs Y, and C and
+// s unless panels_expand has written the panels (`expanded`).
+void panels_terms(tci_plan& P, int build, bool expanded, const double* x, const IoSlot* io, hipStream_t st) {
+  auto& Z = P.pp;
+  const int precision = panels_precision(P, build);
   const bool split = precision != TCI_SIGMA_FP64;
   auto& F = split ? Z.s16 : Z.f64;
   const int n = P.n_int, nv = P.n_v;
@@ -805,7 +1248,7 @@ void panels_terms(tci_plan& P, int precision, hipStream_t st) {
   const PanelTab K = ptab(P);
   const int nt = (P.dmax + 31) / 32;
   auto run = [&](const std::string& role, const NProgram& g, int prec) {
-    if (!g.tasks.empty()) P.kt_run(pn + " " + role, g, precision, st, [&] { g.launch(prec, st, 0, sc); });
+    if (!g.tasks.empty()) P.kt_run(pn + " " + role, g, build, st, [&] { g.launch(prec, st, 0, sc); });
   };
   auto panels = [&](int what) {
     const dim3 g(nt * nt, P.n_pairs);
@@ -816,14 +1259,17 @@ void panels_terms(tci_plan& P, int precision, hipStream_t st) {
       hipLaunchKernelGGL(panels_kernel<false>, g, dim3(256), 0, st, P.tab, K, P.C.as<double>(), F.CR.p, F.CC.p, F.CT.p,
                          nullptr, nullptr, 0, 3);
   };
-  int e0 = P.kt_begin(st);
-  if (f16) hipLaunchKernelGGL(panel_scales_kernel, dim3(1), dim3(64), 0, st, 0, mx, sc);
-  panels(f16 ? 2 : 3);  // fp16x3: the scale of CR and CC waits for max|U|
-  hipLaunchKernelGGL(st_kernel, dim3(gsz((int64_t)nv * Z.nk)), dim3(256), 0, st, P.s.as<double>(), n, nv, Z.nk,
-                     Z.sTp.as<double>());
-  TCI_HIP(hipGetLastError());
-  P.kt_end(e0, pn + " pair panels", 0.0, precision, st);
-  run("pair product W", F.W, precision);
+  int e0 = -1;
+  if (!expanded) {
+    e0 = P.kt_begin(st);
+    if (f16) hipLaunchKernelGGL(panel_scales_kernel, dim3(1), dim3(64), 0, st, 0, mx, sc);
+    panels(f16 ? 2 : 3);  // fp16x3: the scale of CR and CC waits for max|U|
+    hipLaunchKernelGGL(st_kernel, dim3(gsz((int64_t)nv * Z.nk)), dim3(256), 0, st, P.s.as<double>(), n, nv, Z.nk,
+                       Z.sTp.as<double>());
+    TCI_HIP(hipGetLastError());
+    P.kt_end(e0, pn + " pair panels", 0.0, build, st);
+  }
+  if (build != TCI_SIGMA_FP64 || !Z.m1on) run("pair product W", F.W, precision);
   e0 = P.kt_begin(st);
   if (f16) {
     hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(64), 0, st, mx + 1);
@@ -833,25 +1279,26 @@ void panels_terms(tci_plan& P, int precision, hipStream_t st) {
     panels(1);
   }
   const dim3 gu((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n);
-  const dim3 gx((unsigned)nv, (unsigned)cdiv(nv, 32), (unsigned)cdiv(P.n_pairs, 32));
   const int64_t wi = P.n_chol * nv;
   if (split) {
     hipLaunchKernelGGL(u_kernel<true>, gu, dim3(256), 0, st, P.Y.as<double>(), P.W.as<double>(), nv, P.n_chol, wi,
                        (int64_t)nv, F.U.p, Z.ldu, sc + 6, f16);
-    hipLaunchKernelGGL(xt_kernel<true>, gx, dim3(256), 0, st, P.tab, P.pos.as<int32_t>(), P.C.as<double>(), F.XTp.p,
-                       F.XTm.p, Z.ldw, sc + 6, f16);
   } else {
     hipLaunchKernelGGL(u_kernel<false>, gu, dim3(256), 0, st, P.Y.as<double>(), P.W.as<double>(), nv, P.n_chol, wi,
                        (int64_t)nv, F.U.p, Z.ldu, nullptr, 0);
-    hipLaunchKernelGGL(xt_kernel<false>, gx, dim3(256), 0, st, P.tab, P.pos.as<int32_t>(), P.C.as<double>(), F.XTp.p,
-                       F.XTm.p, Z.ldw, nullptr, 0);
   }
   TCI_HIP(hipGetLastError());
-  P.kt_end(e0, pn + " pair panels", 0.0, precision, st);
-  for (const auto& g : F.pair) run("pair products", g, precision);
+  const bool hole = !panels_hole_in_ladder(P, build);
+  if (hole) panels_xt(P, precision, x, io, st);
+  P.kt_end(e0, pn + " pair panels", 0.0, build, st);
+  if (build == TCI_SIGMA_FP64 && Z.m2on) {
+    run("pair products, gW", Z.m2, precision);
+  } else {
+    for (const auto& g : F.pair) run("pair products", g, precision);
+  }
   if (split && !Z.rank.tasks.empty())
-    P.kt_run(pn + " 3-internal products", Z.rank, precision, st, [&] { Z.rank.launch(TCI_SIGMA_FP64, st); });
-  run("4-internal product", F.hole, precision);
+    P.kt_run(pn + " 3-internal products", Z.rank, build, st, [&] { Z.rank.launch(TCI_SIGMA_FP64, st); });
+  if (hole) run("4-internal product", F.hole, precision);
 }
 
 // sigma from the pair terms' partials, the ladder (packed S+- when `packed`,
@@ -859,23 +1306,26 @@ void panels_terms(tci_plan& P, int precision, hipStream_t st) {
 void panels_pack(tci_plan& P, int precision, bool packed, bool use_r, const double* x, const IoSlot* io, int flags,
                  double* y, hipStream_t st) {
   auto& Z = P.pp;
-  const bool split = precision != TCI_SIGMA_FP64;
+  const bool split = precision != TCI_SIGMA_FP64, psplit = split && Z.split;
   PackSrc S{};
   S.Rp = Z.Rp.as<double>();
   S.rstride = P.sum_d2;
-  S.nrp = (split ? Z.s16.ks : Z.f64.ks) + (split ? 1 : 0);
+  // an FP64 build may have merged its pair products on another K-split
+  S.nrp = psplit ? Z.s16.ks + 1 : split || !Z.m2on ? Z.f64.ks : Z.m2_ks;
   S.R = use_r ? P.R.as<double>() : nullptr;
   S.np = Z.np;
   S.nm = Z.nm;
   if (packed) {
-    S.nsp = split ? P.vv.ksx : P.vv.ks;
+    S.nsp = split ? P.vv.ksx : Z.m1on ? Z.m1_ks : P.vv.ks;
     S.Sp = P.vv.Sp.as<double>();
     S.Sm = P.vv.Sm.as<double>();
     S.sp_part = (int64_t)P.n_pairs * Z.np;
     S.sm_part = (int64_t)std::max(Z.ncm, 1) * Z.nm;
   }
-  S.Hp = Z.Hp.as<double>();
-  S.Hm = Z.Hm.as<double>();
+  if (!panels_hole_in_ladder(P, precision)) {
+    S.Hp = Z.Hp.as<double>();
+    S.Hm = Z.Hm.as<double>();
+  }
   S.colm = Z.colm.as<int32_t>();
   S.Kov = P.Kov.as<double>();
   const int nt = (P.dmax + 31) / 32;

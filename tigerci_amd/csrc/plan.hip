@@ -471,15 +471,15 @@ void tci_plan::build(const tci_problem& p) {
     fockvv.upload_tables(st);
   }
   if (pp.on) panels_build(*this, o4, st);
-  // Y[i][J][a] = sum_c L^J_ac s_i^c: s rows against the rows (J, a) of L^J on
-  // the NT GEMM where those rows are 16-byte aligned FP64; otherwise L^J sT on
-  // the dense kernel, its columns i stored n_chol n_v apart
-  const bool nt_ok = !lvv_f32 && n_v % 2 == 0;
+  // Y[i][J][a] = sum_c L^J_ac s_i^c: on the NT GEMM where the rows of L^J are
+  // 16-byte aligned FP64; otherwise L^J sT on the dense kernel, its columns i
+  // stored n_chol n_v apart
+  const bool nt_ok = singles_nt();
   progY.clear();
   nprogY.clear();
   if (nt_ok) {
     nprogY.shape = N64;
-    nprogY.add(Y.as<double>(), n_chol * n_v, n_int, (int)(n_chol * n_v), {nseg(s.p, n_v, Lvv.p, n_v, n_v, 8)}, false);
+    add_singles_Y(nprogY);
     nprogY.upload_tables(st);
   } else {
     Blocking by;
@@ -514,28 +514,23 @@ void tci_plan::build(const tci_problem& p) {
   // gW[s][i][a] = sum_{J in split s} sum_b W[i][J][b] L^J_ab
   progGW.clear();
   nprogGW.clear();
-  progGW.dense = true;
-  progGW.tile = 64;
   nprogGW.shape = N64;
-  for (int sp = 0; sp < n_split; ++sp) {
-    const int64_t J0 = n_chol * sp / n_split, J1 = n_chol * (sp + 1) / n_split;
-    double* out = gW.as<double>() + (int64_t)sp * niv;
-    if (nt_ok) {
-      std::vector<NSeg> sg;
-      for (int64_t J = J0; J < J1; ++J)
-        sg.push_back(nseg(W.as<double>() + J * n_v, n_chol * n_v, Lvv.as<double>() + J * n_v * n_v, n_v, n_v, 8));
-      nprogGW.add(out, n_v, n_int, n_v, sg, false);
-      continue;
+  if (nt_ok) {
+    add_singles_GW(nprogGW);
+  } else {
+    progGW.dense = true;
+    progGW.tile = 64;
+    for (int sp = 0; sp < n_split; ++sp) {
+      const int64_t J0 = n_chol * sp / n_split, J1 = n_chol * (sp + 1) / n_split;
+      const void* Lb = lvv_f32 ? (const void*)(Lvv.as<float>() + J0 * n_v * n_v) : (const void*)(Lvv.as<double>() + J0 * n_v * n_v);
+      progGW.add(gW.as<double>() + (int64_t)sp * niv, n_v, n_int, n_v,
+                 {seg(op(W.as<double>() + J0 * n_v, n_chol * n_v, 1), op(Lb, n_v, 1, nullptr, nullptr, lvv_f32),
+                      (int)((J1 - J0) * n_v), 1.0)},
+                 false);
     }
-    const void* Lb = lvv_f32 ? (const void*)(Lvv.as<float>() + J0 * n_v * n_v) : (const void*)(Lvv.as<double>() + J0 * n_v * n_v);
-    progGW.add(out, n_v, n_int, n_v,
-               {seg(op(W.as<double>() + J0 * n_v, n_chol * n_v, 1), op(Lb, n_v, 1, nullptr, nullptr, lvv_f32),
-                    (int)((J1 - J0) * n_v), 1.0)},
-               false);
   }
   progGW.upload_tables(st);
   nprogGW.upload_tables(st);
-  // gss = (2K - J) s runs as a GEMV (launch_gemv) inside every sigma
 
   // ---- ladder work items -------------------------------------------------------
   {
@@ -566,6 +561,13 @@ void tci_plan::build(const tci_problem& p) {
       ladder.build(items, cost, dmax, st);
       lad_part.alloc((size_t)lad_chunks * sum_d2 * 8);
     }
+  }
+  // schedules are timed on a random vector: zero operands draw less power and
+  // rank the candidates differently (34/192/1200: 64 x 64 pair tiles 6.5 ms on
+  // zeros and 7.9 ms on data, tiles by domain size 6.8 and 7.1 ms)
+  if (autotune_enabled()) {
+    DevBuf x;
+    tune_vector(x, st);
   }
   if (!ladder_fused) build_two_phase_ladder(st);
   // ladder from the resident (ab|cd) block: with autotuning, built when it
@@ -612,7 +614,10 @@ void tci_plan::build(const tci_problem& p) {
     }
   }
 
-  if (pp.on) panels_tune(*this, TCI_SIGMA_FP64, st);
+  if (pp.on) {
+    panels_tune(*this, TCI_SIGMA_FP64, st);
+    panels_merge(*this, st);
+  }
 
   // ---- accounting ---------------------------------------------------------------
   flops_ladder = 0.0;
@@ -637,12 +642,29 @@ void tci_plan::build(const tci_problem& p) {
   flops_sigma = flops_ladder + f_ring + 2.0 * (double)n_chol * n_v * niv * 3.0 + 2.0 * (double)niv * niv;
   TCI_HIP(hipDeviceSynchronize());
   device_bytes = 0;
-  for (DevBuf* b : {&pairs, &dom_off, &dom_idx, &cd_off, &aa_off, &ab_off, &eps, &pos, &xmap, &isect_off, &isect,
+  for (DevBuf* b : {&pairs, &dom_off, &dom_idx, &cd_off, &aa_off, &ab_off, &eps, &pos, &xmap, &cw_off, &isect_off, &isect,
                     &inv_off, &inv_q, &inv_pos, &gpart_off, &Lvv, &Lov, &Kov, &Jvv, &Mss, &O4, &O3, &vvd, &vvx,
                     &diag, &C, &Ct, &R, &s, &sT, &g, &gss, &gW, &Y, &W, &gpart, &part, &sig0, &lad_part, &Tbuf, &Rpart, &Lp, &Cw, &lp_off_all, &Fm,
                     &Fvvp, &Fov})
     device_bytes += (int64_t)b->bytes;
   device_bytes += vv_device_bytes(*this) + panels_device_bytes(*this);
+}
+
+// Y[i][(J,a)]: s rows against the rows (J, a) of L^J
+void tci_plan::add_singles_Y(NProgram& g) const {
+  g.add(Y.as<double>(), n_chol * n_v, n_int, (int)(n_chol * n_v), {nseg(s.p, n_v, Lvv.p, n_v, n_v, 8)}, false);
+}
+
+// gW[split][i][a]: one repeated range over the Cholesky vectors of a split
+void tci_plan::add_singles_GW(NProgram& g) const {
+  for (int sp = 0; sp < n_split; ++sp) {
+    const int64_t J0 = n_chol * sp / n_split, J1 = n_chol * (sp + 1) / n_split;
+    NSeg q = nseg(W.as<double>() + J0 * n_v, n_chol * n_v, Lvv.as<double>() + J0 * n_v * n_v, n_v, n_v, 8);
+    q.reps = J1 - J0;
+    q.sa = (int64_t)n_v * 8;
+    q.sb = (int64_t)n_v * n_v * 8;
+    g.add(gW.as<double>() + (int64_t)sp * n_int * n_v, n_v, n_int, n_v, {q}, false);
+  }
 }
 
 void tci_plan::drop_graphs() {
@@ -700,57 +722,77 @@ void tci_plan::kt_collect() {
   kev_used = 0;
 }
 
-// Two-phase ladder tables (dense FP64 MFMA programs).  Per chunk of Lc
-// Cholesky vectors starting at J0:
-//   pack    Lp_P[jj] = L^{J0+jj}[D_P, D_P]  (local-domain pairs only; full-domain
-//           pairs read L^J directly)
-//   phase 1 T_P[(jj,a)][c] = sum_k Lp_P[jj][a][k] C_P[k][c]       (128-wide tiles)
-//   phase 2 R_P[a][n]    += sum_jj sum_c T_P[jj][a][c] Lp_P[jj][c][n]
-//           (64-wide tiles, one K-segment per jj, K split into partial R
-//           buffers when the outputs alone cannot fill the chip)
-// Lc bounds T (8 bytes) plus Lp (4 or 8 bytes) per element of sum_P d_P^2.
+// A fixed random vector x, and its C, Ct and s, for timing schedules.
+void tci_plan::tune_vector(DevBuf& x, hipStream_t st) {
+  x.alloc((size_t)n_csf * 8);
+  launch_random(x.as<double>(), n_csf, st);
+  launch_unpack(tab, dmax, x.as<double>(), C.as<double>(), Ct.as<double>(), s.as<double>(), st);
+  TCI_HIP(hipStreamSynchronize(st));
+}
+
+// Y of the current s
+void tci_plan::run_Y(int precision, hipStream_t st) {
+  if (!nprogY.tasks.empty()) {
+    kt_run("singles Y", nprogY, precision, st, [&] { nprogY.launch(TCI_SIGMA_FP64, st); });
+  } else {
+    launch_transpose_small(s.as<double>(), n_int, n_v, sT.as<double>(), st);
+    kt_run("singles Y", progY, precision, st, [&] { progY.launch(st); });
+  }
+}
+
+// Two-phase ladder tables (FP64, on the NT GEMM).  Per chunk of Lc Cholesky
+// vectors starting at J0, dp = d rounded up to even (16-byte rows):
+//   pack    Lp_P[jj] = L^{J0+jj}[D_P, D_P], rows of dp (full-domain walks of an
+//           even n_v read an FP64 L^J itself)
+//   phase 1 T'_P[(jj,a)][c] = sum_k Lp_P[jj][a][k] C_P[c][k]
+//   phase 2 R_P[n][a]      += sum_jj sum_c Lp_P[jj][n][c] T'_P[jj][a][c]
+//           (one repeated K-range over the jj of a K-split, split into partial
+//           R buffers when the outputs alone cannot fill the chip)
+// L^J is symmetric, so R = L (L C^T)^T = L C L, and both phases read their
+// operands along k.  Lc bounds T' plus Lp per element of sum_P d_P dp.
 void tci_plan::build_two_phase_ladder(hipStream_t st) {
   lphase.clear();
   lchunks.clear();
-  const size_t lsz = lvv_f32 ? 4 : 8;
-  int64_t sum_local = 0;
+  auto dsz = [&](int P) { return h_dom_off[P + 1] - h_dom_off[P]; };
+  auto even = [](int64_t d) { return (d + 1) & ~(int64_t)1; };
+  const bool direct = !lvv_f32 && n_v % 2 == 0;  // full domains read L^J
+  int64_t sum_local = 0, sum_dp = 0;
   std::vector<int32_t> loc;
+  std::vector<int64_t> cpo(n_pairs + 1, 0);
   for (int P = 0; P < n_pairs; ++P) {
-    const int64_t d = h_dom_off[P + 1] - h_dom_off[P];
-    if (d != n_v) {
+    const int64_t e = dsz(P) * even(dsz(P));
+    cpo[P + 1] = cpo[P] + e;
+    sum_dp += e;
+    if (dsz(P) != n_v || !direct) {
       loc.push_back(P);
-      sum_local += d * d;
+      sum_local += e;
     }
   }
   n_local = (int)loc.size();
   upload(pairs_local, loc, st);
-  {
-    const char* env = std::getenv("TCI_LADDER_MERGED");
-    ladder_merged = n_local == 0 && n_pairs > 0 && !(env && env[0] == '0');
-  }
-  // L^J[D_P, D_P] of every local walk packed once per plan when that takes at
-  // most 96 GB and leaves 64 GB free (the split ladder's copies and the
-  // Davidson vectors); otherwise packed per chunk inside every sigma
+  upload(cw_off, cpo, st);
+  Cw.alloc((size_t)std::max<int64_t>(sum_dp, 1) * 8);
+  launch_fill(Cw.as<double>(), sum_dp, 0.0, st);  // padding columns stay zero
+  // L^J[D_P, D_P] of every packed walk once per plan when that takes at most 96
+  // GB and leaves 64 GB free (the split ladder's copies and the Davidson
+  // vectors); otherwise packed per chunk inside every sigma
   {
     const char* env = std::getenv("TCI_FP64_PREPACK");
-    const double need = (double)sum_local * (double)n_chol * (double)lsz;
+    const double need = (double)sum_local * (double)n_chol * 8.0;
     size_t freeb = 0, totalb = 0;
     TCI_HIP(hipMemGetInfo(&freeb, &totalb));
     lp_all = sum_local > 0 && !(env && env[0] == '0') && need <= 96.0e9 && need + 64.0e9 <= (double)freeb;
   }
   std::vector<int64_t> lpo_all(loc.size() + 1, 0);
   if (lp_all) {
-    for (size_t q = 0; q < loc.size(); ++q) {
-      const int64_t d = h_dom_off[loc[q] + 1] - h_dom_off[loc[q]];
-      lpo_all[q + 1] = lpo_all[q] + n_chol * d * d;
-    }
+    for (size_t q = 0; q < loc.size(); ++q) lpo_all[q + 1] = lpo_all[q] + n_chol * dsz(loc[q]) * even(dsz(loc[q]));
     upload(lp_off_all, lpo_all, st);
-    Lp.alloc((size_t)lpo_all.back() * lsz);
+    Lp.alloc((size_t)lpo_all.back() * 8);
     PackTab K{pairs_local.as<int32_t>(), lp_off_all.as<int64_t>(), n_local};
-    launch_pack_L(tab, K, Lvv.p, lvv_f32, 0, n_chol, Lp.p, st);
+    launch_pack_L(tab, K, Lvv.p, lvv_f32, 0, n_chol, Lp.as<double>(), st);
   }
-  const double budget = 8.0e9;  // bytes of T + Lp per chunk
-  const double per_J = 8.0 * (double)std::max<int64_t>(sum_d2, 1) + (lp_all ? 0.0 : (double)lsz * sum_local);
+  const double budget = 8.0e9;  // bytes of T' + Lp per chunk
+  const double per_J = 8.0 * (double)std::max<int64_t>(sum_dp, 1) + (lp_all ? 0.0 : 8.0 * sum_local);
   int64_t Lc = std::max<int64_t>(1, std::min<int64_t>(n_chol, (int64_t)(budget / per_J)));
   for (int64_t q = Lc; q >= std::max<int64_t>(1, Lc / 2); --q)
     if (n_chol % q == 0) { Lc = q; break; }
@@ -766,33 +808,30 @@ void tci_plan::build_two_phase_ladder(hipStream_t st) {
     }
     lchunks.push_back({J0, idx});
   }
-  if (ladder_merged) Cw.alloc((size_t)sum_d2 * 8);
-  Tbuf.alloc((size_t)Lc * sum_d2 * 8);
-  if (sum_local && !lp_all) Lp.alloc((size_t)Lc * sum_local * lsz);
-  // programs for a K-split fill target: phase 2 is split along K until it has
-  // about `target` workgroups (at most 16 splits)
-  // tile2: phase-2 tile of the per-walk programs (64 or 128)
-  // tile1: phase-1 tile of the per-walk programs for domains above 64 (64 or
-  //        128; 192 puts the domains of 129-192 on 192 x 192 tiles, 65-128 on 128)
-  // big: both phases of local domains of 129-192 on 192 x 192 tiles (one
-  //      workgroup per CU, so their K-split target is a quarter)
-  auto is_big = [&](int64_t d) { return d > 128 && d <= 192 && d != n_v; };
-  auto build = [&](int64_t target, int tile2, int tile1, bool big) {
-    int64_t tiles2 = 0, tiles_big = 0;
+  // T' of walk P starts at Lc cpo[P] for every chunk length, so that its
+  // padding columns, which phase 1 does not write, stay zero
+  Tbuf.alloc((size_t)Lc * std::max<int64_t>(sum_dp, 1) * 8);
+  launch_fill(Tbuf.as<double>(), Lc * sum_dp, 0.0, st);
+  if (sum_local && !lp_all) Lp.alloc((size_t)Lc * sum_local * 8);
+  // tile of a d-wide side: the one with the least padding among 64 (up to 64),
+  // 128 and 192
+  auto shape_of = [&](int64_t d) {
+    if (d <= 64) return (int)N64;
+    return cdiv(d, 192) * 192 < cdiv(d, 128) * 128 ? (int)N192 : (int)N128;
+  };
+  // programs for a K-split fill target (phase 2 is split along J until it has
+  // about that many workgroups, at most 16) and a phase-2 tiling: 0 by domain
+  // size, 1 all 64 x 64
+  auto build = [&](int64_t target, int p2) {
+    int64_t tiles2 = 0;
     for (int P = 0; P < n_pairs; ++P) {
-      const int64_t d = h_dom_off[P + 1] - h_dom_off[P];
-      if (big && is_big(d)) ++tiles_big;
-      else tiles2 += cdiv(d, tile2) * cdiv(d, tile2);
+      const int sh = p2 ? (int)N64 : shape_of(dsz(P));
+      const int64_t t = sh == N64 ? 64 : sh == N192 ? 192 : 128;
+      // a 192 x 192 workgroup has a compute unit to itself, four 64 x 64 share one
+      tiles2 += cdiv(dsz(P), t) * cdiv(dsz(P), t) * (sh == N192 ? 4 : sh == N128 ? 2 : 1);
     }
-    const int nsp_small = tiles2 ? (int)std::max<int64_t>(1, std::min<int64_t>(16, cdiv(target, tiles2))) : 1;
-    const int nsp_big =
-        tiles_big ? (int)std::max<int64_t>(1, std::min<int64_t>(16, cdiv(std::max<int64_t>(target / 4, 1), tiles_big)))
-                  : 1;
-    rpart_n = std::max(nsp_small, nsp_big);
-    if (ladder_merged) {
-      const int64_t tm = cdiv((int64_t)n_pairs * n_v, 128) * cdiv(n_v, 128);
-      rpart_n = (int)std::max<int64_t>(1, std::min<int64_t>(16, cdiv(target, tm)));
-    }
+    const int nsp_max = (int)std::max<int64_t>(1, std::min<int64_t>(16, cdiv(target, std::max<int64_t>(tiles2, 1))));
+    rpart_n = nsp_max;
     if (rpart_n > 1 && Rpart.bytes < (size_t)rpart_n * sum_d2 * 8) Rpart.alloc((size_t)rpart_n * sum_d2 * 8);
     lphase.clear();
     const int64_t nv2 = (int64_t)n_v * n_v;
@@ -800,192 +839,87 @@ void tci_plan::build_two_phase_ladder(hipStream_t st) {
       lphase.emplace_back();
       LadderPhase& ph = lphase.back();
       ph.Lc = len;
-      ph.nsplit = (int)std::min<int64_t>(rpart_n, len);
+      const int nsp = (int)std::min<int64_t>(rpart_n, len);
       std::vector<int64_t> lpo(n_local + 1, 0);
-      for (int q = 0; q < n_local; ++q) {
-        const int64_t d = h_dom_off[loc[q] + 1] - h_dom_off[loc[q]];
-        lpo[q + 1] = lpo[q] + len * d * d;
-      }
+      for (int q = 0; q < n_local; ++q) lpo[q + 1] = lpo[q] + len * dsz(loc[q]) * even(dsz(loc[q]));
       upload(ph.lp_off, lpo, st);
-      ph.p1.clear();
-      ph.p2.clear();
-      ph.p1.dense = ph.p2.dense = true;
-      ph.p1.tile = 128;
-      ph.p2.tile = 64;
-      if (ladder_merged) {
-        // phase 1: T[(jj,a)][(P,c)] = sum_k L^J[a][k] Cw[k][(P,c)], stored as T[jj][P][a][c]
-        // phase 2: R[(P,a)][n] += sum_jj sum_c T[jj][(P,a)][c] L^J[c][n]  (R blocks back to back)
-        const int d = n_v, NP = n_pairs * n_v;
-        const int64_t Sjj = (int64_t)n_pairs * d * d;
-        Blocking bk;
-        bk.rdiv = d;
-        bk.rstride = Sjj;
-        bk.cdiv = d;
-        bk.cstride = (int64_t)d * d;
-        ph.p1.add(Tbuf.as<double>(), d, (int)(len * d), NP,
-                  {seg(op(Lvv.p, n_v, 1, nullptr, nullptr, lvv_f32, nv2), op(Cw.p, NP, 1), d, 1.0)}, false, false, 0, bk);
-        ph.p2.tile = 128;
-        for (int sp = 0; sp < ph.nsplit; ++sp) {
-          const int64_t j0 = len * sp / ph.nsplit, j1 = len * (sp + 1) / ph.nsplit;
-          std::vector<Seg> sg;
-          for (int64_t jj = j0; jj < j1; ++jj)
-            sg.push_back(seg(op(Tbuf.as<double>() + jj * Sjj, d, 1),
-                             op(static_cast<const char*>(Lvv.p) + (size_t)(jj * nv2) * lsz, n_v, 1, nullptr, nullptr,
-                                lvv_f32, nv2),
-                             d, 1.0));
-          double* Rout = rpart_n > 1 ? Rpart.as<double>() + (int64_t)sp * sum_d2 : R.as<double>();
-          ph.p2.add(Rout, d, NP, d, sg, true);
-        }
-        ph.p1.upload_tables(st);
-        ph.p2.upload_tables(st);
-        continue;
-      }
-      // per-walk programs: phase 1 (M = len d) on 64- or 128-wide tiles by domain
-      // size; phase 2 on 64-wide tiles (4 workgroups per CU measure faster than
-      // 128-wide tiles for the long-K d x d outputs)
-      ph.p1x.clear();
-      ph.p2x.clear();
-      ph.p1x.resize(3);
-      ph.p2x.resize(2);
-      for (int v = 0; v < 3; ++v) {
-        ph.p1x[v].dense = true;
-        ph.p1x[v].tile = v == 2 ? 192 : (v ? (tile1 == 192 ? 128 : tile1) : 64);
-      }
-      ph.p2x[0].dense = ph.p2x[1].dense = true;
-      ph.p2x[0].tile = tile2;
-      ph.p2x[1].tile = 192;
-      int64_t toff = 0;
+      ph.n1.resize(3);
+      ph.n2.resize(3);
+      for (int v = 0; v < 3; ++v) ph.n1[v].shape = ph.n2[v].shape = v;  // N128, N192, N64
       int qloc = 0;
       for (int P = 0; P < n_pairs; ++P) {
-        const int d = (int)(h_dom_off[P + 1] - h_dom_off[P]);
-        const bool full = d == n_v;
-        const bool b192 = big && is_big(d);
-        // tile1 == 192: phase 1 of the domains of 129-192 on 192 x 192 tiles, phase 2 on tile2
-        const int v = (b192 || (tile1 == 192 && is_big(d))) ? 2 : (d <= 64 ? 0 : 1);
-        const int nsp = (int)std::min<int64_t>(b192 ? nsp_big : nsp_small, len);
-        double* T = Tbuf.as<double>() + toff;
-        // L operand of this pair: rows (jj, a) with leading dimension ld, one
-        // jj-block every jstep elements; full domains read L^J itself (J0 via jstride)
-        const void* Lb;
-        int64_t ld, jstep, jstride;
-        if (full) {
-          Lb = Lvv.p;
+        const int64_t d = dsz(P), dp = even(d);
+        double* T = Tbuf.as<double>() + Lc * cpo[P];
+        const double* Lb;
+        int64_t ld = dp, jstep = d * dp, jstride = 0;  // rows, one jj to the next, one J0 to the next
+        if (d == n_v && direct) {
+          Lb = Lvv.as<double>();
           ld = n_v;
-          jstep = nv2;
-          jstride = nv2;
-        } else if (lp_all) {  // [q][J][r][c]: chunk start through jstride
-          Lb = static_cast<const char*>(Lp.p) + (size_t)lpo_all[qloc++] * lsz;
-          ld = d;
-          jstep = (int64_t)d * d;
+          jstep = jstride = nv2;
+        } else if (lp_all) {
+          Lb = Lp.as<double>() + lpo_all[qloc++];
           jstride = jstep;
         } else {
-          Lb = static_cast<const char*>(Lp.p) + (size_t)lpo[qloc++] * lsz;
-          ld = d;
-          jstep = (int64_t)d * d;
-          jstride = 0;
+          Lb = Lp.as<double>() + lpo[qloc++];
         }
-        // phase 1: rows (jj, a) of L (M = len*d); rows jj*ld.. are contiguous when
-        // ld == d, and for full domains ld == n_v == d as well
-        ph.p1x[v].add(T, d, (int)(len * d), d, {seg(op(Lb, ld, 1, nullptr, nullptr, lvv_f32, jstride),
-                                                    op(C.as<double>() + h_cd_off[P], d, 1), d, 1.0)},
-                      false);
+        NSeg s1 = nseg(Lb, ld, Cw.as<double>() + cpo[P], dp, dp, 8);
+        s1.ja = jstride * 8;
+        ph.n1[shape_of(d)].add(T, dp, (int)(len * d), (int)d, {s1}, false);
         for (int sp = 0; sp < nsp; ++sp) {
           const int64_t j0 = len * sp / nsp, j1 = len * (sp + 1) / nsp;
-          std::vector<Seg> sg;
-          for (int64_t jj = j0; jj < j1; ++jj) {
-            const void* Lj = static_cast<const char*>(Lb) + (size_t)(jj * jstep) * lsz;
-            sg.push_back(seg(op(T + jj * d * d, d, 1), op(Lj, ld, 1, nullptr, nullptr, lvv_f32, jstride), d, 1.0));
-          }
+          NSeg s2 = nseg(Lb + j0 * jstep, ld, T + j0 * d * dp, dp, dp, 8);
+          s2.ja = jstride * 8;
+          s2.reps = j1 - j0;
+          s2.sa = jstep * 8;
+          s2.sb = d * dp * 8;
           double* Rout = (rpart_n > 1 ? Rpart.as<double>() + (int64_t)sp * sum_d2 : R.as<double>()) + h_cd_off[P];
-          ph.p2x[b192 ? 1 : 0].add(Rout, d, d, d, sg, true);
+          ph.n2[p2 ? (int)N64 : shape_of(d)].add(Rout, d, (int)d, (int)d, {s2}, true);
         }
-        toff += len * (int64_t)d * d;
       }
-      for (auto& g : ph.p1x) g.upload_tables(st);
-      for (auto& g : ph.p2x) g.upload_tables(st);
+      for (auto& g : ph.n1) g.upload_tables(st);
+      for (auto& g : ph.n2) g.upload_tables(st);
     }
   };
-  // 64-wide phase-2 tiles run 4 workgroups per CU, 128-wide ones 2
-  const int64_t def_target = ladder_merged ? 512 : 2048;
   if (!autotune_enabled()) {
-    // untuned: no 192 x 192 tiles unless TCI_FP64_P192=1 (both phases of
-    // 129-192) or TCI_FP64_P1_192=1 (their phase 1)
-    const char* e = std::getenv("TCI_FP64_P192");
-    const char* e1 = std::getenv("TCI_FP64_P1_192");
-    build(def_target, 64, e1 && e1[0] == '1' ? 192 : 128, e && e[0] == '1');
+    build(2048, 0);
     return;
   }
-  // autotuning on the first chunk (C holds no vector yet; the timing does
-  // not depend on the values) over fill targets and, for per-walk programs,
-  // the phase-2 tile and the 192 x 192 tiles; then the phase-1 tile and each
-  // program's workgroup order
-  bool any_big = false;
-  for (int P = 0; P < n_pairs; ++P) any_big = any_big || is_big(h_dom_off[P + 1] - h_dom_off[P]);
+  // autotuning on the first chunk, then each program's workgroup order
+  launch_pad_blocks(tab, dmax, cw_off.as<int64_t>(), C.as<double>(), Cw.as<double>(), st);
   double best = 1e300;
-  int64_t bt = def_target;
-  int btile = 64;
-  bool bbig = false;
-  std::string log = "fp64 ladder: (K-split target, phase-2 tile, 192-tiles)";
-  for (int big = 0; big <= (any_big && !ladder_merged ? 1 : 0); ++big)
-    for (int tile2 : {64, 128}) {
-      if ((ladder_merged || big) && tile2 == 128) break;  // merged programs have their own tiles
-      const int64_t base = tile2 == 64 ? def_target : def_target / 4;
-      for (int64_t t : {base / 2, base, 2 * base, 4 * base}) {
-        build(t, tile2, 128, big != 0);
-        TCI_HIP(hipStreamSynchronize(st));
-        const double ms = time_ms(st, 2, [&] { ladder_chunk(lchunks[0], st); });
-        log += " " + std::to_string(t) + "/" + std::to_string(tile2) + (big ? "b" : "") + ":" + fmt_ms(ms);
-        if (ms < best * 0.98) {
-          best = ms;
-          bt = t;
-          btile = tile2;
-          bbig = big != 0;
-        }
-      }
-    }
-  int btile1 = 128;
-  if (!ladder_merged && n_local > 0) {  // then the phase-1 tile of domains above 64
-    build(bt, btile, 64, bbig);
-    TCI_HIP(hipStreamSynchronize(st));
-    const double ms = time_ms(st, 2, [&] { ladder_chunk(lchunks[0], st); });
-    log += "; phase-1 tile 64:" + fmt_ms(ms);
-    if (ms < best * 0.98) {
-      best = ms;
-      btile1 = 64;
-    }
-    if (any_big && !bbig) {  // phase 1 of 129-192 alone on 192 x 192 tiles
-      build(bt, btile, 192, bbig);
+  int64_t bt = 2048;
+  int b2 = 0;
+  std::string log = "fp64 ladder: (K-split target, phase-2 tiles)";
+  for (int p2 = 0; p2 < 2; ++p2)
+    for (int64_t t : {1024, 2048, 4096, 8192}) {
+      build(t, p2);
       TCI_HIP(hipStreamSynchronize(st));
-      const double m2 = time_ms(st, 2, [&] { ladder_chunk(lchunks[0], st); });
-      log += " 192:" + fmt_ms(m2);
-      if (m2 < best * 0.98) {
-        best = m2;
-        btile1 = 192;
+      const double ms = time_ms(st, 2, [&] { ladder_chunk(lchunks[0], st); });
+      log += " " + std::to_string(t) + (p2 ? "/64:" : "/size:") + fmt_ms(ms);
+      if (ms < best * 0.98) {
+        best = ms;
+        bt = t;
+        b2 = p2;
       }
     }
-  }
-  build(bt, btile, btile1, bbig);
+  build(bt, b2);
   TCI_HIP(hipStreamSynchronize(st));
-  log += " -> " + std::to_string(bt) + "/" + std::to_string(btile) + (bbig ? "b" : "") + "/p1 " +
-         std::to_string(btile1) + "; order";
-  auto progs = [&](LadderPhase& ph) {
-    std::vector<GemmProgram*> v;
-    if (ladder_merged) {
-      v.push_back(&ph.p1);
-      v.push_back(&ph.p2);
-    }
-    for (auto& g : ph.p1x) v.push_back(&g);
-    for (auto& g : ph.p2x) v.push_back(&g);
-    return v;
-  };
+  log += " -> " + std::to_string(bt) + (b2 ? "/64" : "/size") + "; order";
   const int64_t J0 = lchunks[0].first;
-  std::vector<GemmProgram*> g0 = progs(lphase[lchunks[0].second]);
-  for (size_t k = 0; k < g0.size(); ++k) {
-    if (g0[k]->tasks.empty()) continue;
-    const int o = tune_order(*g0[k], st, [&] { g0[k]->launch(st, J0); });
-    log += " " + std::to_string(o);
-    for (auto& ph : lphase) progs(ph)[k]->remap = o;
-  }
+  for (int which = 0; which < 2; ++which)
+    for (int v = 0; v < 3; ++v) {
+      LadderPhase& p0 = lphase[lchunks[0].second];
+      NProgram& g = which ? p0.n2[v] : p0.n1[v];
+      if (g.tasks.empty() || xcd_remap_forced()) continue;
+      double t[2];
+      for (int o = 0; o < 2; ++o) {
+        g.remap = o;
+        t[o] = time_ms(st, 2, [&] { g.launch(TCI_SIGMA_FP64, st, J0); });
+      }
+      const int o = t[1] < 0.97 * t[0] ? 1 : 0;
+      log += " " + std::to_string(o);
+      for (auto& ph : lphase) (which ? ph.n2[v] : ph.n1[v]).remap = o;
+    }
   tuning += log + "\n";
 }
 
@@ -996,19 +930,14 @@ void tci_plan::ladder_chunk(const std::pair<int64_t, int>& ch, hipStream_t st) {
   if (n_local && !lp_all) {
     PackTab K{pairs_local.as<int32_t>(), ph.lp_off.as<int64_t>(), n_local};
     const int e0 = kt_begin(st);
-    launch_pack_L(tab, K, Lvv.p, lvv_f32, ch.first, ph.Lc, Lp.p, st);
+    launch_pack_L(tab, K, Lvv.p, lvv_f32, ch.first, ph.Lc, Lp.as<double>(), st);
     kt_end(e0, "fp64 ladder pack_L_kernel", 0.0, TCI_SIGMA_FP64, st);
   }
-  auto run = [&](const char* role, const GemmProgram& g) {
-    kt_run(role, g, TCI_SIGMA_FP64, st, [&] { g.launch(st, ch.first); });
-  };
-  if (ladder_merged) {
-    run("fp64 ladder phase 1", ph.p1);
-    run("fp64 ladder phase 2", ph.p2);
-  } else {
-    for (const auto& g : ph.p1x) run("fp64 ladder phase 1", g);
-    for (const auto& g : ph.p2x) run("fp64 ladder phase 2", g);
-  }
+  for (const auto* v : {&ph.n1, &ph.n2})
+    for (const auto& g : *v)
+      if (!g.tasks.empty())
+        kt_run(v == &ph.n1 ? "fp64 ladder phase 1" : "fp64 ladder phase 2", g, TCI_SIGMA_FP64, st,
+               [&] { g.launch(TCI_SIGMA_FP64, st, ch.first); });
 }
 
 // The FP64 two-phase ladder of one sigma: R (zeroed here) += sum over the
@@ -1016,27 +945,32 @@ void tci_plan::ladder_chunk(const std::pair<int64_t, int>& ch, hipStream_t st) {
 void tci_plan::two_phase_ladder(hipStream_t st) {
   double* Rz = rpart_n > 1 ? Rpart.as<double>() : R.as<double>();
   launch_fill(Rz, (int64_t)(rpart_n > 1 ? rpart_n : 1) * sum_d2, 0.0, st);
-  if (ladder_merged) launch_concat_cols(C.as<double>(), n_pairs, n_v, Cw.as<double>(), st);
+  launch_pad_blocks(tab, dmax, cw_off.as<int64_t>(), C.as<double>(), Cw.as<double>(), st);
   for (const auto& ch : lchunks) ladder_chunk(ch, st);
   if (timing()) TCI_HIP(hipEventRecord(ev[3], st));
   if (rpart_n > 1) ladder_reduce(Rpart.as<double>(), sum_d2, rpart_n, R.as<double>(), sum_d2, st);
 }
 
-void tci_plan::unpack_and_ladder(const double* x, const IoSlot* io, int precision, hipStream_t st) {
-  launch_unpack(tab, dmax, x, C.as<double>(), Ct.as<double>(), s.as<double>(), st, io);
+// returns whether panels_expand wrote the operands of x
+bool tci_plan::unpack_and_ladder(const double* x, const IoSlot* io, int precision, hipStream_t st) {
+  if (precision != TCI_SIGMA_FP64) mixed_prepare(*this, precision, st);
+  const bool expanded = panels_expand(*this, precision, x, io, st);
+  if (!expanded) launch_unpack(tab, dmax, x, C.as<double>(), Ct.as<double>(), s.as<double>(), st, io);
   if (timing()) TCI_HIP(hipEventRecord(ev[2], st));
   if (precision != TCI_SIGMA_FP64) {
-    mixed_ladder(*this, precision, st);
-    return;
+    mixed_ladder(*this, precision, expanded, x, io, st);
+    return expanded;
   }
   if (vv.fp64) {
-    vv_ladder(*this, TCI_SIGMA_FP64, st, !pp.on);
+    if (panels_hole_in_ladder(*this, precision)) panels_xt(*this, precision, x, io, st);
+    if (pp.m1on) kt_run("fp64 products S, W, Y", pp.m1, precision, st, [&] { pp.m1.launch(TCI_SIGMA_FP64, st); });
+    else vv_ladder(*this, TCI_SIGMA_FP64, st, !expanded, !pp.on);
     if (timing()) TCI_HIP(hipEventRecord(ev[3], st));
-    return;
+    return expanded;
   }
   if (!ladder_fused) {
     two_phase_ladder(st);
-    return;
+    return expanded;
   }
   LadderArgs a;
   a.dom_off = dom_off.as<int64_t>();
@@ -1053,30 +987,27 @@ void tci_plan::unpack_and_ladder(const double* x, const IoSlot* io, int precisio
   kt_end(e0, "fp64 fused ladder", flops_ladder, TCI_SIGMA_FP64, st);
   if (timing()) TCI_HIP(hipEventRecord(ev[3], st));
   ladder_reduce(lad_part.as<double>(), sum_d2, lad_chunks, R.as<double>(), sum_d2, st);
+  return expanded;
 }
 
 void tci_plan::sigma_body(const double* x, double* y, const IoSlot* io, int flags, hipStream_t st) {
-  unpack_and_ladder(x, io, flags & 0xff, st);
-  sigma_rest(x, y, io, flags, st);
+  const bool expanded = unpack_and_ladder(x, io, flags & 0xff, st);
+  sigma_rest(x, y, io, flags, expanded, st);
 }
 
-// every term after the ladder: needs C, Ct and s of x (unpacked) and the
-// ladder's R
-void tci_plan::sigma_rest(const double* x, double* y, const IoSlot* io, int flags, hipStream_t st) {
+// every term after the ladder: needs Ct and s of x, C or the panels (expanded),
+// and the ladder's R or S+-
+void tci_plan::sigma_rest(const double* x, double* y, const IoSlot* io, int flags, bool expanded, hipStream_t st) {
   const int precision = flags & 0xff;
   int e0;
-  if (!nprogY.tasks.empty()) {
-    kt_run("singles Y", nprogY, precision, st, [&] { nprogY.launch(TCI_SIGMA_FP64, st); });
-  } else {
-    launch_transpose_small(s.as<double>(), n_int, n_v, sT.as<double>(), st);
-    kt_run("singles Y", progY, precision, st, [&] { progY.launch(st); });
-  }
+  const bool m1 = pp.m1on && precision == TCI_SIGMA_FP64, m2 = pp.m2on && precision == TCI_SIGMA_FP64;
+  if (!(m1 && pp.m1_singles)) run_Y(precision, st);
   // with the panels the ladder's packed S+- and the pair terms meet in the
   // final kernel; R then holds a Cholesky-direct ladder and the virtual Fock
   // products only
   const bool packed = pp.on && (precision == TCI_SIGMA_FP64 ? vv.fp64 : vv.split);
   if (pp.on) {
-    panels_terms(*this, precision, st);
+    panels_terms(*this, precision, expanded, x, io, st);
   } else {
     e0 = kt_begin(st);
     launch_rterms(tab, dmax, x, s.as<double>(), Kov.as<double>(), O3.as<double>(), R.as<double>(), st, io);
@@ -1088,18 +1019,20 @@ void tci_plan::sigma_rest(const double* x, double* y, const IoSlot* io, int flag
     kt_run("ring and 3-external", ring, precision, st, [&] { ring.launch(st); });
     kt_run("singles W", progW, precision, st, [&] { progW.launch(st); });
   }
-  launch_gemv(Mss.as<double>(), (int64_t)n_int * n_v, s.as<double>(), gss.as<double>(), st);
-  if (!nprogGW.tasks.empty()) nprogGW.launch(TCI_SIGMA_FP64, st);
-  else progGW.launch(st);
-  launch_s3int_singles(tab, dmax, gpart_off.as<int64_t>(), Ct.as<double>(), O3.as<double>(), gpart.as<double>(), st);
+  launch_singles_terms(tab, dmax, Mss.as<double>(), s.as<double>(), gss.as<double>(), gpart_off.as<int64_t>(),
+                       Ct.as<double>(), O3.as<double>(), gpart.as<double>(), Kov.as<double>(), part.as<double>(), st);
+  if (m2 && pp.m2_singles) {
+  } else if (!nprogGW.tasks.empty()) {
+    nprogGW.launch(TCI_SIGMA_FP64, st);
+  } else {
+    progGW.launch(st);
+  }
   InvTab I{inv_off.as<int64_t>(), inv_q.as<int32_t>(), inv_pos.as<int32_t>()};
   launch_singles_reduce(tab, I, gpart_off.as<int64_t>(), gpart.as<double>(), gss.as<double>(), gW.as<double>(), n_split,
-                        g.as<double>(), st);
-  launch_ref_dot(tab, Kov.as<double>(), Ct.as<double>(), part.as<double>(), sig0.as<double>(), st);
+                        g.as<double>(), x, s.as<double>(), has_fov ? Fov.as<double>() : nullptr, part.as<double>(),
+                        sig0.as<double>(), st, io);
   if (has_fvv && packed) launch_fill(R.as<double>(), sum_d2, 0.0, st);
   if (has_fvv) kt_run("virtual Fock", fockvv, precision, st, [&] { fockvv.launch(st); });
-  if (has_fov) launch_fov_terms(x, s.as<double>(), Fov.as<double>(), (int64_t)n_int * n_v, g.as<double>(),
-                                sig0.as<double>(), st, io);
   if (pp.on) panels_pack(*this, precision, packed, !packed || has_fvv, x, io, flags, y, st);
   else launch_pack(tab, dmax, x, R.as<double>(), g.as<double>(), sig0.as<double>(), e_ref, flags, y, st, io);
 }
@@ -1183,7 +1116,7 @@ void tci_plan::sigma_batch(const double* const* x, double* const* y, int nvec, i
     launch_unpack(tab, dmax, x[v], C.as<double>(), Ct.as<double>(), s.as<double>(), st);
     TCI_HIP(hipMemcpyAsync(R.p, mx.bat.Rb.as<double>() + (int64_t)v * sum_d2, (size_t)sum_d2 * 8,
                            hipMemcpyDeviceToDevice, st));
-    sigma_rest(x[v], y[v], nullptr, fl, st);
+    sigma_rest(x[v], y[v], nullptr, fl, false, st);
   }
   if (profiling) {
     TCI_HIP(hipEventRecord(ev[1], st));

@@ -43,7 +43,7 @@ struct tci_plan {
   tci::NProgram nprogY, nprogGW;   // the same on the NT GEMM (even n_v, FP64 L^J)
   // pair terms as per-walk products over packed panels (pair_panels.hip)
   struct PairPanels {
-    bool on = false;
+    bool on = false, split = false;           // split: split builds run them in split precision
     std::vector<int32_t> h_koff;
     std::vector<int64_t> h_ld, h_poff, h_jpoff, h_lpoff;
     tci::DevBuf koff, ld, poff, jpoff, lpoff, pairid, colm;
@@ -58,8 +58,13 @@ struct tci_plan {
       std::vector<tci::NProgram> pair;        // one per tile shape
       int ks = 1;
     } f64, s16;
+    // small FP64 builds: the ladder's S+-, W and Y as one launch, the pair
+    // products and gW as another (m*_singles: Y / gW are part of them)
+    tci::NProgram m1, m2;
+    bool m1on = false, m2on = false, m1_singles = false, m2_singles = false;
+    int m1_ks = 1, m2_ks = 1;
     tci::NProgram rank;                       // FP64 3-internal products of a split sigma
-    int tuned_mode = -1, tuned_ks = 1, tuned_order = 0;  // split schedule, kept for both split precisions
+    int tuned_mode = -1, tuned_ks = 1, tuned_order = 0, tuned_w = 0;  // split schedule, kept for both split precisions
   } pp;
   tci::LadderLaunch ladder;        // fused single-kernel ladder (TCI_LADDER=fused)
   bool ladder_fused = false;
@@ -67,7 +72,8 @@ struct tci_plan {
   struct LadderPhase {
     int64_t Lc = 0;                 // chunk length these tables are built for
     int nsplit = 1;                 // K-splits of phase 2 (partial R buffers)
-    tci::GemmProgram p1, p2;        // dense programs (FP64, or split for the mixed ladder)
+    tci::GemmProgram p1, p2;        // split programs over all walks (full domains)
+    std::vector<tci::NProgram> n1, n2;       // FP64 programs, one per tile shape
     std::vector<tci::GemmProgram> p1x, p2x;  // split per-walk programs, one per tile shape
     std::vector<tci::GemmProgram> pp1, pp2;  // one program per walk (TCI_LADDER_PER_PAIR=1)
     tci::DevBuf lp_off;             // packed-L offsets of the local-domain pairs
@@ -80,10 +86,7 @@ struct tci_plan {
   std::vector<std::pair<int64_t, int>> lchunks;  // (J0, index into lphase)
   tci::DevBuf Tbuf, Rpart;
   int rpart_n = 1;
-  // every walk has the full domain: both phases run as single products over all
-  // walks (C blocks side by side in Cw)
-  bool ladder_merged = false;
-  tci::DevBuf Cw;
+  tci::DevBuf Cw, cw_off;           // C blocks with rows padded to an even count, their offsets
   // split-precision (bf16x3) two-phase ladder, built on first use:
   //   phase 1 T'_P[(jj,a)][c] = sum_k L^J[a][k] C_P[c][k]   (T' = L C^T, split rows)
   //   phase 2 R_P[n][a]     += sum_jj sum_c L^J[n][c] T'_P[jj][a][c]
@@ -234,12 +237,18 @@ struct tci_plan {
   void build(const tci_problem& p);
   void sigma(const double* x, double* y, int flags, hipStream_t st);
   void sigma_body(const double* x, double* y, const tci::IoSlot* io, int flags, hipStream_t st);
-  void sigma_rest(const double* x, double* y, const tci::IoSlot* io, int flags, hipStream_t st);
+  void sigma_rest(const double* x, double* y, const tci::IoSlot* io, int flags, bool expanded, hipStream_t st);
   // several vectors at once: the split ladder of local domains runs as one
   // batched pass (L^J read once per batch), every other term per vector
   void sigma_batch(const double* const* x, double* const* y, int nvec, int flags, hipStream_t st);
   void sigma_graph(const double* x, double* y, int flags, hipStream_t st);
-  void unpack_and_ladder(const double* x, const tci::IoSlot* io, int precision, hipStream_t st);
+  bool unpack_and_ladder(const double* x, const tci::IoSlot* io, int precision, hipStream_t st);
+  // are the rows of L^J 16-byte aligned FP64 (singles products on the NT GEMM)?
+  bool singles_nt() const { return !lvv_f32 && n_v % 2 == 0; }
+  void add_singles_Y(tci::NProgram& g) const;
+  void add_singles_GW(tci::NProgram& g) const;
+  void tune_vector(tci::DevBuf& x, hipStream_t st);
+  void run_Y(int precision, hipStream_t st);
   void build_two_phase_ladder(hipStream_t st);
   void two_phase_ladder(hipStream_t st);
   void ladder_chunk(const std::pair<int64_t, int>& ch, hipStream_t st);
@@ -250,7 +259,8 @@ namespace tci {
 // from the FP64 C blocks of the plan; records ev[3] before the final reduction
 // when profiling
 void mixed_prepare(tci_plan& P, int precision, hipStream_t st);
-void mixed_ladder(tci_plan& P, int precision, hipStream_t st);
+// expanded: panels_expand has written the operands of x
+void mixed_ladder(tci_plan& P, int precision, bool expanded, const double* x, const tci::IoSlot* io, hipStream_t st);
 void mixed_ladder_chunk(tci_plan& P, int precision, const std::pair<int64_t, int>& ch, hipStream_t st);
 // the split ladder of one sigma after preparation (C split, chunks, fused walks, reduction)
 void mixed_ladder_run(tci_plan& P, int precision, hipStream_t st);
@@ -273,17 +283,23 @@ void vv_build(tci_plan& P, hipStream_t st);
 // shape: an NShape of ngemm.hpp
 void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t st);
 void vv_prepare_split(tci_plan& P, int precision, hipStream_t st);
-// gather: unpack S+- into R (otherwise the caller reads the packed S+-)
-void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool gather);
+// scatter: write X+- from C; gather: unpack S+- into R (otherwise the caller
+// reads the packed S+-)
+void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool scatter, bool gather);
 double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log);
 int64_t vv_device_bytes(const tci_plan& P);
 // pair terms over packed panels (pair_panels.hip)
 bool panels_choose(const tci_plan& P);
 void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st);
 void panels_build_split(tci_plan& P, hipStream_t st);
-void panels_programs(tci_plan& P, bool split, int mode, int ks, hipStream_t st);
+bool panels_hole_in_ladder(const tci_plan& P, int precision);
+bool panels_expand(tci_plan& P, int precision, const double* x, const tci::IoSlot* io, hipStream_t st);
+void panels_xt(tci_plan& P, int precision, const double* x, const tci::IoSlot* io, hipStream_t st);
 void panels_tune(tci_plan& P, int precision, hipStream_t st);
-void panels_terms(tci_plan& P, int precision, hipStream_t st);
+void panels_merge(tci_plan& P, hipStream_t st);
+// tasks of the resident ladder's product appended to g (g.shape set)
+void vv_add_products(tci_plan& P, NProgram& g, bool split, int ks);
+void panels_terms(tci_plan& P, int precision, bool expanded, const double* x, const tci::IoSlot* io, hipStream_t st);
 void panels_pack(tci_plan& P, int precision, bool packed, bool use_r, const double* x, const tci::IoSlot* io,
                  int flags, double* y, hipStream_t st);
 int64_t panels_device_bytes(const tci_plan& P);

@@ -204,9 +204,9 @@ __global__ void hole_kernel(PairTab T, HoleTab H, const double* __restrict__ C, 
 // (coalesced reads of C and of the gathered row of Kov).
 constexpr int kRefSlices = 8;
 
-__global__ __launch_bounds__(256) void ref_dot_kernel(PairTab T, const double* __restrict__ Kov,
-                                                      const double* __restrict__ Ct, double* __restrict__ part) {
-  const int P = blockIdx.x, y = blockIdx.y;
+__device__ __forceinline__ void ref_dot_block(const PairTab& T, const double* __restrict__ Kov,
+                                              const double* __restrict__ Ct, double* __restrict__ part, int P, int y,
+                                              double* red) {
   const int i = T.pairs[2 * P], j = T.pairs[2 * P + 1];
   const int64_t off = T.dom_off[P];
   const int d = (int)(T.dom_off[P + 1] - off);
@@ -222,37 +222,33 @@ __global__ __launch_bounds__(256) void ref_dot_kernel(PairTab T, const double* _
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-  __shared__ double red[4];
   if (lane == 0) red[wv] = acc;
   __syncthreads();
   if (threadIdx.x == 0)
     part[(int64_t)P * kRefSlices + y] = (i == j ? 1.0 : 2.0) * ((red[0] + red[1]) + (red[2] + red[3]));
 }
 
-__global__ void sum_kernel(const double* __restrict__ part, int n, double* __restrict__ out) {
-  __shared__ double red[256];
-  double acc = 0.0;
-  for (int e = threadIdx.x; e < n; e += blockDim.x) acc += part[e];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = red[0];
-}
-
-// block (Q, o): ordered pair (j,k) = o==0 ? (qi,qj) : (qj,qi)
+// s3int block (Q, o): ordered pair (j,k) = o==0 ? (qi,qj) : (qj,qi)
 // out[i][r] = -sum_c Ct'[r][c] W[i][c], W[i][c] = (jj i|kk D[c]) (a row of O3),
-// Ct' = Ct (o = 0) or Ct^T (o = 1).  Block (Q, o, 64 rows of r); c in chunks of
-// 32 staged in LDS with coalesced reads of Ct, i in groups of 64 (16 per thread).
-constexpr int S3R = 64, S3C = 32;
+// Ct' = Ct (o = 0) or Ct^T (o = 1).  Block (Q, o, 64 rows of r), one wave per
+// 16 of them; c in chunks of 32 staged in LDS with coalesced reads of Ct, i in
+// groups of 64 as four 16 x 16 MFMA blocks (blocks beyond n_int are skipped).
+// v_mfma_f64_16x16x4: A[i][k] lane i + 16k, B[k][j] lane j + 16k, D[i][j] lane
+// j + 16 (i % 4), register i / 4.  The sums on the vector ALU from LDS took
+// 247-276 us at 34/192/1200: two LDS reads per multiply-add; the MFMA
+// form, which reads each staged value once per 16 products, takes 225 us
+// together with ref_dot.
+// LDS rows of 34: 16 rows x 2 columns of a half-wave read fall on distinct banks.
+constexpr int S3R = 64, S3C = 32, S3P = S3C + 2;
 
-__global__ __launch_bounds__(256) void s3int_singles_kernel(PairTab T, const int64_t* __restrict__ gpart_off,
-                                                            const double* __restrict__ Ct,
-                                                            const double* __restrict__ O3,
-                                                            double* __restrict__ gpart) {
-  const int Q = blockIdx.x, o = blockIdx.y, r0 = blockIdx.z * S3R;
+struct S3Lds {
+  double sC[S3R][S3P];
+  double sW[64][S3P];
+};
+
+__device__ __forceinline__ void s3int_block(const PairTab& T, const int64_t* __restrict__ gpart_off,
+                                            const double* __restrict__ Ct, const double* __restrict__ O3,
+                                            double* __restrict__ gpart, int Q, int o, int r0, S3Lds& L) {
   const int qi = T.pairs[2 * Q], qj = T.pairs[2 * Q + 1];
   const int64_t off = T.dom_off[Q];
   const int d = (int)(T.dom_off[Q + 1] - off);
@@ -261,52 +257,120 @@ __global__ __launch_bounds__(256) void s3int_singles_kernel(PairTab T, const int
   const int n = T.n_int, nv = T.n_v;
   const double* Cb = Ct + T.cd_off[Q];
   double* out = gpart + gpart_off[2 * Q + o];  // [n_int][d]
-  __shared__ double sC[S3R][S3C + 1];
-  __shared__ double sW[64][S3C + 1];
-  const int t = threadIdx.x, r = t & 63, ig = t >> 6;
+  auto& sC = L.sC;
+  auto& sW = L.sW;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  // element e = t + 256 q of a chunk: C (row rr, column cc) along the block's
+  // rows for o = 0, its columns for o = 1; W (row e / 32, column e % 32)
   for (int i0 = 0; i0 < n; i0 += 64) {
-    double acc[16];
+    const int nib = min(4, (n - i0 + 15) >> 4);
+    d4 acc[4];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = 0.0;
+    for (int q = 0; q < 4; ++q) acc[q] = d4{0.0, 0.0, 0.0, 0.0};
+    double rc[8], rw[8];
+    auto load = [&](int c0) {  // all of a chunk's loads in flight together
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int e = t + 256 * q;
+        const int rr = o == 0 ? e / S3C : e % S3R, cc = o == 0 ? e % S3C : e / S3R;
+        const int gr = r0 + rr, gc = c0 + cc;
+        const int64_t a = o == 0 ? (int64_t)min(gr, d - 1) * d + min(gc, d - 1) : (int64_t)min(gc, d - 1) * d + min(gr, d - 1);
+        const double v = Cb[a];
+        rc[q] = gr < d && gc < d ? v : 0.0;
+      }
+      const int gc = c0 + (t & 31);
+      const int64_t col = T.dom_idx[off + min(gc, d - 1)];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int ii = (t >> 5) + 8 * q, gi = i0 + ii;
+        if (8 * q < 16 * nib) {
+          const double v = O3[(((int64_t)jj * n + min(gi, n - 1)) * n + kk) * nv + col];
+          rw[q] = gi < n && gc < d ? v : 0.0;
+        }
+      }
+    };
+    load(0);
     for (int c0 = 0; c0 < d; c0 += S3C) {
       __syncthreads();
-      for (int e = t; e < S3R * S3C; e += 256) {
-        int rr, cc;
-        if (o == 0) {
-          rr = e / S3C;
-          cc = e % S3C;
-        } else {
-          rr = e % S3R;
-          cc = e / S3R;
-        }
-        const int gr = r0 + rr, gc = c0 + cc;
-        sC[rr][cc] = (gr < d && gc < d) ? (o == 0 ? Cb[(int64_t)gr * d + gc] : Cb[(int64_t)gc * d + gr]) : 0.0;
-      }
-      for (int e = t; e < 64 * S3C; e += 256) {
-        const int ii = e / S3C, cc = e % S3C;
-        const int gi = i0 + ii, gc = c0 + cc;
-        sW[ii][cc] = (gi < n && gc < d) ? O3[(((int64_t)jj * n + gi) * n + kk) * nv + T.dom_idx[off + gc]] : 0.0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int e = t + 256 * q;
+        sC[o == 0 ? e / S3C : e % S3R][o == 0 ? e % S3C : e / S3R] = rc[q];
+        if (8 * q < 16 * nib) sW[(t >> 5) + 8 * q][t & 31] = rw[q];
       }
       __syncthreads();
-      // rows i >= n hold zeros: skip them (ig is the wave index, so the test
-      // is uniform over a wave)
+      if (c0 + S3C < d) load(c0 + S3C);
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        if (i0 + ig + 4 * q >= n) continue;
-        double a = 0.0;
-#pragma unroll 8
-        for (int cc = 0; cc < S3C; ++cc) a += sW[ig + 4 * q][cc] * sC[r][cc];
-        acc[q] += a;
+      for (int k4 = 0; k4 < S3C / 4; ++k4) {
+        const double b = sC[16 * w + li][4 * k4 + lg];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (q < nib) acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(sW[16 * q + li][4 * k4 + lg], b, acc[q], 0, 0, 0);
       }
     }
-    if (r0 + r < d)
+    const int r = r0 + 16 * w + li;
+    if (r < d)
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int i = i0 + ig + 4 * q;
-        if (i < n) out[(int64_t)i * d + r0 + r] = -acc[q];
-      }
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const int i = i0 + 16 * q + lg + 4 * p;
+          if (i < n) out[(int64_t)i * d + r] = -acc[q][p];
+        }
   }
 }
+
+// The terms that need only Ct and s, in one launch (none of them fills the chip
+// at small sizes, and each launch of its own cost about as much as its work at
+// 5 internal, 30 virtual orbitals): block ranges for
+//   gss = Mss s        one wave per row
+//   the 3-internal singles partials (s3int_block)
+//   sigma_0 partials   (ref_dot_block)
+struct SinglesArgs {
+  const double *Mss, *s;
+  double* gss;
+  int64_t niv;
+  const int64_t* gpart_off;
+  const double *Ct, *O3;
+  double* gpart;
+  const double* Kov;
+  double* part;
+  int n_s3, nz, n_ref, n_gemv;  // blocks of each range (s3: n_pairs x 2 x nz)
+};
+
+__device__ __forceinline__ void gemv_block(const SinglesArgs& A, int b) {
+  const int lane = threadIdx.x & 63;
+  for (int64_t r = (int64_t)b * 4 + (threadIdx.x >> 6); r < A.niv; r += (int64_t)A.n_gemv * 4) {
+    const double* a = A.Mss + r * A.niv;
+    double acc = 0.0;
+    for (int64_t c = lane; c < A.niv; c += 64) acc += a[c] * A.s[c];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+    if (lane == 0) A.gss[r] = acc;
+  }
+}
+
+__global__ __launch_bounds__(256) void singles_terms_kernel(PairTab T, SinglesArgs A) {
+  __shared__ S3Lds lds;
+  int b = blockIdx.x;
+  if (b < A.n_s3) {
+    const int z = b % A.nz, qo = b / A.nz;
+    s3int_block(T, A.gpart_off, A.Ct, A.O3, A.gpart, qo >> 1, qo & 1, z * S3R, lds);
+    return;
+  }
+  b -= A.n_s3;
+  if (b < A.n_ref) {
+    ref_dot_block(T, A.Kov, A.Ct, A.part, b / kRefSlices, b % kRefSlices, &lds.sC[0][0]);
+    return;
+  }
+  gemv_block(A, b - A.n_ref);
+}
+
+// gss alone, without the LDS of the other ranges: at 34/192/1200 the product
+// streams 341 MB and wants every wave slot (88 us against 193 us inside
+// singles_terms_kernel)
+__global__ __launch_bounds__(256) void gemv_kernel(SinglesArgs A) { gemv_block(A, blockIdx.x); }
 
 // g[i][a] = gss + sum of the K-split partials of gW + every gpart entry of a
 // walk whose domain holds a.  One block per virtual a; thread (i, slice) sums
@@ -316,13 +380,31 @@ __global__ __launch_bounds__(256) void s3int_singles_kernel(PairTab T, const int
 // walk tables, then the partial) short: a launch has only n_v blocks.
 constexpr int kRedSlices = 16;
 
-__global__ __launch_bounds__(64 * kRedSlices) void singles_reduce_kernel(PairTab T, InvTab I,
-                                                                         const int64_t* __restrict__ gpart_off,
-                                                                         const double* __restrict__ gpart,
-                                                                         const double* __restrict__ gss,
-                                                                         const double* __restrict__ gW, int n_split,
-                                                                         double* __restrict__ g) {
+// Reference <-> singles through f_ia (Fov not null): g[i][a] += c0 f_ia and
+// sigma_0 += 2 sum_ia f_ia s_i^a.  Block n_v sums sigma_0 from its partials.
+__global__ __launch_bounds__(64 * kRedSlices) void singles_reduce_kernel(
+    PairTab T, InvTab I, const int64_t* __restrict__ gpart_off, const double* __restrict__ gpart,
+    const double* __restrict__ gss, const double* __restrict__ gW, int n_split, double* __restrict__ g,
+    const double* __restrict__ x, const IoSlot* __restrict__ io, const double* __restrict__ s,
+    const double* __restrict__ Fov, const double* __restrict__ ref_part, int n_ref, double* __restrict__ sig0) {
+  if (io) x = io->x;
   const int nv = T.n_v, no = T.n_int, a = blockIdx.x;
+  if (a == nv) {
+    constexpr int NT = 64 * kRedSlices;
+    __shared__ double red[NT];
+    double acc = 0.0;
+    for (int e = threadIdx.x; e < n_ref; e += NT) acc += ref_part[e];
+    if (Fov)
+      for (int e = threadIdx.x; e < no * nv; e += NT) acc += 2.0 * Fov[e] * s[e];
+    red[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = NT / 2; w > 0; w >>= 1) {
+      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *sig0 = red[0];
+    return;
+  }
   const int64_t n = (int64_t)no * nv;
   const int il = threadIdx.x & 63, sl = threadIdx.x >> 6;
   __shared__ double part[kRedSlices][64];
@@ -344,9 +426,9 @@ __global__ __launch_bounds__(64 * kRedSlices) void singles_reduce_kernel(PairTab
     part[sl][il] = v;
     __syncthreads();
     if (sl == 0 && i < no) {
-      double s = part[0][il];
-      for (int k = 1; k < kRedSlices; ++k) s += part[k][il];
-      g[(int64_t)i * nv + a] = s;
+      double r = part[0][il];
+      for (int k = 1; k < kRedSlices; ++k) r += part[k][il];
+      g[(int64_t)i * nv + a] = Fov ? r + x[0] * Fov[(int64_t)i * nv + a] : r;
     }
     __syncthreads();
   }
@@ -543,52 +625,52 @@ __global__ void build_mss_kernel(const double* __restrict__ Kov, const double* _
   }
 }
 
-// block (local pair q, jj): copy the d x d gathered block of L^{J0+jj}
+// block (local pair q, jj): copy the d x d gathered block of L^{J0+jj}, rows of
+// d rounded up to even (a zero beyond d)
 template <class LT>
 __global__ void pack_L_kernel(PairTab T, PackTab K, const LT* __restrict__ Lvv, int64_t J0, int64_t len,
-                              LT* __restrict__ Lp) {
+                              double* __restrict__ Lp) {
   const int q = blockIdx.x;
   const int64_t jj = blockIdx.y;
   const int P = K.pairs_local[q];
   const int64_t off = T.dom_off[P];
-  const int d = (int)(T.dom_off[P + 1] - off);
+  const int d = (int)(T.dom_off[P + 1] - off), dp = (d + 1) & ~1;
   const int64_t nv = T.n_v;
   const LT* L = Lvv + (J0 + jj) * nv * nv;
-  LT* out = Lp + K.lp_off[q] + jj * (int64_t)d * d;
+  double* out = Lp + K.lp_off[q] + jj * (int64_t)d * dp;
   for (int r = threadIdx.y; r < d; r += blockDim.y) {
     const int64_t row = (int64_t)T.dom_idx[off + r] * nv;
-    for (int c = threadIdx.x; c < d; c += blockDim.x) out[(int64_t)r * d + c] = L[row + T.dom_idx[off + c]];
+    for (int c = threadIdx.x; c < dp; c += blockDim.x)
+      out[(int64_t)r * dp + c] = c < d ? (double)L[row + T.dom_idx[off + c]] : 0.0;
   }
 }
 
-// Cw[k][P d + c] = C_P[k][c]: the C blocks of equal size d side by side
-__global__ void concat_cols_kernel(const double* __restrict__ C, int n_pairs, int d, double* __restrict__ Cw) {
-  const int64_t d2 = (int64_t)d * d, n = (int64_t)n_pairs * d2, ld = (int64_t)n_pairs * d;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t P = e / d2, rem = e - P * d2;
-    const int64_t k = rem / d, c = rem - k * d;
-    Cw[k * ld + P * d + c] = C[e];
-  }
-}
-
-// y = A x for a square row-major n x n matrix: one wave per row
-__global__ void gemv_kernel(const double* __restrict__ A, int64_t n, const double* __restrict__ x,
-                            double* __restrict__ y) {
-  const int lane = threadIdx.x & 63;
-  for (int64_t r = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); r < n;
-       r += (int64_t)gridDim.x * (blockDim.x >> 6)) {
-    const double* a = A + r * n;
-    double acc = 0.0;
-    for (int64_t c = lane; c < n; c += 64) acc += a[c] * x[c];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-    if (lane == 0) y[r] = acc;
+// block rows of C_P copied into rows of d rounded up to even
+__global__ void pad_blocks_kernel(PairTab T, const int64_t* __restrict__ cw_off, const double* __restrict__ C,
+                                  double* __restrict__ Cw) {
+  const int P = blockIdx.y;
+  const int d = (int)(T.dom_off[P + 1] - T.dom_off[P]), dp = (d + 1) & ~1;
+  const double* src = C + T.cd_off[P];
+  double* dst = Cw + cw_off[P];
+  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < d * d; e += gridDim.x * blockDim.x) {
+    const int r = e / d;
+    dst[(int64_t)r * dp + (e - r * d)] = src[e];
   }
 }
 
 __global__ void fill_kernel(double* p, int64_t n, double v) {
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
     p[e] = v;
+}
+
+__global__ void random_kernel(double* p, int64_t n) {
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
+    uint64_t h = (uint64_t)(e + 1) * 0x9E3779B97F4A7C15ull;  // splitmix64 finaliser
+    h = (h ^ (h >> 30)) * 0xBF58476D1CE4E5B9ull;
+    h = (h ^ (h >> 27)) * 0x94D049BB133111EBull;
+    h ^= h >> 31;
+    p[e] = (double)(h >> 11) * 0x1.0p-53 - 0.5;
+  }
 }
 
 // ---- explicit one-electron integrals ---------------------------------------
@@ -650,30 +732,6 @@ __global__ void fold_mss_kernel(double* __restrict__ Mss, const double* __restri
   }
 }
 
-// Reference <-> singles through f_ia: g[i][a] += c0 f_ia and
-// sigma_0 += 2 sum_ia f_ia s_i^a (one workgroup; after the singles reduction
-// and the reference dot of the same build)
-__global__ void fov_terms_kernel(const double* x, const IoSlot* io, const double* __restrict__ s,
-                                 const double* __restrict__ Fov, int64_t niv, double* __restrict__ g,
-                                 double* __restrict__ sig0) {
-  if (io) x = io->x;
-  const double c0 = x[0];
-  __shared__ double red[256];
-  double acc = 0.0;
-  for (int64_t e = threadIdx.x; e < niv; e += blockDim.x) {
-    const double f = Fov[e];
-    g[e] += c0 * f;
-    acc += f * s[e];
-  }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *sig0 += 2.0 * red[0];
-}
-
 inline unsigned gx(int64_t work) { return (unsigned)std::min<int64_t>(std::max<int64_t>(cdiv(work, 256), 1), 4096); }
 
 // out[c][r] = in[r][c] (rows x cols, small matrices)
@@ -718,28 +776,42 @@ void launch_hole(const PairTab& T, const HoleTab& H, int dmax, const double* C, 
 
 int ref_dot_slices() { return kRefSlices; }
 
-void launch_ref_dot(const PairTab& T, const double* Kov, const double* Ct, double* pair_part, double* sig0,
-                    hipStream_t st) {
-  if (T.n_pairs > 0) {
-    hipLaunchKernelGGL(ref_dot_kernel, dim3(T.n_pairs, kRefSlices), dim3(256), 0, st, T, Kov, Ct, pair_part);
-    TCI_HIP(hipGetLastError());
+void launch_singles_terms(const PairTab& T, int dmax, const double* Mss, const double* s, double* gss,
+                          const int64_t* gpart_off, const double* Ct, const double* O3, double* gpart,
+                          const double* Kov, double* ref_part, hipStream_t st) {
+  SinglesArgs A;
+  A.Mss = Mss;
+  A.s = s;
+  A.gss = gss;
+  A.niv = (int64_t)T.n_int * T.n_v;
+  A.gpart_off = gpart_off;
+  A.Ct = Ct;
+  A.O3 = O3;
+  A.gpart = gpart;
+  A.Kov = Kov;
+  A.part = ref_part;
+  A.nz = (int)cdiv(dmax, S3R);
+  A.n_s3 = T.n_pairs * 2 * A.nz;
+  A.n_ref = T.n_pairs * kRefSlices;
+  A.n_gemv = (int)std::min<int64_t>(cdiv(A.niv, 4), 8192);
+  // one launch while all of it fits the chip at once (four workgroups a compute
+  // unit); beyond that gss goes out alone
+  const int all = A.n_s3 + A.n_ref + A.n_gemv;
+  if (all > 1024) {
+    hipLaunchKernelGGL(gemv_kernel, dim3((unsigned)A.n_gemv), dim3(256), 0, st, A);
+    A.n_gemv = 0;
   }
-  hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, st, pair_part, T.n_pairs * kRefSlices, sig0);
-  TCI_HIP(hipGetLastError());
-}
-
-void launch_s3int_singles(const PairTab& T, int dmax, const int64_t* gpart_off, const double* Ct, const double* O3,
-                          double* gpart, hipStream_t st) {
-  if (T.n_pairs == 0) return;
-  hipLaunchKernelGGL(s3int_singles_kernel, dim3(T.n_pairs, 2, (unsigned)cdiv(dmax, S3R)), dim3(256), 0, st, T,
-                     gpart_off, Ct, O3, gpart);
+  if (A.n_s3 + A.n_ref + A.n_gemv > 0)
+    hipLaunchKernelGGL(singles_terms_kernel, dim3((unsigned)(A.n_s3 + A.n_ref + A.n_gemv)), dim3(256), 0, st, T, A);
   TCI_HIP(hipGetLastError());
 }
 
 void launch_singles_reduce(const PairTab& T, const InvTab& I, const int64_t* gpart_off, const double* gpart,
-                           const double* gss, const double* gW, int n_split, double* g, hipStream_t st) {
-  hipLaunchKernelGGL(singles_reduce_kernel, dim3((unsigned)T.n_v), dim3(64 * kRedSlices), 0, st, T, I, gpart_off,
-                     gpart, gss, gW, n_split, g);
+                           const double* gss, const double* gW, int n_split, double* g, const double* x,
+                           const double* s, const double* Fov, const double* ref_part, double* sig0, hipStream_t st,
+                           const IoSlot* io) {
+  hipLaunchKernelGGL(singles_reduce_kernel, dim3((unsigned)T.n_v + 1), dim3(64 * kRedSlices), 0, st, T, I, gpart_off,
+                     gpart, gss, gW, n_split, g, x, io, s, Fov, ref_part, T.n_pairs * kRefSlices, sig0);
   TCI_HIP(hipGetLastError());
 }
 
@@ -790,31 +862,31 @@ void launch_build_mss(const double* Kov, const double* Jvv, int n_int, int n_v, 
   TCI_HIP(hipGetLastError());
 }
 
-void launch_pack_L(const PairTab& T, const PackTab& K, const void* Lvv, bool f32, int64_t J0, int64_t len, void* Lp,
+void launch_pack_L(const PairTab& T, const PackTab& K, const void* Lvv, bool f32, int64_t J0, int64_t len, double* Lp,
                    hipStream_t st) {
   if (K.n_local == 0 || len == 0) return;
   dim3 grid(K.n_local, (unsigned)len), block(64, 4);
-  if (f32) hipLaunchKernelGGL(pack_L_kernel<float>, grid, block, 0, st, T, K, (const float*)Lvv, J0, len, (float*)Lp);
-  else hipLaunchKernelGGL(pack_L_kernel<double>, grid, block, 0, st, T, K, (const double*)Lvv, J0, len, (double*)Lp);
+  if (f32) hipLaunchKernelGGL(pack_L_kernel<float>, grid, block, 0, st, T, K, (const float*)Lvv, J0, len, Lp);
+  else hipLaunchKernelGGL(pack_L_kernel<double>, grid, block, 0, st, T, K, (const double*)Lvv, J0, len, Lp);
   TCI_HIP(hipGetLastError());
 }
 
-void launch_concat_cols(const double* C, int n_pairs, int d, double* Cw, hipStream_t st) {
-  const int64_t n = (int64_t)n_pairs * d * d;
-  if (n <= 0) return;
-  hipLaunchKernelGGL(concat_cols_kernel, dim3(gx(n)), dim3(256), 0, st, C, n_pairs, d, Cw);
-  TCI_HIP(hipGetLastError());
-}
-
-void launch_gemv(const double* A, int64_t n, const double* x, double* y, hipStream_t st) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(gemv_kernel, dim3((unsigned)std::min<int64_t>(cdiv(n, 4), 8192)), dim3(256), 0, st, A, n, x, y);
+void launch_pad_blocks(const PairTab& T, int dmax, const int64_t* cw_off, const double* C, double* Cw, hipStream_t st) {
+  if (T.n_pairs == 0) return;
+  hipLaunchKernelGGL(pad_blocks_kernel, dim3(std::min<unsigned>(gx((int64_t)dmax * dmax), 256), T.n_pairs), dim3(256), 0,
+                     st, T, cw_off, C, Cw);
   TCI_HIP(hipGetLastError());
 }
 
 void launch_fill(double* p, int64_t n, double v, hipStream_t st) {
   if (n <= 0) return;
   hipLaunchKernelGGL(fill_kernel, dim3(gx(n)), dim3(256), 0, st, p, n, v);
+  TCI_HIP(hipGetLastError());
+}
+
+void launch_random(double* p, int64_t n, hipStream_t st) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(random_kernel, dim3(gx(n)), dim3(256), 0, st, p, n);
   TCI_HIP(hipGetLastError());
 }
 
@@ -830,12 +902,6 @@ void launch_fold_fock(const double* F, int n_int, int n_v, double* O3, double* M
   hipLaunchKernelGGL(fold_o3_kernel, dim3(gx(n)), dim3(256), 0, st, O3, F, n_int, n_v);
   TCI_HIP(hipGetLastError());
   hipLaunchKernelGGL(fold_mss_kernel, dim3(gx(n)), dim3(256), 0, st, Mss, F, n_int, n_v);
-  TCI_HIP(hipGetLastError());
-}
-
-void launch_fov_terms(const double* x, const double* s, const double* Fov, int64_t niv, double* g, double* sig0,
-                      hipStream_t st, const IoSlot* io) {
-  hipLaunchKernelGGL(fov_terms_kernel, dim3(1), dim3(256), 0, st, x, io, s, Fov, niv, g, sig0);
   TCI_HIP(hipGetLastError());
 }
 
