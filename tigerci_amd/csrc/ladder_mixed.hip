@@ -253,47 +253,12 @@ void mixed_ladder_chunk(tci_plan& P, int precision, const std::pair<int64_t, int
   }
 }
 
-void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
+// Operand copies, buffers and tuned programs of the two-phase (and fused) split
+// ladder.
+static void mixed_layout(tci_plan& P, int precision, hipStream_t st) {
   tci_plan::MixedLadder& M = P.mx;
-  TCI_REQUIRE(precision == TCI_SIGMA_BF16X3 || precision == TCI_SIGMA_FP16X3, "not a split precision");
-  if (M.ready && M.prec == precision) return;
-  TCI_REQUIRE(!P.capturing, "split operands are prepared outside graph capture");
-  // captured graphs point into the copies rebuilt below
-  P.drop_graphs();
-  M.ready = false;
-  M.bat.nvec = 0;  // batched programs point into the copies rebuilt below
-  M.prec = precision;
   const int f16 = precision == TCI_SIGMA_FP16X3 ? 1 : 0;
-  // scales: all 1 for bf16x3 (FP32 exponent range); for fp16x3 the constants'
-  // scale now, the per-sigma ones inside every sigma
-  {
-    std::vector<float> one(16, 1.f);
-    upload(M.scales, one, st);
-    std::vector<unsigned> z(4, 0u);
-    upload(M.maxbits, z, st);
-  }
   float* sc = M.scales.as<float>();
-  if (f16) {
-    unsigned* mx = M.maxbits.as<unsigned>();
-    const int64_t nvv = P.n_chol * (int64_t)P.n_v * P.n_v, nov = P.n_chol * (int64_t)P.n_int * P.n_v;
-    if (P.lvv_f32)
-      hipLaunchKernelGGL(absmax_kernel<float>, dim3(blocks_for(nvv, 1024)), dim3(256), 0, st, P.Lvv.as<float>(), nvv,
-                         mx + 2);
-    else
-      hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(nvv, 1024)), dim3(256), 0, st, P.Lvv.as<double>(), nvv,
-                         mx + 2);
-    if (P.pp.on && P.pp.split) {
-      auto amax = [&](const DevBuf& x, int64_t n) {
-        hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(n, 1024)), dim3(256), 0, st, x.as<double>(), n, mx + 2);
-      };
-      amax(P.Jvv, (int64_t)(P.Jvv.bytes / 8));
-      amax(P.Lov, nov);
-      amax(P.pp.holeP, (int64_t)(P.pp.holeP.bytes / 8));  // 4-internal coefficients
-      amax(P.pp.holeM, (int64_t)(P.pp.holeM.bytes / 8));
-    }
-    hipLaunchKernelGGL(set_scales_kernel, dim3(1), dim3(64), 0, st, 0, mx, sc, (float)P.dmax);
-    TCI_HIP(hipGetLastError());
-  }
   const int n_pairs = P.n_pairs, n_v = P.n_v;
   const int64_t nvp = xpad(n_v), n_chol = P.n_chol;
   std::vector<int64_t> cxo(n_pairs + 1, 0);
@@ -312,7 +277,6 @@ void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
       sum_local_x += x;
     }
   }
-  M.bytes = 0;
   upload(M.cx_off, cxo, st);
   M.Cx.alloc((size_t)std::max<int64_t>(sum_x, 16) * 2);
   M.n_local = (int)loc.size();
@@ -862,17 +826,65 @@ void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
     M.tuned_fused_target = bft;
     P.tuning += log + "\n";
   }
+}
+
+void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
+  tci_plan::MixedLadder& M = P.mx;
+  TCI_REQUIRE(precision == TCI_SIGMA_BF16X3 || precision == TCI_SIGMA_FP16X3, "not a split precision");
+  if (M.ready && M.prec == precision) return;
+  TCI_REQUIRE(!P.capturing, "split operands are prepared outside graph capture");
+  // captured graphs point into the copies rebuilt below
+  P.drop_graphs();
+  M.ready = false;
+  M.bat.nvec = 0;  // batched programs point into the copies rebuilt below
+  M.prec = precision;
+  const int f16 = precision == TCI_SIGMA_FP16X3 ? 1 : 0;
+  // scales: all 1 for bf16x3 (FP32 exponent range); for fp16x3 the constants'
+  // scale now, the per-sigma ones inside every sigma
+  {
+    std::vector<float> one(16, 1.f);
+    upload(M.scales, one, st);
+    std::vector<unsigned> z(4, 0u);
+    upload(M.maxbits, z, st);
+  }
+  float* sc = M.scales.as<float>();
+  if (f16) {
+    unsigned* mx = M.maxbits.as<unsigned>();
+    const int64_t nvv = P.n_chol * (int64_t)P.n_v * P.n_v, nov = P.n_chol * (int64_t)P.n_int * P.n_v;
+    if (P.lvv_f32)
+      hipLaunchKernelGGL(absmax_kernel<float>, dim3(blocks_for(nvv, 1024)), dim3(256), 0, st, P.Lvv.as<float>(), nvv,
+                         mx + 2);
+    else
+      hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(nvv, 1024)), dim3(256), 0, st, P.Lvv.as<double>(), nvv,
+                         mx + 2);
+    if (P.pp.on && P.pp.split) {
+      auto amax = [&](const DevBuf& x, int64_t n) {
+        hipLaunchKernelGGL(absmax_kernel<double>, dim3(blocks_for(n, 1024)), dim3(256), 0, st, x.as<double>(), n, mx + 2);
+      };
+      amax(P.Jvv, (int64_t)(P.Jvv.bytes / 8));
+      amax(P.Lov, nov);
+      amax(P.pp.holeP, (int64_t)(P.pp.holeP.bytes / 8));  // 4-internal coefficients
+      amax(P.pp.holeM, (int64_t)(P.pp.holeM.bytes / 8));
+    }
+    hipLaunchKernelGGL(set_scales_kernel, dim3(1), dim3(64), 0, st, 0, mx, sc, (float)P.dmax);
+    TCI_HIP(hipGetLastError());
+  }
+  // ladder from the resident (ab|cd) block when the plan holds it; timed
+  // against the Cholesky-direct one unless it wins by a wide margin
+  // (vv_clear_win), is forced (TCI_LADDER_VV=1) or autotuning is off
+  const char* env_vv = std::getenv("TCI_LADDER_VV");
+  const bool force = env_vv && env_vv[0] == '1';
+  const bool untimed = P.vv.built && (force || P.vv.split_use == 1 ||
+                                      (P.vv.split_use < 0 && (!autotune_enabled() || vv_clear_win(P))));
+  M.bytes = 0;
+  if (!untimed) mixed_layout(P, precision, st);
+  else if (autotune_enabled() && P.vv.split_use < 0) P.tuning += "split ladder: Cholesky-direct not laid out\n";
   if (P.pp.on && P.pp.split) {
     panels_build_split(P, st);
     panels_tune(P, precision, st);
   }
-  // ladder from the resident (ab|cd) block when the plan holds it: timed
-  // against the split Cholesky-direct ladder above (kept when faster) unless
-  // autotuning is off or TCI_LADDER_VV=1; the loser's operand copies are freed
   P.vv.split = false;
   if (P.vv.built) {
-    const char* env = std::getenv("TCI_LADDER_VV");
-    const bool force = env && env[0] == '1';
     const std::string pn = precision == TCI_SIGMA_FP16X3 ? "fp16x3" : "bf16x3";
     vv_prepare_split(P, precision, st);
     std::string log = pn + " ladder (ab|cd) resident:";
@@ -886,7 +898,7 @@ void mixed_prepare(tci_plan& P, int precision, hipStream_t st) {
       log += " kept";
     } else if (autotune_enabled()) {
       const double tv = vv_tune(P, precision, st, log);
-      if (!force) {
+      if (!untimed) {
         const double tc = time_ms(st, 1, [&] { mixed_ladder_run(P, precision, st); });
         log += "; resident " + fmt_ms(tv) + ", Cholesky-direct " + fmt_ms(tc);
         use = tv < tc;

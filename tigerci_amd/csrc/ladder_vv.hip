@@ -319,6 +319,22 @@ double vv_flops(const tci_plan& P) {
   return 2.0 * np * np * P.n_pairs + 2.0 * nm * nm * ncm;
 }
 
+// Whether the resident product wins without being timed: 2.5 times its flops,
+// counting rows of X as whole tiles of 128, stay below the Cholesky-direct
+// flops.  Both run on the same tiles; the Cholesky-direct phases add the traffic
+// of T' and of two passes over L^J.  With f_chol over the padded flops at 6.9 (10/100/400), 11 (16/203/811), 7.2
+// (34/192/1200) and 3.6 (13/151/607) the resident FP64 ladder measured 17, 20, 12
+// and 8 times faster, the split ones 14 and more.  Below the line both are timed.
+bool vv_clear_win(const tci_plan& P) {
+  const double np = (double)tri(P.n_v), nm = (double)tri(P.n_v - 1);
+  int ncm = 0;
+  for (int Q = 0; Q < P.n_pairs; ++Q) ncm += P.h_pairs[2 * Q] != P.h_pairs[2 * Q + 1];
+  double f_chol = 0.0;
+  for (int Q = 0; Q < P.n_pairs; ++Q)
+    f_chol += 4.0 * std::pow((double)(P.h_dom_off[Q + 1] - P.h_dom_off[Q]), 3) * (double)P.n_chol;
+  return 2.5 * 2.0 * 128.0 * (np * np * cdiv(P.n_pairs, 128) + nm * nm * cdiv(ncm, 128)) <= f_chol;
+}
+
 // Assemble V+- (FP64) from L^J, in slabs of outer virtuals: W = LT[(a,c)][J]
 // L^J[(b,d)] on the dense FP64 GEMM, then the symmetric and antisymmetric
 // combinations.  Sets up X, the column map of X- and FP64 product tables.

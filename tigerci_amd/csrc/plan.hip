@@ -569,10 +569,10 @@ void tci_plan::build(const tci_problem& p) {
     DevBuf x;
     tune_vector(x, st);
   }
-  if (!ladder_fused) build_two_phase_ladder(st);
   // ladder from the resident (ab|cd) block: with autotuning, built when it
   // fits and its product costs under twice the Cholesky-direct flops, then
-  // timed against the Cholesky-direct ladder (the faster is kept);
+  // timed against the Cholesky-direct ladder (the faster is kept) unless it wins
+  // by a wide margin (vv_clear_win);
   // TCI_LADDER_VV=1 forces it whenever it fits (with or without autotuning),
   // TCI_LADDER_VV=0 switches it off
   if (!ladder_fused && n_pairs > 0) {
@@ -584,8 +584,10 @@ void tci_plan::build(const tci_problem& p) {
     double need = 0.0;
     const bool fits = force != 0 && vv_fits(*this, &need);
     const bool tune = autotune_enabled();
+    const bool untimed = force == 1 || vv_clear_win(*this);
     const bool try_vv = fits && (force == 1 || (tune && f_vv < 2.0 * f_chol));
     if (force == 1 && !fits) tuning += "fp64 ladder (ab|cd) resident: does not fit (" + std::to_string(need / 1e9) + " GB)\n";
+    if (!try_vv || !untimed) build_two_phase_ladder(st);
     if (try_vv) {
       vv_build(*this, st);
       char head[160];
@@ -595,7 +597,7 @@ void tci_plan::build(const tci_problem& p) {
       bool use = true;
       if (tune) {
         const double tv = vv_tune(*this, TCI_SIGMA_FP64, st, log);
-        if (force != 1) {
+        if (!untimed) {
           const double tc = time_ms(st, 1, [&] { two_phase_ladder(st); });
           log += "; resident " + fmt_ms(tv) + ", Cholesky-direct " + fmt_ms(tc);
           use = tv < tc;
@@ -612,6 +614,8 @@ void tci_plan::build(const tci_problem& p) {
         lphase.clear();
       }
     }
+  } else if (!ladder_fused) {
+    build_two_phase_ladder(st);
   }
 
   if (pp.on) {

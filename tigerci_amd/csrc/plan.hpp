@@ -279,6 +279,7 @@ void launch_split_scales(int mode, const double* x, int64_t n, unsigned* mx, int
 // ladder from the resident (ab|cd) block (ladder_vv.hip)
 bool vv_fits(const tci_plan& P, double* bytes_out);
 double vv_flops(const tci_plan& P);
+bool vv_clear_win(const tci_plan& P);
 void vv_build(tci_plan& P, hipStream_t st);
 // shape: an NShape of ngemm.hpp
 void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t st);
