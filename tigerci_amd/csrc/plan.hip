@@ -19,7 +19,6 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
-#include <mutex>
 #include <set>
 
 namespace tci {
@@ -685,6 +684,9 @@ tci_plan::~tci_plan() {
   for (auto& kv : graphs) (void)hipGraphExecDestroy(kv.second);
   for (auto& kv : iter_graphs) (void)hipGraphExecDestroy(kv.second);
   if (iter_host) (void)hipHostFree(iter_host);
+  if (hs.pin) (void)hipHostFree(hs.pin);
+  for (hipEvent_t& e : hs.ev)
+    if (e) (void)hipEventDestroy(e);
   if (gstream) (void)hipStreamDestroy(gstream);
   for (hipEvent_t& e : ev)
     if (e) (void)hipEventDestroy(e);
@@ -1041,6 +1043,51 @@ void tci_plan::sigma_rest(const double* x, double* y, const IoSlot* io, int flag
   else launch_pack(tab, dmax, x, R.as<double>(), g.as<double>(), sig0.as<double>(), e_ref, flags, y, st, io);
 }
 
+// sigmavec += H civec on host vectors.  The host copies each piece of civec
+// into a pinned slot while the GPU fetches the piece before it, and adds each
+// piece of H civec to sigmavec while the next one arrives; sigmavec itself
+// never crosses the bus.  At 10/100/400 (4.3 MB a vector, sigma 0.41 ms):
+// 0.75 ms,
+// against 1.21 with two device allocations and three pageable copies per call.
+// Pieces of 512 KB take about 10 us on the bus and on the host; kernels move
+// them, since an asynchronous copy of that size costs about 50 us to start.
+void tci_plan::htimesc(const double* civec, double* sigmavec) {
+  std::lock_guard<std::mutex> guard(hs.lock);
+  const hipStream_t st = nullptr;
+  const int64_t n = n_csf;
+  if (!hs.c.p) hs.c.alloc((size_t)n * 8);
+  if (!hs.s.p) hs.s.alloc((size_t)n * 8);
+  if (!hs.pin)
+    TCI_HIP(hipHostMalloc(reinterpret_cast<void**>(&hs.pin), (size_t)(HostStage::kSlots * HostStage::kSlot * 8),
+                          hipHostMallocDefault));
+  for (hipEvent_t& e : hs.ev)
+    if (!e) TCI_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  const int64_t np = cdiv(n, HostStage::kSlot);
+  auto slot = [&](int64_t k) { return hs.pin + (k % HostStage::kSlots) * HostStage::kSlot; };
+  auto len = [&](int64_t k) { return std::min(HostStage::kSlot, n - k * HostStage::kSlot); };
+  for (int64_t k = 0; k < np; ++k) {
+    hipEvent_t e = hs.ev[k % HostStage::kSlots];
+    if (k >= HostStage::kSlots) TCI_HIP(hipEventSynchronize(e));
+    std::memcpy(slot(k), civec + k * HostStage::kSlot, (size_t)len(k) * 8);
+    launch_copy(slot(k), hs.c.as<double>() + k * HostStage::kSlot, len(k), st);
+    TCI_HIP(hipEventRecord(e, st));
+  }
+  sigma(hs.c.as<double>(), hs.s.as<double>(), TCI_SIGMA_FP64 | TCI_ADD_EREF, st);
+  auto fetch = [&](int64_t k) {
+    launch_copy(hs.s.as<double>() + k * HostStage::kSlot, slot(k), len(k), st);
+    TCI_HIP(hipEventRecord(hs.ev[k % HostStage::kSlots], st));
+  };
+  // the copies of the last pieces of civec precede these on the stream
+  for (int64_t k = 0; k < std::min<int64_t>(np, HostStage::kSlots); ++k) fetch(k);
+  for (int64_t k = 0; k < np; ++k) {
+    TCI_HIP(hipEventSynchronize(hs.ev[k % HostStage::kSlots]));
+    const double* w = slot(k);
+    double* out = sigmavec + k * HostStage::kSlot;
+    for (int64_t q = 0, m = len(k); q < m; ++q) out[q] += w[q];
+    if (k + HostStage::kSlots < np) fetch(k + HostStage::kSlots);
+  }
+}
+
 // The whole build as one graph launch: the first call with a flag set captures
 // the launch sequence of sigma_body on a private stream (x and y read from the
 // io slot), later calls set the slot and replay.  Split precisions prepare
@@ -1264,13 +1311,7 @@ int tci_htimesc(tci_plan* plan, const double* civec, double* sigmavec, int64_t n
   TCI_GUARD_BEGIN
   TCI_REQUIRE(plan && civec && sigmavec, "null argument");
   TCI_REQUIRE(n == plan->n_csf, "vector length does not match the plan's CSF count");
-  DevBuf dc, ds;
-  dc.alloc((size_t)n * 8);
-  ds.alloc((size_t)n * 8);
-  TCI_HIP(hipMemcpy(dc.p, civec, (size_t)n * 8, hipMemcpyHostToDevice));
-  TCI_HIP(hipMemcpy(ds.p, sigmavec, (size_t)n * 8, hipMemcpyHostToDevice));
-  plan->sigma(dc.as<double>(), ds.as<double>(), TCI_SIGMA_FP64 | TCI_ACCUMULATE | TCI_ADD_EREF, nullptr);
-  TCI_HIP(hipMemcpy(sigmavec, ds.p, (size_t)n * 8, hipMemcpyDeviceToHost));
+  plan->htimesc(civec, sigmavec);
   return TCI_OK;
   TCI_GUARD_END
 }

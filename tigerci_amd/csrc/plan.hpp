@@ -2,6 +2,7 @@
 #pragma once
 
 #include <map>
+#include <mutex>
 
 #include "common.hpp"
 #include "ladder.hpp"
@@ -204,6 +205,18 @@ struct tci_plan {
   void* iter_host = nullptr;
   size_t iter_host_bytes = 0;
   int iter_clock_khz = 0;
+  // staging of tci_htimesc, laid out on its first call: device vectors, a ring
+  // of pinned host slots and the event of each slot's last copy; one call at a
+  // time
+  struct HostStage {
+    static constexpr int kSlots = 4;
+    static constexpr int64_t kSlot = 65536;  // doubles
+    std::mutex lock;
+    tci::DevBuf c, s;
+    double* pin = nullptr;
+    hipEvent_t ev[kSlots] = {};
+  } hs;
+  void htimesc(const double* civec, double* sigmavec);
   bool timing() const { return profiling && !capturing; }
   // per-kernel event timing of profiled eager builds (tci_profile_kernels):
   // kt_begin records a start event (-1 when not timing), kt_end the stop event

@@ -645,6 +645,14 @@ __global__ void pack_L_kernel(PairTab T, PackTab K, const LT* __restrict__ Lvv, 
   }
 }
 
+// pairs of doubles (both ends 16-byte aligned), an odd last one alone
+__global__ __launch_bounds__(256) void copy_kernel(const double* __restrict__ src, double* __restrict__ dst, int64_t n) {
+  const int64_t h = n >> 1;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < h; e += (int64_t)gridDim.x * blockDim.x)
+    reinterpret_cast<double2*>(dst)[e] = reinterpret_cast<const double2*>(src)[e];
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) dst[n - 1] = src[n - 1];
+}
+
 // block rows of C_P copied into rows of d rounded up to even
 __global__ void pad_blocks_kernel(PairTab T, const int64_t* __restrict__ cw_off, const double* __restrict__ C,
                                   double* __restrict__ Cw) {
@@ -868,6 +876,12 @@ void launch_pack_L(const PairTab& T, const PackTab& K, const void* Lvv, bool f32
   dim3 grid(K.n_local, (unsigned)len), block(64, 4);
   if (f32) hipLaunchKernelGGL(pack_L_kernel<float>, grid, block, 0, st, T, K, (const float*)Lvv, J0, len, Lp);
   else hipLaunchKernelGGL(pack_L_kernel<double>, grid, block, 0, st, T, K, (const double*)Lvv, J0, len, Lp);
+  TCI_HIP(hipGetLastError());
+}
+
+void launch_copy(const double* src, double* dst, int64_t n, hipStream_t st) {
+  const unsigned g = (unsigned)std::min<int64_t>(std::max<int64_t>(cdiv(n, 512), 1), 1024);
+  hipLaunchKernelGGL(copy_kernel, dim3(g), dim3(256), 0, st, src, dst, n);
   TCI_HIP(hipGetLastError());
 }
 
