@@ -31,6 +31,7 @@
 // X+- as split rows (hi/lo 16-bit parts, common.hpp).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "plan.hpp"
 
@@ -184,8 +185,9 @@ __global__ void vv_scatter_kernel(PairTab T, const double* __restrict__ C, const
 }
 
 // R_P[r][s] (overwritten) from the K-split partials of S+ [P][n_p] and S- [P'][n_m]
-__global__ void vv_gather_kernel(PairTab T, const double* __restrict__ Sp, int64_t sp_part, int64_t ldp,
-                                 const double* __restrict__ Sm, int64_t sm_part, int64_t ldm, int nparts,
+template <class TS>
+__global__ void vv_gather_kernel(PairTab T, const TS* __restrict__ Sp, int64_t sp_part, int64_t ldp,
+                                 const TS* __restrict__ Sm, int64_t sm_part, int64_t ldm, int nparts,
                                  const int32_t* __restrict__ colm, double* __restrict__ R) {
   const int P = blockIdx.y;
   const int64_t o = T.dom_off[P];
@@ -197,13 +199,13 @@ __global__ void vv_gather_kernel(PairTab T, const double* __restrict__ Sp, int64
     const int r = (int)(t / d), c = (int)(t - (int64_t)r * d);
     const int gr = T.dom_idx[o + r], gc = T.dom_idx[o + c];
     const int hi = max(gr, gc), lo = min(gr, gc);
-    const double* sp = Sp + P * ldp + tri(hi) + lo;
+    const TS* sp = Sp + P * ldp + tri(hi) + lo;
     double v = 0.0;
-    for (int k = 0; k < nparts; ++k) v += sp[k * sp_part];
+    for (int k = 0; k < nparts; ++k) v += (double)sp[k * sp_part];
     if (cm >= 0 && hi != lo) {
-      const double* sm = Sm + cm * ldm + tri(hi - 1) + lo;
+      const TS* sm = Sm + cm * ldm + tri(hi - 1) + lo;
       double w = 0.0;
-      for (int k = 0; k < nparts; ++k) w += sm[k * sm_part];
+      for (int k = 0; k < nparts; ++k) w += (double)sm[k * sm_part];
       v += gr > gc ? w : -w;
     }
     Rp[t] = v;
@@ -280,7 +282,10 @@ void vv_add_products(tci_plan& P, NProgram& g, bool split, int ks) {
           const int64_t ldw = P.pp.ldw;
           sg.push_back(nseg(pt.hc, ldw, static_cast<const char*>(pt.hx) + n0 * ldw * esz, ldw, ldw, esz));
         }
-        g.add(pt.S + k * spart + n0, pt.n, (int)pt.rows, nn, sg, false, Blocking(), split ? kScOut : -1);
+        // the sums of a split product are FP32: stored as such
+        double* S = split ? reinterpret_cast<double*>(reinterpret_cast<float*>(pt.S) + k * spart + n0)
+                          : pt.S + k * spart + n0;
+        g.add(S, pt.n, (int)pt.rows, nn, sg, false, Blocking(), split ? kScOut : -1, split);
       }
     }
   }
@@ -296,7 +301,9 @@ void build_products(tci_plan& P, NProgram& g, bool split, int shape, int ks, hip
   g.upload_tables(st);
 }
 
-constexpr int kMaxSplits = 4;  // K-splits of the products
+// K-splits of the products: partials S in FP64, and in FP32 (split) in the same
+// memory
+constexpr int kMaxSplits = 4, kMaxSplits32 = 2 * kMaxSplits;
 
 }  // namespace
 
@@ -402,7 +409,7 @@ void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t 
   tci_plan::VVLadder& V = P.vv;
   // every K-split range non-empty (at least 64 long), so every partial of S is written
   const int64_t kmin = V.ncm > 0 ? std::min(V.np, V.nm) : V.np;
-  ks = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(ks, kMaxSplits), kmin / 64));
+  ks = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(ks, precision == TCI_SIGMA_FP64 ? kMaxSplits : kMaxSplits32), kmin / 64));
   if (precision == TCI_SIGMA_FP64) {
     V.ks = ks;
     build_products(P, V.g64, false, shape, ks, st);
@@ -483,9 +490,14 @@ void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool scatter, bool ga
            precision, st, [&] { g.launch(precision, st, 0, sc); });
   if (!gather) return;
   e0 = P.kt_begin(st);
-  hipLaunchKernelGGL(vv_gather_kernel, dim3(blocks((int64_t)P.dmax * P.dmax, 64), (unsigned)P.n_pairs), dim3(256), 0,
-                     st, P.tab, V.Sp.as<double>(), (int64_t)P.n_pairs * V.np, V.np, V.Sm.as<double>(),
-                     (int64_t)std::max(V.ncm, 1) * V.nm, V.nm, ks, V.colm.as<int32_t>(), P.R.as<double>());
+  auto gather_to_r = [&](auto* sp, auto* sm) {
+    hipLaunchKernelGGL((vv_gather_kernel<std::remove_pointer_t<decltype(sp)>>),
+                       dim3(blocks((int64_t)P.dmax * P.dmax, 64), (unsigned)P.n_pairs), dim3(256), 0, st, P.tab, sp,
+                       (int64_t)P.n_pairs * V.np, V.np, sm, (int64_t)std::max(V.ncm, 1) * V.nm, V.nm, ks,
+                       V.colm.as<int32_t>(), P.R.as<double>());
+  };
+  if (split) gather_to_r(V.Sp.as<float>(), V.Sm.as<float>());
+  else gather_to_r(V.Sp.as<double>(), V.Sm.as<double>());
   TCI_HIP(hipGetLastError());
   P.kt_end(e0, pn + " ladder vv_gather_kernel", 0.0, precision, st);
 }
@@ -509,8 +521,8 @@ double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
   int bs = N128, bk = kmin, bo = 0;
   NProgram& g = split ? V.gx : V.g64;
   const int orders = xcd_remap_forced() ? 1 : 2;
-  for (int ks : {1, 2, 4}) {
-    if (ks < kmin) continue;
+  for (int ks : {1, 2, 4, 6}) {
+    if (ks < kmin || ks > (split ? kMaxSplits32 : kMaxSplits)) continue;
     for (int sh : shapes) {
       vv_set_schedule(P, precision, sh, ks, st);
       for (int o = 0; o < orders; ++o) {

@@ -71,10 +71,10 @@ struct NProgram {
   int tm() const { return shape == N192 ? 192 : shape == N64 ? 64 : shape == N32K4 ? 32 : shape == N256 ? 256 : 128; }
   int tn() const { return shape == N128x192 ? 192 : tm(); }
   // adds the tiles of one M x N output; rows / cols of the stored element are
-  // offset by the blocking as in GemmProgram.  out_split: C is a split-row
-  // matrix (the operand of a following split product), ldc in 16-bit elements
+  // offset by the blocking as in GemmProgram.  out32 (split programs, no
+  // accumulation): C points to FP32 values, the sums as they were accumulated
   void add(double* C, int64_t ldc, int M, int N, const std::vector<NSeg>& s, bool accumulate, Blocking blk = Blocking(),
-           int oscale = -1, bool out_split = false);
+           int oscale = -1, bool out32 = false);
   void upload_tables(hipStream_t st);
   void launch(int precision, hipStream_t st, int64_t J0 = 0, const float* scales = nullptr) const;
   std::string kernel_name() const;

@@ -31,12 +31,10 @@ void launch_ngemm64(int shape, const Task* tasks, const NSeg* segs, int64_t ntas
 }
 
 void NProgram::add(double* C, int64_t ldc, int M, int N, const std::vector<NSeg>& s, bool accumulate, Blocking blk,
-                   int oscale, bool out_split) {
+                   int oscale, bool out32) {
   if (M <= 0 || N <= 0) return;
   TCI_REQUIRE(oscale < 0 || split, "output scales belong to split programs");
-  TCI_REQUIRE(!out_split || (split && !accumulate && blk.rdiv == 0 && blk.cdiv == 0 && ldc % 16 == 0 &&
-                             (reinterpret_cast<uintptr_t>(C) & 31) == 0),
-              "split-row output needs a split program, no accumulation or blocking, and 32-byte rows");
+  TCI_REQUIRE(!out32 || (split && !accumulate), "FP32 output needs a split program and no accumulation");
   for (const NSeg& x : s)
     TCI_REQUIRE(x.A && x.B && x.kbytes % 16 == 0 && x.lda % 16 == 0 && x.ldb % 16 == 0 && x.ja % 16 == 0 &&
                     x.jb % 16 == 0 && x.kbytes < ((int64_t)1 << 30) && x.reps >= 1 && x.reps < ((int64_t)1 << 30) && x.sa % 16 == 0 && x.sb % 16 == 0 &&
@@ -63,7 +61,7 @@ void NProgram::add(double* C, int64_t ldc, int M, int N, const std::vector<NSeg>
       t.seg0 = seg0;
       t.seg1 = seg1;
       t.accumulate = accumulate ? 1 : 0;
-      t.out_split = out_split ? 1 : 0;
+      t.out_split = out32 ? 1 : 0;
       t.rdiv = blk.rdiv;
       t.cdiv = blk.cdiv;
       t.rstride = blk.rstride;

@@ -272,31 +272,27 @@ __device__ __forceinline__ void nstore(const Task& t, const float*, const d4 (&a
     }
 }
 
-// four consecutive columns col .. col+3 of one row; split-row output writes
-// their hi and lo parts as 8-byte groups (columns beyond N up to the padding
-// to a multiple of 8 receive zeros: the caller's B rows are clamped, so they
-// are masked here)
-template <class T16>
+// four consecutive columns col .. col+3 of one row.  out_split (see NProgram):
+// C holds FP32 values.
 __device__ __forceinline__ void nput4(const Task& t, int row, int col, const float* v) {
   const int64_t ro = nrow_off(t, row);
+  const int cc = t.cdiv ? col % t.cdiv : col;
+  const bool whole = t.cdiv ? ((cc & 3) == 0 && cc + 3 < t.cdiv && col + 3 < t.N) : col + 3 < t.N;
   if (t.out_split) {
-    typedef T16 b4 __attribute__((ext_vector_type(4)));
-    b4 h, l;
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // ldc is arbitrary
+    __attribute__((address_space(1))) float* C = (__attribute__((address_space(1))) float*)t.C;
+    if (whole) {
+      const f4u o = {v[0], v[1], v[2], v[3]};
+      *(__attribute__((address_space(1))) f4u*)(C + ro + ncol_off(t, col)) = o;
+    } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float x = col + r < t.N ? v[r] : 0.f;
-      h[r] = (T16)x;
-      l[r] = (T16)(x - (float)h[r]);
+      for (int r = 0; r < 4; ++r)
+        if (col + r < t.N) C[ro + ncol_off(t, col + r)] = v[r];
     }
-    __attribute__((address_space(1))) b4* p =
-        (__attribute__((address_space(1))) b4*)(reinterpret_cast<uint16_t*>(t.C) + ro + xidx(col));
-    p[0] = h;
-    p[2] = l;
     return;
   }
-  const int cc = t.cdiv ? col % t.cdiv : col;
-  if (t.cdiv ? ((cc & 3) == 0 && cc + 3 < t.cdiv && col + 3 < t.N) : col + 3 < t.N) {
-    typedef double d4u __attribute__((ext_vector_type(4), aligned(8)));  // ldc is arbitrary
+  if (whole) {
+    typedef double d4u __attribute__((ext_vector_type(4), aligned(8)));
     __attribute__((address_space(1))) d4u* p = (__attribute__((address_space(1))) d4u*)(t.C + ro + ncol_off(t, col));
     const d4u o = {(double)v[0], (double)v[1], (double)v[2], (double)v[3]};
     if (t.accumulate) *p = *p + o;
@@ -322,7 +318,7 @@ __device__ __forceinline__ void nstore(const Task& t, const float* scales, const
       const int col = t.n0 + 16 * (wc + NWN * j) + 4 * lg;
       const f4 v = acc[i][j] * osc;
       const float x[4] = {v[0], v[1], v[2], v[3]};
-      if (col < t.N) nput4<typename TT::T16>(t, row, col, x);
+      if (col < t.N) nput4(t, row, col, x);
     }
   }
 }
@@ -343,7 +339,7 @@ __device__ __forceinline__ void nstore(const Task& t, const float* scales, const
         const int col = t.n0 + 32 * (wc + NWN * j) + 8 * g + 4 * hs;
         const float x[4] = {acc[i][j][4 * g] * osc, acc[i][j][4 * g + 1] * osc, acc[i][j][4 * g + 2] * osc,
                             acc[i][j][4 * g + 3] * osc};
-        if (col < t.N) nput4<typename TT::T16>(t, row, col, x);
+        if (col < t.N) nput4(t, row, col, x);
       }
   }
 }

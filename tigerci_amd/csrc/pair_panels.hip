@@ -502,12 +502,13 @@ __global__ void st_kernel(const double* __restrict__ s, int n, int nv, int nk, d
 // Block: one walk, one pair of 32 x 32 tiles (X >= Y); the transposed elements
 // come through LDS.  blockIdx.y == n_pairs: valence and singles.
 struct PackSrc {
-  const double* Rp;     // [nrp][sum_d2]
+  const void* Rp;       // [nrp][sum_d2]
   int64_t rstride;
   int nrp;
+  const double* rank;   // [sum_d2] FP64 products next to FP32 partials Rp, or null
   const double* R;      // null: no further terms
-  const double* Sp;     // [nsp][n_pairs][np], null: no resident ladder
-  const double* Sm;     // [nsp][ncm][nm]
+  const void* Sp;       // [nsp][n_pairs][np] (nsp = 0: no resident ladder)
+  const void* Sm;       // [nsp][ncm][nm]
   int64_t sp_part, sm_part;
   int nsp;
   const double* Hp;     // [n_pairs][np], null: part of S+-
@@ -517,6 +518,10 @@ struct PackSrc {
   const double* Kov;
 };
 
+// TR, TS: FP64, or FP32 where the sums were accumulated in FP32 (split products).
+// Bound by the partials it reads: at
+// 34/192/1200 (bf16x3) 208 us with all of them in FP64, 165 in FP32.
+template <class TR, class TS>
 __global__ __launch_bounds__(256) void pack_panels_kernel(PairTab T, PackSrc S, const double* __restrict__ x,
                                                           const double* __restrict__ g,
                                                           const double* __restrict__ sig0, double e_ref, int flags,
@@ -551,7 +556,9 @@ __global__ __launch_bounds__(256) void pack_panels_kernel(PairTab T, PackSrc S, 
   const int x0 = X * 32, y0 = Yt * 32;
   const int i = T.pairs[2 * P], j = T.pairs[2 * P + 1];
   const int64_t niv = (int64_t)no * nv, m2 = (int64_t)d * (d - 1) / 2;
-  const double* Rp = S.Rp + T.cd_off[P];
+  const TR* Rp = static_cast<const TR*>(S.Rp) + T.cd_off[P];
+  const double* rank = S.rank ? S.rank + T.cd_off[P] : nullptr;
+  const TS *Sp = static_cast<const TS*>(S.Sp), *Sm = static_cast<const TS*>(S.Sm);
   const double* R = S.R ? S.R + T.cd_off[P] : nullptr;
   const int32_t* D = T.dom_idx + off;
   const int cm = S.colm[P];
@@ -575,7 +582,10 @@ __global__ __launch_bounds__(256) void pack_panels_kernel(PairTab T, PackSrc S, 
 #pragma unroll 2
     for (int q = 0; q < S.nrp; ++q)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] += Rp[q * S.rstride + e[u]];
+      for (int u = 0; u < 4; ++u) v[u] += (double)Rp[q * S.rstride + e[u]];
+    if (rank)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] += rank[e[u]];
     if (R)
 #pragma unroll
       for (int u = 0; u < 4; ++u) v[u] += R[e[u]];
@@ -607,8 +617,8 @@ __global__ __launch_bounds__(256) void pack_panels_kernel(PairTab T, PackSrc S, 
   for (int q = 0; q < S.nsp; ++q)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      sp[u] += S.Sp[q * S.sp_part + p[u]];
-      if (m[u] >= 0) sm[u] += S.Sm[q * S.sm_part + m[u]];
+      sp[u] += (double)Sp[q * S.sp_part + p[u]];
+      if (m[u] >= 0) sm[u] += (double)Sm[q * S.sm_part + m[u]];
     }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
@@ -670,13 +680,16 @@ void zero(DevBuf& b, size_t bytes, hipStream_t st) {
 }
 
 // tile shape of a d x d pair block under a tiling mode: 0 by size (64, 128,
-// 192; 128-wide tiles above), 1 all 128, 2 all 64, 3 all 32 x 32 in four K-groups
-int shape_of(int mode, int d) {
+// 192, in split precision 256; 128-wide tiles above), 1 all 128, 2 all 64, 3 all
+// 32 x 32 in four K-groups.  A block on one tile reads its panels once: at
+// 16/203/811 (fp16x3) 0.76 ms on 256 x 256 tiles, 0.83 on 128 x 128
+int shape_of(int mode, int d, bool split) {
   if (mode == 3) return N32K4;
   if (mode == 2 || d <= 64) return N64;
   if (mode == 1 || d <= 128) return N128;
-  return d <= 192 ? N192 : N128;
+  return d <= 192 ? N192 : split && d <= 256 ? N256 : N128;
 }
+constexpr int kShapes = 6;
 
 }  // namespace
 
@@ -907,9 +920,9 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, int order, hipSt
   F.ks = ks;
   if (!into) {
     F.pair.clear();
-    F.pair.resize(4);
+    F.pair.resize(kShapes);
   }
-  for (int s = 0; s < (into ? 0 : 4); ++s) {
+  for (int s = 0; s < (into ? 0 : kShapes); ++s) {
     F.pair[s].split = split;
     F.pair[s].shape = s;
     F.pair[s].remap = order;
@@ -955,14 +968,14 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, int order, hipSt
     const double* Oji = Z.O3T.as<double>() + ((int64_t)j * n + i) * nv * Z.nk;
     const NSeg r1 = nseg(Z.sTp.p, Z.nk, Oij, Z.nk, Z.nk, 8, D, D), r2 = nseg(Oji, Z.nk, Z.sTp.p, Z.nk, Z.nk, 8, D, D);
     if (split) {
-      Z.rank.add(Z.Rp.as<double>() + (int64_t)ks * P.sum_d2 + P.h_cd_off[Q], d, d, d, {r1, r2}, false);
+      Z.rank.add(Z.Rp.as<double>() + (int64_t)kMaxKs * P.sum_d2 + P.h_cd_off[Q], d, d, d, {r1, r2}, false);
     } else {
       sg.push_back(r1);
       sg.push_back(r2);
     }
     int64_t tot = 0;
     for (const NSeg& s : sg) tot += s.kbytes;
-    NProgram& g = into ? *into : F.pair[shape_of(mode, d)];
+    NProgram& g = into ? *into : F.pair[shape_of(mode, d, split)];
     for (int s = 0; s < ks; ++s) {
       const int64_t b0 = (tot * s / ks) & ~(int64_t)127, b1 = s + 1 == ks ? tot : (tot * (s + 1) / ks) & ~(int64_t)127;
       std::vector<NSeg> part;
@@ -978,8 +991,9 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, int order, hipSt
         }
         pos += q.kbytes;
       }
-      g.add(Z.Rp.as<double>() + (int64_t)s * P.sum_d2 + P.h_cd_off[Q], d, d, d, part, false, Blocking(),
-            split ? 5 : -1);
+      const int64_t o = (int64_t)s * P.sum_d2 + P.h_cd_off[Q];
+      double* Rout = split ? reinterpret_cast<double*>(Z.Rp.as<float>() + o) : Z.Rp.as<double>() + o;
+      g.add(Rout, d, d, d, part, false, Blocking(), split ? 5 : -1, split);
     }
   }
   if (into) return;
@@ -1054,7 +1068,8 @@ void panels_tune(tci_plan& P, int precision, hipStream_t st) {
       for (int o = 0; o < (xcd_remap_forced() ? 1 : 2); ++o) {
         panels_programs(P, split, mode, ks, o, st);
         const double ms = time_ms(st, 2, [&] {
-          for (const auto& g : F.pair) g.launch(precision, st, 0, sc);
+          for (const auto& g : F.pair)
+            if (!g.tasks.empty()) g.launch(precision, st, 0, sc);
         });
         log += std::string(" ") + mname[mode] + "/" + std::to_string(ks) + (o ? "x:" : ":") + fmt_ms(ms);
         if (ms < best * 0.98) {
@@ -1132,7 +1147,8 @@ void panels_merge(tci_plan& P, hipStream_t st) {
   }
   // pair products, gW
   t0 = time_ms(st, 3, [&] {
-    for (const auto& g : F.pair) g.launch(TCI_SIGMA_FP64, st);
+    for (const auto& g : F.pair)
+      if (!g.tasks.empty()) g.launch(TCI_SIGMA_FP64, st);
     if (sing) P.nprogGW.launch(TCI_SIGMA_FP64, st);
   });
   log += "; pairs, gW separate:" + fmt_ms(t0);
@@ -1308,17 +1324,18 @@ void panels_pack(tci_plan& P, int precision, bool packed, bool use_r, const doub
   auto& Z = P.pp;
   const bool split = precision != TCI_SIGMA_FP64, psplit = split && Z.split;
   PackSrc S{};
-  S.Rp = Z.Rp.as<double>();
+  S.Rp = Z.Rp.p;
   S.rstride = P.sum_d2;
   // an FP64 build may have merged its pair products on another K-split
-  S.nrp = psplit ? Z.s16.ks + 1 : split || !Z.m2on ? Z.f64.ks : Z.m2_ks;
+  S.nrp = psplit ? Z.s16.ks : split || !Z.m2on ? Z.f64.ks : Z.m2_ks;
+  S.rank = psplit ? Z.Rp.as<double>() + (int64_t)kMaxKs * P.sum_d2 : nullptr;
   S.R = use_r ? P.R.as<double>() : nullptr;
   S.np = Z.np;
   S.nm = Z.nm;
   if (packed) {
     S.nsp = split ? P.vv.ksx : Z.m1on ? Z.m1_ks : P.vv.ks;
-    S.Sp = P.vv.Sp.as<double>();
-    S.Sm = P.vv.Sm.as<double>();
+    S.Sp = P.vv.Sp.p;
+    S.Sm = P.vv.Sm.p;
     S.sp_part = (int64_t)P.n_pairs * Z.np;
     S.sm_part = (int64_t)std::max(Z.ncm, 1) * Z.nm;
   }
@@ -1329,8 +1346,13 @@ void panels_pack(tci_plan& P, int precision, bool packed, bool use_r, const doub
   S.colm = Z.colm.as<int32_t>();
   S.Kov = P.Kov.as<double>();
   const int nt = (P.dmax + 31) / 32;
-  hipLaunchKernelGGL(pack_panels_kernel, dim3((unsigned)std::max<int64_t>(nt * (nt + 1) / 2, 4), P.n_pairs + 1),
-                     dim3(256), 0, st, P.tab, S, x, P.g.as<double>(), P.sig0.as<double>(), P.e_ref, flags, y, io);
+  auto pack = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::max<int64_t>(nt * (nt + 1) / 2, 4), P.n_pairs + 1), dim3(256), 0, st,
+                       P.tab, S, x, P.g.as<double>(), P.sig0.as<double>(), P.e_ref, flags, y, io);
+  };
+  if (psplit) packed ? pack(pack_panels_kernel<float, float>) : pack(pack_panels_kernel<float, double>);
+  else if (split && packed) pack(pack_panels_kernel<double, float>);
+  else pack(pack_panels_kernel<double, double>);
   TCI_HIP(hipGetLastError());
 }
 
