@@ -143,6 +143,8 @@ __global__ __launch_bounds__(256) void panels_kernel(PairTab T, PanelTab K, cons
 struct ExpandOut {
   double *C, *Ct, *s, *sT;  // C null: not needed
   int nk;
+  double* sP;               // s with rows of ldw, or null
+  int64_t ldw;
   void *CR, *CC, *CT;
   void *Xp, *Xm;            // null: no resident ladder
   int64_t ldp, ldm;         // values
@@ -168,6 +170,7 @@ __global__ __launch_bounds__(256) void expand_kernel(PairTab T, PanelTab K, cons
       const int k = (int)(e / nv), a = (int)(e - (int64_t)k * nv);
       const double v = k < n ? x[1 + (int64_t)(n - 1 - k) * nv + a] * INV_SQRT2 : 0.0;
       if (k < n) O.s[e] = v;
+      if (k < n && O.sP) O.sP[k * O.ldw + a] = v;
       O.sT[(int64_t)a * O.nk + k] = v;
     }
     return;
@@ -289,10 +292,13 @@ __global__ __launch_bounds__(256) void expand_kernel(PairTab T, PanelTab K, cons
   }
 }
 
-// JP_ij block k: rows x of D_ij, columns c of D_ik.  Grid (k, (i,j)).
+// JP_ij block k: rows x of D_ij, columns c of D_ik.  Grid (k, (i,j)).  F (FP64,
+// or null): the off-diagonal virtual Fock elements; block k = j of JP_ij (i >= j)
+// multiplies C_ij from both sides, so adding F there (half for i = j, whose
+// products come twice) makes F C + C F part of the pair products.
 template <bool SPLIT>
-__global__ __launch_bounds__(256) void jp_kernel(PairTab T, PanelTab K, const double* __restrict__ Jvv, void* JP,
-                                                 const float* scl, int f16) {
+__global__ __launch_bounds__(256) void jp_kernel(PairTab T, PanelTab K, const double* __restrict__ Jvv,
+                                                 const double* __restrict__ F, void* JP, const float* scl, int f16) {
   const int n = T.n_int, k = blockIdx.x, i = blockIdx.y / n, j = blockIdx.y % n;
   const int P = K.pairid[i * n + j], Q = K.pairid[i * n + k];
   if (P < 0 || Q < 0) return;
@@ -315,9 +321,13 @@ __global__ __launch_bounds__(256) void jp_kernel(PairTab T, PanelTab K, const do
       put_split8(srow(JP, base + x * ld, col + c), w, s, f16 != 0);
     }
   } else {
+    const double f = F && k == j && i >= j ? (i == j ? 0.5 : 1.0) : 0.0;
     for (int t = threadIdx.x; t < dP * dQ; t += 256) {
       const int x = t / dQ, c = t - x * dQ;
-      static_cast<double*>(JP)[base + x * ld + col + c] = -J[(int64_t)T.dom_idx[oP + x] * nv + T.dom_idx[oQ + c]];
+      const int64_t e = (int64_t)T.dom_idx[oP + x] * nv + T.dom_idx[oQ + c];
+      double v = -J[e];
+      if (f != 0.0) v += f * F[e];
+      static_cast<double*>(JP)[base + x * ld + col + c] = v;
     }
   }
 }
@@ -367,9 +377,8 @@ __global__ __launch_bounds__(256) void u_kernel(const double* __restrict__ Y, co
     const int a = a0 + tx;
     double v = 0.0;
     if (J < n_chol && a < n_v) {
-      const int64_t e = i * wstride_i + J * wstride_J + a;
-      v = W[e];
-      if (Y) v += Y[e];
+      v = W[i * wstride_i + J * wstride_J + a];
+      if (Y) v += Y[(i * n_chol + J) * n_v + a];
     }
     tile[r][tx] = v;
   }
@@ -394,11 +403,11 @@ __global__ __launch_bounds__(256) void u_kernel(const double* __restrict__ Y, co
 
 // max |Y + W| into *out (float bits)
 __global__ __launch_bounds__(256) void u_absmax_kernel(const double* __restrict__ Y, const double* __restrict__ W,
-                                                       int64_t n, unsigned* __restrict__ out) {
+                                                       int64_t n, int n_v, int pad, unsigned* __restrict__ out) {
   __shared__ float part[4];
   float m = 0.f;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
-    m = fmaxf(m, fabsf((float)(Y[e] + W[e])));
+    m = fmaxf(m, fabsf((float)(Y[e] + W[pad ? e + e / n_v * pad : e])));
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_down(m, off, 64));
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
@@ -828,7 +837,8 @@ void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st) {
   zero(F.XTp, (size_t)Z.np * Z.ldw * 8, st);
   zero(F.XTm, (size_t)std::max<int64_t>(Z.nm, 1) * Z.ldw * 8, st);
   const PanelTab K = ptab(P);
-  hipLaunchKernelGGL(jp_kernel<false>, dim3(n, n * n), dim3(256), 0, st, P.tab, K, P.Jvv.as<double>(), F.JP.p, nullptr, 0);
+  hipLaunchKernelGGL(jp_kernel<false>, dim3(n, n * n), dim3(256), 0, st, P.tab, K, P.Jvv.as<double>(),
+                     P.has_fvv ? P.Fvvp.as<double>() : nullptr, F.JP.p, nullptr, 0);
   hipLaunchKernelGGL(lp_kernel<false>, dim3((unsigned)P.n_chol, n), dim3(256), 0, st, P.tab, K, P.Lov.as<double>(),
                      F.LP.p, nullptr, 0);
   // LovT[(i,a)][J] = Lov[J][(i,a)]
@@ -854,7 +864,8 @@ void panels_build_split(tci_plan& P, hipStream_t st) {
   zero(F.hP, (size_t)P.n_pairs * Z.ldw * 4, st);
   zero(F.hM, (size_t)std::max(Z.ncm, 1) * Z.ldw * 4, st);
   const PanelTab K = ptab(P);
-  hipLaunchKernelGGL(jp_kernel<true>, dim3(n, n * n), dim3(256), 0, st, P.tab, K, P.Jvv.as<double>(), F.JP.p, s0, f16);
+  hipLaunchKernelGGL(jp_kernel<true>, dim3(n, n * n), dim3(256), 0, st, P.tab, K, P.Jvv.as<double>(), nullptr,
+                     F.JP.p, s0, f16);
   hipLaunchKernelGGL(lp_kernel<true>, dim3((unsigned)P.n_chol, n), dim3(256), 0, st, P.tab, K, P.Lov.as<double>(),
                      F.LP.p, s0, f16);
   hipLaunchKernelGGL(u_kernel<true>, dim3((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n), dim3(256), 0, st,
@@ -875,7 +886,7 @@ void add_w(tci_plan& P, NProgram& g, bool split) {
   const int n = P.n_int, nv = P.n_v, es = split ? 4 : 8;
   auto at = [&](const DevBuf& b, int64_t values) { return static_cast<const char*>(b.p) + values * es; };
   for (int i = 0; i < n; ++i)
-    g.add(P.W.as<double>() + (int64_t)i * P.n_chol * nv, nv, (int)P.n_chol, nv,
+    g.add(P.W.as<double>() + (int64_t)i * P.n_chol * P.ldw, P.ldw, (int)P.n_chol, nv,
             {nseg(at(F.LP, Z.h_lpoff[i]), Z.h_ld[i], at(F.CT, Z.h_poff[i]), Z.h_ld[i], Z.h_ld[i], es)}, false,
             Blocking(), split ? 12 : -1);
 }
@@ -1032,7 +1043,7 @@ void panels_tune(tci_plan& P, int precision, hipStream_t st) {
   if (precision == TCI_SIGMA_FP16X3)
     launch_split_scales(1, P.C.as<double>(), P.sum_d2, P.mx.maxbits.as<unsigned>(), 0, P.mx.scales.as<float>(),
                         (float)P.dmax, st);
-  P.run_Y(precision, st);
+  P.run_Y(precision, st, false);
   panels_terms(P, precision, false, xr.as<double>(), nullptr, st);
   TCI_HIP(hipStreamSynchronize(st));
   static const char* mname[4] = {"by size", "128", "64", "32k4"};
@@ -1189,6 +1200,13 @@ int panels_precision(const tci_plan& P, int precision) {
   return precision != TCI_SIGMA_FP64 && P.pp.split ? precision : (int)TCI_SIGMA_FP64;
 }
 
+// Are the virtual Fock products part of the pair products (FP64 ones only: split
+// operands would round F)?  A launch of their own took 114 us of 1.54 ms at
+// 13/151/607.
+bool panels_hold_fock(const tci_plan& P, int precision) {
+  return P.pp.on && panels_precision(P, precision) == TCI_SIGMA_FP64;
+}
+
 // Is the 4-internal product a K-range of the resident ladder's product?  Then
 // its operand XT+- is written before the ladder and no H+- exists.  Not where
 // the two differ in arithmetic or (fp16x3) in their scales.
@@ -1209,11 +1227,13 @@ bool panels_expand(tci_plan& P, int precision, const double* x, const IoSlot* io
   auto& F = split ? Z.s16 : Z.f64;
   ExpandOut O{};
   // C itself is read by the Cholesky-direct ladders and the virtual Fock products
-  O.C = !vv || P.has_fvv ? P.C.as<double>() : nullptr;
+  O.C = !vv || (P.has_fvv && split) ? P.C.as<double>() : nullptr;
   O.Ct = P.Ct.as<double>();
   O.s = P.s.as<double>();
   O.sT = Z.sTp.as<double>();
   O.nk = Z.nk;
+  O.sP = P.sP.as<double>();
+  O.ldw = P.ldw;
   O.CR = F.CR.p;
   O.CC = F.CC.p;
   O.CT = F.CT.p;
@@ -1290,18 +1310,17 @@ void panels_terms(tci_plan& P, int build, bool expanded, const double* x, const 
   if (f16) {
     hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(64), 0, st, mx + 1);
     hipLaunchKernelGGL(u_absmax_kernel, dim3(gsz((int64_t)n * nv * P.n_chol, 1024)), dim3(256), 0, st,
-                       P.Y.as<double>(), P.W.as<double>(), (int64_t)n * nv * P.n_chol, mx + 1);
+                       P.Y.as<double>(), P.W.as<double>(), (int64_t)n * nv * P.n_chol, nv, (int)(P.ldw - nv), mx + 1);
     hipLaunchKernelGGL(panel_scales_kernel, dim3(1), dim3(64), 0, st, 1, mx, sc);
     panels(1);
   }
   const dim3 gu((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n);
-  const int64_t wi = P.n_chol * nv;
   if (split) {
-    hipLaunchKernelGGL(u_kernel<true>, gu, dim3(256), 0, st, P.Y.as<double>(), P.W.as<double>(), nv, P.n_chol, wi,
-                       (int64_t)nv, F.U.p, Z.ldu, sc + 6, f16);
+    hipLaunchKernelGGL(u_kernel<true>, gu, dim3(256), 0, st, P.Y.as<double>(), P.W.as<double>(), nv, P.n_chol,
+                       P.n_chol * P.ldw, P.ldw, F.U.p, Z.ldu, sc + 6, f16);
   } else {
-    hipLaunchKernelGGL(u_kernel<false>, gu, dim3(256), 0, st, P.Y.as<double>(), P.W.as<double>(), nv, P.n_chol, wi,
-                       (int64_t)nv, F.U.p, Z.ldu, nullptr, 0);
+    hipLaunchKernelGGL(u_kernel<false>, gu, dim3(256), 0, st, P.Y.as<double>(), P.W.as<double>(), nv, P.n_chol,
+                       P.n_chol * P.ldw, P.ldw, F.U.p, Z.ldu, nullptr, 0);
   }
   TCI_HIP(hipGetLastError());
   const bool hole = !panels_hole_in_ladder(P, build);

@@ -386,7 +386,24 @@ void tci_plan::build(const tci_problem& p) {
   g.alloc((size_t)niv * 8);
   gss.alloc((size_t)niv * 8);
   Y.alloc((size_t)n_chol * niv * 8);
-  W.alloc((size_t)n_chol * niv * 8);
+  // the singles products of an odd n_v read rows that are not 16-byte aligned;
+  // a padded copy of L^J (up to 4 GB) puts them on the NT GEMM and into the
+  // merged launches of small builds: 13/151/607 Y and gW 131 -> 80 us
+  ldw = n_v;
+  {
+    size_t freeb = 0, totalb = 0;
+    TCI_HIP(hipMemGetInfo(&freeb, &totalb));
+    const double need = (double)n_chol * n_v * (n_v + 1) * 8.0;
+    if (!lvv_f32 && n_v % 2 != 0 && need <= 4.0e9 && 8.0 * need <= (double)freeb) {
+      ldw = n_v + 1;
+      LvvP.alloc((size_t)n_chol * n_v * ldw * 8);
+      launch_pad_rows(Lvv.as<double>(), n_chol * n_v, n_v, ldw, LvvP.as<double>(), st);
+      sP.alloc((size_t)n_int * ldw * 8);
+      launch_fill(sP.as<double>(), n_int * ldw, 0.0, st);
+    }
+  }
+  W.alloc((size_t)n_chol * n_int * ldw * 8);
+  if (ldw != n_v) launch_fill(W.as<double>(), n_chol * n_int * ldw, 0.0, st);
   part.alloc((size_t)std::max(n_pairs, 1) * ref_dot_slices() * 8);
   sig0.alloc(8);
   {
@@ -507,7 +524,7 @@ void tci_plan::build(const tci_problem& p) {
                 : op(b, 1, dq, nullptr, pos.as<int32_t>() + (size_t)Q * n_v);
       sg.push_back(seg(op(Lov.as<double>() + (int64_t)j * n_v, niv, 1, nullptr, DL(Q)), B, dq, 1.0));
     }
-    progW.add(W.as<double>() + (int64_t)i * n_chol * n_v, n_v, (int)n_chol, n_v, sg, false);
+    progW.add(W.as<double>() + (int64_t)i * n_chol * ldw, ldw, (int)n_chol, n_v, sg, false);
   }
   progW.upload_tables(st);
   // gW[s][i][a] = sum_{J in split s} sum_b W[i][J][b] L^J_ab
@@ -645,7 +662,7 @@ void tci_plan::build(const tci_problem& p) {
   flops_sigma = flops_ladder + f_ring + 2.0 * (double)n_chol * n_v * niv * 3.0 + 2.0 * (double)niv * niv;
   TCI_HIP(hipDeviceSynchronize());
   device_bytes = 0;
-  for (DevBuf* b : {&pairs, &dom_off, &dom_idx, &cd_off, &aa_off, &ab_off, &eps, &pos, &xmap, &cw_off, &isect_off, &isect,
+  for (DevBuf* b : {&pairs, &dom_off, &dom_idx, &cd_off, &aa_off, &ab_off, &eps, &pos, &xmap, &cw_off, &LvvP, &sP, &isect_off, &isect,
                     &inv_off, &inv_q, &inv_pos, &gpart_off, &Lvv, &Lov, &Kov, &Jvv, &Mss, &O4, &O3, &vvd, &vvx,
                     &diag, &C, &Ct, &R, &s, &sT, &g, &gss, &gW, &Y, &W, &gpart, &part, &sig0, &lad_part, &Tbuf, &Rpart, &Lp, &Cw, &lp_off_all, &Fm,
                     &Fvvp, &Fov})
@@ -655,17 +672,19 @@ void tci_plan::build(const tci_problem& p) {
 
 // Y[i][(J,a)]: s rows against the rows (J, a) of L^J
 void tci_plan::add_singles_Y(NProgram& g) const {
-  g.add(Y.as<double>(), n_chol * n_v, n_int, (int)(n_chol * n_v), {nseg(s.p, n_v, Lvv.p, n_v, n_v, 8)}, false);
+  const DevBuf &L = LvvP.p ? LvvP : Lvv, &sr = LvvP.p ? sP : s;
+  g.add(Y.as<double>(), n_chol * n_v, n_int, (int)(n_chol * n_v), {nseg(sr.p, ldw, L.p, ldw, ldw, 8)}, false);
 }
 
 // gW[split][i][a]: one repeated range over the Cholesky vectors of a split
 void tci_plan::add_singles_GW(NProgram& g) const {
+  const DevBuf& L = LvvP.p ? LvvP : Lvv;
   for (int sp = 0; sp < n_split; ++sp) {
     const int64_t J0 = n_chol * sp / n_split, J1 = n_chol * (sp + 1) / n_split;
-    NSeg q = nseg(W.as<double>() + J0 * n_v, n_chol * n_v, Lvv.as<double>() + J0 * n_v * n_v, n_v, n_v, 8);
+    NSeg q = nseg(W.as<double>() + J0 * ldw, n_chol * ldw, L.as<double>() + J0 * n_v * ldw, ldw, ldw, 8);
     q.reps = J1 - J0;
-    q.sa = (int64_t)n_v * 8;
-    q.sb = (int64_t)n_v * n_v * 8;
+    q.sa = ldw * 8;
+    q.sb = (int64_t)n_v * ldw * 8;
     g.add(gW.as<double>() + (int64_t)sp * n_int * n_v, n_v, n_int, n_v, {q}, false);
   }
 }
@@ -736,9 +755,10 @@ void tci_plan::tune_vector(DevBuf& x, hipStream_t st) {
   TCI_HIP(hipStreamSynchronize(st));
 }
 
-// Y of the current s
-void tci_plan::run_Y(int precision, hipStream_t st) {
+// Y of the current s (expanded: sP holds it already)
+void tci_plan::run_Y(int precision, hipStream_t st, bool expanded) {
   if (!nprogY.tasks.empty()) {
+    if (sP.p && !expanded) launch_pad_rows(s.as<double>(), n_int, n_v, ldw, sP.as<double>(), st);
     kt_run("singles Y", nprogY, precision, st, [&] { nprogY.launch(TCI_SIGMA_FP64, st); });
   } else {
     launch_transpose_small(s.as<double>(), n_int, n_v, sT.as<double>(), st);
@@ -1007,7 +1027,7 @@ void tci_plan::sigma_rest(const double* x, double* y, const IoSlot* io, int flag
   const int precision = flags & 0xff;
   int e0;
   const bool m1 = pp.m1on && precision == TCI_SIGMA_FP64, m2 = pp.m2on && precision == TCI_SIGMA_FP64;
-  if (!(m1 && pp.m1_singles)) run_Y(precision, st);
+  if (!(m1 && pp.m1_singles)) run_Y(precision, st, expanded);
   // with the panels the ladder's packed S+- and the pair terms meet in the
   // final kernel; R then holds a Cholesky-direct ladder and the virtual Fock
   // products only
@@ -1037,9 +1057,10 @@ void tci_plan::sigma_rest(const double* x, double* y, const IoSlot* io, int flag
   launch_singles_reduce(tab, I, gpart_off.as<int64_t>(), gpart.as<double>(), gss.as<double>(), gW.as<double>(), n_split,
                         g.as<double>(), x, s.as<double>(), has_fov ? Fov.as<double>() : nullptr, part.as<double>(),
                         sig0.as<double>(), st, io);
-  if (has_fvv && packed) launch_fill(R.as<double>(), sum_d2, 0.0, st);
-  if (has_fvv) kt_run("virtual Fock", fockvv, precision, st, [&] { fockvv.launch(st); });
-  if (pp.on) panels_pack(*this, precision, packed, !packed || has_fvv, x, io, flags, y, st);
+  const bool fock = has_fvv && !panels_hold_fock(*this, precision);
+  if (fock && packed) launch_fill(R.as<double>(), sum_d2, 0.0, st);
+  if (fock) kt_run("virtual Fock", fockvv, precision, st, [&] { fockvv.launch(st); });
+  if (pp.on) panels_pack(*this, precision, packed, !packed || fock, x, io, flags, y, st);
   else launch_pack(tab, dmax, x, R.as<double>(), g.as<double>(), sig0.as<double>(), e_ref, flags, y, st, io);
 }
 

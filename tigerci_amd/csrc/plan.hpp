@@ -41,7 +41,11 @@ struct tci_plan {
   int lad_chunks = 1;
   // programs
   tci::GemmProgram ring, progY, progW, progGW;
-  tci::NProgram nprogY, nprogGW;   // the same on the NT GEMM (even n_v, FP64 L^J)
+  tci::NProgram nprogY, nprogGW;   // the same on the NT GEMM (FP64 L^J, see singles_nt)
+  // odd n_v: L^J and s with rows of n_v + 1, the last column zero, for those
+  // products; ldw: row stride of W (n_v, or n_v + 1 with them)
+  tci::DevBuf LvvP, sP;
+  int64_t ldw = 0;
   // pair terms as per-walk products over packed panels (pair_panels.hip)
   struct PairPanels {
     bool on = false, split = false;           // split: split builds run them in split precision
@@ -256,12 +260,12 @@ struct tci_plan {
   void sigma_batch(const double* const* x, double* const* y, int nvec, int flags, hipStream_t st);
   void sigma_graph(const double* x, double* y, int flags, hipStream_t st);
   bool unpack_and_ladder(const double* x, const tci::IoSlot* io, int precision, hipStream_t st);
-  // are the rows of L^J 16-byte aligned FP64 (singles products on the NT GEMM)?
-  bool singles_nt() const { return !lvv_f32 && n_v % 2 == 0; }
+  // FP64 rows of L^J at a 16-byte aligned stride (singles products on the NT GEMM)?
+  bool singles_nt() const { return !lvv_f32 && (n_v % 2 == 0 || LvvP.p); }
   void add_singles_Y(tci::NProgram& g) const;
   void add_singles_GW(tci::NProgram& g) const;
   void tune_vector(tci::DevBuf& x, hipStream_t st);
-  void run_Y(int precision, hipStream_t st);
+  void run_Y(int precision, hipStream_t st, bool expanded);
   void build_two_phase_ladder(hipStream_t st);
   void two_phase_ladder(hipStream_t st);
   void ladder_chunk(const std::pair<int64_t, int>& ch, hipStream_t st);
@@ -306,6 +310,7 @@ int64_t vv_device_bytes(const tci_plan& P);
 bool panels_choose(const tci_plan& P);
 void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st);
 void panels_build_split(tci_plan& P, hipStream_t st);
+bool panels_hold_fock(const tci_plan& P, int precision);
 bool panels_hole_in_ladder(const tci_plan& P, int precision);
 bool panels_expand(tci_plan& P, int precision, const double* x, const tci::IoSlot* io, hipStream_t st);
 void panels_xt(tci_plan& P, int precision, const double* x, const tci::IoSlot* io, hipStream_t st);

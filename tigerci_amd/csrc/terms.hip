@@ -645,6 +645,14 @@ __global__ void pack_L_kernel(PairTab T, PackTab K, const LT* __restrict__ Lvv, 
   }
 }
 
+__global__ void pad_rows_kernel(const double* __restrict__ src, int64_t rows, int n, int64_t ld, double* __restrict__ dst) {
+  const int64_t tot = rows * ld;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot; e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r = e / ld, c = e - r * ld;
+    dst[e] = c < n ? src[r * n + c] : 0.0;
+  }
+}
+
 // pairs of doubles (both ends 16-byte aligned), an odd last one alone
 __global__ __launch_bounds__(256) void copy_kernel(const double* __restrict__ src, double* __restrict__ dst, int64_t n) {
   const int64_t h = n >> 1;
@@ -876,6 +884,12 @@ void launch_pack_L(const PairTab& T, const PackTab& K, const void* Lvv, bool f32
   dim3 grid(K.n_local, (unsigned)len), block(64, 4);
   if (f32) hipLaunchKernelGGL(pack_L_kernel<float>, grid, block, 0, st, T, K, (const float*)Lvv, J0, len, Lp);
   else hipLaunchKernelGGL(pack_L_kernel<double>, grid, block, 0, st, T, K, (const double*)Lvv, J0, len, Lp);
+  TCI_HIP(hipGetLastError());
+}
+
+void launch_pad_rows(const double* src, int64_t rows, int n, int64_t ld, double* dst, hipStream_t st) {
+  const unsigned g = (unsigned)std::min<int64_t>(std::max<int64_t>(cdiv(rows * ld, 256), 1), 65536);
+  hipLaunchKernelGGL(pad_rows_kernel, dim3(g), dim3(256), 0, st, src, rows, n, ld, dst);
   TCI_HIP(hipGetLastError());
 }
 

@@ -98,6 +98,8 @@ void launch_fock(const double* h_packed, const double* O4, const double* O3, con
                  int n_int, int n_v, double* F, hipStream_t st);
 // O3[k][k][q][b] -= f_qb and Mss += delta_ij f'_ab - delta_ab f'_ij (f' = F off its diagonal)
 void launch_fold_fock(const double* F, int n_int, int n_v, double* O3, double* Mss, hipStream_t st);
+// dst rows of ld values = src rows of n, zero-padded
+void launch_pad_rows(const double* src, int64_t rows, int n, int64_t ld, double* dst, hipStream_t st);
 // dst[0..n) = src[0..n), either of them pinned host memory
 void launch_copy(const double* src, double* dst, int64_t n, hipStream_t st);
 // Cw_P[r][c] = C_P[r][c], rows padded to an even count (block P at cw_off[P])
