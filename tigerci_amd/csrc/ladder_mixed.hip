@@ -980,7 +980,7 @@ void mixed_ladder_run(tci_plan& P, int precision, hipStream_t st) {
 void mixed_ladder(tci_plan& P, int precision, bool expanded, const double* x, const IoSlot* io, hipStream_t st) {
   mixed_prepare(P, precision, st);
   if (P.vv.split) {
-    if (panels_hole_in_ladder(P, precision)) panels_xt(P, precision, x, io, st);
+    if (!expanded && panels_hole_in_ladder(P, precision)) panels_xt(P, precision, x, io, st);
     vv_ladder(P, precision, st, !expanded, !P.pp.on);
     if (P.timing()) TCI_HIP(hipEventRecord(P.ev[3], st));
     return;

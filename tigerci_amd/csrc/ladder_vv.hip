@@ -527,7 +527,10 @@ double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
       vv_set_schedule(P, precision, sh, ks, st);
       for (int o = 0; o < orders; ++o) {
         g.remap = o;
-        const double ms = time_ms(st, 2, [&] { vv_ladder(P, precision, st, true, !P.pp.on); });
+        // with the partials read back by the final kernel, at about 4 TB/s
+        const double ms = time_ms(st, 2, [&] { vv_ladder(P, precision, st, true, !P.pp.on); }) +
+                          (P.pp.on ? (double)ks * (double)(P.n_pairs * V.np + V.ncm * V.nm) * (split ? 4.0 : 8.0) / 4.0e9
+                                   : 0.0);
         log += " " + std::to_string(g.tm()) + "x" + std::to_string(g.tn()) + "/" + std::to_string(ks) + (o ? "x:" : ":") +
                fmt_ms(ms);
         if (ms < best * 0.98) {

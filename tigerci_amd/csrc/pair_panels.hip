@@ -132,14 +132,81 @@ __global__ __launch_bounds__(256) void panels_kernel(PairTab T, PanelTab K, cons
   }
 }
 
+// XT+[p(a,b)][Q] = C+_ab, XT-[q(a,b)][Q] = C-_ab of walk Q (0 outside its
+// domain), rows of ldw values, from the CI vector (the symmetric part of C_Q
+// is its singlet-coupled block, the antisymmetric part its triplet-coupled
+// one).  Block: one a, 32 b and 32 walks; the walks' elements are read along b
+// and leave through LDS along Q.
+template <bool SPLIT>
+__device__ __forceinline__ void xt_block(const PairTab& T, const int32_t* __restrict__ pos, const double* __restrict__ x,
+                                         void* XTp, void* XTm, int64_t ldw, const float* scl, int f16, int a, int b0,
+                                         int Q0, double (&tp)[32][33], double (&tm)[32][33]) {
+  const int nv = T.n_v;
+  if (b0 > a) return;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int b = b0 + tx;
+  for (int r = ty; r < 32; r += 8) {
+    const int Q = Q0 + r;
+    double vp = 0.0, vm = 0.0;
+    if (Q < T.n_pairs && b <= a) {
+      const int32_t* ps = pos + (int64_t)Q * nv;
+      const int pa = ps[a], pb = ps[b];
+      if (pa >= 0 && pb >= 0) {
+        const int d = (int)(T.dom_off[Q + 1] - T.dom_off[Q]);
+        const bool same = T.pairs[2 * Q] == T.pairs[2 * Q + 1];
+        if (pa == pb) {
+          vp = same ? x[T.aa_off[Q] + pa] : -x[T.aa_off[Q] + pa] * INV_SQRT2;
+        } else {  // domains are sorted: pa > pb
+          const int64_t idx = T.ab_off[Q] + (int64_t)pa * (pa - 1) / 2 + pb;
+          vp = same ? x[idx] * INV_SQRT2 : -0.5 * x[idx];
+          if (!same) vm = -x[idx + (int64_t)d * (d - 1) / 2] * 0.28867513459481288225;  // 1 / (2 sqrt3)
+        }
+      }
+    }
+    tp[r][tx] = vp;
+    tm[r][tx] = vm;
+  }
+  __syncthreads();
+  if (!SPLIT) {
+    for (int r = ty; r < 32; r += 8) {
+      const int bb = b0 + r, Q = Q0 + tx;
+      if (bb > a || Q >= T.n_pairs) continue;
+      static_cast<double*>(XTp)[(tri(a) + bb) * ldw + Q] = tp[tx][r];
+      if (bb < a) static_cast<double*>(XTm)[(tri(a - 1) + bb) * ldw + Q] = tm[tx][r];
+    }
+  } else {
+    const int t = threadIdx.x & 127, r = t >> 2, c = 8 * (t & 3);
+    const bool minus = threadIdx.x >= 128;
+    const int bb = b0 + r;
+    if (bb <= a && Q0 + c < T.n_pairs && !(minus && bb == a)) {
+      float w[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w[q] = (float)(minus ? tm[c + q][r] : tp[c + q][r]);
+      put_split8(srow(minus ? XTm : XTp, (minus ? tri(a - 1) + bb : tri(a) + bb) * ldw, Q0 + c), w, scale_at(scl),
+                 f16 != 0);
+    }
+  }
+}
+
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void xt_kernel(PairTab T, const int32_t* __restrict__ pos, const double* __restrict__ x,
+                                                 const IoSlot* __restrict__ io, void* XTp, void* XTm, int64_t ldw,
+                                                 const float* scl, int f16) {
+  if (io) x = io->x;
+  __shared__ double tp[32][33], tm[32][33];
+  xt_block<SPLIT>(T, pos, x, XTp, XTm, ldw, scl, f16, blockIdx.x, blockIdx.y * 32, blockIdx.z * 32, tp, tm);
+}
+
 // Everything a sigma derives from the CI vector alone, in one pass over it:
 // the panels, Ct (and C where a term reads it), the rows X+- of the resident
-// ladder, s and its transpose.  Block: one walk, one pair of 32 x 32 tiles
+// ladder, s and its transpose, and (blocks past the walks') XT+-.  Block: one walk, one pair of 32 x 32 tiles
 // (X >= Y) of the packed triangle; each vector element is read once and both
 // orientations leave along rows.  FP64 and bf16x3 (the scales of fp16x3 need
 // max|C| first: unpack_kernel, vv_scatter_kernel and panels_kernel there).
 // Bound by its writes: 116 us (bf16x3) and 157 us (FP64) at 34/192/1200, against
-// 98 + 50 + 100 us for unpack, scatter and panels one after the other.
+// 98 + 50 + 100 us for unpack, scatter and panels one after the other.  XT+-
+// in a launch of its own took 5 us at 5/30/175, 11 at 10/100/400 and 95-125 at
+// 34/192/1200; here XTMEASURED.
 struct ExpandOut {
   double *C, *Ct, *s, *sT;  // C null: not needed
   int nk;
@@ -149,6 +216,9 @@ struct ExpandOut {
   void *Xp, *Xm;            // null: no resident ladder
   int64_t ldp, ldm;         // values
   const int32_t* colm;
+  const int32_t* pos;
+  void *XTp, *XTm;
+  int64_t ldx;              // row stride of XT+-
 };
 
 __device__ __forceinline__ void put_bf(uint16_t* p, double v) {
@@ -164,6 +234,17 @@ __global__ __launch_bounds__(256) void expand_kernel(PairTab T, PanelTab K, cons
                                                      const IoSlot* __restrict__ io, ExpandOut O) {
   if (io) x = io->x;
   const int Q = blockIdx.y, n = T.n_int, nv = T.n_v;
+  __shared__ double ta[32][33], tb[32][33];  // C[x][y] and C[y][x], x in tile X, y in tile Y
+  if (Q > T.n_pairs) {  // XT+-
+    const int64_t l = (int64_t)(Q - T.n_pairs - 1) * gridDim.x + blockIdx.x;
+    const int nb = (nv + 31) >> 5;
+    const int64_t r = l / nv;
+    const int z = (int)(r / nb);
+    if (z * 32 < T.n_pairs)
+      xt_block<SPLIT>(T, O.pos, x, O.XTp, O.XTm, O.ldx, nullptr, 0, (int)(l - r * nv), (int)(r - (int64_t)z * nb) * 32,
+                      z * 32, ta, tb);
+    return;
+  }
   if (Q == T.n_pairs) {  // singles (walks by descending hole)
     const int64_t tot = (int64_t)nv * O.nk;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot; e += (int64_t)gridDim.x * blockDim.x) {
@@ -175,7 +256,6 @@ __global__ __launch_bounds__(256) void expand_kernel(PairTab T, PanelTab K, cons
     }
     return;
   }
-  __shared__ double ta[32][33], tb[32][33];  // C[x][y] and C[y][x], x in tile X, y in tile Y
   const int64_t o = T.dom_off[Q];
   const int d = (int)(T.dom_off[Q + 1] - o), nt = (d + 31) >> 5;
   if ((int)blockIdx.x >= nt * (nt + 1) / 2) return;
@@ -413,63 +493,6 @@ __global__ __launch_bounds__(256) void u_absmax_kernel(const double* __restrict_
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) atomicMax(out, __float_as_uint(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]))));
-}
-
-// XT+[p(a,b)][Q] = C+_ab, XT-[q(a,b)][Q] = C-_ab of walk Q (0 outside its
-// domain), rows of ldw values, from the CI vector (the symmetric part of C_Q
-// is its singlet-coupled block, the antisymmetric part its triplet-coupled
-// one).  Block: one a, 32 b and 32 walks; the walks' elements are read along b
-// and leave through LDS along Q.
-template <bool SPLIT>
-__global__ __launch_bounds__(256) void xt_kernel(PairTab T, const int32_t* __restrict__ pos, const double* __restrict__ x,
-                                                 const IoSlot* __restrict__ io, void* XTp, void* XTm, int64_t ldw, const float* scl, int f16) {
-  if (io) x = io->x;
-  __shared__ double tp[32][33], tm[32][33];
-  const int nv = T.n_v, a = blockIdx.x, b0 = blockIdx.y * 32, Q0 = blockIdx.z * 32;
-  if (b0 > a) return;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const int b = b0 + tx;
-  for (int r = ty; r < 32; r += 8) {
-    const int Q = Q0 + r;
-    double vp = 0.0, vm = 0.0;
-    if (Q < T.n_pairs && b <= a) {
-      const int32_t* ps = pos + (int64_t)Q * nv;
-      const int pa = ps[a], pb = ps[b];
-      if (pa >= 0 && pb >= 0) {
-        const int d = (int)(T.dom_off[Q + 1] - T.dom_off[Q]);
-        const bool same = T.pairs[2 * Q] == T.pairs[2 * Q + 1];
-        if (pa == pb) {
-          vp = same ? x[T.aa_off[Q] + pa] : -x[T.aa_off[Q] + pa] * INV_SQRT2;
-        } else {  // domains are sorted: pa > pb
-          const int64_t idx = T.ab_off[Q] + (int64_t)pa * (pa - 1) / 2 + pb;
-          vp = same ? x[idx] * INV_SQRT2 : -0.5 * x[idx];
-          if (!same) vm = -x[idx + (int64_t)d * (d - 1) / 2] * 0.28867513459481288225;  // 1 / (2 sqrt3)
-        }
-      }
-    }
-    tp[r][tx] = vp;
-    tm[r][tx] = vm;
-  }
-  __syncthreads();
-  if (!SPLIT) {
-    for (int r = ty; r < 32; r += 8) {
-      const int bb = b0 + r, Q = Q0 + tx;
-      if (bb > a || Q >= T.n_pairs) continue;
-      static_cast<double*>(XTp)[(tri(a) + bb) * ldw + Q] = tp[tx][r];
-      if (bb < a) static_cast<double*>(XTm)[(tri(a - 1) + bb) * ldw + Q] = tm[tx][r];
-    }
-  } else {
-    const int t = threadIdx.x & 127, r = t >> 2, c = 8 * (t & 3);
-    const bool minus = threadIdx.x >= 128;
-    const int bb = b0 + r;
-    if (bb <= a && Q0 + c < T.n_pairs && !(minus && bb == a)) {
-      float w[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) w[q] = (float)(minus ? tm[c + q][r] : tp[c + q][r]);
-      put_split8(srow(minus ? XTm : XTp, (minus ? tri(a - 1) + bb : tri(a) + bb) * ldw, Q0 + c), w, scale_at(scl),
-                 f16 != 0);
-    }
-  }
 }
 
 // split rows of an FP64 matrix (rows x K values, stride ld) into stride ldo values
@@ -1245,7 +1268,14 @@ bool panels_expand(tci_plan& P, int precision, const double* x, const IoSlot* io
   }
   O.colm = Z.colm.as<int32_t>();
   const int nt = (P.dmax + 31) / 32;
-  const dim3 g((unsigned)std::max(nt * (nt + 1) / 2, 4), P.n_pairs + 1);
+  O.pos = P.pos.as<int32_t>();
+  O.XTp = F.XTp.p;
+  O.XTm = F.XTm.p;
+  O.ldx = Z.ldw;
+  // blocks of XT+-, in rows of the grid's width (at most 32768 rows)
+  const int64_t nxt = (int64_t)P.n_v * cdiv(P.n_v, 32) * cdiv(P.n_pairs, 32);
+  const int64_t gx = std::max<int64_t>({(int64_t)nt * (nt + 1) / 2, 4, cdiv(nxt, 32768)});
+  const dim3 g((unsigned)gx, (unsigned)(P.n_pairs + 1 + cdiv(nxt, gx)));
   const PanelTab K = ptab(P);
   if (split) hipLaunchKernelGGL(expand_kernel<true>, g, dim3(256), 0, st, P.tab, K, x, io, O);
   else hipLaunchKernelGGL(expand_kernel<false>, g, dim3(256), 0, st, P.tab, K, x, io, O);
@@ -1324,7 +1354,7 @@ void panels_terms(tci_plan& P, int build, bool expanded, const double* x, const 
   }
   TCI_HIP(hipGetLastError());
   const bool hole = !panels_hole_in_ladder(P, build);
-  if (hole) panels_xt(P, precision, x, io, st);
+  if (hole && !expanded) panels_xt(P, precision, x, io, st);
   P.kt_end(e0, pn + " pair panels", 0.0, build, st);
   if (build == TCI_SIGMA_FP64 && Z.m2on) {
     run("pair products, gW", Z.m2, precision);

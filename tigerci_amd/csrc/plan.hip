@@ -988,7 +988,7 @@ bool tci_plan::unpack_and_ladder(const double* x, const IoSlot* io, int precisio
     return expanded;
   }
   if (vv.fp64) {
-    if (panels_hole_in_ladder(*this, precision)) panels_xt(*this, precision, x, io, st);
+    if (!expanded && panels_hole_in_ladder(*this, precision)) panels_xt(*this, precision, x, io, st);
     if (pp.m1on) kt_run("fp64 products S, W, Y", pp.m1, precision, st, [&] { pp.m1.launch(TCI_SIGMA_FP64, st); });
     else vv_ladder(*this, TCI_SIGMA_FP64, st, !expanded, !pp.on);
     if (timing()) TCI_HIP(hipEventRecord(ev[3], st));
