@@ -401,10 +401,6 @@ void launch_xgemm192_bf16(const Task* tasks, const Seg* segs, int64_t ntasks, in
                           hipStream_t st, int remap);
 void launch_xgemm192_f16(const Task* tasks, const Seg* segs, int64_t ntasks, int64_t J0, const float* scales,
                          hipStream_t st, int remap);
-// 256 x 256 tiles on 32 x 32 MFMAs with direct-load stages (xgemm256.hip);
-// FP64 output only
-void launch_xgemm256(int precision, int waves, const Task* tasks, const Seg* segs, int64_t ntasks, int64_t J0,
-                     const float* scales, hipStream_t st, int remap);
 // LDS stages filled by direct loads (xgemm192d.hip): 192 x 192 with 3 stages,
 // 128 x 192 with 2 or 3
 void launch_xgemmd(int precision, int tm, int tn, int nst, const Task* tasks, const Seg* segs, int64_t ntasks,
