@@ -77,3 +77,15 @@ def test_synthetic_generator_matches_oracle():
         b = make_synthetic(**args, chunk_rows=17)
         for f in ("eps", "L", "pairs", "dom_off", "dom_idx"):
             assert np.array_equal(getattr(a, f), getattr(b, f)), f
+
+
+def test_long_rows_rule():
+    """Rows of one tile the NT GEMM's 32-bit byte offsets reach: (rows - 1) ld
+    plus the staged 512 bytes stay below 2^32, whatever a single row's length."""
+    ok = tci.load_library().tci_selftest_nt_rows
+    ok.argtypes, ok.restype = [ctypes.c_int64] * 3, ctypes.c_int
+    top = 2 ** 32 - 512
+    assert ok(1, 64, 2 ** 40) == 1
+    for rows in (2, 34, 64):
+        assert ok(rows, 64, top // (rows - 1)) == 1 and ok(rows, 64, top // (rows - 1) + 1) == 0
+    assert ok(500, 64, top // 63) == 1 and ok(500, 64, top // 63 + 1) == 0

@@ -16,6 +16,8 @@ import numpy as np
 import pytest
 
 import tigerci_amd as tci
+from oracle.problem import make_problem, random_ci_vector
+from oracle.sigma import Integrals, sigma as oracle_sigma
 from tigerci_amd.synthetic import workload, random_vector
 
 pytestmark = pytest.mark.gpu
@@ -94,3 +96,18 @@ def test_config3_split_vs_fp64(big, precision, tol):
     err = np.linalg.norm(smx - s64) / np.linalg.norm(s64)
     _say(f"  {precision} rel err {err:.2e}, Rayleigh diff {abs(x @ smx - x @ s64):.2e}")
     assert err < tol
+
+
+@pytest.mark.parametrize("n_chol", [43690, 43691])
+def test_long_rows_of_w(n_chol):
+    """W has rows of n_chol n_v values: plans on both sides of 2^21 of them
+    (16 MiB a row), FP64 L^J, against the oracle."""
+    _say("case: 2x48 with", n_chol, "Cholesky vectors")
+    prob = make_problem(2, 48, n_chol, 9, domain_range=(4, 9))
+    x = random_ci_vector(prob, 3)
+    plan = tci.Plan.from_problem(prob)
+    ref = oracle_sigma(prob, x, Integrals(prob))
+    got = _sigma(plan, x)
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    _say(f"  rel err {err:.2e}")
+    assert err < 1e-10

@@ -26,6 +26,8 @@
 // mostly idle chip).
 #pragma once
 
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace tci {
@@ -79,6 +81,14 @@ struct NProgram {
   void launch(int precision, hipStream_t st, int64_t J0 = 0, const float* scales = nullptr) const;
   std::string kernel_name() const;
 };
+
+// May a task address `rows` plain rows of ld_bytes from one tile of `tile` rows?
+// A lane holds the distance from the tile's first row, and the place within the
+// staged part of a row (at most 512 bytes), as a 32-bit byte offset.
+inline bool nrows_addressable(int64_t rows, int64_t tile, int64_t ld_bytes) {
+  const int64_t last = std::min(rows, tile) - 1;
+  return last <= 0 || ld_bytes <= ((((int64_t)1 << 32) - 512) / last);
+}
 
 // segment over rows of elements of `esz` bytes per value of k (8: FP64, 4: split rows)
 inline NSeg nseg(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t K, int esz,

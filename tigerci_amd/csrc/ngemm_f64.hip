@@ -41,10 +41,9 @@ void NProgram::add(double* C, int64_t ldc, int M, int N, const std::vector<NSeg>
                     (reinterpret_cast<uintptr_t>(x.A) & 15) == 0 &&
                     (reinterpret_cast<uintptr_t>(x.B) & 15) == 0,
                 "NT GEMM operands need 16-byte aligned rows and ranges");
-  // plain rows: a lane's offset spans one tile (gathered rows: the caller keeps
-  // the operand below 4 GiB)
+  // (gathered rows: the caller keeps the operand below 4 GiB)
   for (const NSeg& x : s)
-    TCI_REQUIRE((x.am || x.lda * 256 < ((int64_t)1 << 32)) && (x.bm || x.ldb * 256 < ((int64_t)1 << 32)),
+    TCI_REQUIRE((x.am || nrows_addressable(M, tm(), x.lda)) && (x.bm || nrows_addressable(N, tn(), x.ldb)),
                 "NT GEMM row stride too large");
   const int seg0 = (int)segs.size();
   for (const NSeg& x : s) segs.push_back(x);

@@ -1139,7 +1139,9 @@ void panels_merge(tci_plan& P, hipStream_t st) {
   for (const auto& g : F.pair) fl += g.alg_flops;
   if (!autotune_enabled() || !P.vv.fp64 || fl + P.vv.g64.alg_flops > 4.0e10) return;
   const bool sing = P.singles_nt();
-  Z.m1_singles = Z.m2_singles = sing;
+  const bool gw = !P.nprogGW.tasks.empty();
+  Z.m1_singles = sing;
+  Z.m2_singles = gw;
   std::string log = "fp64 merged launches:";
   const int kp0 = F.ks;
   // S, W, Y
@@ -1183,7 +1185,7 @@ void panels_merge(tci_plan& P, hipStream_t st) {
   t0 = time_ms(st, 3, [&] {
     for (const auto& g : F.pair)
       if (!g.tasks.empty()) g.launch(TCI_SIGMA_FP64, st);
-    if (sing) P.nprogGW.launch(TCI_SIGMA_FP64, st);
+    if (gw) P.nprogGW.launch(TCI_SIGMA_FP64, st);
   });
   log += "; pairs, gW separate:" + fmt_ms(t0);
   best = t0 * 0.98;
@@ -1192,7 +1194,7 @@ void panels_merge(tci_plan& P, hipStream_t st) {
     Z.m2.clear();
     Z.m2.shape = sh;
     panels_programs(P, false, 0, ks, 0, st, &Z.m2);
-    if (sing) P.add_singles_GW(Z.m2);
+    if (gw) P.add_singles_GW(Z.m2);
     Z.m2.upload_tables(st);
   };
   for (int sh : {(int)N64, (int)N32K4})

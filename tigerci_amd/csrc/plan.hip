@@ -394,7 +394,7 @@ void tci_plan::build(const tci_problem& p) {
     size_t freeb = 0, totalb = 0;
     TCI_HIP(hipMemGetInfo(&freeb, &totalb));
     const double need = (double)n_chol * n_v * (n_v + 1) * 8.0;
-    if (!lvv_f32 && n_v % 2 != 0 && need <= 4.0e9 && 8.0 * need <= (double)freeb) {
+    if (!lvv_f32 && n_v % 2 != 0 && need <= 4.0e9 && 8.0 * need <= (double)freeb && gw_nt(n_v + 1)) {
       ldw = n_v + 1;
       LvvP.alloc((size_t)n_chol * n_v * ldw * 8);
       launch_pad_rows(Lvv.as<double>(), n_chol * n_v, n_v, ldw, LvvP.as<double>(), st);
@@ -529,9 +529,10 @@ void tci_plan::build(const tci_problem& p) {
   progW.upload_tables(st);
   // gW[s][i][a] = sum_{J in split s} sum_b W[i][J][b] L^J_ab
   progGW.clear();
+  // (on the dense kernel too where W's row stride leaves the NT GEMM's 32-bit offsets)
   nprogGW.clear();
   nprogGW.shape = N64;
-  if (nt_ok) {
+  if (nt_ok && gw_nt(ldw)) {
     add_singles_GW(nprogGW);
   } else {
     progGW.dense = true;

@@ -262,6 +262,8 @@ struct tci_plan {
   bool unpack_and_ladder(const double* x, const tci::IoSlot* io, int precision, hipStream_t st);
   // FP64 rows of L^J at a 16-byte aligned stride (singles products on the NT GEMM)?
   bool singles_nt() const { return !lvv_f32 && (n_v % 2 == 0 || LvvP.p); }
+  // ... and rows of W (n_chol values of ld each) its tiles of at most 64 rows can address?
+  bool gw_nt(int64_t ld) const { return tci::nrows_addressable(n_int, 64, n_chol * ld * 8); }
   void add_singles_Y(tci::NProgram& g) const;
   void add_singles_GW(tci::NProgram& g) const;
   void tune_vector(tci::DevBuf& x, hipStream_t st);

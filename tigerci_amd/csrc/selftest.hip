@@ -10,7 +10,7 @@
 //   bf16/f16 32x32x16: A[i][k] lane i+32(k/8), element k%8; B likewise
 //                  D[i][j] lane j+32((i/4)%2), register 4(i/8)+i%4
 // Inputs are small integers so every product and sum is exact.
-#include "common.hpp"
+#include "ngemm.hpp"
 
 namespace tci {
 namespace {
@@ -113,4 +113,9 @@ extern "C" int tci_selftest_mfma(void) {
     set_last_error(e.what());
     return e.code;
   }
+}
+
+// the dispatch rule of ngemm.hpp, for its test on the host
+extern "C" int tci_selftest_nt_rows(int64_t rows, int64_t tile, int64_t ld_bytes) {
+  return tci::nrows_addressable(rows, tile, ld_bytes) ? 1 : 0;
 }
