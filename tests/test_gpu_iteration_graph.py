@@ -13,6 +13,7 @@ mixed -> FP64 switch, roots that stop on their residual norm inside a replay,
 repeated solves that reuse the captured graphs, and the generalized (ACPF)
 problem.
 """
+import ctypes
 import sys
 
 import numpy as np
@@ -165,3 +166,50 @@ def test_iteration_graphs_across_solves_on_one_plan():
         assert r0["converged"] and r1["converged"]
         assert r1["iterations"] == r0["iterations"]
         assert np.abs(e0 - e1).max() < 1e-10
+
+
+@pytest.mark.parametrize("graph", [False, "iteration"])
+def test_solves_keep_their_vector_store(graph):
+    """A plan's solves share one store of expansion vectors: the first lays it
+    out for the vectors it uses (not for the thousand its budget allows) and the
+    next allocates nothing.  A solve past the first slots grows the store and
+    gives what the grown store gives; one of fewer roots, a small budget with
+    collapses and the generalized problem use it in turn."""
+    _say("case: vector store of solves, graph", graph)
+    prob = make_problem(6, 100, 90, 31, l_scale=0.03)
+    plan = tci.Plan.from_problem(prob)
+    n = plan.n_csf
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert tci.load_library().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    kw = dict(energy_tol=1e-8, norm_tol=1e-6)
+    vec = tci.DeviceArray(2 * n)
+    out = tci.DeviceArray(n)
+    plan.sigma(vec, out)
+    f0 = free()
+    e1, r1 = plan.davidson(roots=2, vectors=vec, graph=graph, **kw)
+    v1, f1 = vec.numpy(), free()
+    e2, r2 = plan.davidson(roots=2, vectors=vec, graph=graph, **kw)
+    kept = f0 - f1
+    _say(f"  {r1['iterations']} iterations, kept {kept / 8 / n:.1f} vectors")
+    assert free() == f1 and 0 < kept < 8 * n * 64 + (160 << 20)
+    assert np.array_equal(e1, e2) and np.array_equal(v1, vec.numpy())
+    # one root to 1e-13: more vectors than the first slots of a new plan hold
+    tight = dict(roots=1, energy_tol=1e-13, norm_tol=1e-9, vectors=out, graph=graph)
+    other = tci.Plan.from_problem(prob)
+    e3, r3 = other.davidson(**tight)
+    v3 = out.numpy()
+    assert r3["converged"] and r3["sigma_fp64"] > 10
+    e4, _ = other.davidson(**tight)
+    assert np.array_equal(e3, e4) and np.array_equal(v3, out.numpy())
+    e5, r5 = other.davidson(max_vectors=8, **tight)
+    assert r5["collapses"] > 0 and abs(e5[0] - e3[0]) < 1e-9
+    g = tci.acpf_gvalues(tci.ACPF, 12)
+    e6, _ = other.davidson(roots=1, g_values=g, graph=graph, **kw)
+    e7, _ = tci.Plan.from_problem(prob).davidson(roots=1, g_values=g, graph=graph, **kw)
+    assert abs(e6[0] - e7[0]) < 1e-9
+    e8, _ = other.davidson(**tight)
+    assert abs(e8[0] - e3[0]) < 1e-11

@@ -610,21 +610,71 @@ void gen_eigh(int m, const std::vector<double>& h, const std::vector<double>& g,
     }
 }
 
+// b at least `bytes` large, its first `used` bytes kept.  Where the old and the
+// new buffer do not fit beside each other, the contents go through host memory.
+void grow_buffer(DevBuf& b, size_t used, size_t bytes) {
+  if (b.bytes >= bytes) return;
+  TCI_HIP(hipDeviceSynchronize());
+  if (!used) b.reset();
+  void* q = nullptr;
+  if (hipMalloc(&q, bytes) == hipSuccess) {
+    DevBuf nb;
+    nb.p = q;
+    nb.bytes = bytes;
+    if (used) TCI_HIP(hipMemcpy(q, b.p, used, hipMemcpyDeviceToDevice));
+    TCI_HIP(hipDeviceSynchronize());
+    b = std::move(nb);
+    return;
+  }
+  (void)hipGetLastError();
+  std::vector<char> host(used);
+  if (used) TCI_HIP(hipMemcpy(host.data(), b.p, used, hipMemcpyDeviceToHost));
+  b.alloc(bytes);
+  if (used) TCI_HIP(hipMemcpy(b.p, host.data(), used, hipMemcpyHostToDevice));
+}
+
+// The store of one solve: the plan's, or one of its own where another solve
+// holds that.  What a solve leaves behind above DavStore::kKeep is given back.
+// A store allocated by every solve for all the vectors its budget allows costs
+// more than the solve once the memory that earlier solves freed has to be
+// cleared for reuse (about 36 GB/s): at 34/192/1200, three roots, 0.90 s a
+// solve against 0.20 s, with 32 GB allocated and 4 GB used.
+struct StoreUse {
+  tci_plan::DavStore own;
+  std::unique_lock<std::mutex> held;
+  tci_plan::DavStore& Q;
+  explicit StoreUse(tci_plan& P) : held(P.dav.lock, std::try_to_lock), Q(held.owns_lock() ? P.dav : own) {}
+  ~StoreUse() {
+    if (Q.V.bytes + Q.S.bytes <= tci_plan::DavStore::kKeep) return;
+    Q.V.reset();
+    Q.S.reset();
+    Q.slots = 0;
+  }
+  // `need` slots (at most `most`) of n values for the vectors and the sigmas, the first m kept
+  void slots(int64_t n, int m, int need, int most) {
+    if (need <= Q.slots) return;
+    const int c = std::min(most, std::max(need, Q.slots + Q.slots / 2));
+    grow_buffer(Q.V, (size_t)m * n * 8, (size_t)c * n * 8);
+    grow_buffer(Q.S, (size_t)m * n * 8, (size_t)c * n * 8);
+    Q.slots = c;
+  }
+};
+
 struct Dav {
   tci_plan& P;
   hipStream_t st = nullptr;
   int64_t n;
   int nblk = 1024;
-  DevBuf ptrs, coefs, partial, dots;
-  std::vector<double*> hptr;
+  DevBuf &ptrs, &coefs, &partial, &dots;
   // pointer table: X vectors from 0, the second operand set from XMAX
   static constexpr int XMAX = 2048, RB = 4;
-  explicit Dav(tci_plan& p) : P(p), n(p.n_csf) {
+  Dav(tci_plan& p, tci_plan::DavStore& Q)
+      : P(p), n(p.n_csf), ptrs(Q.ptrs), coefs(Q.coefs), partial(Q.partial), dots(Q.dots) {
     nblk = (int)std::min<int64_t>(1024, std::max<int64_t>(1, cdiv(n, 256 * 4)));
-    ptrs.alloc((XMAX + RB) * sizeof(double*));
-    coefs.alloc((size_t)RB * XMAX * sizeof(double));
-    partial.alloc((size_t)RB * XMAX * nblk * sizeof(double));
-    dots.alloc((size_t)RB * XMAX * sizeof(double));
+    if (!ptrs.p) ptrs.alloc((XMAX + RB) * sizeof(double*));
+    if (!coefs.p) coefs.alloc((size_t)RB * XMAX * sizeof(double));
+    if (!partial.p) partial.alloc((size_t)RB * XMAX * nblk * sizeof(double));
+    if (!dots.p) dots.alloc((size_t)RB * XMAX * sizeof(double));
   }
   // out[k R + j] = X_k . V_j (R = V.size()): one pass over X per group of RB
   // vectors V_j
@@ -1026,17 +1076,22 @@ int davidson_impl(tci_plan* plan, const tci_davidson_params* prm, const double* 
     const int prec0 = prm->precision & 0xff;
     TCI_REQUIRE(prec0 == TCI_SIGMA_FP64 || prec0 == TCI_SIGMA_BF16X3 || prec0 == TCI_SIGMA_FP16X3, "unknown precision");
     const int64_t n = plan->n_csf;
-    Dav D(*plan);
+    StoreUse store(*plan);
+    Dav D(*plan, store.Q);
     hipStream_t st = D.st;
     auto t_start = std::chrono::steady_clock::now();
     double t_sigma = 0.0;
     int n64 = 0, nmix = 0, n_collapse = 0;
-    DevBuf Vb, Sb, work;
-    Vb.alloc((size_t)mslots * n * 8);
-    Sb.alloc((size_t)mslots * n * 8);
-    work.alloc((size_t)n * 8);
-    double* Vp = Vb.as<double>();
-    double* Sp = Sb.as<double>();
+    // slots for ten vectors a root at first (most solves converge in them)
+    double *Vp = nullptr, *Sp = nullptr;
+    auto slots = [&](int m, int need) {
+      store.slots(n, m, need, mslots);
+      Vp = store.Q.V.as<double>();
+      Sp = store.Q.S.as<double>();
+    };
+    slots(0, std::min(mslots, 10 * roots));
+    DevBuf &work = store.Q.work, &gbuf = store.Q.g, &sel = store.Q.sel;
+    if (!work.p) work.alloc((size_t)n * 8);
     auto Vk = [&](int k) { return Vp + (int64_t)k * n; };
     auto Sk = [&](int k) { return Sp + (int64_t)k * n; };
     double* tmp = work.as<double>();  // G c of the generalized residual
@@ -1044,11 +1099,10 @@ int davidson_impl(tci_plan* plan, const tci_davidson_params* prm, const double* 
     const unsigned gxn = (unsigned)std::min<int64_t>(cdiv(n, 256), 8192);
     // generalized problem: G on the device, its subspace matrix gs beside h
     const bool gen = gvals != nullptr;
-    DevBuf gbuf;
     const double* gd = nullptr;
     if (gen) {
       for (int q = 0; q < 5; ++q) TCI_REQUIRE(std::isfinite(gvals[q]) && gvals[q] > 0.0, "g values must be positive");
-      gbuf.alloc((size_t)n * 8);
+      if (!gbuf.p) gbuf.alloc((size_t)n * 8);
       hipLaunchKernelGGL(gdiag_kernel, dim3(gxn), dim3(256), 0, st, gbuf.as<double>(), n,
                          (int64_t)plan->n_int * plan->n_v, gvals[0], gvals[3], gvals[4]);
       TCI_HIP(hipGetLastError());
@@ -1095,8 +1149,7 @@ int davidson_impl(tci_plan* plan, const tci_davidson_params* prm, const double* 
     std::vector<int64_t> idx;
     {
       const int nb = (int)std::min<int64_t>(1024, std::max<int64_t>(1, cdiv(n, 256 * 4)));
-      DevBuf sel;
-      sel.alloc((size_t)nb * 16);
+      if (!sel.p) sel.alloc((size_t)nb * 16);
       double* bv = sel.as<double>();
       int64_t* bi = reinterpret_cast<int64_t*>(bv + nb);
       std::vector<double> hv(nb);
@@ -1161,6 +1214,8 @@ int davidson_impl(tci_plan* plan, const tci_davidson_params* prm, const double* 
       iter_ensure(*plan, IL);
     }
     for (it = 1; it <= maxit; ++it) {
+      // a collapse takes 2 roots slots beyond the basis, new vectors at most as many
+      slots(m, std::min(mslots, m + 2 * roots));
       if (!sig_done) {
         // new vectors of the unsettled roots: their sigmas, then
         // h(q,k) = <c_q, sigma_k> for q <= k in one pass over the basis

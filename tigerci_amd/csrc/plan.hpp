@@ -209,6 +209,17 @@ struct tci_plan {
   void* iter_host = nullptr;
   size_t iter_host_bytes = 0;
   int iter_clock_khz = 0;
+  // stores of the Davidson solver (davidson.hip), kept from one solve to the
+  // next up to kKeep bytes: the expansion vectors and their sigmas (`slots` of
+  // each, grown as a solve needs them), G c and G of the generalized problem,
+  // and the solver's tables.  One solve at a time uses them; a solve that finds
+  // them taken brings its own.
+  struct DavStore {
+    static constexpr size_t kKeep = (size_t)16 << 30;
+    std::mutex lock;
+    int slots = 0;
+    tci::DevBuf V, S, work, g, sel, ptrs, coefs, partial, dots;
+  } dav;
   // staging of tci_htimesc, laid out on its first call: device vectors, a ring
   // of pinned host slots and the event of each slot's last copy; one call at a
   // time
