@@ -149,3 +149,24 @@ def test_vv_transposed_split_product(args, precision, tile):
         for x, g in zip(xs, got):
             assert _rel(g, oracle_sigma(prob, x, ints)) < SPLIT_TOL[precision]
         assert np.array_equal(_sigma(plan, xs[0], precision=precision, graph=True), got[0])
+
+
+@pytest.mark.parametrize("autotune", ["0", "1"])
+@pytest.mark.parametrize("first", ["bf16x3", "fp16x3"])
+def test_fp16x3_k_splits(first, autotune):
+    """fp16x3 keeps its FP32 chains at a quarter of the contraction whichever
+    split precision is prepared first and without autotuning: the product that
+    ran names at least four K-splits."""
+    _say("case: fp16x3 K-splits,", first, "first, autotune", autotune)
+    prob = make_problem(4, 60, 70, 12)
+    x = random_ci_vector(prob, 5)
+    with _env(TCI_LADDER_VV=1, TCI_AUTOTUNE=autotune):
+        plan = tci.Plan.from_problem(prob)
+        _sigma(plan, x, precision=first)
+        plan.profile(True)
+        got = _sigma(plan, x, precision="fp16x3")
+        names = [k["name"] for k in plan.profile_kernels("fp16x3") if "(ab|cd) product" in k["name"]]
+        plan.profile(False)
+    _say("  ", names)
+    assert len(names) == 1 and any(f"K-split {k} " in names[0] for k in (4, 5, 6, 7, 8))
+    assert _rel(got, oracle_sigma(prob, x, Integrals(prob))) < SPLIT_TOL["fp16x3"]

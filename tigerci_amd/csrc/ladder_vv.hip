@@ -304,6 +304,10 @@ void build_products(tci_plan& P, NProgram& g, bool split, int shape, int ks, hip
 // K-splits of the products: partials S in FP64, and in FP32 (split) in the same
 // memory
 constexpr int kMaxSplits = 4, kMaxSplits32 = 2 * kMaxSplits;
+// FP32 sums of scaled fp16x3 products lose about as much to the length of the
+// chain as the operands do to their split: four K-splits at least, whichever
+// split precision chose the schedule and with or without autotuning
+constexpr int kMinSplits16 = 4;
 
 }  // namespace
 
@@ -409,6 +413,7 @@ void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t 
   tci_plan::VVLadder& V = P.vv;
   // every K-split range non-empty (at least 64 long), so every partial of S is written
   const int64_t kmin = V.ncm > 0 ? std::min(V.np, V.nm) : V.np;
+  if (precision == TCI_SIGMA_FP16X3) ks = std::max(ks, kMinSplits16);
   ks = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(ks, precision == TCI_SIGMA_FP64 ? kMaxSplits : kMaxSplits32), kmin / 64));
   if (precision == TCI_SIGMA_FP64) {
     V.ks = ks;
@@ -514,9 +519,7 @@ double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
     shapes.push_back(N64);
     shapes.push_back(N32K4);
   }
-  // FP32 sums of scaled fp16x3 products lose about as much to the length of
-  // the chain as the operands do to their split: four K-splits at least
-  const int kmin = precision == TCI_SIGMA_FP16X3 ? 4 : 1;
+  const int kmin = precision == TCI_SIGMA_FP16X3 ? kMinSplits16 : 1;
   double best = 1e300;
   int bs = N128, bk = kmin, bo = 0;
   NProgram& g = split ? V.gx : V.g64;
