@@ -1,7 +1,7 @@
 """GPU parity of the pair-panel sigma (pair_panels.hip, ngemm_kernel.hpp) at the
 sizes where its tiles and K-ranges end: against the oracle, and against the
-gathered pair terms (TCI_DENSE_PAIRS=0) that accept every layout.  Odd and even
-virtual spaces, domains on both sides of 64, 128, 192 and 256, explicit
+gathered pair terms (TCI_DENSE_PAIRS=0) that accept every layout; with panels
+over the domains and with wide ones (TCI_DENSE_PAIRS=2).  Odd and even virtual spaces, domains on both sides of 64, 128, 192 and 256, explicit
 one-electron parts, FP32 L^J, both ladders, tuned and fixed schedules, graph
 replays; the host-vector htimesc around its slot length.
 
@@ -18,6 +18,7 @@ import pytest
 import tigerci_amd as tci
 from oracle.problem import make_problem, random_ci_vector
 from oracle.sigma import Integrals, sigma as oracle_sigma
+from tigerci_amd.synthetic import make_synthetic, random_vector
 
 pytestmark = pytest.mark.gpu
 TOL = {"fp64": 1e-10, "bf16x3": 5e-5, "fp16x3": 2e-6}
@@ -63,7 +64,8 @@ CASES = [
     dict(n_int=3, n_v=260, n_chol=13, seed=307, domain_range=(190, 260)),
     dict(n_int=4, n_v=200, n_chol=18, seed=308, domain_range=(60, 200), weak_below=70),
 ]
-ENVS = [{}, {"TCI_AUTOTUNE": "0"}, {"TCI_LADDER_VV": "0"}, {"TCI_LADDER_VV": "1", "TCI_AUTOTUNE": "0"}]
+ENVS = [{}, {"TCI_AUTOTUNE": "0"}, {"TCI_LADDER_VV": "0"}, {"TCI_LADDER_VV": "1", "TCI_AUTOTUNE": "0"},
+        {"TCI_DENSE_PAIRS": "2"}, {"TCI_DENSE_PAIRS": "2", "TCI_LADDER_VV": "0", "TCI_AUTOTUNE": "0"}]
 
 
 @pytest.mark.parametrize("env", ENVS, ids=lambda e: ",".join(e) or "tuned")
@@ -74,7 +76,7 @@ def test_panels_match_oracle_and_gathered_terms(args, env):
     ints = Integrals(prob)
     x = random_ci_vector(prob, 21)
     ref = oracle_sigma(prob, x, ints)
-    with _env(TCI_DENSE_PAIRS="0", **env):
+    with _env(**{**env, "TCI_DENSE_PAIRS": "0"}):
         gathered = _sigma(tci.Plan.from_problem(prob), x)
     with _env(**env):
         plan = tci.Plan.from_problem(prob)
@@ -92,6 +94,25 @@ def test_panels_match_oracle_and_gathered_terms(args, env):
             f32 = tci.Plan.from_problem(prob, ladder_dtype="f32")
             assert _rel(_sigma(f32, x), ref) < 1e-6  # L^J rounded to FP32: 24 bits
             assert _rel(_sigma(f32, x, precision="bf16x3"), ref) < TOL["bf16x3"]
+
+
+def test_wide_panels_where_the_others_do_not_fit():
+    """60 internal orbitals with 168 full virtuals: panels over the domains would
+    take 75 GB, the plan takes the wide ones; against the gathered products."""
+    _say("case: wide panels at 60x168x24")
+    syn = make_synthetic(60, 168, 24, 309)
+    with _env(TCI_DENSE_PAIRS="0", TCI_LADDER_VV="1"):
+        plan = tci.Plan.from_problem(syn)
+        x = random_vector(plan.n_csf, 7)
+        ref = _sigma(plan, x)
+        del plan
+    with _env(TCI_LADDER_VV="1"):
+        plan = tci.Plan.from_problem(syn)
+        assert "wide pair panels" in plan.tuning()
+        y = _sigma(plan, x)
+        z = _sigma(plan, x, precision="bf16x3")
+    _say(f"  fp64 {_rel(y, ref):.2e} bf16x3 {_rel(z, ref):.2e}")
+    assert _rel(y, ref) < 1e-12 and _rel(z, ref) < TOL["bf16x3"]
 
 
 @pytest.mark.parametrize("n_int,n_v", [(2, 5), (3, 174), (9, 81)])

@@ -88,21 +88,6 @@ __global__ void vv_assemble_kernel(const double* __restrict__ W, int n_v, int a0
   }
 }
 
-__device__ __forceinline__ void put_split1(uint16_t* p, double v, float s, int f16) {
-  const float x = (float)v * s;
-  if (f16) {
-    const _Float16 h = (_Float16)x;
-    const _Float16 l = (_Float16)(x - (float)h);
-    p[0] = __builtin_bit_cast(uint16_t, h);
-    p[8] = __builtin_bit_cast(uint16_t, l);
-  } else {
-    const __bf16 h = (__bf16)x;
-    const __bf16 l = (__bf16)(x - (float)h);
-    p[0] = __builtin_bit_cast(uint16_t, h);
-    p[8] = __builtin_bit_cast(uint16_t, l);
-  }
-}
-
 // split rows of a row-major FP64 n x n matrix of row stride ld: out[r ldo + xidx(k)] (k padded to 8)
 __global__ void split_square_kernel(const double* __restrict__ src, int64_t n, int64_t ld, uint16_t* __restrict__ out,
                                     int64_t ldo, const float* scl, int f16) {
@@ -173,12 +158,12 @@ __global__ void vv_scatter_kernel(PairTab T, const double* __restrict__ C, const
     }
     const double vp = r == c ? 0.5 * hr : 0.5 * (hr + rh);
     const int64_t kp = tri(gr) + gc;
-    if (SPLIT) put_split1(static_cast<uint16_t*>(Xp) + P * ldp + xidx(kp), vp, s, f16);
+    if (SPLIT) put_split1(static_cast<uint16_t*>(Xp) + P * ldp + xidx(kp), vp, s, f16 != 0);
     else static_cast<double*>(Xp)[P * ldp + kp] = vp;
     if (cm >= 0 && gr != gc) {
       const double vm = 0.5 * (hr - rh);
       const int64_t km = tri(gr - 1) + gc;
-      if (SPLIT) put_split1(static_cast<uint16_t*>(Xm) + cm * ldm + xidx(km), vm, s, f16);
+      if (SPLIT) put_split1(static_cast<uint16_t*>(Xm) + cm * ldm + xidx(km), vm, s, f16 != 0);
       else static_cast<double*>(Xm)[cm * ldm + km] = vm;
     }
   }

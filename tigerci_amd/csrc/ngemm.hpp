@@ -32,6 +32,22 @@
 
 namespace tci {
 
+// one value of a split-row chunk: its parts 8 elements apart
+__device__ __forceinline__ void put_split1(uint16_t* p, double v, float s, bool f16) {
+  const float x = (float)v * s;
+  if (f16) {
+    const _Float16 h = (_Float16)x;
+    const _Float16 l = (_Float16)(x - (float)h);
+    p[0] = __builtin_bit_cast(uint16_t, h);
+    p[8] = __builtin_bit_cast(uint16_t, l);
+  } else {
+    const __bf16 h = (__bf16)x;
+    const __bf16 l = (__bf16)(x - (float)h);
+    p[0] = __builtin_bit_cast(uint16_t, h);
+    p[8] = __builtin_bit_cast(uint16_t, l);
+  }
+}
+
 // One contraction range of a task.  kbytes: valid bytes of k per row, a
 // multiple of 16; lda / ldb row strides in bytes (multiples of 16); am / bm
 // row maps or null; ja / jb bytes per unit of the launch argument J0.  The range

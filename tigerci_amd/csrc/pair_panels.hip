@@ -16,6 +16,9 @@
 //        + U_i Lov_j + (U_j Lov_i)^T
 // and the 3-internal singles terms are two more ranges of it (FP64):
 //        + s_i O_ij^T + O_ji s^T,   O_ij[b][k] = -(ki|bj).
+// Where the JP_ij of all pairs do not fit, the columns (k, c) run over all
+// virtuals instead (wide panels): JP_ij then is the rows D_ij of one JP_j, and
+// LP_i one LP, for four N x N matrices (N = n_int n_v) in all.
 // All operands have their k contiguous and rows gathered through D_P, so they
 // run on the NT GEMM (ngemm.hpp): flops 2 d_P^2 (2 |K_i| + 2 |K_j| + 2 n_chol)
 // per walk, the count of the gathered per-walk products, at the rate of the
@@ -65,10 +68,33 @@ struct PanelTab {
   const int64_t* jpoff;  // [i n_int + j] start of JP_ij
   const int64_t* lpoff;  // [i] start of LP_i (n_chol rows)
   const int32_t* pairid;
+  int wide;              // columns of a block: 0 positions in its domain, 1 virtuals
 };
+
+// column, within its block, of position y of the domain D
+__device__ __forceinline__ int pcol(const PanelTab& K, const int32_t* __restrict__ D, int y) { return K.wide ? D[y] : y; }
 
 __device__ __forceinline__ uint16_t* srow(void* base, int64_t row_start, int64_t col) {
   return static_cast<uint16_t*>(base) + 2 * row_start + xidx(col);
+}
+
+// Eight values of a panel row (its block starts at value `at`), positions y ..
+// y + 7 of the domain D of size d, as split parts.  A wide block has them
+// together only where D holds eight aligned consecutive virtuals.
+__device__ __forceinline__ void put_cols(const PanelTab& K, void* dst, int64_t row, int64_t at,
+                                         const int32_t* __restrict__ D, int y, int d, const float (&w)[8], float s, bool f16) {
+  if (!K.wide) {
+    put_split8(srow(dst, row, at + y), w, s, f16);
+    return;
+  }
+  const int g = D[y];
+  if (y + 7 < d && (g & 7) == 0 && D[y + 7] == g + 7) {
+    put_split8(srow(dst, row, at + g), w, s, f16);
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (y + q < d) put_split1(srow(dst, row, at + D[y + q]), w[q], s, f16);
 }
 
 // CR, CC and CT of both panels of walk Q from its C block: 32 x 32 tiles, the
@@ -103,7 +129,7 @@ __global__ __launch_bounds__(256) void panels_kernel(PairTab T, PanelTab K, cons
         const int x = x0 + r, y = y0 + tx;
         if (x >= d || y >= d) continue;
         const double a = p ? tb[r][tx] : ta[r][tx], b = p ? ta[r][tx] : tb[r][tx];
-        const int64_t e = base + (int64_t)T.dom_idx[o + x] * ld + y;
+        const int64_t e = base + (int64_t)T.dom_idx[o + x] * ld + pcol(K, T.dom_idx + o, y);
         static_cast<double*>(CR)[e] = a;
         static_cast<double*>(CC)[e] = b;
         static_cast<double*>(CT)[e] = 2.0 * a - b;
@@ -126,8 +152,8 @@ __global__ __launch_bounds__(256) void panels_kernel(PairTab T, PanelTab K, cons
         w[q] = (float)(arr == 0 ? a : arr == 1 ? b : 2.0 * a - b);
       }
       void* dst = arr == 0 ? CR : arr == 1 ? CC : CT;
-      put_split8(srow(dst, K.poff[u] + (int64_t)T.dom_idx[o + x] * K.ld[u], K.koff[u * T.n_int + v] + y), w,
-                 arr == 2 ? st : s, f16 != 0);
+      put_cols(K, dst, K.poff[u] + (int64_t)T.dom_idx[o + x] * K.ld[u], K.koff[u * T.n_int + v], T.dom_idx + o, y, d, w,
+               arr == 2 ? st : s, f16 != 0);
     }
   }
 }
@@ -339,7 +365,7 @@ __global__ __launch_bounds__(256) void expand_kernel(PairTab T, PanelTab K, cons
         const int64_t g = T.dom_idx[o + row];
         for (int p = 0; p < two; ++p) {
           const int iu = p ? j : i, iv = p ? i : j;
-          const int64_t q = K.poff[iu] + K.koff[iu * n + iv] + g * K.ld[iu] + col;
+          const int64_t q = K.poff[iu] + K.koff[iu * n + iv] + g * K.ld[iu] + pcol(K, T.dom_idx + o, col);
           const double aa = p ? b : a, bb = p ? a : b;
           static_cast<double*>(O.CR)[q] = aa;
           static_cast<double*>(O.CC)[q] = bb;
@@ -366,7 +392,8 @@ __global__ __launch_bounds__(256) void expand_kernel(PairTab T, PanelTab K, cons
           v[q] = col + q < d ? (float)(arr == 0 ? a : arr == 1 ? b : 2.0 * a - b) : 0.f;
         }
         void* dst = arr == 0 ? O.CR : arr == 1 ? O.CC : O.CT;
-        put_split8(srow(dst, K.poff[iu] + (int64_t)T.dom_idx[o + row] * K.ld[iu], K.koff[iu * n + iv] + col), v);
+        put_cols(K, dst, K.poff[iu] + (int64_t)T.dom_idx[o + row] * K.ld[iu], K.koff[iu * n + iv], T.dom_idx + o, col, d,
+                 v, 1.f, false);
       }
     }
   }
@@ -437,6 +464,55 @@ __global__ __launch_bounds__(256) void lp_kernel(PairTab T, PanelTab K, const do
     } else {
       for (int c = threadIdx.x; c < d; c += 256) static_cast<double*>(LP)[row + col + c] = L[T.dom_idx[o + c]];
     }
+  }
+}
+
+// The same for wide panels, whose columns (k, c) run over all virtuals of all
+// internal orbitals: one JP_j[x][(k,c)] for every i, rows x over all virtuals.
+// Half of F goes into block k = j: the walk (i, j) meets it once in JP_j and
+// once in JP_i.  Grid (k, j).
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void jp_wide_kernel(PairTab T, PanelTab K, const double* __restrict__ Jvv,
+                                                      const double* __restrict__ F, void* JP, const float* scl, int f16) {
+  const int k = blockIdx.x, j = blockIdx.y, nv = T.n_v;
+  const int hi = max(k, j), lo = min(k, j);
+  const double* J = Jvv + ((int64_t)hi * (hi + 1) / 2 + lo) * nv * nv;
+  const int64_t ld = K.ld[j], base = K.jpoff[j], col = (int64_t)k * ((nv + 7) & ~7);
+  const float s = SPLIT ? scale_at(scl) : 1.f;
+  if (SPLIT) {
+    const int nch = (nv + 7) >> 3;
+    for (int t = threadIdx.x; t < nv * nch; t += 256) {
+      const int x = t / nch, c = 8 * (t - x * nch);
+      float w[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w[q] = c + q < nv ? (float)-J[(int64_t)x * nv + c + q] : 0.f;
+      put_split8(srow(JP, base + x * ld, col + c), w, s, f16 != 0);
+    }
+  } else {
+    for (int t = threadIdx.x; t < nv * nv; t += 256) {
+      const int x = t / nv, c = t - x * nv;
+      static_cast<double*>(JP)[base + x * ld + col + c] = F && k == j ? 0.5 * F[t] - J[t] : -J[t];
+    }
+  }
+}
+
+// ... and one LP[J][(k,c)].  Grid (J, k).
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void lp_wide_kernel(PairTab T, PanelTab K, const double* __restrict__ Lov, void* LP,
+                                                      const float* scl, int f16) {
+  const int k = blockIdx.y, nv = T.n_v;
+  const int64_t row = (int64_t)blockIdx.x * K.ld[0], col = (int64_t)k * ((nv + 7) & ~7);
+  const double* L = Lov + ((int64_t)blockIdx.x * T.n_int + k) * nv;
+  const float s = SPLIT ? scale_at(scl) : 1.f;
+  if (SPLIT) {
+    for (int c = 8 * (int)threadIdx.x; c < nv; c += 8 * 256) {
+      float w[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w[q] = c + q < nv ? (float)L[c + q] : 0.f;
+      put_split8(srow(LP, row, col + c), w, s, f16 != 0);
+    }
+  } else {
+    for (int c = threadIdx.x; c < nv; c += 256) static_cast<double*>(LP)[row + col + c] = L[c];
   }
 }
 
@@ -703,7 +779,23 @@ inline unsigned gsz(int64_t work, unsigned cap = 16384) {
 PanelTab ptab(const tci_plan& P) {
   const auto& Z = P.pp;
   return PanelTab{Z.koff.as<int32_t>(), Z.ld.as<int64_t>(), Z.poff.as<int64_t>(), Z.jpoff.as<int64_t>(),
-                  Z.lpoff.as<int64_t>(), Z.pairid.as<int32_t>()};
+                  Z.lpoff.as<int64_t>(), Z.pairid.as<int32_t>(), Z.wide ? 1 : 0};
+}
+
+// JP and LP of one element type from the integrals
+template <bool SPLIT>
+void fill_jp_lp(tci_plan& P, tci_plan::PairPanels::Set& F, const double* Fvv, const float* scl, int f16, hipStream_t st) {
+  const int n = P.n_int;
+  const PanelTab K = ptab(P);
+  const dim3 lg((unsigned)P.n_chol, n), b(256);
+  if (P.pp.wide) {
+    hipLaunchKernelGGL(jp_wide_kernel<SPLIT>, dim3(n, n), b, 0, st, P.tab, K, P.Jvv.as<double>(), Fvv, F.JP.p, scl, f16);
+    hipLaunchKernelGGL(lp_wide_kernel<SPLIT>, lg, b, 0, st, P.tab, K, P.Lov.as<double>(), F.LP.p, scl, f16);
+  } else {
+    hipLaunchKernelGGL(jp_kernel<SPLIT>, dim3(n, n * n), b, 0, st, P.tab, K, P.Jvv.as<double>(), Fvv, F.JP.p, scl, f16);
+    hipLaunchKernelGGL(lp_kernel<SPLIT>, lg, b, 0, st, P.tab, K, P.Lov.as<double>(), F.LP.p, scl, f16);
+  }
+  TCI_HIP(hipGetLastError());
 }
 
 void zero(DevBuf& b, size_t bytes, hipStream_t st) {
@@ -725,16 +817,29 @@ constexpr int kShapes = 6;
 
 }  // namespace
 
-// Panels hold |K_i| columns for n_v rows three times, for every ordered strong
-// pair's domain once (JP) and for n_chol rows once (LP).
-bool panels_choose(const tci_plan& P) {
-  if (P.n_pairs == 0) return false;
+// Layout of the panels: 0 none (gathered products), 1 columns over the domains,
+// 2 wide (columns over all virtuals).
+//
+// Panels over the domains hold |K_i| columns for n_v rows three times, for every
+// ordered strong pair's domain once (JP) and for n_chol rows once (LP): JP grows
+// as n_int^3 d^2, 72 GB at about 50 full domains of 200.  Beyond that the wide
+// ones share JP and LP between the internal orbitals (4 N^2 values, N = n_int
+// n_v) for products of K = N.  They are taken while their flops stay below 2.5
+// times the gathered products' (domains of a quarter of the virtuals and more):
+// the NT GEMM runs at 42-58 TF (FP64), the gathered products at 15-28.  Sigma at
+// 60/200/600, gathered -> wide: full domains 2938 -> 234 ms (FP64), 2901 -> 42.5
+// (bf16x3); domains of 100-200 1180 -> 150 and 1145 -> 34 ms.
+int panels_choose(const tci_plan& P) {
+  if (P.n_pairs == 0) return 0;
   const char* env = std::getenv("TCI_DENSE_PAIRS");
-  if (env && env[0] == '0') return false;
+  if (env && env[0] == '0') return 0;
   const int n = P.n_int;
-  double vals = 0.0, kmax = 0.0;
+  if (n > 255) return 0;  // grids of n_int^2 rows
+  const double nv = P.n_v, nc = (double)P.n_chol, np = (double)tri(P.n_v), nw = (double)up(P.n_pairs, 16);
+  const double ldw = (double)up(n * up(P.n_v, 8), 16);  // row stride of a wide panel
+  double vals = 0.0, kmax = 0.0, f_gather = 0.0, f_wide = 2.0 * n * nc * nv * ldw;
   for (int i = 0; i < n; ++i) {
-    double kp = 0.0, rows = 3.0 * P.n_v + (double)P.n_chol;
+    double kp = 0.0, rows = 3.0 * nv + nc;
     for (int k = 0; k < n; ++k) {
       const int Q = P.pairid[(size_t)i * n + k];
       if (Q < 0) continue;
@@ -745,16 +850,31 @@ bool panels_choose(const tci_plan& P) {
     vals += (kp + 16.0) * rows;
     kmax = std::max(kmax, kp + 16.0);
   }
-  const double np = (double)tri(P.n_v);
-  vals += 2.0 * np * (double)up(P.n_pairs, 16) + 2.0 * np * P.n_pairs;  // XT+-, H+-
-  vals += (double)n * n * P.n_v * (n + 1);
+  for (int Q = 0; Q < P.n_pairs; ++Q) {
+    const double d = (double)(P.h_dom_off[Q + 1] - P.h_dom_off[Q]);
+    for (int e = 0; e < 2; ++e)
+      for (int k = 0; k < n; ++k) {
+        const int R = P.pairid[(size_t)P.h_pairs[2 * Q + e] * n + k];
+        if (R >= 0) f_gather += 6.0 * d * d * (double)(P.h_dom_off[R + 1] - P.h_dom_off[R]);
+      }
+    f_gather += 4.0 * d * d * nc + 2.0 * d * nv * nc;
+    f_wide += 2.0 * d * d * (4.0 * ldw + 2.0 * nc);
+  }
+  // XT+-, H+-, the 4- and 3-internal factors, U and LovT
+  const double common = 2.0 * np * nw + 2.0 * np * P.n_pairs + 2.0 * nw * P.n_pairs + (double)n * n * nv * (n + 1) +
+                        2.0 * n * nv * (nc + 16.0);
   size_t freeb = 0, totalb = 0;
-  if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) return false;
+  if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) return 0;
   // FP64 and one split copy and the K-split partials, with room left for the
-  // ladder; gathered rows are addressed by 32-bit byte offsets from a panel
-  const double need = 12.0 * vals + 8.0 * 9.0 * (double)P.sum_d2;
-  return need <= 72.0e9 && need + 64.0e9 <= (double)freeb && 8.0 * kmax * P.n_v < 4.0e9 &&
-         8.0 * ((double)P.n_chol + 16.0) * P.n_v < 4.0e9;
+  // ladder's smallest form (T' of a chunk in either precision); gathered rows
+  // are addressed by 32-bit byte offsets from a panel
+  auto fits = [&](double v, double k) {
+    const double need = 12.0 * (v + common) + 8.0 * 9.0 * (double)P.sum_d2;
+    return need <= 72.0e9 && need + 24.0e9 <= (double)freeb && 8.0 * k * nv < 4.0e9 && 8.0 * (nc + 16.0) * nv < 4.0e9;
+  };
+  const bool force = env && env[0] == '2';
+  if (!force && fits(vals, kmax)) return 1;
+  return fits((4.0 * n * nv + nc) * ldw, ldw) && (force || f_wide <= 2.5 * f_gather) ? 2 : 0;
 }
 
 // Do the pair terms of a split build run in split precision?  Where the
@@ -767,7 +887,7 @@ bool panels_split_rule(const tci_plan& P) {
   const double N = (double)P.n_int * P.n_v;
   if (8.0 * (6.0 * N * N + 3.0 * P.n_pairs * (double)P.n_v * P.n_v) > 48.0e9 || N >= 46340.0) return false;
   const char* env = std::getenv("TCI_DENSE_PAIRS");
-  if (env && env[0] == '1') return true;
+  if (env && (env[0] == '1' || env[0] == '2')) return true;
   double f = 0.0;
   for (int Q = 0; Q < P.n_pairs; ++Q) {
     const double d = (double)(P.h_dom_off[Q + 1] - P.h_dom_off[Q]);
@@ -793,6 +913,19 @@ void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st) {
   Z.n_panel = Z.n_jp = Z.n_lp = 0;
   for (int i = 0; i < n; ++i) {
     int64_t w = 0;
+    if (Z.wide) {  // JP_j for every i at j, one LP
+      w = n * up(nv, 8);
+      Z.h_ld[i] = std::max<int64_t>(up(w, 16), 16);
+      Z.h_poff[i] = Z.n_panel;
+      Z.n_panel += nv * Z.h_ld[i];
+      for (int k = 0; k < n; ++k) {
+        if (P.pairid[(size_t)i * n + k] >= 0) Z.h_koff[(size_t)i * n + k] = (int32_t)(k * up(nv, 8));
+        Z.h_jpoff[(size_t)i * n + k] = k * nv * Z.h_ld[i];
+      }
+      Z.n_jp = Z.n_panel;
+      Z.n_lp = P.n_chol * Z.h_ld[i];
+      continue;
+    }
     for (int k = 0; k < n; ++k) {
       const int Q = P.pairid[(size_t)i * n + k];
       if (Q < 0) continue;
@@ -859,11 +992,7 @@ void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st) {
   zero(F.LovT, (size_t)n * nv * Z.ldu * 8, st);
   zero(F.XTp, (size_t)Z.np * Z.ldw * 8, st);
   zero(F.XTm, (size_t)std::max<int64_t>(Z.nm, 1) * Z.ldw * 8, st);
-  const PanelTab K = ptab(P);
-  hipLaunchKernelGGL(jp_kernel<false>, dim3(n, n * n), dim3(256), 0, st, P.tab, K, P.Jvv.as<double>(),
-                     P.has_fvv ? P.Fvvp.as<double>() : nullptr, F.JP.p, nullptr, 0);
-  hipLaunchKernelGGL(lp_kernel<false>, dim3((unsigned)P.n_chol, n), dim3(256), 0, st, P.tab, K, P.Lov.as<double>(),
-                     F.LP.p, nullptr, 0);
+  fill_jp_lp<false>(P, F, P.has_fvv ? P.Fvvp.as<double>() : nullptr, nullptr, 0, st);
   // LovT[(i,a)][J] = Lov[J][(i,a)]
   hipLaunchKernelGGL(u_kernel<false>, dim3((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n), dim3(256), 0, st,
                      nullptr, P.Lov.as<double>(), nv, P.n_chol, (int64_t)nv, (int64_t)n * nv, F.LovT.p, Z.ldu, nullptr, 0);
@@ -886,11 +1015,7 @@ void panels_build_split(tci_plan& P, hipStream_t st) {
   zero(F.XTm, (size_t)std::max<int64_t>(Z.nm, 1) * Z.ldw * 4, st);
   zero(F.hP, (size_t)P.n_pairs * Z.ldw * 4, st);
   zero(F.hM, (size_t)std::max(Z.ncm, 1) * Z.ldw * 4, st);
-  const PanelTab K = ptab(P);
-  hipLaunchKernelGGL(jp_kernel<true>, dim3(n, n * n), dim3(256), 0, st, P.tab, K, P.Jvv.as<double>(), nullptr,
-                     F.JP.p, s0, f16);
-  hipLaunchKernelGGL(lp_kernel<true>, dim3((unsigned)P.n_chol, n), dim3(256), 0, st, P.tab, K, P.Lov.as<double>(),
-                     F.LP.p, s0, f16);
+  fill_jp_lp<true>(P, F, nullptr, s0, f16, st);
   hipLaunchKernelGGL(u_kernel<true>, dim3((unsigned)cdiv(P.n_chol, 32), (unsigned)cdiv(nv, 32), n), dim3(256), 0, st,
                      nullptr, P.Lov.as<double>(), nv, P.n_chol, (int64_t)nv, (int64_t)n * nv, F.LovT.p, Z.ldu, s0, f16);
   hipLaunchKernelGGL(split_matrix_kernel, dim3(gsz(P.n_pairs * Z.ldw / 8)), dim3(256), 0, st, Z.holeP.as<double>(),
@@ -994,8 +1119,9 @@ void panels_programs(tci_plan& P, bool split, int mode, int ks, int order, hipSt
           sg.push_back(c);
         }
     };
-    two(nseg(CRi, li, Jij, li, li, es, D, nullptr), nseg(Jij, li, CCi, li, li, es, nullptr, D));
-    two(nseg(Jji, lj, CRj, lj, lj, es, nullptr, D), nseg(CCj, lj, Jji, lj, lj, es, D, nullptr));
+    const int32_t* DJ = Z.wide ? D : nullptr;  // rows of JP: all virtuals, or the walk's own
+    two(nseg(CRi, li, Jij, li, li, es, D, DJ), nseg(Jij, li, CCi, li, li, es, DJ, D));
+    two(nseg(Jji, lj, CRj, lj, lj, es, DJ, D), nseg(CCj, lj, Jji, lj, lj, es, D, DJ));
     sg.push_back(nseg(Ui, Z.ldu, Lj, Z.ldu, Z.ldu, es, D, D));
     sg.push_back(nseg(Li, Z.ldu, Uj, Z.ldu, Z.ldu, es, D, D));
     const double* Oij = Z.O3T.as<double>() + ((int64_t)i * n + j) * nv * Z.nk;
@@ -1075,7 +1201,7 @@ void panels_tune(tci_plan& P, int precision, hipStream_t st) {
     const int64_t c = cdiv(P.h_dom_off[Q + 1] - P.h_dom_off[Q], 128);
     tiles128 += (double)(c * c);
   }
-  std::string log = std::string(split ? "split" : "fp64") + " pair panels: W";
+  std::string log = std::string(split ? "split" : "fp64") + (Z.wide ? " wide pair panels: W" : " pair panels: W");
   double best = 1e300;
   int bw = N128;
   std::vector<int> wshapes = {N128, N192, N64};

@@ -432,7 +432,9 @@ void tci_plan::build(const tci_problem& p) {
     const double* b = X + h_cd_off[Q];
     return transposed ? op(b, 1, d, rm, cm) : op(b, d, 1, rm, cm);
   };
-  pp.on = panels_choose(*this);
+  const int layout = panels_choose(*this);
+  pp.on = layout > 0;
+  pp.wide = layout == 2;
   ring.clear();
   ring.tile = 128;
   for (int P = 0; P < n_pairs; ++P) {

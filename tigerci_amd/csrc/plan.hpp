@@ -49,6 +49,7 @@ struct tci_plan {
   // pair terms as per-walk products over packed panels (pair_panels.hip)
   struct PairPanels {
     bool on = false, split = false;           // split: split builds run them in split precision
+    bool wide = false;                        // columns over all (k, virtual): see panels_choose
     std::vector<int32_t> h_koff;
     std::vector<int64_t> h_ld, h_poff, h_jpoff, h_lpoff;
     tci::DevBuf koff, ld, poff, jpoff, lpoff, pairid, colm;
@@ -320,7 +321,7 @@ void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool scatter, bool ga
 double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log);
 int64_t vv_device_bytes(const tci_plan& P);
 // pair terms over packed panels (pair_panels.hip)
-bool panels_choose(const tci_plan& P);
+int panels_choose(const tci_plan& P);
 void panels_build(tci_plan& P, const std::vector<double>& o4, hipStream_t st);
 void panels_build_split(tci_plan& P, hipStream_t st);
 bool panels_hold_fock(const tci_plan& P, int precision);
