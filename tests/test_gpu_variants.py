@@ -111,3 +111,38 @@ def test_fused_fp64_ladder(args):
     b = _gpu_sigma(tci.Plan.from_problem(prob), x)
     _say(f"  fused rel err {_rel(a, ref):.2e}  two-phase {_rel(b, ref):.2e}")
     assert _rel(a, ref) < TOL and _rel(b, ref) < TOL
+
+
+@pytest.mark.parametrize("prepack", ["1", "0"])
+@pytest.mark.parametrize("storage", ["f64", "f32"])
+@pytest.mark.parametrize("n_v", [61, 62])
+def test_full_domains_share_one_block(n_v, storage, prepack):
+    """Cholesky-direct FP64 ladder with full domains next to smaller ones, odd
+    and even n_v, both storages of L^J, packed once per plan and per chunk: the
+    oracle's sigma; and the full-domain walks hold at most one packed copy of
+    L^J between them."""
+    _say("case: full domains sharing L^J", n_v, storage, "prepack", prepack)
+    args = dict(n_int=5, n_v=n_v, n_chol=150)
+    p64, p32 = _fp32_records(make_problem(seed=21, domain_range=(n_v - 1, n_v), **args))
+    d = np.diff(p64.dom_off)
+    assert (d == n_v).sum() >= 3 and (d < n_v).sum() >= 3
+    x = random_ci_vector(p64, 41)
+    old = {k: os.environ.get(k) for k in ("TCI_LADDER_VV", "TCI_FP64_PREPACK")}
+    os.environ.update(TCI_LADDER_VV="0", TCI_FP64_PREPACK=prepack)
+    try:
+        plan = tci.Plan.from_problem(p32, ladder_dtype=storage)
+        _, full32 = _fp32_records(make_problem(seed=22, **args))
+        one = args["n_chol"] * n_v * (n_v + 1) * 8
+        size = {s: tci.Plan.from_problem(full32, ladder_dtype=s).info.device_bytes for s in ("f32", "f64")}
+        even = tci.Plan.from_problem(make_problem(args["n_int"], 62, args["n_chol"], 22)).info.device_bytes
+    finally:
+        for k, v in old.items():
+            if v is None:
+                os.environ.pop(k, None)
+            else:
+                os.environ[k] = v
+    err = _rel(_gpu_sigma(plan, x), oracle_sigma(p64, x, Integrals(p64)))
+    _say(f"  rel err {err:.2e}; bytes {size}, even {even}, one copy {one}")
+    assert err < TOL
+    # the even FP64 plan packs nothing: two copies leave room for the odd n_v's padded one
+    assert max(size.values()) - even < 2 * one

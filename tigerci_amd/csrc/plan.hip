@@ -771,8 +771,8 @@ void tci_plan::run_Y(int precision, hipStream_t st, bool expanded) {
 
 // Two-phase ladder tables (FP64, on the NT GEMM).  Per chunk of Lc Cholesky
 // vectors starting at J0, dp = d rounded up to even (16-byte rows):
-//   pack    Lp_P[jj] = L^{J0+jj}[D_P, D_P], rows of dp (full-domain walks of an
-//           even n_v read an FP64 L^J itself)
+//   pack    Lp_P[jj] = L^{J0+jj}[D_P, D_P], rows of dp (full-domain walks read an
+//           FP64 L^J of even rows itself, or else share one block)
 //   phase 1 T'_P[(jj,a)][c] = sum_k Lp_P[jj][a][k] C_P[c][k]
 //   phase 2 R_P[n][a]      += sum_jj sum_c Lp_P[jj][n][c] T'_P[jj][a][c]
 //           (one repeated K-range over the jj of a K-split, split into partial
@@ -784,18 +784,28 @@ void tci_plan::build_two_phase_ladder(hipStream_t st) {
   lchunks.clear();
   auto dsz = [&](int P) { return h_dom_off[P + 1] - h_dom_off[P]; };
   auto even = [](int64_t d) { return (d + 1) & ~(int64_t)1; };
-  const bool direct = !lvv_f32 && n_v % 2 == 0;  // full domains read L^J
+  // full domains read L^J itself (or its copy with even rows); where there is no
+  // FP64 L^J of even rows they share one packed block
+  const DevBuf* fullL = lvv_f32 ? nullptr : n_v % 2 == 0 ? &Lvv : LvvP.p ? &LvvP : nullptr;
   int64_t sum_local = 0, sum_dp = 0;
   std::vector<int32_t> loc;
+  std::vector<int> slot(n_pairs, -1);  // packed block of each walk, -1: fullL
+  int full_slot = -1;
   std::vector<int64_t> cpo(n_pairs + 1, 0);
   for (int P = 0; P < n_pairs; ++P) {
     const int64_t e = dsz(P) * even(dsz(P));
     cpo[P + 1] = cpo[P] + e;
     sum_dp += e;
-    if (dsz(P) != n_v || !direct) {
-      loc.push_back(P);
-      sum_local += e;
+    const bool full = dsz(P) == n_v;
+    if (full && fullL) continue;
+    if (full && full_slot >= 0) {
+      slot[P] = full_slot;
+      continue;
     }
+    slot[P] = (int)loc.size();
+    if (full) full_slot = slot[P];
+    loc.push_back(P);
+    sum_local += e;
   }
   n_local = (int)loc.size();
   upload(pairs_local, loc, st);
@@ -863,7 +873,6 @@ void tci_plan::build_two_phase_ladder(hipStream_t st) {
     rpart_n = nsp_max;
     if (rpart_n > 1 && Rpart.bytes < (size_t)rpart_n * sum_d2 * 8) Rpart.alloc((size_t)rpart_n * sum_d2 * 8);
     lphase.clear();
-    const int64_t nv2 = (int64_t)n_v * n_v;
     for (int64_t len : lens) {
       lphase.emplace_back();
       LadderPhase& ph = lphase.back();
@@ -875,21 +884,19 @@ void tci_plan::build_two_phase_ladder(hipStream_t st) {
       ph.n1.resize(3);
       ph.n2.resize(3);
       for (int v = 0; v < 3; ++v) ph.n1[v].shape = ph.n2[v].shape = v;  // N128, N192, N64
-      int qloc = 0;
       for (int P = 0; P < n_pairs; ++P) {
         const int64_t d = dsz(P), dp = even(d);
         double* T = Tbuf.as<double>() + Lc * cpo[P];
         const double* Lb;
         int64_t ld = dp, jstep = d * dp, jstride = 0;  // rows, one jj to the next, one J0 to the next
-        if (d == n_v && direct) {
-          Lb = Lvv.as<double>();
-          ld = n_v;
-          jstep = jstride = nv2;
+        if (slot[P] < 0) {  // rows of dp = n_v rounded up to even
+          Lb = fullL->as<double>();
+          jstride = jstep;
         } else if (lp_all) {
-          Lb = Lp.as<double>() + lpo_all[qloc++];
+          Lb = Lp.as<double>() + lpo_all[slot[P]];
           jstride = jstep;
         } else {
-          Lb = Lp.as<double>() + lpo[qloc++];
+          Lb = Lp.as<double>() + lpo[slot[P]];
         }
         NSeg s1 = nseg(Lb, ld, Cw.as<double>() + cpo[P], dp, dp, 8);
         s1.ja = jstride * 8;
