@@ -138,10 +138,11 @@ def test_dense_pair_path_matches_gather_path():
 
 @pytest.mark.parametrize("env", [{}, {"TCI_LADDER_MERGED": "0"}, {"TCI_LADDER_MERGED": "0", "TCI_DENSE_PAIRS": "0"}])
 def test_full_domain_variants(env):
-    """Full domains run the ladder as single products over all walks; the
-    per-walk programs (TCI_LADDER_MERGED=0) must give the same sigma, in FP64
-    and bf16x3, including a domain size that is not a multiple of 4 or 8."""
+    """Full domains run the Cholesky-direct split ladder as single products
+    over all walks; the per-walk programs (TCI_LADDER_MERGED=0) must give the
+    same sigma, including a domain size that is not a multiple of 4 or 8."""
     _say("case: full-domain variants", env)
+    env = {"TCI_LADDER_VV": "0", **env}
     for args in [dict(n_int=4, n_v=37, n_chol=30, seed=31), dict(n_int=3, n_v=64, n_chol=20, seed=32)]:
         prob = make_problem(**args)
         ints = Integrals(prob)
@@ -150,11 +151,11 @@ def test_full_domain_variants(env):
         os.environ.update(env)
         try:
             plan = tci.Plan.from_problem(prob)
+            assert _rel(_gpu_sigma(plan, x), ref) < TOL
+            assert _rel(_gpu_sigma(plan, x, precision="bf16x3"), ref) < 5e-5
         finally:
             for k in env:
                 del os.environ[k]
-        assert _rel(_gpu_sigma(plan, x), ref) < TOL
-        assert _rel(_gpu_sigma(plan, x, precision="bf16x3"), ref) < 5e-5
 
 
 @pytest.mark.parametrize("dense", ["0", "1"])
@@ -177,22 +178,17 @@ def test_local_domain_pair_paths(dense):
         assert _rel(_gpu_sigma(plan, x, precision="bf16x3"), ref) < 5e-5
 
 
-@pytest.mark.parametrize("z", ["0", "1"])
-def test_dense_pair_z_forms(z):
-    """Z = C~R Kov - CR Jbig + Yt Lov of the dense pair products directly
-    (TCI_Z_LOWRANK=0) and as U Lov - CR Jbig with U = Yt + C~R Lov^T (=1, the
-    default; FP64 and bf16x3, fp16x3 keeps the direct form): both reproduce the
-    oracle with local domains and weak pairs, in every precision."""
-    _say("case: dense pair Z form, TCI_Z_LOWRANK =", z)
+def test_pair_panels_across_precisions():
+    """The panels of one plan through every precision and back, with local
+    domains and weak pairs: each against the oracle."""
+    _say("case: pair panels across precisions")
     prob = make_problem(6, 45, 40, 43, domain_range=(9, 45), weak_below=14)
     ints = Integrals(prob)
     os.environ["TCI_DENSE_PAIRS"] = "1"
-    os.environ["TCI_Z_LOWRANK"] = z
     try:
         plan = tci.Plan.from_problem(prob)
     finally:
         del os.environ["TCI_DENSE_PAIRS"]
-        del os.environ["TCI_Z_LOWRANK"]
     for k in range(2):
         x = random_ci_vector(prob, 64 + k)
         ref = oracle_sigma(prob, x, ints)
@@ -222,30 +218,76 @@ def test_sigma_pair_block_strips(args):
     assert _rel(_gpu_sigma(plan, x, precision="bf16x3"), ref) < 5e-5
 
 
-@pytest.mark.parametrize("waves", ["256", "256w8", "256w16", "128x192d2", "128d2"])
-@pytest.mark.parametrize("precision", ["bf16x3", "fp16x3"])
-def test_split_products_on_256_tiles(precision, waves):
-    """Every split pair product (U, W, Z, Z3, the 4-internal product) on the
-    256 x 256 tiles of the 32 x 32-MFMA kernel (TCI_PAIRS_TILE=256, or 256w8
-    and 256w16 for its eight- and sixteen-wave forms) or on 128 x 192 tiles
-    with two direct-load stages (128x192d2), and the resident ladder's
-    product on them too
-    (TCI_VV_TILE): sigma against the
-    oracle, with outputs that are partial tiles (n_v = 45, 6 internal), W's
-    blocked columns and U's accumulation."""
-    _say("case: split products on 256 tiles", precision)
-    prob = make_problem(6, 45, 40, 47, domain_range=(9, 45), weak_below=14)
+TILES = {"128": "128x128", "192": "192x192", "64": "64x64", "32k4": "32x32,k4", "256": "256x256", "128x192": "128x192"}
+
+
+@pytest.mark.parametrize("schedule", ["128/1", "128/4x", "192/2", "64/8", "64/1x", "32k4/4", "256/4", "256/8x",
+                                      "128x192/5"])
+@pytest.mark.parametrize("args", [
+    dict(n_int=6, n_v=45, n_chol=40, seed=47, domain_range=(9, 45), weak_below=14),
+    dict(n_int=3, n_v=200, n_chol=33, seed=48, domain_range=(60, 200)),
+], ids=["6x45", "3x200"])
+def test_pair_panels_on_every_tile(args, schedule):
+    """W and the pair products on every tile of the NT GEMM, on several K-splits
+    and both workgroup orders (TCI_PANEL_TILE): outputs of less than a tile and
+    of a whole and a ragged one.  Every precision against the oracle; the tile
+    is the one that ran."""
+    _say("case: pair panels on", schedule, args)
+    tile = schedule.split("/")[0]
+    split_only = tile in ("256", "128x192")
+    prob = make_problem(**args)
     ints = Integrals(prob)
-    env = {"TCI_DENSE_PAIRS": "1", "TCI_PAIRS_TILE": waves, "TCI_VV_TILE": waves, "TCI_LADDER_VV": "1",
-           "TCI_AUTOTUNE": "0"}
+    env = {"TCI_DENSE_PAIRS": "1", "TCI_PANEL_TILE": schedule, "TCI_LADDER_VV": "1", "TCI_AUTOTUNE": "0",
+           "TCI_MERGE": "0"}
     os.environ.update(env)
     try:
         plan = tci.Plan.from_problem(prob)
-        for k in range(2):
-            x = random_ci_vector(prob, 66 + k)
-            ref = oracle_sigma(prob, x, ints)
-            assert _rel(_gpu_sigma(plan, x, precision=precision), ref) < (5e-5 if precision == "bf16x3" else 2e-6)
-        assert "-> resident" in plan.tuning()
+        plan.profile(True)
+        for precision, tol in (("bf16x3", 5e-5), ("fp16x3", 2e-6)) if split_only else \
+                (("fp64", TOL), ("bf16x3", 5e-5), ("fp16x3", 2e-6)):
+            x = random_ci_vector(prob, 66)
+            err = _rel(_gpu_sigma(plan, x, precision=precision), oracle_sigma(prob, x, ints))
+            names = [k["name"] for k in plan.profile_kernels(precision) if "pair product" in k["name"]]
+            _say(f"  {precision} rel err {err:.2e} {names}")
+            assert err < tol
+            assert len(names) == 2 and all(TILES[tile] + ">" in n for n in names)
     finally:
         for k in env:
             del os.environ[k]
+
+
+@pytest.mark.parametrize("merge", ["64/1", "64/3", "32k4/1", "32k4/8"])
+@pytest.mark.parametrize("args", [
+    dict(n_int=5, n_v=30, n_chol=40, seed=49),
+    dict(n_int=5, n_v=33, n_chol=41, seed=50, domain_range=(5, 33), weak_below=9, h_offdiag=0.2),
+    dict(n_int=3, n_v=70, n_chol=20, seed=51),
+], ids=["5x30", "5x33", "3x70"])
+def test_merged_launches(args, merge):
+    """S, W and Y as one launch, the pair products and gW as another
+    (TCI_MERGE), against the separate launches (summation order only) and the
+    oracle, even and odd n_v; FP32 L^J keeps the singles products apart."""
+    _say("case: merged launches", merge, args)
+    prob = make_problem(**args)
+    x = random_ci_vector(prob, 67)
+    ref = oracle_sigma(prob, x, Integrals(prob))
+    env = {"TCI_LADDER_VV": "1", "TCI_AUTOTUNE": "0"}
+    os.environ.update(env, TCI_MERGE="0")
+    try:
+        apart = _gpu_sigma(tci.Plan.from_problem(prob), x)
+        os.environ["TCI_MERGE"] = merge
+        plan = tci.Plan.from_problem(prob)
+        f32 = tci.Plan.from_problem(prob, ladder_dtype="f32")
+    finally:
+        for k in [*env, "TCI_MERGE"]:
+            del os.environ[k]
+    plan.profile(True)
+    y = _gpu_sigma(plan, x)
+    names = [k["name"] for k in plan.profile_kernels("fp64")]
+    _say(f"  rel err {_rel(y, ref):.2e}, against separate launches {_rel(y, apart):.2e}")
+    tile = TILES[merge.split("/")[0]] + ">"
+    assert any(n.startswith("fp64 products S, W, Y") and tile in n for n in names)
+    assert any("pair products, gW" in n and tile in n for n in names)
+    assert _rel(y, ref) < TOL and _rel(y, apart) < 1e-12
+    assert np.array_equal(_gpu_sigma(plan, x, graph=True), y)
+    assert _rel(_gpu_sigma(f32, x), ref) < 1e-6  # L^J rounded to FP32
+    assert _rel(_gpu_sigma(plan, x, precision="bf16x3"), ref) < 5e-5  # the separate programs

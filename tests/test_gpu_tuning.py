@@ -92,29 +92,28 @@ def test_phase2_192_tiles():
     assert _rel(b, a) < 1e-5
 
 
-@pytest.mark.parametrize("env", ["TCI_FP64_P192", "TCI_FP64_P1_192"])
-def test_fp64_192_tiles(env):
-    """Both FP64 ladder phases (TCI_FP64_P192), or phase 1 alone
-    (TCI_FP64_P1_192), of domains of 129-192 on 192 x 192 tiles (eight waves
-    per workgroup) reproduce the oracle and the default tiles."""
-    _say("case: FP64 ladder on 192 x 192 tiles", env)
+def test_fp64_192_tiles():
+    """Both FP64 ladder phases of domains of 129-192 run on 192 x 192 tiles
+    (eight waves per workgroup), beside 128 x 128 ones for the others, and
+    reproduce the oracle."""
+    _say("case: FP64 ladder on 192 x 192 tiles")
     prob = make_problem(3, 200, 24, 53, domain_range=(100, 192), weak_below=0)
     ints = Integrals(prob)
-    xs = [random_ci_vector(prob, 11 + k) for k in range(2)]
-    os.environ["TCI_AUTOTUNE"] = "0"
+    os.environ.update(TCI_AUTOTUNE="0", TCI_LADDER_VV="0")
     try:
-        base = tci.Plan.from_problem(prob)
-        os.environ[env] = "1"
-        big = tci.Plan.from_problem(prob)
+        plan = tci.Plan.from_problem(prob)
     finally:
-        os.environ.pop(env, None)
-        del os.environ["TCI_AUTOTUNE"]
-    for x in xs:
-        ref = oracle_sigma(prob, x, ints)
-        a, b = _sigma(base, x), _sigma(big, x)
-        _say(f"  rel err default {_rel(a, ref):.2e}  192-tiles {_rel(b, ref):.2e}")
-        assert _rel(a, ref) < 1e-10 and _rel(b, ref) < 1e-10
-        assert _rel(b, a) < 1e-12
+        del os.environ["TCI_AUTOTUNE"], os.environ["TCI_LADDER_VV"]
+    plan.profile(True)
+    for k in range(2):
+        x = random_ci_vector(prob, 11 + k)
+        err = _rel(_sigma(plan, x), oracle_sigma(prob, x, ints))
+        _say(f"  rel err {err:.2e}")
+        assert err < 1e-10
+    names = [k["name"] for k in plan.profile_kernels("fp64") if "ladder phase" in k["name"]]
+    for phase in "12":
+        for tile in ("128x128", "192x192"):
+            assert any(f"phase {phase}" in n and tile in n for n in names), names
 
 
 @pytest.mark.parametrize("precision", ["bf16x3", "fp16x3"])

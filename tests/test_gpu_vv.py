@@ -128,27 +128,35 @@ def test_vv_davidson_roots():
     assert np.max(np.abs(np.asarray(e2) - np.asarray(e0))) < 1e-6
 
 
-@pytest.mark.parametrize("tile", ["128x192T", "128x192T2", "128x192d2", "128x192d3", "128x128d2"])
-@pytest.mark.parametrize("precision", ["bf16x3", "fp16x3"])
-@pytest.mark.parametrize("args", CASES)
-def test_vv_transposed_split_product(args, precision, tile):
-    """S^T = V X^T (walks along the tiles' N side), one and two K-splits,
-    transposed back before the gather, and the untransposed product with two
-    or three direct-load stages: against the oracle at the split bound, and
-    against the default schedule to FP32 summation order."""
-    _say("case: resident ladder transposed", precision, tile, args)
+@pytest.mark.parametrize("schedule", ["128/1", "128/2x", "192/4", "192/1x", "64/1", "32k4/4x", "256/6", "256/1x",
+                                      "128x192/2"])
+@pytest.mark.parametrize("args", CASES[2:])
+def test_vv_product_on_every_tile(args, schedule):
+    """The product S = X V on every tile of the NT GEMM, on several K-splits
+    (the last one with the 4-internal range behind it) and both workgroup
+    orders (TCI_VV_TILE), without and with the autotuner's route: against the
+    oracle; the tile is the one that ran."""
+    _say("case: resident ladder on", schedule, args)
+    tile, ks = schedule.rstrip("x").split("/")
+    shape = {"32k4": "32x32,k4"}.get(tile, tile if "x" in tile else f"{tile}x{tile}")
     prob = make_problem(**args)
     ints = Integrals(prob)
-    xs = [random_ci_vector(prob, 110 + k) for k in range(2)]
-    with _env(TCI_LADDER_VV=1, TCI_AUTOTUNE=0):
-        ref = [_sigma(tci.Plan.from_problem(prob), x, precision=precision) for x in xs[:1]]
-    with _env(TCI_LADDER_VV=1, TCI_AUTOTUNE=0, TCI_VV_TILE=tile):
-        plan = tci.Plan.from_problem(prob)
-        got = [_sigma(plan, x, precision=precision) for x in xs]
-        assert _rel(got[0], ref[0]) < 1e-6
-        for x, g in zip(xs, got):
-            assert _rel(g, oracle_sigma(prob, x, ints)) < SPLIT_TOL[precision]
-        assert np.array_equal(_sigma(plan, xs[0], precision=precision, graph=True), got[0])
+    x = random_ci_vector(prob, 110)
+    ref = oracle_sigma(prob, x, ints)
+    for autotune in "01":
+        with _env(TCI_LADDER_VV=1, TCI_AUTOTUNE=autotune, TCI_VV_TILE=schedule, TCI_MERGE=0):
+            plan = tci.Plan.from_problem(prob)
+            plan.profile(True)
+            for precision in ("bf16x3", "fp16x3") if tile in ("256", "128x192") else ("fp64", "bf16x3", "fp16x3"):
+                y = _sigma(plan, x, precision=precision)
+                names = [k["name"] for k in plan.profile_kernels(precision) if "(ab|cd) product" in k["name"]]
+                _say(f"  {precision} rel err {_rel(y, ref):.2e} {names}")
+                assert _rel(y, ref) < SPLIT_TOL.get(precision, TOL)
+                assert len(names) == 1 and shape + ">" in names[0]
+                most = min(int(ks), 4 if precision == "fp64" else 8)
+                least = max(most, 4) if precision == "fp16x3" else most
+                assert (f"K-split {least} " in names[0]) if least > 1 else "K-split" not in names[0]
+                assert np.array_equal(_sigma(plan, x, precision=precision, graph=True), y)
 
 
 @pytest.mark.parametrize("autotune", ["0", "1"])

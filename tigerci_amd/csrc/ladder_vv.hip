@@ -390,7 +390,7 @@ void vv_build(tci_plan& P, hipStream_t st) {
   V.Sp.alloc((size_t)kMaxSplits * P.n_pairs * V.np * 8);
   V.Sm.alloc((size_t)kMaxSplits * std::max(V.ncm, 1) * V.nm * 8);
   V.built = true;
-  vv_set_schedule(P, TCI_SIGMA_FP64, N128, 1, st);
+  vv_untuned(P, TCI_SIGMA_FP64, st);
   TCI_HIP(hipStreamSynchronize(st));
 }
 
@@ -407,6 +407,16 @@ void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t 
     V.ksx = ks;
     build_products(P, V.gx, true, shape, ks, st);
   }
+}
+
+// The schedule without timing: 128 x 128 tiles (FP64) or 128 x 192 ones, or
+// what TCI_VV_TILE asks for; returns whether it asks.
+bool vv_untuned(tci_plan& P, int precision, hipStream_t st) {
+  const bool split = precision != TCI_SIGMA_FP64;
+  const NSchedule f = asked_schedule("TCI_VV_TILE", split);
+  vv_set_schedule(P, precision, f.shape >= 0 ? f.shape : split ? N128x192 : N128, f.shape >= 0 ? f.ks : 1, st);
+  (split ? P.vv.gx : P.vv.g64).remap = f.shape >= 0 ? f.order : 0;
+  return f.shape >= 0;
 }
 
 // Split copies of V for a split precision (fp16x3: scaled by a power of two
@@ -441,11 +451,7 @@ void vv_prepare_split(tci_plan& P, int precision, hipStream_t st) {
   launch_fill(static_cast<double*>(V.Xpx.p), (int64_t)(V.Xpx.bytes / 8), 0.0, st);
   launch_fill(static_cast<double*>(V.Xmx.p), (int64_t)(V.Xmx.bytes / 8), 0.0, st);
   V.prec = precision;
-  // untuned schedule: 128 x 192 tiles; TCI_VV_TILE=256.. or 128x128.. for the others
-  const char* te = std::getenv("TCI_VV_TILE");
-  const std::string ts = te ? te : "";
-  const int shape = ts.rfind("256", 0) == 0 ? N256 : ts.rfind("128x128", 0) == 0 || ts.rfind("128d", 0) == 0 ? N128 : N128x192;
-  vv_set_schedule(P, precision, shape, 1, st);
+  vv_untuned(P, precision, st);
   TCI_HIP(hipStreamSynchronize(st));
 }
 
@@ -497,6 +503,10 @@ void vv_ladder(tci_plan& P, int precision, hipStream_t st, bool scatter, bool ga
 double vv_tune(tci_plan& P, int precision, hipStream_t st, std::string& log) {
   tci_plan::VVLadder& V = P.vv;
   const bool split = precision != TCI_SIGMA_FP64;
+  if (vv_untuned(P, precision, st)) {
+    log += " as asked";
+    return time_ms(st, 2, [&] { vv_ladder(P, precision, st, true, !P.pp.on); });
+  }
   std::vector<int> shapes = {N128, N192};
   if (split) shapes = {N128, N128x192, N192, N256};
   // tiles that leave the chip idle at 128 x 128 also try the small ones

@@ -74,6 +74,14 @@ enum NShape {
   N128x192 = 5 // split only: 128 x 192, 4 waves
 };
 
+// A schedule asked for in the environment, "tile/ks" or "tile/ksx" (XCD-contiguous
+// order), tile 128, 192, 64, 32k4 and for split products 256 or 128x192: shape
+// -1 where the variable is unset or names no tile of this element type.
+struct NSchedule {
+  int shape = -1, ks = 1, order = 0;
+};
+NSchedule asked_schedule(const char* env, bool split);
+
 struct NProgram {
   int shape = N128;
   bool split = false;

@@ -803,11 +803,14 @@ void zero(DevBuf& b, size_t bytes, hipStream_t st) {
   launch_fill(b.as<double>(), (int64_t)(b.bytes / 8), 0.0, st);
 }
 
+constexpr int kAsked = 16;  // modes from here on: one tile shape for all
+
 // tile shape of a d x d pair block under a tiling mode: 0 by size (64, 128,
 // 192, in split precision 256; 128-wide tiles above), 1 all 128, 2 all 64, 3 all
 // 32 x 32 in four K-groups.  A block on one tile reads its panels once: at
 // 16/203/811 (fp16x3) 0.76 ms on 256 x 256 tiles, 0.83 on 128 x 128
 int shape_of(int mode, int d, bool split) {
+  if (mode >= kAsked) return mode - kAsked;
   if (mode == 3) return N32K4;
   if (mode == 2 || d <= 64) return N64;
   if (mode == 1 || d <= 128) return N128;
@@ -1174,6 +1177,12 @@ void panels_tune(tci_plan& P, int precision, hipStream_t st) {
     auto fill = [&](int t) { return cdiv(P.n_chol, t) * cdiv(P.n_v, t) * P.n_int; };
     return fill(128) >= 512 ? N128 : fill(64) >= 256 ? N64 : N32K4;
   };
+  const NSchedule asked = asked_schedule("TCI_PANEL_TILE", split);
+  if (asked.shape >= 0) {
+    panels_w_program(P, split, asked.shape, st);
+    panels_programs(P, split, kAsked + asked.shape, std::min(std::max(kmin, asked.ks), kMaxKs), asked.order, st);
+    return;
+  }
   if (!autotune_enabled()) {
     panels_w_program(P, split, wrule(), st);
     panels_programs(P, split, 0, kmin, 0, st);
@@ -1263,7 +1272,12 @@ void panels_merge(tci_plan& P, hipStream_t st) {
   Z.m1on = Z.m2on = false;
   double fl = F.W.alg_flops;
   for (const auto& g : F.pair) fl += g.alg_flops;
-  if (!autotune_enabled() || !P.vv.fp64 || fl + P.vv.g64.alg_flops > 4.0e10) return;
+  // TCI_MERGE=tile/ks merges both groups so (64 or 32k4), =0 neither
+  const NSchedule asked = asked_schedule("TCI_MERGE", false);
+  const bool force = asked.shape == N64 || asked.shape == N32K4;
+  const char* env = std::getenv("TCI_MERGE");
+  if (!P.vv.fp64 || (env && env[0] == '0')) return;
+  if (!force && (!autotune_enabled() || fl + P.vv.g64.alg_flops > 4.0e10)) return;
   const bool sing = P.singles_nt();
   const bool gw = !P.nprogGW.tasks.empty();
   Z.m1_singles = sing;
@@ -1288,9 +1302,14 @@ void panels_merge(tci_plan& P, hipStream_t st) {
     Z.m1.upload_tables(st);
   };
   const int64_t kmin = P.vv.ncm > 0 ? std::min(P.vv.np, P.vv.nm) : P.vv.np;
+  if (force) {
+    best = 0.0;
+    bs = asked.shape;
+    bk = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)asked.ks, 4, kmin / 64}));
+  }
   for (int sh : {(int)N64, (int)N32K4})
     for (int ks : {1, 2, 4}) {
-      if (ks > 1 && ks > kmin / 64) continue;
+      if (force || (ks > 1 && ks > kmin / 64)) continue;
       build1(sh, ks);
       const double ms = time_ms(st, 3, [&] { Z.m1.launch(TCI_SIGMA_FP64, st); });
       log += std::string(sh == N64 ? " 64/" : " 32k4/") + std::to_string(ks) + ":" + fmt_ms(ms);
@@ -1316,6 +1335,11 @@ void panels_merge(tci_plan& P, hipStream_t st) {
   log += "; pairs, gW separate:" + fmt_ms(t0);
   best = t0 * 0.98;
   bs = -1;
+  if (force) {
+    best = 0.0;
+    bs = asked.shape;
+    bk = std::min(asked.ks, kMaxKs);
+  }
   auto build2 = [&](int sh, int ks) {
     Z.m2.clear();
     Z.m2.shape = sh;
@@ -1325,6 +1349,7 @@ void panels_merge(tci_plan& P, hipStream_t st) {
   };
   for (int sh : {(int)N64, (int)N32K4})
     for (int ks : {1, 2, 4, 8}) {
+      if (force) continue;
       build2(sh, ks);
       const double ms = time_ms(st, 3, [&] { Z.m2.launch(TCI_SIGMA_FP64, st); });
       log += std::string(sh == N64 ? " 64/" : " 32k4/") + std::to_string(ks) + ":" + fmt_ms(ms);

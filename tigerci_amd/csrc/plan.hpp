@@ -314,6 +314,7 @@ bool vv_clear_win(const tci_plan& P);
 void vv_build(tci_plan& P, hipStream_t st);
 // shape: an NShape of ngemm.hpp
 void vv_set_schedule(tci_plan& P, int precision, int shape, int ks, hipStream_t st);
+bool vv_untuned(tci_plan& P, int precision, hipStream_t st);
 void vv_prepare_split(tci_plan& P, int precision, hipStream_t st);
 // scatter: write X+- from C; gather: unpack S+- into R (otherwise the caller
 // reads the packed S+-)

@@ -9,7 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 
-#include "common.hpp"
+#include "ngemm.hpp"
 
 namespace tci {
 
@@ -44,6 +44,22 @@ double time_ms(hipStream_t st, int reps, const std::function<void()>& fn) {
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   return (double)ms / reps;
+}
+
+NSchedule asked_schedule(const char* env, bool split) {
+  static const struct {
+    const char* name;
+    int shape;
+  } tiles[] = {{"128x192", N128x192}, {"128", N128}, {"192", N192}, {"256", N256}, {"64", N64}, {"32k4", N32K4}};
+  NSchedule f;
+  const char* e = std::getenv(env);
+  if (!e) return f;
+  const std::string s(e), t = s.substr(0, s.find('/'));
+  for (const auto& x : tiles)
+    if (t == x.name && (split || (x.shape != N256 && x.shape != N128x192))) f.shape = x.shape;
+  if (s.size() > t.size()) f.ks = std::max(1, std::atoi(s.c_str() + t.size() + 1));
+  f.order = !s.empty() && s.back() == 'x' ? 1 : 0;
+  return f;
 }
 
 int tune_order(GemmProgram& g, hipStream_t st, const std::function<void()>& launch) {
