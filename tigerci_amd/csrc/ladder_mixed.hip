@@ -296,7 +296,14 @@ static void mixed_layout(tci_plan& P, int precision, hipStream_t st) {
   }
   // local-domain L^J[D,D] for all J packed once when it fits 64 GB; otherwise
   // packed per chunk of Cholesky vectors inside every sigma
-  M.prepacked = sum_local_x > 0 && 2.0 * (double)sum_local_x * (double)n_chol <= 64.0e9;
+  {
+    // (12 GB left beside them for T' of a chunk and the partials; the copies of
+    // the other split precision are replaced)
+    const double need = 2.0 * (double)sum_local_x * (double)n_chol;
+    size_t freeb = 0, totalb = 0;
+    TCI_HIP(hipMemGetInfo(&freeb, &totalb));
+    M.prepacked = sum_local_x > 0 && need <= 64.0e9 && need + 12.0e9 <= (double)(freeb + M.Lpx.bytes);
+  }
   std::vector<int64_t> lpo_all(loc.size() + 1, 0);
   if (M.prepacked) {
     for (size_t q = 0; q < loc.size(); ++q) {
