@@ -116,8 +116,8 @@ def test_sigma_config1_size():
 
 
 def test_dense_pair_path_matches_gather_path():
-    """Full domains take the dense ordered-pair products for the ring and
-    4-internal terms; TCI_DENSE_PAIRS=0 forces the per-walk gather GEMMs.
+    """Full domains take the pair panels for the ring and 4-internal terms;
+    TCI_DENSE_PAIRS=0 forces the per-walk gather GEMMs.
     Both must agree with the oracle (and so with each other)."""
     _say("case: dense pair products vs gather path")
     prob = make_problem(5, 37, 50, 21)
@@ -161,8 +161,8 @@ def test_full_domain_variants(env):
 @pytest.mark.parametrize("dense", ["0", "1"])
 def test_local_domain_pair_paths(dense):
     """Local domains with weak pairs: the ring, 3-external and 4-internal terms
-    as products over embedded blocks (TCI_DENSE_PAIRS=1) and as per-walk
-    gathered programs (=0) both reproduce the oracle."""
+    as products over packed panels (TCI_DENSE_PAIRS=1) and as per-walk gathered
+    programs (=0) both reproduce the oracle."""
     _say("case: local-domain pair paths, TCI_DENSE_PAIRS =", dense)
     prob = make_problem(6, 45, 40, 41, domain_range=(9, 45), weak_below=14)
     ints = Integrals(prob)

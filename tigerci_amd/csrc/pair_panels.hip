@@ -229,10 +229,10 @@ __global__ __launch_bounds__(256) void xt_kernel(PairTab T, const int32_t* __res
 // (X >= Y) of the packed triangle; each vector element is read once and both
 // orientations leave along rows.  FP64 and bf16x3 (the scales of fp16x3 need
 // max|C| first: unpack_kernel, vv_scatter_kernel and panels_kernel there).
-// Bound by its writes: 116 us (bf16x3) and 157 us (FP64) at 34/192/1200, against
-// 98 + 50 + 100 us for unpack, scatter and panels one after the other.  XT+-
-// in a launch of its own took 5 us at 5/30/175, 11 at 10/100/400 and 95-125 at
-// 34/192/1200; here XTMEASURED.
+// Bound by its writes: 230 us (bf16x3) and 304 us (FP64) at 34/192/1200 (its
+// part without XT+- 116 and 157, against 98 + 50 + 100 us for unpack, scatter
+// and panels one after the other; XT+- in a launch of its own 95-125), FP64 at
+// 10/100/400 15.6 us and at 5/30/175 6.5 us, where XT+- alone took 11 and 5.
 struct ExpandOut {
   double *C, *Ct, *s, *sT;  // C null: not needed
   int nk;
@@ -880,10 +880,10 @@ int panels_choose(const tci_plan& P) {
   return fits((4.0 * n * nv + nc) * ldw, ldw) && (force || f_wide <= 2.5 * f_gather) ? 2 : 0;
 }
 
-// Do the pair terms of a split build run in split precision?  Where the
-// embedded products (6 N^3 + 4 N^2 n_chol, N = n_int n_v) cost at most eight
-// times the per-walk ones, i.e. the domains fill a good part of the virtual
-// space.  Elsewhere (small domains in a wide space) the pair terms are a few
+// Do the pair terms of a split build run in split precision?  Where products
+// over whole pair blocks (6 N^3 + 4 N^2 n_chol flops, N = n_int n_v) cost at most
+// eight times the per-walk ones, i.e. the domains fill a good part of the
+// virtual space.  Elsewhere (small domains in a wide space) the pair terms are a few
 // percent of the ladder's work: they stay FP64, and the split error is the
 // ladder's alone.
 bool panels_split_rule(const tci_plan& P) {

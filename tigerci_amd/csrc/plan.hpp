@@ -105,8 +105,8 @@ struct tci_plan {
     int n_local = 0;
     bool prepacked = false;         // Lpx holds every J (packed once per plan)
     int prec = -1;                  // split precision the copies are made for
-    // scales (fp16x3; all 1 for bf16x3): [0] constants (L, Kov, Jbig, Lov,
-    // the 4-internal coefficients),
+    // scales (fp16x3; all 1 for bf16x3): [0] constants (L, J, Lov, the
+    // 4-internal coefficients),
     // [1] C of the ladder, [2] ladder intermediate, [3] phase-1 output,
     // [4] phase-2 output, [5] pair-product output, [6] C and U of the pair
     // products, [8] max of the constants, [9] and [10] V and the output of the
